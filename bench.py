@@ -617,9 +617,9 @@ def secondary_record(workload, steps, warmup, single_stream=False, with_cpu_base
     extra = {}
     total_us = lambda name: stats[name]["launches"] * stats[name]["avg_us"] if name in stats else 0.0
     if kernel == "gemm_f32" and total_us("gemm_f32_as_bf16x6") > total_us(kernel):
-        # the large fp32 products run as six bf16 MFMA products of split operands: that launch (operand split,
-        # bf16 GEMM over the six-fold reduction, and the sum of partial products where the output is narrow) is
-        # the dominant one, measured against the bf16 MFMA peak with the flop it executes (6 x 2 M N K)
+        # the large fp32 products run as six bf16 MFMA products of operands that are split inside the kernel: that
+        # launch (with the sum of partial products where the output is narrow) is the dominant one, measured
+        # against the bf16 MFMA peak with the flop it executes (6 x 2 M N K)
         kernel, peak = "gemm_f32_as_bf16x6", 2500.0
         k = dict(stats[kernel])
         extra = {"f32_equivalent": k["TFLOP/s"],
@@ -655,14 +655,13 @@ def secondary_record(workload, steps, warmup, single_stream=False, with_cpu_base
     if with_kernels:
         out["kernels"] = stats
     if workload in ("gnmt", "gnmt_criterion") and "gemm_f32_as_bf16x6" in stats:
-        # Products of at least 2^32 multiply-adds with wide outputs (the LSTM input projections, the classifier's
-        # forward and weight-gradient products) run as six bf16 MFMA products of three-way split fp32 operands
-        # with fp32 accumulation (ops.set_gemm_f32_algorithm): closer to the fp64 product than the fp32 MFMA
-        # kernel, and faster.  The same steps with every product on the fp32 MFMA kernels, for comparison:
+        # The large fp32 products (the LSTM projections, their gradients, the classifier) run as six bf16 MFMA
+        # products of three-way split fp32 operands with fp32 accumulation (ops.set_gemm_f32_algorithm): closer to
+        # the fp64 product than the fp32 MFMA kernel, and faster.  The same steps with every product on the fp32
+        # MFMA kernels, for comparison:
         from pipedream_amd import ops
-        out["config"]["workload"] += ("; fp32 products of at least 2^32 multiply-adds with at least 192 output tiles of "
-                                      "256 x 256 computed as six bf16 MFMA products of three-way split operands, "
-                                      "fp32 accumulation")
+        out["config"]["workload"] += ("; large fp32 products computed as six bf16 MFMA products of three-way split "
+                                      "operands, fp32 accumulation")
         out["dtype"] = "f32 (large products: 3 x bf16 split operands, f32 accumulation)"
         ops.set_gemm_f32_algorithm("mfma_f32")
         try:

@@ -369,6 +369,16 @@ int pd_gemm_bf16(int trans_a, int trans_b, int M, int N, int K,
  * not thread-safe against concurrent GEMM calls.  No counterpart in the reference (its GEMMs are library calls). */
 int pd_gemm_bf16_set_tile(int bm, int bn);
 
+/* The product of pd_gemm_f32 (same operands and layout flags, no ReLU) on the bf16 matrix pipes: the operands are
+ * split into three bf16 terms each as they enter the kernel, six bf16 MFMAs stand for one fp32 MFMA, accumulation is
+ * fp32.  At least as close to the exact product as the fp32 MFMA kernel, infinities and NaNs included.  
+ * splits > 1: the reduction is cut into that many ranges, whose partial products go to partials[splits][M][N]
+ * (16-byte aligned, N and ldc multiples of 4) and are added in index order.
+ * An operand whose rows hold the reduction index (A not transposed, B transposed) must be 16-byte aligned with K and
+ * its leading dimension multiples of 4. */
+int pd_gemm_f32x6(int trans_a, int trans_b, int M, int N, int K, const float* A, int lda, const float* B, int ldb,
+                  float beta, float* C, int ldc, const float* bias, int splits, float* partials, void* stream);
+
 /* Operand preparation for an fp32 product computed on the bf16 matrix pipes (no counterpart in the reference,
  * whose fp32 products are library calls).  x[rows][ld] (cols used) is written as six bf16 slots of three terms
  * x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2) (x = x1 + x2 + x3 exactly): slots 1 3 2 2 1 1 for the

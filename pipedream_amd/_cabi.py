@@ -69,6 +69,7 @@ SIGNATURES = {
                            True),
     "pd_gemm_f32": (_i, [_i, _i, _i, _i, _i, _vp, _i, _vp, _i, _f, _vp, _i, _vp, _i, _vp], True),
     "pd_gemm_splitk_f32": (_i, [_i, _i, _i, _i, _i, _vp, _i, _vp, _i, _vp, _i, _vp], True),
+    "pd_gemm_f32x6": (_i, [_i, _i, _i, _i, _i, _vp, _i, _vp, _i, _f, _vp, _i, _vp, _i, _vp, _vp], True),
     "pd_splitk_reduce_f32": (_i, [_vp, _i, _i, _i, _vp, _i, _f, _vp, _i, _vp], True),
     "pd_colsum_f32": (_i, [_vp, _vp, _u64, _i, _u64, _i, _f, _vp], True),
     "pd_relu_fwd_f32": (_i, [_vp, _vp, _u64, _vp], True),

@@ -6,6 +6,7 @@ never launched on operands it was not written for), allocates the output with to
 torch's current stream.
 """
 import ctypes
+import functools
 
 import torch
 
@@ -81,6 +82,13 @@ def gemm(a, b, trans_a=False, trans_b=False, bias=None, relu=False, out=None, be
     lda = a.stride(0) if a.size(0) > 1 else a.size(1)
     ldb = b.stride(0) if b.size(0) > 1 else b.size(1)
     ldc = out.stride(0) if out.size(0) > 1 else out.size(1)
+    if _use_x6(M, N, K, trans_a, trans_b, relu, a, b, out, lda, ldb, ldc):
+        splits = _x6_splits(M, N, K, out.data_ptr() % 16 == 0 and ldc % 4 == 0)
+        part = torch.empty((splits, M, N), dtype=torch.float32, device=a.device) if splits > 1 else None
+        with _timed("gemm_f32_as_bf16x6", 2.0 * M * N * K):
+            _cabi.lib().pd_gemm_f32x6(int(trans_a), int(trans_b), M, N, K, _ptr(a), lda, _ptr(b), ldb, float(beta),
+                                      _ptr(out), ldc, _ptr(bias), splits, _ptr(part), _cabi.stream_ptr())
+        return out
     if _use_split_bf16(M, N, K, trans_a, trans_b, relu, a, b, out):
         return _gemm_split_bf16(a, b, trans_a, trans_b, M, N, K, bias, out, beta)
     splits = splitk_factor(M, N, K, trans_a)
@@ -119,22 +127,74 @@ def gemm(a, b, trans_a=False, trans_b=False, bias=None, relu=False, out=None, be
     return out
 
 
-# Large fp32 products on the bf16 matrix pipes: "auto" (products of at least SPLIT_BF16_MIN_WORK multiply-adds
-# whose shape the bf16 kernel takes), "never" (always the fp32 MFMA kernels), "always" (whenever the shape allows).
+# fp32 products on the bf16 matrix pipes: "auto" (where they are faster), "never" (always the fp32 MFMA kernels),
+# "always" (whenever the operands allow).
 _GEMM_F32_ALGO = "auto"
 SPLIT_BF16_MIN_WORK = 1 << 32
 
 
 def set_gemm_f32_algorithm(mode):
-    """How ``gemm`` computes large fp32 products.  "mfma_f32": the fp32 MFMA kernels.  "split_bf16": each operand
-    as the exact sum of three bf16 terms, six bf16 MFMA products per term pair, fp32 accumulation
-    (pd_split3_bf16_f32 + pd_gemm_bf16 over a six-fold reduction) -- 1.5 to 1.7 times as fast on the LSTM
-    projections and the classifier, and closer to the fp64 product than the fp32 MFMA kernel (fewer roundings of the
-    running sum).  "auto" (default): split_bf16 for products of at least 2^32 multiply-adds, else mfma_f32."""
+    """How ``gemm`` computes fp32 products.  "mfma_f32": the fp32 MFMA kernels.  "split_bf16": each operand as the exact
+    sum of three bf16 terms, six bf16 MFMA products per term pair, fp32 accumulation (pd_gemm_f32x6) -- 1.3 to 1.8 times
+    as fast on the LSTM projections and the classifier, and closer to the fp64 product than the fp32 MFMA kernel
+    (fewer roundings of the running sum).  "auto" (default): split_bf16 where it is faster."""
     global _GEMM_F32_ALGO
     _GEMM_F32_ALGO = {"auto": "auto", "mfma_f32": "never", "split_bf16": "always"}[mode]
 
 
+def _use_x6(M, N, K, trans_a, trans_b, relu, a, b, out, lda, ldb, ldc):
+    """Whether ``gemm`` takes pd_gemm_f32x6.  Measured over 90 shapes of 2^17 to 2^34 multiply-adds: its blocks own
+    at least 128 x 128 and start with two round trips to memory (about 10 us for the shallowest product, 5 us for the
+    fp32 kernel's 64 x 64 tiles), so it needs depth (from 2^26 multiply-adds with k >= 256 and both sides of a tile
+    filled: 1.3 to 1.7 times as fast, 2^27.7 652 x 940 x 368 32 -> 20 us) or size (from 2^28.5: 1.04 to 2.7 times;
+    below it with k < 256 0.6 to 1.2).  At most 128 rows of an untransposed A are the streaming kernel's."""
+    if _GEMM_F32_ALGO == "never" or relu:
+        return False
+    if _GEMM_F32_ALGO == "auto":
+        work = M * N * K
+        if not trans_a and M <= 128:
+            return False
+        if work < X6_MIN_WORK and not (work >= 1 << 26 and K >= 256 and M >= 128 and N >= 128):
+            return False
+    if lda >= 1 << 20 or ldb >= 1 << 20:              # 32-bit byte offsets within a tile
+        return False
+    # an operand whose rows hold the reduction index is fetched 16 bytes at a time
+    if not trans_a and (K % 4 or lda % 4 or a.data_ptr() % 16):
+        return False
+    return not trans_b or (K % 4 == 0 and ldb % 4 == 0 and b.data_ptr() % 16 == 0)
+
+
+X6_MIN_WORK = 380 << 20      # 2^28.57 multiply-adds
+
+
+@functools.lru_cache(maxsize=1024)
+def _x6_splits(M, N, K, may_split):
+    """Number of k ranges of a pd_gemm_f32x6 product.  Cost in us, fitted to thirty measured (shape, split) pairs of the
+    LSTM and classifier products, most within 8 %: rounds of 512 work items (two blocks per CU) at 0.77 TFLOP/s a CU; a
+    last round of at most 256 items, one per CU, runs at 0.9 (at 0.7 where it is the only one), a fuller one at 0.85.
+    Partial products are written once and read once by the reduction, at about 5 TB/s."""
+    best, best_cost = 1, None
+    tiles = -(-M // 128) * -(-N // 128)
+    for splits in (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16):
+        if splits > 1 and (not may_split or N % 4 or K // splits < SPLITK_MIN_K):
+            break
+        item = 2.0 * 128 * 128 * (-(-K // splits)) / 1e6
+        rounds, rest = divmod(tiles * splits, 512)
+        cost = rounds * 2 * item / 0.77
+        if rest > 256:
+            cost += 2 * item / 0.85
+        elif rest > 0:
+            cost += item / (0.9 if rounds else 0.7)
+        if splits > 1:
+            cost += 3 + (splits + 1) * M * N * 4 / 5e6
+        if best_cost is None or cost < best_cost:
+            best, best_cost = splits, cost
+    return best
+
+
+# The same arithmetic through memory: six bf16 slots of each operand written by pd_split3_bf16_f32 and multiplied by
+# the bf16 GEMM over a six-fold reduction.  Slower than pd_gemm_f32x6 everywhere; for operands whose leading dimension
+# is beyond that kernel's offsets.
 def _split_bf16_parts(M, N, K):
     """Number of ranges the six-fold reduction is cut into (partial products, one batch entry each, added by
     pd_splitk_reduce_f32) so that the bf16 kernel's 256 x 256 tiles fill the chip: 1 for at least 192 tiles, else

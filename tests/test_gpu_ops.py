@@ -11,7 +11,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from pipedream_amd import layers, ops
+from pipedream_amd import _cabi, layers, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -391,3 +391,41 @@ def test_three_way_bf16_split_is_exact_and_keeps_special_values():
         assert torch.isinf(t[0][0, 0]) and torch.isinf(t[0][0, 1]) and torch.isnan(t[0][0, 2])
         assert float(t[1][0, :3].abs().sum()) == 0.0 and float(t[2][0, :3].abs().sum()) == 0.0
         assert torch.isfinite(t[0][0, 3]) and torch.isfinite(t[0][0, 4])
+
+
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(128, 256, 64),      # whole tiles, whole pairs of chunks
+                                   (129, 260, 100),     # one row and four columns more: blocks with a single row
+                                   (1, 4, 4), (257, 36, 20), (640, 516, 1004), (300, 1000, 16),
+                                   (2944, 2820, 48)])   # 529 work items: more than the resident blocks
+def test_gemm_f32x6_tiles_remainders_and_splits(ta, tb, M, N, K):
+    """pd_gemm_f32x6 at the edges of its tiles and of its chunks of 16 k, unsplit and with k ranges that leave a short
+    last one, against fp64.  Every product of two terms is exact, so what remains is the three products left out
+    (2^-24 of a term each) and one rounding of the running sum per 16 k: rel-L2 well below 4e-7."""
+    g = torch.Generator().manual_seed(31)
+    a = torch.randn((K, M) if ta else (M, K), generator=g).cuda()
+    b = torch.randn((N, K) if tb else (K, N), generator=g).cuda()
+    bias, prior = torch.randn(N, generator=g).cuda(), torch.randn(M, N, generator=g).cuda()
+    want = (a.double().t() if ta else a.double()) @ (b.double().t() if tb else b.double()) + bias.double() + 0.5 * prior.double()
+    for splits in (1, 3):
+        out = prior.clone()
+        part = torch.full((splits, M, N), float("nan")).cuda()
+        _cabi.lib().pd_gemm_f32x6(int(ta), int(tb), M, N, K, ops._ptr(a), a.stride(0), ops._ptr(b), b.stride(0), 0.5,
+                                  ops._ptr(out), N, ops._ptr(bias), splits, ops._ptr(part), _cabi.stream_ptr())
+        assert float((out.double() - want).norm() / want.norm()) < 4e-7
+
+
+def test_gemm_f32x6_infinities_nans_and_values_that_round_to_infinity():
+    """A NaN, an infinity and a value above the largest bf16 give what the fp32 MFMA kernel gives."""
+    g = torch.Generator().manual_seed(32)
+    a, b = torch.randn(256, 64, generator=g), torch.randn(384, 64, generator=g)
+    a[3, 5], a[100, 1], b[7, 7] = float("inf"), float("nan"), 3.4e38
+    a, b, outs = a.cuda(), b.cuda(), {}
+    for mode in ("mfma_f32", "split_bf16"):
+        ops.set_gemm_f32_algorithm(mode)
+        try:
+            outs[mode] = ops.gemm(a, b, trans_b=True)
+        finally:
+            ops.set_gemm_f32_algorithm("auto")
+    assert bool(torch.isinf(outs["mfma_f32"]).any()) and bool(torch.isnan(outs["mfma_f32"]).any())
+    torch.testing.assert_close(outs["split_bf16"], outs["mfma_f32"], rtol=1e-5, atol=1e-4, equal_nan=True)
