@@ -193,7 +193,8 @@ def stream_ptr(stream=None):
     """hipStream_t of a torch stream (default: the current one) as a void*."""
     import torch
     if stream is None:
-        stream = torch.cuda.current_stream()
+        # (torch.cuda.current_stream() builds a Stream object around this number: 3 us of a 12 us call, measured)
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
     return ctypes.c_void_p(stream.cuda_stream)
 
 

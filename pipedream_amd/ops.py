@@ -5,6 +5,7 @@ never launched on operands it was not written for), allocates the output with to
 (device memory and streams are the only things torch provides here) and launches on
 torch's current stream.
 """
+import contextlib
 import ctypes
 import functools
 
@@ -20,7 +21,7 @@ _vp = ctypes.c_void_p
 kernel_timer = None
 
 
-class _timed(object):
+class _Timing(object):
     __slots__ = ("name", "work", "start")
 
     def __init__(self, name, work):
@@ -28,20 +29,25 @@ class _timed(object):
         self.work = work
 
     def __enter__(self):
-        if kernel_timer is not None:
-            self.start = torch.cuda.Event(enable_timing=True)
-            self.start.record()
+        self.start = torch.cuda.Event(enable_timing=True)
+        self.start.record()
 
     def __exit__(self, *exc):
-        if kernel_timer is not None:
-            end = torch.cuda.Event(enable_timing=True)
-            end.record()
-            kernel_timer.setdefault(self.name, []).append((self.start, end, self.work))
+        end = torch.cuda.Event(enable_timing=True)
+        end.record()
+        kernel_timer.setdefault(self.name, []).append((self.start, end, self.work))
         return False
 
 
+_UNTIMED = contextlib.nullcontext()
+
+
+def _timed(name, work):
+    return _UNTIMED if kernel_timer is None else _Timing(name, work)
+
+
 def _ptr(t):
-    return _vp(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _check(t, name, dtype=torch.float32):
