@@ -469,13 +469,13 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int DK = 32;   // k per ring stage
 constexpr int NS = 4;    // ring stages
 
-// One operand's part of the ring (4 waves): where each lane fetches from and where the
-// fragments are read.
-template <int ROWS, bool KC>
+// One operand's part of the ring: where each lane fetches from and where the fragments are read.  NW waves fill it
+// together (4), or one fills and reads a ring of its own (1).
+template <int ROWS, bool KC, int NW = 4>
 struct DmaTile {
     static constexpr int BYTES = ROWS * DK * 2;     // one stage
-    static constexpr int PER_WAVE = ROWS / 64;      // 1 KB transfers per wave and chunk
-    static_assert(ROWS % 64 == 0 && NS * BYTES + 16 * ROWS * 2 + 4 * ROWS * 2 <= 65536 + BYTES,
+    static constexpr int PER_WAVE = ROWS / (16 * NW);      // 1 KB transfers per wave and chunk
+    static_assert(ROWS % (16 * NW) == 0 && NS * BYTES + 16 * ROWS * 2 + 4 * ROWS * 2 <= 65536 + BYTES,
                   "stage offsets must fit the 16-bit LDS instruction offset");
 
     uint32_t off[PER_WAVE];   // byte offset of this lane's 16 bytes from the tile origin, chunk 0
@@ -483,7 +483,7 @@ struct DmaTile {
     __device__ __forceinline__ void init(int ld, int row0, int rows, int wave, int lane) {
 #pragma unroll
         for (int t = 0; t < PER_WAVE; ++t) {
-            const int n = wave + 4 * t;
+            const int n = wave + NW * t;
             if (KC) {
                 const int row = n * 16 + lane / 4;
                 const int kq = (lane % 4) ^ ((row >> 2) & 3);
@@ -491,12 +491,16 @@ struct DmaTile {
             } else {
                 const int e = n * 512 + lane * 8;
                 const int k = e / ROWS, c = (e % ROWS) / 8;
-                int col = ((((c / 4) ^ (k % 4)) * 4) + c % 4) * 8;
+                int col = ((((c / 4) ^ granule_xor(k)) * 4) + c % 4) * 8;
                 if (row0 + col >= rows) col = 0;
                 off[t] = (uint32_t)(k * ld + col) * 2u;
             }
         }
     }
+    // what the 64-byte granule index of row k is XORed with, so that the four k-rows of a transposing read start in
+    // different banks (256 bytes of them): a row of 128 or more elements always starts in the same bank, of 64 every
+    // second row does, of 32 every fourth
+    __device__ __forceinline__ static int granule_xor(int k) { return ROWS >= 128 ? k % 4 : ROWS == 64 ? (k >> 1) & 1 : 0; }
     // tile origin and per-chunk advance, in bytes (both wave-uniform)
     __device__ __forceinline__ static const char* origin(const uint16_t* g, int ld, int row0) {
         return (const char*)(KC ? g + (size_t)row0 * ld : g + row0);
@@ -511,7 +515,7 @@ struct DmaTile {
         } else {
             const int g = lane / 16, i = lane % 16;
             const int k = 8 * (g / 2) + i / 4;       // k-step and second half go into the instruction offset
-            const int gran = blk ^ (k % 4);
+            const int gran = blk ^ granule_xor(k);
             return (uint32_t)((k * ROWS + gran * 32 + 16 * (g % 2) + 4 * (i % 4)) * 2);
         }
     }
@@ -761,6 +765,216 @@ __global__ __launch_bounds__(256, (BM * BN <= 128 * 128 ? 2 : 1)) void pd_gemm_b
     store_tile<TM, TN>(a, acc, m0 + wm * TM * 32, n0 + wn * TN * 32, c_off, (float*)ring + wave * (32 * (32 * TN + 8)), lane);
 }
 
+// ---------------------------------------------------------------------------------------
+// Products with few output tiles (a sequence or a micro-batch of a few hundred tokens): the reduction is split over
+// the waves of a block.  Such a product is a matter of latency: with 128 x 128 tiles the 8 to 30 blocks of
+// 128 x 1024..3072 x 1024 walk 32 chunks each with four in flight, i.e. eight round trips to memory, 9-10 us whatever
+// the size (28 us at k = 4096).  Here a block owns only 32 x 32 to 64 x 64 of C and its eight waves an eighth of the k
+// range each, with a ring of their own and no barrier until the end: 128 KB in flight per CU from the start, one to
+// four round trips in all (5 to 9 us; figures at the choice of the kernel below).  The eight partial tiles meet in LDS and are added in wave order (deterministic) by all threads,
+// which apply the epilogue to 8 consecutive elements of a row.
+// A k-contiguous, K a multiple of 32; rows beyond M or N are fetched from a clamped row and not stored.
+template <int TM, int TN, bool B_KC>
+__global__ __launch_bounds__(512, 2) void pd_gemm_bf16_ksplit_kernel(const GemmBf16Args a) {
+    constexpr int BM = 32 * TM, BN = 32 * TN, NW = 8;
+    constexpr int RS = 5 - TM * TN > 1 ? 5 - TM * TN : 2;        // ring stages of a wave: 4, 3, 2 for 1, 2, 4 MFMA tiles
+    using TA = DmaTile<BM, true, 1>;
+    using TB = DmaTile<BN, B_KC, 1>;
+    using FB = Frag<B_KC>;
+    constexpr int IPT = TA::PER_WAVE + TB::PER_WAVE;
+    constexpr int STAGE = TA::BYTES + TB::BYTES;
+    constexpr int P = BN + 4;                                    // pitch of a partial tile (floats)
+    constexpr int PART = BM * P * 4;
+    constexpr int LDS = NW * (RS * STAGE > PART ? RS * STAGE : PART);
+    static_assert(LDS <= 160 * 1024, "LDS budget of one CU");
+    __shared__ __attribute__((aligned(1024))) char lds[LDS];
+
+    const int lane = threadIdx.x % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int lin = (blockIdx.x % N_XCD) * a.tiles_per_xcd + blockIdx.x / N_XCD;
+    if (lin >= a.total_tiles) return;
+    // (down the rows first: the blocks of one die share columns of B, the weights)
+    const int m0 = (lin % a.tiles_m) * BM, n0 = (lin / a.tiles_m) * BN;
+
+    const int nk = a.K / DK;
+    const int c0 = nk * wave / NW, n = nk * (wave + 1) / NW - c0;      // this wave's chunks
+    TA ta;
+    TB tb;
+    ta.init(a.lda, m0, a.M, 0, lane);
+    tb.init(a.ldb, n0, a.N, 0, lane);
+    const char* const a_org = TA::origin(a.A, a.lda, m0) + c0 * TA::chunk_bytes(a.lda);
+    const char* const b_org = TB::origin(a.B, a.ldb, n0) + c0 * TB::chunk_bytes(a.ldb);
+    const size_t a_step = TA::chunk_bytes(a.lda), b_step = TB::chunk_bytes(a.ldb);
+    char* const ring = lds + wave * (RS * STAGE);
+
+    float16_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+    // chunk `c` of this wave (clamped: past the end the last one is fetched again, so that the number of loads in
+    // flight is the same in every turn) into ring stage ST
+    auto fetch = [&](auto st, int c) {
+        constexpr int ST = decltype(st)::value;
+        const int cc = min(c, n - 1);
+#pragma unroll
+        for (int t = 0; t < TA::PER_WAVE; ++t)
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(a_org + cc * a_step + ta.off[t]),
+                                             (lds_void_ptr)(ring + ST * STAGE + t * 1024), 16, 0, 0);
+#pragma unroll
+        for (int t = 0; t < TB::PER_WAVE; ++t)
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(b_org + cc * b_step + tb.off[t]),
+                                             (lds_void_ptr)(ring + ST * STAGE + TA::BYTES + t * 1024), 16, 0, 0);
+    };
+    using std::integral_constant;
+    if (n > 0) {
+        fetch(integral_constant<int, 0>{}, 0);
+        fetch(integral_constant<int, 1>{}, 1);
+        if constexpr (RS > 2) fetch(integral_constant<int, 2>{}, 2);
+        if constexpr (RS > 3) fetch(integral_constant<int, 3>{}, 3);
+        const uint32_t base = (uint32_t)(size_t)(lds_void_ptr)ring;
+        uint32_t fa[TM][2], fb[TN][2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) fa[i][s] = base + TA::frag_offset(i, lane, s);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) fb[j][s] = base + TA::BYTES + TB::frag_offset(j, lane, B_KC ? s : 0);
+        }
+        auto turn = [&](auto st, int c) {
+            constexpr int ST = decltype(st)::value;
+            constexpr int OFF = ST * STAGE;
+            wait_vmcnt<(RS - 1) * IPT>();                        // the oldest chunk has landed
+            u32x4 va[TM][2];
+            u32x4 vb[TN][2];
+            u32x2 blo[TN][2], bhi[TN][2];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(va[i][s]) : "v"(fa[i][s]), "n"(OFF) : "memory");
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    if (B_KC) {
+                        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(vb[j][s]) : "v"(fb[j][s]), "n"(OFF) : "memory");
+                    } else if (s == 0) {
+                        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(blo[j][s]) : "v"(fb[j][s]), "n"(OFF) : "memory");
+                        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(bhi[j][s]) : "v"(fb[j][s]), "n"(OFF + 4 * BN * 2) : "memory");
+                    } else {
+                        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(blo[j][s]) : "v"(fb[j][s]), "n"(OFF + 16 * BN * 2) : "memory");
+                        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(bhi[j][s]) : "v"(fb[j][s]), "n"(OFF + 20 * BN * 2) : "memory");
+                    }
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(va[i][s]));
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    if (B_KC) asm volatile("" : "+v"(vb[j][s]));
+                    else asm volatile("" : "+v"(blo[j][s]), "+v"(bhi[j][s]));
+                }
+            }
+            fetch(st, c + RS);                                   // the fragments are in registers: the stage is free
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        if (!B_KC) vb[j][s] = u32x4{blo[j][s][0], blo[j][s][1], bhi[j][s][0], bhi[j][s][1]};
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va[i][s]),
+                                                                            __builtin_bit_cast(bf16x8, vb[j][s]), acc[i][j], 0, 0, 0);
+                    }
+        };
+        for (int c = 0; c < n; c += RS) {
+            turn(integral_constant<int, 0>{}, c);
+            if (c + 1 < n) turn(integral_constant<int, 1>{}, c + 1);
+            if constexpr (RS > 2) if (c + 2 < n) turn(integral_constant<int, 2>{}, c + 2);
+            if constexpr (RS > 3) if (c + 3 < n) turn(integral_constant<int, 3>{}, c + 3);
+        }
+        wait_vmcnt<0>();                                         // the ring becomes staging space
+    }
+    __syncthreads();
+    {
+        float* const part = (float*)(lds + wave * PART);
+        const int idx = lane % 32, h = lane / 32;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) part[(i * 32 + 8 * (e / 4) + 4 * h + e % 4) * P + j * 32 + idx] = acc[i][j][e];
+    }
+    __syncthreads();
+    constexpr int VPR = BN / 8;                                  // 16-byte results per row
+    if (threadIdx.x < BM * VPR) {
+        const int r = threadIdx.x / VPR, c8 = (threadIdx.x % VPR) * 8;
+        const int row = m0 + r, col = n0 + c8;
+        if (row < a.M && col < a.N) {
+            float4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const float* src = (const float*)(lds + w * PART) + r * P + c8;
+                s0 += *(const float4_t*)src;
+                s1 += *(const float4_t*)(src + 4);
+            }
+            float v[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = a.alpha * v[q] + (a.bias ? a.bias[col + q] : 0.f);
+            if (a.out_f32) {
+                float4_t* p = (float4_t*)((float*)a.C + (long long)row * a.ldc + col);
+                float4_t w0 = {v[0], v[1], v[2], v[3]}, w1 = {v[4], v[5], v[6], v[7]};
+                if (a.beta != 0.f) {
+                    w0 += a.beta * p[0];
+                    w1 += a.beta * p[1];
+                }
+                p[0] = w0;
+                p[1] = w1;
+                return;
+            }
+            if (a.residual) {
+                const u16x8 rr = *(const u16x8*)(a.residual + (long long)row * a.ldr + col);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[q] += bf2f(rr[q]);
+            }
+            if (a.act == 2) {
+                const u16x8 xx = *(const u16x8*)(a.aux_in + (long long)row * a.ld_aux + col);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[q] *= gelu_grad_f(bf2f(xx[q]));
+            }
+            u16x8 o;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) o[q] = f2bf(v[q]);
+            *(u16x8*)((uint16_t*)a.C + (long long)row * a.ldc + col) = o;
+            if (a.act == 1) {
+                u16x8 gg;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) gg[q] = f2bf(gelu_f(bf2f(o[q])));
+                *(u16x8*)(a.aux_out + (long long)row * a.ld_aux + col) = gg;
+            }
+        }
+    }
+}
+
+template <int TM, int TN>
+int launch_gemm_bf16_ksplit(int tb, GemmBf16Args g, hipStream_t s) {
+    g.tiles_m = (g.M + 32 * TM - 1) / (32 * TM);
+    g.tiles_n = (g.N + 32 * TN - 1) / (32 * TN);
+    g.total_tiles = g.tiles_m * g.tiles_n;
+    g.tiles_per_xcd = (g.total_tiles + N_XCD - 1) / N_XCD;
+    const dim3 grid(g.tiles_per_xcd * N_XCD);
+    if (tb) pd_gemm_bf16_ksplit_kernel<TM, TN, true><<<grid, 512, 0, s>>>(g);
+    else pd_gemm_bf16_ksplit_kernel<TM, TN, false><<<grid, 512, 0, s>>>(g);
+    PD_CHECK_LAUNCH("pd_gemm_bf16");
+    return PD_OK;
+}
+
 template <int BM, int BN>
 int launch_gemm_bf16_dma(int ta, int tb, GemmBf16Args g, int batch, hipStream_t s) {
     g.tiles_m = (g.M + BM - 1) / BM;
@@ -847,6 +1061,17 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     if (g_force_bm && dma_ok) {
         if (g_force_bm == 256 && g_force_bn == 256) return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
         if (g_force_bm == 128 && g_force_bn == 128) return launch_gemm_bf16_dma<128, 128>(trans_a, trans_b, g, batch, s);
+    }
+    // Few output tiles: the reduction split over the waves of a block, with the smallest tile whose blocks still find a
+    // CU each (32 x 32, 32 x 64, 64 x 64).  us, weights from memory, against 128 x 128 tiles: 128 x 1024 x 4096 10.6 / 28,
+    // 128 x 1024 x 1024 5.0 / 8.8, 128 x 3072 x 1024 8.2 / 10.4, 600 x 768 x 3072 15.9 / 28.9, 600 x 768 x 768 8.1 / 8.8,
+    // 256 x 4096 x 1024 (256 blocks of 64 x 64) 10.4 / 10.4; with 360 blocks (600 x 2304 x 768) 15.2 / 9.4.
+    if (!g_force_bm && !trans_a && batch == 1 && g.vec_store && K % DK == 0 &&
+        (long long)64 * (lda > ldb ? lda : ldb) * 2 < (1ll << 31)) {
+        const auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+        if (blocks(32, 32) <= 256) return launch_gemm_bf16_ksplit<1, 1>(trans_b, g, s);
+        if (blocks(32, 64) <= 256) return launch_gemm_bf16_ksplit<1, 2>(trans_b, g, s);
+        if (blocks(64, 64) <= 256) return launch_gemm_bf16_ksplit<2, 2>(trans_b, g, s);
     }
     // 256 x 256 tiles (one block per CU, half the LDS reads per MFMA) from 192 tiles on, i.e. three quarters of
     // the CUs busy: 4096 x 4096 x 1024 takes 41 us against 49 with 128 x 128 tiles, 4096 x 3072 x 1024 (192

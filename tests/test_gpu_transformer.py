@@ -440,3 +440,36 @@ def test_gemm_with_gelu_in_its_epilogue(M, N, K, gemm_tile):
     ff = f.float().cpu().requires_grad_()
     F.gelu(ff).backward(dy.float().cpu() @ w2.float().cpu())
     assert _rel(df, ff.grad) < 6e-3
+
+
+@pytest.mark.parametrize("tb", [True, False])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 32), (33, 40, 32),        # one chunk: seven of a block's eight waves have none
+                                   (128, 1024, 1024), (65, 136, 288),      # 32 x 32 tiles, whole and with remainders
+                                   (128, 3072, 512), (601, 776, 96),       # 32 x 64
+                                   (250, 4000, 1056), (1024, 1024, 64)])   # 64 x 64
+def test_gemm_bf16_with_few_tiles_splits_k_over_the_waves(M, N, K, tb):
+    """Every tile of the kernel behind products with at most 256 small tiles, all its epilogues, against fp64.  A bf16
+    result carries one rounding of an fp32 sum: neighbouring values are up to 2^-7 of a value apart, so every value is
+    within 2^-8 of itself and so is the whole in rel-L2 (2^-8 / sqrt(3) and less for many values; the smallest case has
+    eight)."""
+    from pipedream_amd import ops
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g).to(BF).cuda()
+    b = torch.randn((N, K) if tb else (K, N), generator=g).to(BF).cuda()
+    bias, res = torch.randn(N, generator=g).cuda(), torch.randn(M, N, generator=g).to(BF).cuda()
+    want = (a.double() @ (b.double().t() if tb else b.double())).cpu()
+    bound = 2.0 ** -8
+    out = ops.gemm_bf16(a, b, trans_b=tb, out_f32=True, alpha=0.5)
+    assert _rel(out, 0.5 * want) < 1e-6
+    ops.gemm_bf16(a, b, trans_b=tb, out=out, beta=2.0)
+    assert _rel(out, 2.0 * want) < 1e-6
+    want_b = want + bias.double().cpu()
+    assert _rel(ops.gemm_bf16(a, b, trans_b=tb, bias=bias, residual=res), want_b + res.double().cpu()) < bound
+    f, act = ops.gemm_bf16_gelu(a, b, trans_b=tb, bias=bias)
+    assert _rel(f, want_b) < bound
+    assert _rel(act, F.gelu(f.double().cpu())) < bound
+    if not tb:
+        df = ops.gemm_bf16_gelu_backward(a, b, res)
+        x = res.double().cpu().requires_grad_()
+        (grad,) = torch.autograd.grad(F.gelu(x).sum(), x)
+        assert _rel(df, want * grad) < bound
