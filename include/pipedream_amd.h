@@ -272,6 +272,20 @@ int pd_conv3x3_winograd_fwd_pool_nhwc_f32(const float* x, const float* u, const 
  * its own that re-reads y.  Needs the full-resolution size to be exactly 2H x 2W. */
 int pd_conv3x3_winograd_fwd_unpool_nhwc_f32(const float* x, const float* u, const uint8_t* idx, float* y,
                                             float* y_full, int N, int H, int W, int C, int K, void* stream);
+/* The same three convolutions (plain, pooled, unpooled) with the sixteen products on the f16 matrix pipes: operands
+ * scaled by powers of two and split into two f16 terms, three products each, sums in fp32; no further from the exact
+ * result than the fp32 kernel above, and infinities give what it gives.  Needs C % 16 == 0 and K % 4 == 0
+ * (.._supported() returns 1).  filter_f32 writes filter_bytes bytes to u (16-byte aligned; meaning of C, K, rot180 as
+ * above).  Of the outputs exactly one set is given, the rest is NULL: y (with bias, relu, in_mask, out_mask as above); y_pool and
+ * pool_idx (with bias, relu); or y, unpool_idx and y_full (without bias, ReLU and mask).
+ * (torch.nn.Conv2d, vgg16/gpus=4_straight/stage0.py:12-14.) */
+int pd_conv3x3_winograd_f16x3_supported(int C, int K);
+int pd_conv3x3_winograd_f16x3_filter_bytes(int C, int K, uint64_t* bytes);
+int pd_conv3x3_winograd_f16x3_filter_f32(const float* w, void* u, int C, int K, int rot180, void* stream);
+int pd_conv3x3_winograd_f16x3_fwd_nhwc_f32(const float* x, const void* u, const float* bias, const float* in_mask,
+                                           const float* out_mask, float* y, float* y_pool, uint8_t* pool_idx, const uint8_t* unpool_idx,
+                                           float* y_full, int N, int H, int W, int C, int K, int relu,
+                                           void* stream);
 /* Weight (and optional bias) gradient of the same convolution in the Winograd domain: sums
  * dU = sum over 2x2 output tiles of (A dY A^T) (B^T d B) in persistent blocks, adds the blocks' partial
  * sums in fixed order and applies G^T . G.  Deterministic; agrees with pd_conv3x3_wgrad_nhwc_f32 to

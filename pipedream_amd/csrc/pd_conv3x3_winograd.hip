@@ -30,25 +30,17 @@
 //     and the optional output mask follow as the tile is stored as whole NHWC pixel rows.
 #include <type_traits>
 
-#include "pd_internal.h"
+#include "pd_winograd.hpp"
 
 namespace {
 
-typedef float float4_t __attribute__((ext_vector_type(4)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
-
-constexpr int WG_THREADS = 512;
-constexpr int WG_PIX = 16;                       // a block covers WG_PIX x WG_PIX output pixels
 constexpr int WG_TILES = 64;                     // = 8 x 8 tiles of 2 x 2 pixels
-constexpr int WG_BN = 64;                        // output channels per block
 constexpr int WG_CC = 8;                         // input channels per reduction chunk
 constexpr int WG_G = 16;                         // positions of the transformed 4 x 4 tile
 constexpr int WG_GW = 8;                         // ... of which a wave accumulates 8
 constexpr int WG_FRAG = 256;                     // floats in one wave-wide fragment (64 lanes x 4)
 constexpr int WG_V_STAGE = WG_G * 2 * WG_FRAG;   // floats of transformed input per chunk: [g][wm][lane][4]
 constexpr int WG_OP = WG_BN + 4;                 // pitch of the output staging tile
-constexpr int WG_XCD = 8;
-constexpr int WG_HALO = WG_PIX + 2;              // input halo tile: 18 rows x (16 + 2 per segment) pixels
 // The halo tile in LDS: four planes (channel half, column parity) of 18 rows x 12 16-byte units; the
 // unit of (half, row, col) is ((half * 2 + (col & 1)) * 18 + row) * 12 + (col >> 1).  The eight tiles
 // of a tile row then read eight consecutive units and the next tile row lands 8 units further
@@ -69,26 +61,6 @@ constexpr int WG_RAW_OFF = 2 * WG_V_STAGE;
 constexpr int WG_OUT_OFF = WG_RAW_OFF + 2 * WG_RAW_STAGE;
 constexpr int WG_LDS_FLOATS = WG_OUT_OFF + 256 * WG_OP;
 static_assert(WG_LDS_FLOATS * 4 <= 160 * 1024, "LDS budget of one CU");
-
-struct WinoArgs {
-    const float* x;         // [N,H,W,C]
-    const float* u;         // transformed filter, see winograd_filter_kernel
-    const float* bias;      // [K] or null
-    const float* mask;      // [N,H,W,C] or null: x is taken as 0 where mask <= 0
-    const float* out_mask;  // [N,H,W,K] or null: y is written as 0 where out_mask <= 0
-    float* y;               // [N,H,W,K]
-    float* pool_y;          // pooling variant: [N,H/2,W/2,K], written instead of y
-    uint8_t* pool_idx;      // pooling variant: [N,H/2,W/2,K] window position (bits 0-1) and sign (bit 2)
-    const uint8_t* unpool_idx;   // unpooling variant: [N,H,W,K] index bytes of the 2x2 pooling that produced this
-                                 // convolution's input (the convolution is an input gradient)
-    float* unpool_y;        // unpooling variant: [N,2H,2W,K], the gradient in front of that pooling
-    int N, H, W, C, K;
-    int img_h;              // stacked variant: rows of one image (N is then 1 and H the rows of the whole batch)
-    int relu;
-    int tiles_x, tiles_y, k_blocks, n_chunks;
-    int segs_per_row, n_segs;     // segmented variant: pieces per 16 rows of the stacked batch, pieces in all
-    int n_items, items_per_xcd;   // work items (pixel tile x channel block) in all / per die
-};
 
 // U = G g G^T for every (out channel k, in channel c), G = [[1,0,0],[.5,.5,.5],[.5,-.5,.5],[0,0,1]].
 // Output order: [k / 64][c / 8][g][(k % 64) / 32][(c % 8) / 4][k % 32][c % 4] -- for a block's 64
@@ -162,41 +134,6 @@ __global__ __launch_bounds__(256) void winograd_filter_kernel(const float* __res
         for (int m = 0; m < 4; ++m)
             *reinterpret_cast<float4*>(dst + (size_t)(i * 4 + m) * (2 * WG_FRAG)) = o[m];
     }
-}
-
-// Decoded work item: one 16 x 16 pixel tile of one image x one block of 64 output channels.
-struct WinoItem { int n, y0, x0, kb; };
-
-__device__ __forceinline__ WinoItem wino_decode(const WinoArgs& a, int item) {
-    WinoItem w;
-    w.kb = item % a.k_blocks;
-    const int tile = item / a.k_blocks;
-    const int per_img = a.tiles_x * a.tiles_y;
-    w.n = tile / per_img;
-    const int rem = tile - w.n * per_img;
-    const int ty = rem / a.tiles_x;
-    w.y0 = ty * WG_PIX;
-    w.x0 = (rem - ty * a.tiles_x) * WG_PIX;
-    return w;
-}
-
-// Piece s of a work item: first output row and column, and whether it exists (the last item may have fewer).
-// SEG = 1: the item's square.
-struct SegPos { int y0, x0; bool ok; };
-template <int SEG>
-__device__ __forceinline__ SegPos seg_pos(const WinoArgs& a, int item, int s) {
-    SegPos p;
-    if (SEG == 1) {
-        const WinoItem w = wino_decode(a, item);
-        p.y0 = w.y0; p.x0 = w.x0; p.ok = true;
-    } else {
-        const int sg = (item / a.k_blocks) * SEG + s;
-        const int rb = sg / a.segs_per_row;
-        p.y0 = rb * WG_PIX;
-        p.x0 = (sg - rb * a.segs_per_row) * (WG_PIX / SEG);
-        p.ok = sg < a.n_segs;
-    }
-    return p;
 }
 
 // Persistent kernel: gridDim.x (a multiple of 8, at most one block per CU) blocks share the work items.
@@ -809,34 +746,22 @@ namespace {
 
 int g_pieces_mode = 0;   // pd_conv3x3_winograd_set_pieces: 0 = by item count, 1 = wherever the shape allows, -1 = never
 
-int wino_fwd_launch(const char* who, const float* x, const float* u, const float* bias, const float* in_mask,
-                    const float* out_mask, float* y, float* pool_y, uint8_t* pool_idx, int N, int H, int W, int C,
-                    int K, int relu, void* stream, const uint8_t* unpool_idx = nullptr, float* unpool_y = nullptr) {
-    PD_REQUIRE(N > 0 && H > 0 && W > 0 && C > 0 && K > 0, PD_ESHAPE, "%s: dimensions must be positive", who);
-    PD_REQUIRE(wino_shape_ok(C, K), PD_ESHAPE, "%s: needs C %% 8 == 0 and K %% 4 == 0 (C=%d K=%d)", who, C, K);
-    PD_REQUIRE((long)H * W * (C > K ? C : K) < (1L << 29), PD_ESHAPE, "%s: image too large", who);
-    PD_REQUIRE((long)C * WG_G * WG_BN * 4 < (1L << 31), PD_ESHAPE, "%s: too many input channels", who);
-    PD_REQUIRE(x && u, PD_EINVAL, "%s: NULL pointer", who);
-    PD_REQUIRE(pd_aligned(x, 16) && pd_aligned(u, 16) && pd_aligned(y, 16) && pd_aligned(in_mask, 16) &&
-                   pd_aligned(out_mask, 16), PD_EINVAL, "%s: tensors must be 16-byte aligned", who);
-    WinoArgs a;
-    a.x = x; a.u = u; a.bias = bias; a.mask = in_mask; a.out_mask = out_mask; a.y = y;
-    a.pool_y = pool_y; a.pool_idx = pool_idx;
-    a.unpool_idx = unpool_idx; a.unpool_y = unpool_y;
+}  // namespace
+
+int pd_wino_plan(const char* who, WinoArgs& a, int N, int H, int W, int C, int K, int chunk, bool may_stack,
+                 WinoPlan* plan) {
     a.N = N; a.H = H; a.W = W; a.C = C; a.K = K;
     a.img_h = 0;
     // images whose height is even but no multiple of the 16-row tile are stacked into one tall image
     // (see the kernel): N * ceil(H / 16) tile rows become ceil(N * H / 16)
-    // (not with an input mask: that variant has no registers to spare for it)
     // (with the unpooling epilogue the full-resolution gradient, four times y, must fit a buffer descriptor too)
-    const bool stacked = !in_mask && N > 1 && H % 2 == 0 && H % WG_PIX != 0 &&
-                         (long)N * H * W * (C > K ? C : K) < (1L << 29) && (!unpool_y || (long)N * H * W * K < (1L << 27));
+    const bool stacked = may_stack && N > 1 && H % 2 == 0 && H % WG_PIX != 0 &&
+                         (long)N * H * W * (C > K ? C : K) < (1L << 29) && (!a.unpool_y || (long)N * H * W * K < (1L << 27));
     if (stacked) { a.img_h = H; a.H = N * H; a.N = 1; }
-    a.relu = relu != 0;
     a.tiles_x = (W + WG_PIX - 1) / WG_PIX;
     a.tiles_y = (a.H + WG_PIX - 1) / WG_PIX;
     a.k_blocks = (K + WG_BN - 1) / WG_BN;
-    a.n_chunks = C / WG_CC;
+    a.n_chunks = C / chunk;
     // one persistent block per CU (the kernel needs a CU's whole register file), in multiples of 8
     int dev = 0, cus = 0;
     PD_HIP(hipGetDevice(&dev));
@@ -864,7 +789,35 @@ int wino_fwd_launch(const char* who, const float* x, const float* u, const float
     a.items_per_xcd = (int)((items + WG_XCD - 1) / WG_XCD);
     long blocks = cu_blocks;
     if (blocks > (long)a.items_per_xcd * WG_XCD) blocks = (long)a.items_per_xcd * WG_XCD;
-    dim3 grid((unsigned)blocks);
+    plan->blocks = (unsigned)blocks;
+    plan->seg = seg;
+    plan->stacked = stacked;
+    return PD_OK;
+}
+
+namespace {
+
+int wino_fwd_launch(const char* who, const float* x, const float* u, const float* bias, const float* in_mask,
+                    const float* out_mask, float* y, float* pool_y, uint8_t* pool_idx, int N, int H, int W, int C,
+                    int K, int relu, void* stream, const uint8_t* unpool_idx = nullptr, float* unpool_y = nullptr) {
+    PD_REQUIRE(N > 0 && H > 0 && W > 0 && C > 0 && K > 0, PD_ESHAPE, "%s: dimensions must be positive", who);
+    PD_REQUIRE(wino_shape_ok(C, K), PD_ESHAPE, "%s: needs C %% 8 == 0 and K %% 4 == 0 (C=%d K=%d)", who, C, K);
+    PD_REQUIRE((long)H * W * (C > K ? C : K) < (1L << 29), PD_ESHAPE, "%s: image too large", who);
+    PD_REQUIRE((long)C * WG_G * WG_BN * 4 < (1L << 31), PD_ESHAPE, "%s: too many input channels", who);
+    PD_REQUIRE(x && u, PD_EINVAL, "%s: NULL pointer", who);
+    PD_REQUIRE(pd_aligned(x, 16) && pd_aligned(u, 16) && pd_aligned(y, 16) && pd_aligned(in_mask, 16) &&
+                   pd_aligned(out_mask, 16), PD_EINVAL, "%s: tensors must be 16-byte aligned", who);
+    WinoArgs a;
+    a.x = x; a.u = u; a.bias = bias; a.mask = in_mask; a.out_mask = out_mask; a.y = y;
+    a.pool_y = pool_y; a.pool_idx = pool_idx;
+    a.unpool_idx = unpool_idx; a.unpool_y = unpool_y;
+    a.relu = relu != 0;
+    WinoPlan plan;
+    // (an input mask goes without stacking: that variant has no registers to spare for it)
+    if (int rc = pd_wino_plan(who, a, N, H, W, C, K, WG_CC, !in_mask, &plan)) return rc;
+    const int seg = plan.seg;
+    const bool stacked = plan.stacked;
+    const dim3 grid(plan.blocks);
     hipStream_t s = (hipStream_t)stream;
     if (seg == 2) {
         if (unpool_y) winograd_fwd_kernel<false, false, true, true, 2><<<grid, WG_THREADS, 0, s>>>(a);

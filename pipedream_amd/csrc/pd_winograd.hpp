@@ -1,0 +1,78 @@
+// What the Winograd F(2x2, 3x3) forward / input-gradient kernels share: the description of a launch and the division of
+// the output into work items of 16 x 16 pixels (64 tiles of 2 x 2) x 64 output channels.
+#pragma once
+#include "pd_internal.h"
+
+namespace {
+
+typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
+
+constexpr int WG_THREADS = 512;
+constexpr int WG_PIX = 16;                       // a block covers WG_PIX x WG_PIX output pixels
+constexpr int WG_BN = 64;                        // output channels per block
+constexpr int WG_XCD = 8;
+constexpr int WG_HALO = WG_PIX + 2;              // input halo tile: 18 rows x (16 + 2 per segment) pixels
+
+}  // namespace
+
+struct WinoArgs {
+    const float* x;         // [N,H,W,C]
+    const float* u;         // transformed filter, see winograd_filter_kernel
+    const float* bias;      // [K] or null
+    const float* mask;      // [N,H,W,C] or null: x is taken as 0 where mask <= 0
+    const float* out_mask;  // [N,H,W,K] or null: y is written as 0 where out_mask <= 0
+    float* y;               // [N,H,W,K]
+    float* pool_y;          // pooling variant: [N,H/2,W/2,K], written instead of y
+    uint8_t* pool_idx;      // pooling variant: [N,H/2,W/2,K] window position (bits 0-1) and sign (bit 2)
+    const uint8_t* unpool_idx;   // unpooling variant: [N,H,W,K] index bytes of the 2x2 pooling that produced this
+                                 // convolution's input (the convolution is an input gradient)
+    float* unpool_y;        // unpooling variant: [N,2H,2W,K], the gradient in front of that pooling
+    int N, H, W, C, K;
+    int img_h;              // stacked variant: rows of one image (N is then 1 and H the rows of the whole batch)
+    int relu;
+    int tiles_x, tiles_y, k_blocks, n_chunks;
+    int segs_per_row, n_segs;     // segmented variant: pieces per 16 rows of the stacked batch, pieces in all
+    int n_items, items_per_xcd;   // work items (pixel tile x channel block) in all / per die
+};
+
+// How a launch divides its work (a's sizes, tiles, segments and items are filled in): persistent blocks, segments
+// per work item, whether the batch is taken as one tall image.  chunk: input channels per reduction step.
+struct WinoPlan { unsigned blocks; int seg; bool stacked; };
+int pd_wino_plan(const char* who, WinoArgs& a, int N, int H, int W, int C, int K, int chunk, bool may_stack,
+                 WinoPlan* plan);
+
+// Decoded work item: one 16 x 16 pixel tile of one image x one block of 64 output channels.
+struct WinoItem { int n, y0, x0, kb; };
+
+__device__ __forceinline__ WinoItem wino_decode(const WinoArgs& a, int item) {
+    WinoItem w;
+    w.kb = item % a.k_blocks;
+    const int tile = item / a.k_blocks;
+    const int per_img = a.tiles_x * a.tiles_y;
+    w.n = tile / per_img;
+    const int rem = tile - w.n * per_img;
+    const int ty = rem / a.tiles_x;
+    w.y0 = ty * WG_PIX;
+    w.x0 = (rem - ty * a.tiles_x) * WG_PIX;
+    return w;
+}
+
+// Piece s of a work item: first output row and column, and whether it exists (the last item may have fewer).
+// SEG = 1: the item's square.
+struct SegPos { int y0, x0; bool ok; };
+template <int SEG>
+__device__ __forceinline__ SegPos seg_pos(const WinoArgs& a, int item, int s) {
+    SegPos p;
+    if (SEG == 1) {
+        const WinoItem w = wino_decode(a, item);
+        p.y0 = w.y0; p.x0 = w.x0; p.ok = true;
+    } else {
+        const int sg = (item / a.k_blocks) * SEG + s;
+        const int rb = sg / a.segs_per_row;
+        p.y0 = rb * WG_PIX;
+        p.x0 = (sg - rb * a.segs_per_row) * (WG_PIX / SEG);
+        p.ok = sg < a.n_segs;
+    }
+    return p;
+}

@@ -17,7 +17,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from pipedream_amd import layers, ops
+from pipedream_amd import _cabi, layers, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -634,3 +634,70 @@ def test_pieces_equal_squares_at_vgg_size(conv_algorithm):
                 (ops.conv3x3_input_grad(dy, w),) + ops.conv3x3_input_grad_unpool(dy, w, idx)
         for mode in ("always", "auto"):
             assert all(torch.equal(p, q) for p, q in zip(out["never"], out[mode])), (C, K, HW, mode)
+
+
+def _fp32_winograd(x, w, bias, relu=False):
+    """The fp32 MFMA kernel through its own entry points."""
+    import ctypes
+    lib = _cabi.lib()
+    n, c, h, wd = x.shape
+    k = w.shape[0]
+    nbytes = ctypes.c_uint64()
+    lib.pd_conv3x3_winograd_filter_bytes(c, k, ctypes.byref(nbytes))
+    u = torch.empty(nbytes.value // 4, device="cuda")
+    lib.pd_conv3x3_winograd_filter_f32(w.data_ptr(), u.data_ptr(), c, k, 0, _cabi.stream_ptr())
+    y = torch.empty((n, k, h, wd), device="cuda", memory_format=torch.channels_last)
+    lib.pd_conv3x3_winograd_fwd_nhwc_f32(x.data_ptr(), u.data_ptr(), bias.data_ptr() if bias is not None else None,
+                                         None, None, y.data_ptr(), n, h, wd, c, k, int(relu), _cabi.stream_ptr())
+    return y
+
+
+# (one chunk of 16 channels; more work items than blocks hold at once; channel blocks that are not full; tiles beyond
+# the image; stacked images whose tiles see their neighbours' rows; pieces of 8 and 4 columns)
+@pytest.mark.parametrize("N,C,K,H,W", [(1, 16, 32, 1, 1), (2, 16, 64, 16, 16), (3, 48, 36, 33, 35), (5, 32, 128, 18, 20),
+                                       (4, 64, 64, 56, 56), (2, 512, 512, 14, 14), (9, 64, 64, 112, 96)])
+@pytest.mark.parametrize("scales", ["plain", "channels", "growing", "pixels"])
+def test_split_f16_convolution_is_no_less_exact_than_fp32(N, C, K, H, W, scales, conv_algorithm):
+    """The f16 kernel splits operands into two terms that hold 2^-24 of the largest value that shares their scale (a
+    tile's patch, an output channel's filter); its error stays within that of the fp32 kernel (1.7 times it where the
+    operands of one sum span 60 binary orders: there nearly all products round away in fp32, and what is left is the few
+    largest ones, exact in fp32 and split here to 2^-24)."""
+    if conv_algorithm != "winograd":
+        pytest.skip("the Winograd kernel's")
+    g = torch.Generator("cuda").manual_seed(N * 1000 + C + H)
+    x = torch.randn(N, C, H, W, generator=g, device="cuda")
+    if scales == "channels":
+        x = x * torch.randint(-30, 30, (N, C, 1, 1), generator=g, device="cuda").float().exp2()
+    elif scales == "growing":
+        x = x * (torch.arange(C, device="cuda").float() * (64.0 / C) - 32).exp2()[None, :, None, None]
+    elif scales == "pixels":
+        x = x * torch.randint(-20, 20, (N, 1, H, W), generator=g, device="cuda").float().exp2()
+    x = x.contiguous(memory_format=torch.channels_last)
+    w = (torch.randn(K, C, 3, 3, generator=g, device="cuda") * (9 * C) ** -0.5).contiguous(memory_format=torch.channels_last)
+    want = torch.nn.functional.conv2d(x.cpu().double(), w.cpu().double(), padding=1)
+    got = ops.conv3x3_forward(x, w).cpu().double()
+    fp32 = _fp32_winograd(x, w, None).cpu().double()
+    error, allowed = (got - want).norm(), (fp32 - want).norm()
+    factor = 1.7 if scales in ("channels", "growing") else 1.1          # (1.1: two samples of the same rounding)
+    assert error <= factor * allowed + 2.0 ** -23 * want.norm() * (C == 16), (error / want.norm(), allowed / want.norm())
+
+
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan")])
+@pytest.mark.parametrize("where", ["input", "filter"])
+@pytest.mark.parametrize("N,C,K,H,W", [(2, 64, 64, 40, 40), (3, 32, 128, 17, 23), (40, 64, 64, 64, 64)])
+def test_split_f16_convolution_of_infinities(value, where, N, C, K, H, W, conv_algorithm):
+    """Infinities cannot be split into terms; the outputs are those of the fp32 kernel, in the work items that hold one
+    and in the later ones of the same block."""
+    if conv_algorithm != "winograd":
+        pytest.skip("the Winograd kernel's")
+    g = torch.Generator("cuda").manual_seed(3)
+    x = torch.randn(N, C, H, W, generator=g, device="cuda").contiguous(memory_format=torch.channels_last)
+    w = (torch.randn(K, C, 3, 3, generator=g, device="cuda") * 0.05).contiguous(memory_format=torch.channels_last)
+    if where == "input":
+        x[0, 5, 7, 9] = value
+        x[N - 1, C - 1, 16, 20] = value
+    else:
+        w[K - 3, 4, 1, 1] = value
+    got, want = ops.conv3x3_forward(x, w), _fp32_winograd(x, w, None)
+    torch.testing.assert_close(got, want, rtol=1e-4, atol=2e-6, equal_nan=True)   # (C = 64: twice fp32's 1e-6 on unit data)
+    assert torch.isfinite(want).any() and not torch.isfinite(want).all()
