@@ -908,7 +908,6 @@ extern "C" int pd_conv3x3_winograd_fwd_pool_nhwc_f32(const float* x, const float
 // =====================================================================================================
 namespace {
 
-constexpr int WW_THREADS = 512;
 constexpr int WW_TILES = 8;                          // tiles per strip
 constexpr int WW_PATCH_W = 2 * WW_TILES + 2;         // input columns of a strip's patch
 constexpr int WW_ROW_PIECES = 320;                   // 16-byte pieces per patch row, padded from 18*16 to 5 waves
@@ -918,21 +917,6 @@ constexpr int WW_RAW_OFF = 2 * WW_V_STAGE;
 constexpr int WW_ZERO_OFF = WW_RAW_OFF + 2 * WW_RAW_STAGE;   // upright strips: one patch row (4 pixels) of zeros
 constexpr int WW_LDS_FLOATS = WW_ZERO_OFF + 4 * 64;
 constexpr int WW_VROWS = 2 * WW_TILES;               // output rows of an upright strip
-constexpr int WW_BLOCKS = 256;                       // persistent blocks: 8 dies x 32
-constexpr int WW_PART_FLOATS = WG_G * 64 * 64;       // one block's partial dU
-constexpr int WW_PART_STRIDE = WW_PART_FLOATS;       // floats between two blocks' partials
-
-struct WinoWgradArgs {
-    const float* x;      // [N,H,W,C]
-    const float* dy;     // [N,H,W,K]
-    float* part;         // [pair][rank][16][64][64]
-    float* part_db;      // [pair][rank][2][64]
-    int N, H, W, C, K;
-    int sx, sy;          // strips per row pair, row pairs per image (upright strips: strips side by side, unused)
-    int n_strips, strips_per_rank;
-    int rows_all;        // upright strips: N * H, the rows of the batch taken as one tall image
-    int c_blocks, n_pairs, ranks;
-};
 
 struct StripPos { int n, y0, x0, row; };      // row = n * H + y0, the strip's first output row counted over all images
 // (upright strips: row = first output row in the stacked batch, y0 = row % H, n unused)
@@ -1000,17 +984,10 @@ __global__ __launch_bounds__(WW_THREADS, 1) void winograd_wgrad_kernel(const Win
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // block -> (pair, rank): the 32 blocks of a die cover all pairs of a contiguous strip range, so the
-    // pairs that read the same x and dY strips run side by side on one L2
+    // behind the f16 kernel: all of it again if any of its blocks met an infinity
+    if (a.failed && !__syncthreads_or(threadIdx.x < WW_BLOCKS && a.failed[threadIdx.x])) return;
     int pair, rank;
-    if (a.n_pairs <= 32) {
-        const int xcd = blockIdx.x % WG_XCD, slot = blockIdx.x / WG_XCD;
-        pair = slot % a.n_pairs;
-        rank = xcd * (32 / a.n_pairs) + slot / a.n_pairs;
-    } else {                                   // more pairs than a die has blocks: plain round robin
-        pair = blockIdx.x % a.n_pairs;
-        rank = blockIdx.x / a.n_pairs;
-    }
+    wino_wgrad_pair_rank(a, pair, rank);
     const int kb = pair / a.c_blocks, cb = pair % a.c_blocks;
     const int s_begin = rank * a.strips_per_rank;
     int s_end = s_begin + a.strips_per_rank;
@@ -1431,8 +1408,8 @@ extern "C" int pd_conv3x3_winograd_wgrad_workspace_bytes(int C, int K, uint64_t*
                "pd_conv3x3_winograd_wgrad_workspace_bytes: needs C and K multiples of 64 with C*K/4096 a power "
                "of two <= 256 (C=%d K=%d)", C, K);
     const uint64_t pairs = (uint64_t)(C / 64) * (K / 64);
-    // per block: partial dU and 2 x 64 partial dbias; per pair and rank group: summed dU and dbias
-    *bytes = ((uint64_t)WW_BLOCKS * (WW_PART_STRIDE + 128) + WW_SUM_GROUPS * pairs * (WW_PART_FLOATS + 64)) * sizeof(float);
+    // per block: partial dU, 2 x 64 partial dbias and the mark of the f16 kernel; per pair and rank group: summed dU and dbias
+    *bytes = ((uint64_t)WW_BLOCKS * (WW_PART_STRIDE + 128) + WW_SUM_GROUPS * pairs * (WW_PART_FLOATS + 64) + WW_BLOCKS) * sizeof(float);
     return PD_OK;
 }
 
@@ -1476,6 +1453,15 @@ extern "C" int pd_conv3x3_winograd_wgrad_nhwc_f32(const float* x, const float* d
     float* du = a.part_db + (size_t)WW_BLOCKS * 128;
     float* dbsum = du + (size_t)WW_SUM_GROUPS * a.n_pairs * WW_PART_FLOATS;
     hipStream_t s = (hipStream_t)stream;
+    // The f16 kernel, where its blocks have at least one full step of 16 tiles (below, its error against 64 bits is up to
+    // 6 % above the fp32 kernel's, which decides nothing about time), x and dY lie within its offsets, and no strips are
+    // asked for.  What it cannot split (infinities) the fp32 kernel does behind it, whose blocks otherwise leave at once.
+    // 64 images, C = K: 64 at 224 x 224 1147 -> 773 us, 128 at 112 975 -> 620, 256 at 56 1013 -> 603, 512 at 28 1021 -> 587,
+    // 512 at 14 292 -> 198.
+    const long tiles = (long)N * ((H + 1) / 2) * ((W + 1) / 2);
+    const bool split = g_wgrad_strips == 0 && tiles >= 16L * a.ranks && (long)N * H * W * (C > K ? C : K) * 4 < (1L << 30);
+    a.failed = split ? (int*)(dbsum + (size_t)WW_SUM_GROUPS * a.n_pairs * 64) : nullptr;
+    if (split) pd_wino_wgrad_f16x3(a, s);
     if (upright) winograd_wgrad_kernel<true><<<WW_BLOCKS, WW_THREADS, 0, s>>>(a);
     else winograd_wgrad_kernel<false><<<WW_BLOCKS, WW_THREADS, 0, s>>>(a);
     PD_CHECK_LAUNCH(who);

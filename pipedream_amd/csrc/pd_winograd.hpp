@@ -14,6 +14,12 @@ constexpr int WG_BN = 64;                        // output channels per block
 constexpr int WG_XCD = 8;
 constexpr int WG_HALO = WG_PIX + 2;              // input halo tile: 18 rows x (16 + 2 per segment) pixels
 
+// weight gradient
+constexpr int WW_THREADS = 512;
+constexpr int WW_BLOCKS = 256;                       // persistent blocks: 8 dies x 32
+constexpr int WW_PART_FLOATS = 16 * 64 * 64;         // one block's partial dU
+constexpr int WW_PART_STRIDE = WW_PART_FLOATS;       // floats between two blocks' partials
+
 }  // namespace
 
 struct WinoArgs {
@@ -76,3 +82,31 @@ __device__ __forceinline__ SegPos seg_pos(const WinoArgs& a, int item, int s) {
     }
     return p;
 }
+
+// Weight gradient: a launch of either kernel.
+struct WinoWgradArgs {
+    const float* x;      // [N,H,W,C]
+    const float* dy;     // [N,H,W,K]
+    float* part;         // [pair][rank][16][64][64]
+    float* part_db;      // [pair][rank][2][64]
+    int N, H, W, C, K;
+    int sx, sy;          // strips per row pair, row pairs per image (upright strips: strips side by side, unused)
+    int n_strips, strips_per_rank;
+    int rows_all;        // upright strips: N * H, the rows of the batch taken as one tall image
+    int c_blocks, n_pairs, ranks;
+    int* failed;         // [WW_BLOCKS], written by the f16 kernel: the block met an infinity; or null
+};
+// block -> (pair, rank): the 32 blocks of a die cover all pairs of a contiguous range of ranks, so that the pairs that
+// read the same x and dY run side by side on one L2
+__device__ __forceinline__ void wino_wgrad_pair_rank(const WinoWgradArgs& a, int& pair, int& rank) {
+    if (a.n_pairs <= 32) {
+        const int xcd = blockIdx.x % WG_XCD, slot = blockIdx.x / WG_XCD;
+        pair = slot % a.n_pairs;
+        rank = xcd * (32 / a.n_pairs) + slot / a.n_pairs;
+    } else {                                   // more pairs than a die has blocks: plain round robin
+        pair = blockIdx.x % a.n_pairs;
+        rank = blockIdx.x / a.n_pairs;
+    }
+}
+// The f16 kernel: writes a.part, a.part_db and a.failed.
+void pd_wino_wgrad_f16x3(const WinoWgradArgs& a, hipStream_t s);

@@ -652,9 +652,10 @@ def set_conv_pieces(mode):
 
 
 def set_conv_wgrad_strips(mode):
-    """Strips of the Winograd weight-gradient kernel: "auto" (upright strips of 16 rows x 2 columns of the stacked
-    batch where the width is no multiple of 16 pixels), "flat" (2 x 16 pixels always), "upright" (wherever the shape
-    allows).  The results differ by the summation order only."""
+    """Strips of the fp32 Winograd weight-gradient kernel: "auto" (long reductions go to the f16 kernel, which has no
+    strips, the others take upright strips of 16 rows x 2 columns of the stacked batch where the width is no multiple
+    of 16 pixels), "flat" (2 x 16 pixels always), "upright" (wherever the shape allows).  The results differ by rounding
+    only."""
     _cabi.lib().pd_conv3x3_winograd_set_wgrad_strips({"auto": 0, "flat": 1, "upright": 2}[mode])
 
 

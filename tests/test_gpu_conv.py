@@ -701,3 +701,54 @@ def test_split_f16_convolution_of_infinities(value, where, N, C, K, H, W, conv_a
     got, want = ops.conv3x3_forward(x, w), _fp32_winograd(x, w, None)
     torch.testing.assert_close(got, want, rtol=1e-4, atol=2e-6, equal_nan=True)   # (C = 64: twice fp32's 1e-6 on unit data)
     assert torch.isfinite(want).any() and not torch.isfinite(want).all()
+
+
+# (one unit of two tiles; ranks without a step; units that end beyond the image; more pairs of channel blocks than ranks;
+# reductions long enough for the rounding of the sums to show)
+@pytest.mark.parametrize("N,C,K,H,W", [(1, 64, 64, 1, 1), (1, 64, 64, 7, 5), (2, 128, 64, 33, 35), (3, 64, 128, 18, 20),
+                                       (4, 512, 512, 14, 14), (1, 1024, 1024, 6, 6), (16, 64, 64, 112, 112)])
+@pytest.mark.parametrize("scales", ["plain", "channels", "growing"])
+def test_split_f16_weight_gradient(N, C, K, H, W, scales, conv_algorithm):
+    """Against 64 bits.  Sums of P = N H W products of two terms each in fp32: 2^-23 for the terms and the transforms in
+    front of them, times 4 for the cancellation in G^T dU G, and 2^-24 sqrt(P / 16) of the running sums; per tap, so
+    that a bias that adds up in one of them shows.  (The small ones take the fp32 kernel.)"""
+    if conv_algorithm != "winograd":
+        pytest.skip("the Winograd kernel's")
+    g = torch.Generator("cuda").manual_seed(N + C + H)
+    x = torch.randn(N, C, H, W, generator=g, device="cuda")
+    if scales == "channels":
+        x = x * torch.randint(-5, 5, (1, C, 1, 1), generator=g, device="cuda").float().exp2()
+    elif scales == "growing":
+        x = x * (torch.arange(H, device="cuda").float() * (60.0 / H) - 30).exp2()[:, None]
+    x = x.contiguous(memory_format=torch.channels_last)
+    dy = (torch.randn(N, K, H, W, generator=g, device="cuda") * 1e-6).contiguous(memory_format=torch.channels_last)
+    dw, db = ops.conv3x3_weight_grad(x, dy)
+    padded, rows = F.pad(x.double(), (1, 1, 1, 1)), dy.double().permute(1, 0, 2, 3).reshape(K, -1)
+    want = torch.stack([rows @ padded[:, :, r:r + H, s:s + W].permute(0, 2, 3, 1).reshape(-1, C)
+                        for r in range(3) for s in range(3)])      # [tap, K, C]
+    error = dw.double().permute(2, 3, 0, 1).reshape(9, K, C) - want
+    # plain: per tap (the middle one alone is not zero on a 1 x 1 image); channels: per channel; growing: as a whole
+    dims = {"plain": (1, 2), "channels": (0, 1), "growing": (0, 1, 2)}[scales]
+    error, scale = error.pow(2).sum(dims).sqrt(), want.pow(2).sum(dims).sqrt()
+    if H * W == 1:
+        error, scale = error.norm(), scale.norm()
+    bound = 2.0 ** -21 + 2.0 ** -24 * (N * H * W / 16) ** 0.5
+    assert (error <= bound * scale).all(), (error / scale).max()
+    torch.testing.assert_close(db.double(), rows.sum(1), rtol=1e-5, atol=1e-6 * 2.0 ** -20 * (N * H * W) ** 0.5)
+    assert torch.equal(dw, ops.conv3x3_weight_grad(x, dy)[0])
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_split_f16_weight_gradient_of_infinities(value, conv_algorithm):
+    """What the fp32 kernel gives: the channel of the infinity has no finite element, the others are as without it."""
+    if conv_algorithm != "winograd":
+        pytest.skip("the Winograd kernel's")
+    g = torch.Generator("cuda").manual_seed(5)
+    x = torch.randn(2, 64, 40, 40, generator=g, device="cuda").contiguous(memory_format=torch.channels_last)
+    dy = torch.randn(2, 64, 40, 40, generator=g, device="cuda").contiguous(memory_format=torch.channels_last)
+    clean = ops.conv3x3_weight_grad(x, dy)[0]
+    x[1, 5, 7, 9] = value
+    dw = ops.conv3x3_weight_grad(x, dy)[0]
+    assert not torch.isfinite(dw[:, 5]).any()
+    rest = [c for c in range(64) if c != 5]
+    torch.testing.assert_close(dw[:, rest], clean[:, rest], rtol=1e-4, atol=1e-4)     # (sums of 3200 products: 57 typically)
