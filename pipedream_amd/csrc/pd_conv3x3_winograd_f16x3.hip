@@ -390,7 +390,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         int n;                                 // image
         size_t img;                            // its first element [.., K]
         uint32_t off;                          // element offset of the first pixel in it
-        float4_t mk[POOL || UNPOOL ? 1 : 4];
+        uint32_t mbits;                        // output mask, four bits a pixel
         uint32_t iw[UNPOOL ? 4 : 1];
     };
     typedef int int4_t __attribute__((ext_vector_type(4)));
@@ -426,12 +426,18 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         } else if (!POOL && a.out_mask) {
             const __amdgpu_buffer_rsrc_t mr =
                 __builtin_amdgcn_make_buffer_rsrc((void*)(a.out_mask + o.img), 0, out_elems * 4, 0x00020000);
+            float4_t mk[4];
 #pragma unroll
             for (int px = 0; px < 4; ++px) {
                 const bool in = o.ok && o.y + (px >> 1) < a.H && o.x + (px & 1) < a.W;
-                o.mk[POOL || UNPOOL ? 0 : px] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                mk[px] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
                     mr, in ? (o.off + ((px >> 1) * a.W + (px & 1)) * a.K) * 4 : 0x80000000u, 0, 2));
             }
+            o.mbits = 0;
+#pragma unroll
+            for (int px = 0; px < 4; ++px)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) o.mbits |= (mk[px][c] > 0.f ? 1u : 0u) << (4 * px + c);
         }
     };
     // bias, ReLU, mask / pooling / unpooling of the tile's pixels (row-major) and the stores; what lies outside the
@@ -503,7 +509,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
                     for (int c = 0; c < 4; ++c) w[c] = (code[c] & 4u) ? w[c] : 0.f;
                 } else if (a.out_mask) {
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) w[c] = o.mk[POOL || UNPOOL ? 0 : px][c] > 0.f ? w[c] : 0.f;
+                    for (int c = 0; c < 4; ++c) w[c] = (o.mbits >> (4 * px + c)) & 1u ? w[c] : 0.f;
                 }
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, w), yr, in ? at * 4 : 0x80000000u, 0, 2);
             }
@@ -694,8 +700,6 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         load_channels(k4);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            Out o;
-            prepare_out(o, m_i, k4, t * 32 + (tid >> 4));
             float* st = (float*)(lds + H3_SLOT1_OFF) + ((j * 2) * 32 + (lane & 31)) * H3_PITCH + kh * 32 + 4 * (lane >> 5);
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
@@ -710,7 +714,12 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
                 }
                 *(float4_t*)(st + 8 * g) = z0;
                 *(float4_t*)(st + 32 * H3_PITCH + 8 * g) = z1;
+                __builtin_amdgcn_sched_barrier(0);
             }
+            __builtin_amdgcn_sched_barrier(0);
+            // (the output mask is kept as bits: its 16 values and what else is live here would spill 53 registers)
+            Out o;
+            prepare_out(o, m_i, k4, t * 32 + (tid >> 4));
             const int tf = exps[((q - 1) & 1) * 64 + t * 32 + (tid >> 4)];
             __syncthreads();
             const float* src = (const float*)(lds + H3_SLOT1_OFF) + (tid >> 4) * H3_PITCH + (tid & 15) * 4;
