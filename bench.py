@@ -9,12 +9,12 @@ plays its downstream neighbour (consumes the sent activation, queues a synthetic
 gradient ~ N(0,1)*1e-3).  All inputs are resident in HBM before the timed region.
 
 Prints ONE JSON line (see the keys below).  `roofline` covers the dominant kernel, the
-MFMA fp32 3x3 convolution by Winograd F(2x2, 3x3) (`winograd_fwd_kernel`, used for forward
-and input gradient): algorithmic flop of its launches in the timed region (those of the
+fp32 3x3 convolution by Winograd F(2x2, 3x3) on the f16 MFMA units, operands split into two terms
+(`winograd_fwd_f16x3_kernel`, used for forward and input gradient): algorithmic flop of its launches in the timed region (those of the
 direct convolution, 2*9*C*K per output pixel) / their summed duration, both measured with
 HIP events around every launch on the launch stream.  The kernel issues 16/36 of those
-multiplications to the MFMA units: `roofline.achieved` / `roofline.frac` are the rate it actually
-executes against the MFMA fp32 peak (never above 1), `roofline.direct_equivalent` is the rate a direct
+multiplications to the MFMA units, three times each: `roofline.achieved` / `roofline.frac` are the rate it
+actually executes against the dense f16 MFMA peak (never above 1), `roofline.direct_equivalent` is the rate a direct
 convolution would need for the same launch time.  `roofline.traffic` is read from the tracked summary of
 the rocprofv3 --pmc runs under profiles/ and is refused if that summary is about another kernel.
 `cpu_baseline` times the CPU oracle (torch.nn on the host cores) on a bounded sample of
@@ -37,6 +37,9 @@ BATCH = 64
 STASH_DEPTH = 4
 SGD_KW = dict(lr=0.01, momentum=0.9, weight_decay=5e-4)
 PEAK_FP32_MFMA_TFLOPS = 157.3
+PEAK_F16_MFMA_TFLOPS = 2500.0
+# flop the Winograd kernel executes per flop of the direct convolution: 16 of 36 multiplications, three products each
+WINO_EXECUTED = 3.0 * 16.0 / 36.0
 # HBM bytes per launch of the dominant kernel: written next to the summary of the rocprofv3 --pmc
 # FETCH_SIZE / WRITE_SIZE runs it comes from
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "winograd_fwd_vgg16_front_stage_bs64_pmc_traffic.json")
@@ -594,7 +597,7 @@ CPU_BASELINES = {"vgg16_pipeline": cpu_vgg16_pipeline, "gnmt": cpu_gnmt, "gnmt_c
                  "transformer": cpu_transformer}
 
 
-_SECONDARY = {"vgg16_pipeline": (vgg16_pipeline_run, "conv3x3_winograd_kernel", PEAK_FP32_MFMA_TFLOPS, "mfma"),
+_SECONDARY = {"vgg16_pipeline": (vgg16_pipeline_run, "conv3x3_winograd_kernel", PEAK_F16_MFMA_TFLOPS, "mfma"),
               "gnmt": (gnmt_run, "gemm_f32", PEAK_FP32_MFMA_TFLOPS, "mfma"),
               "gnmt_criterion": (gnmt_criterion_run, "label_smoothing_bwd", 8000.0, "hbm"),
               "transformer": (transformer_run, "gemm_bf16", 2500.0, "mfma")}
@@ -634,9 +637,9 @@ def secondary_record(workload, steps, warmup, single_stream=False, with_cpu_base
             stats[name]["GB/s"] = round(stats[name].pop("TFLOP/s") * 1e3, 1)
         k["TFLOP/s"] = stats[kernel]["GB/s"]
     if kernel == "conv3x3_winograd_kernel":
-        # the Winograd kernel executes 16/36 of the direct convolution's multiplications
-        extra = {"direct_equivalent": k["TFLOP/s"]}
-        k["TFLOP/s"] = k["TFLOP/s"] * 16.0 / 36.0
+        extra = {"direct_equivalent": k["TFLOP/s"],
+                 "note": "three f16 MFMA products per fp32 product of 16/36 of the direct convolution's"}
+        k["TFLOP/s"] = k["TFLOP/s"] * WINO_EXECUTED
     out = {
         "metric": "samples/sec per stage (fwd+bwd+stashed update)", "value": batch * steps / elapsed,
         "unit": "samples/s", "n_gpus": 1, "steps": steps, "warmup": warmup,
@@ -727,10 +730,11 @@ def main():
     elapsed, stats, _ = gpu_run(args.steps, args.warmup)
     wino = "conv3x3_winograd_kernel" in stats
     conv = stats["conv3x3_winograd_kernel" if wino else "conv3x3_fwd_kernel"]
-    kernel = "winograd_fwd_kernel" if wino else "conv3x3_fwd_kernel"
+    kernel = "winograd_fwd_f16x3_kernel" if wino else "conv3x3_fwd_kernel"
     direct = conv["rate"] / 1e12
-    # what the MFMA units execute: 16 multiplies per 2x2 outputs and channel pair instead of 36
-    executed = direct * (16.0 / 36.0 if wino else 1.0)
+    # what the MFMA units execute: 16 products per 2x2 outputs and channel pair instead of 36, three f16 MFMAs each
+    executed = direct * (WINO_EXECUTED if wino else 1.0)
+    peak = PEAK_F16_MFMA_TFLOPS if wino else PEAK_FP32_MFMA_TFLOPS
     traffic = args.traffic_bytes if args.traffic_bytes is not None else measured_traffic(kernel)
     out = {
         "metric": "samples/sec per stage (fwd+bwd+stashed update), VGG16 bs64; optimizer HBM GB/s",
@@ -748,12 +752,12 @@ def main():
         "config": {"workload": "VGG16 stage 0 (conv1_1..pool2), batch 64, fp32, stash depth 4, SGD momentum 0.9, "
                                "1F1B with 4 minibatches in flight",
                    "global_batch": BATCH, "parallelism": "1 stage on 1 GPU"},
-        "roofline": {"bound": "mfma", "achieved": executed, "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
-                     "frac": executed / PEAK_FP32_MFMA_TFLOPS, "traffic": traffic,
+        "roofline": {"bound": "mfma", "achieved": executed, "peak": peak, "unit": "TFLOP/s",
+                     "frac": executed / peak, "traffic": traffic,
                      "kernel": kernel + (" (F(2x2,3x3); forward + input gradient)" if wino
                                          else "<.,.,16> (forward + input gradient)"),
                      "launches": conv["launches"], "avg_us": conv["avg_us"],
-                     "flop_per_launch": conv["work_per_launch"] * (16.0 / 36.0 if wino else 1.0),
+                     "flop_per_launch": conv["work_per_launch"] * (WINO_EXECUTED if wino else 1.0),
                      "direct_flop_per_launch": conv["work_per_launch"],
                      # the rate a direct convolution (2*9*C*K flop per output pixel) would need for this time
                      "direct_equivalent": direct},
