@@ -686,7 +686,11 @@ def _winograd_run(x, w, bias, in_mask, out_mask, y, y_pool, pool_idx, unpool_idx
     lib = _cabi.lib()
     stream = _cabi.stream_ptr()
     nbytes = ctypes.c_uint64()
-    split = lib.pd_conv3x3_winograd_f16x3_supported(c, k)
+    # one chunk of 16 channels saves less than the launch for the filter's scales costs (3 us) unless every block has two
+    # work items (16 x 16 pixels x 64 channels) or more: 16 -> 32 channels, 8 images of 64 x 64: 15.6 us fp32, 18.1 f16;
+    # 64 images of 112 x 112: 104 and 85; 32 -> 32 channels there 153 and 110
+    split = (lib.pd_conv3x3_winograd_f16x3_supported(c, k)
+             and (c >= 32 or n * h * wd * ((k + 63) // 64) > 512 * 256))
     if split:
         lib.pd_conv3x3_winograd_f16x3_filter_bytes(c, k, ctypes.byref(nbytes))
         u = torch.empty(nbytes.value // 4, dtype=torch.float32, device=x.device)

@@ -652,10 +652,11 @@ def _fp32_winograd(x, w, bias, relu=False):
     return y
 
 
-# (one chunk of 16 channels; more work items than blocks hold at once; channel blocks that are not full; tiles beyond
-# the image; stacked images whose tiles see their neighbours' rows; pieces of 8 and 4 columns)
-@pytest.mark.parametrize("N,C,K,H,W", [(1, 16, 32, 1, 1), (2, 16, 64, 16, 16), (3, 48, 36, 33, 35), (5, 32, 128, 18, 20),
-                                       (4, 64, 64, 56, 56), (2, 512, 512, 14, 14), (9, 64, 64, 112, 96)])
+# (one chunk of 16 channels, on the fp32 kernel and with work items enough for the f16 one; more work items than blocks
+# hold at once; channel blocks that are not full; tiles beyond the image; stacked images whose tiles see their
+# neighbours' rows; pieces of 8 and 4 columns)
+@pytest.mark.parametrize("N,C,K,H,W", [(1, 16, 32, 1, 1), (2, 32, 64, 16, 16), (3, 48, 36, 33, 35), (5, 32, 128, 18, 20),
+                                       (9, 16, 64, 128, 128), (4, 64, 64, 56, 56), (2, 512, 512, 14, 14), (9, 64, 64, 112, 96)])
 @pytest.mark.parametrize("scales", ["plain", "channels", "growing", "pixels"])
 def test_split_f16_convolution_is_no_less_exact_than_fp32(N, C, K, H, W, scales, conv_algorithm):
     """The f16 kernel splits operands into two terms that hold 2^-24 of the largest value that shares their scale (a
