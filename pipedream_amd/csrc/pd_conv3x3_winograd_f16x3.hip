@@ -2,26 +2,38 @@
 // the reference) on the f16 matrix pipes, with fp32 operands, fp32 accumulation and fp32 accuracy.  For input channel
 // counts that are multiples of 16.
 //
-// An fp32 value, scaled by a power of two into f16's range, is the sum of two f16 values up to 2^-24 of it
-// (x1 = f16(x), x2 = f16(x - x1)); products of f16 values are exact in fp32, so  u v = u1 v1 + u1 v2 + u2 v1  up to
-// 2^-24 u v, three sixteenths of the time of the fp32 MFMA (v_mfma_f32_32x32x16_f16 runs at sixteen times its rate),
-// and unlike an fp32 MFMA it runs beside vector instructions.  Splitting two values takes four instructions
-// (v_cvt_pk_f16_f32, two v_fma_mix_f32 for the remainders, v_cvt_pk_f16_f32).
+// An fp32 value, scaled by a power of two into f16's range, is the sum of two f16 values (x1 = f16(x), x2 = f16(x - x1))
+// up to 2^-23 of it, or 2^-25 of f16's unit where that is more; products of f16 values are exact in fp32, so
+// u v = u1 v1 + u1 v2 + u2 v1  up to 2^-21 u v (4 million products: 2^-21.1 at most, 2^-23.6 rms; the rounding of the
+// running sum, eight times a chunk in the fp32 kernel and three times here, is what decides the error), three sixteenths
+// of the time of the fp32 MFMA (v_mfma_f32_32x32x16_f16 runs at sixteen times its rate), and unlike an fp32 MFMA it runs
+// beside vector instructions.  Splitting two values takes four instructions (v_cvt_pk_f16_f32, two v_fma_mix_f32 for the
+// remainders, v_cvt_pk_f16_f32).
 //
-// The scales are powers of two that are constant along the reduction, so they come out of the sums:
-//   * filter: one per output channel, from the largest |w| of the channel (winograd_amax_kernel), which becomes 8 to 16
-//     (|U| is at most 2.25 times that);
-//   * input: one per 2x2-output tile, from the largest |x| of its patch in the first chunk of 16 channels that holds
-//     anything; that becomes 4 to 8 (|V| at most four times it).  The tile keeps its scale while later chunks stay
-//     below 2^9 times that, else the scale follows and the waves that hold the tile's sums multiply them accordingly
-//     (a test per chunk, hardly ever more).  What is less than 2^-14 of f16's unit there is held to an absolute 2^-25, i.e.
-//     2^-27 of the largest value of the patch.
-// Infinities cannot be split: a block that meets one goes on with fp32 MFMAs from that work item.
+// f16 ends at 2^-24 below its unit, so a value far below the largest of its scale loses bits.  The scales are powers of two:
+//   * filter, per output channel k and per input channel c: with e(k, c) the exponent of the largest tap, R(k) = max over c
+//     of e and s(c) = max over k of e - R, w 2^-(R + s) is at most 1 to 2 everywhere and reaches it in every row and column;
+//     it is split at 2^13 times that (|U| is at most 2.25 times |w|).  R comes out of the sums, s goes into the input: a
+//     channel that is small and has large weights counts as much as one that is large and has small ones;
+//   * input: x 2^s, one scale per 2x2-output tile, from the largest value of its patch in the first chunk of 16 channels;
+//     that becomes 2^11 to 2^12 (|V| at most four times it).  The tile keeps its scale while later chunks stay below twice
+//     that, else the scale follows and the waves that hold the tile's sums multiply them accordingly (a test per chunk,
+//     hardly ever more).
+// A value is then held to 2^-37.8 (rms) of the largest of its patch over all channels, and what that costs is bounded by what
+// the largest contributes, provided that the channel it lies in has weights to speak of and that the pixel is one that the
+// output sees.  Hence two tests, and fp32 MFMAs for the work items that fail one:
+//   * a block of 64 output channels that holds a kernel w(k, c) which is zero, or below 2^-P of what its row and column
+//     have, with 2^P sqrt(C) = 2^13 (the error is then 2^-24.8 even where all of an output comes through that kernel; random
+//     filters of 512 x 512 channels reach 2^-4 of it);
+//   * a tile whose four inner pixels, which all four outputs see, are below 2^-8 of its patch in all channels.
+// Infinities, and values of 2^64 and more, cannot be split either.  A block that met one of those or such a tile stays on
+// the fp32 MFMAs for one item, then for two, four, ... if it goes on.
 //
 // Bound: f16 MFMAs, vector instructions and LDS traffic side by side.  Per chunk of 16 channels a SIMD's two waves issue
 // 48 MFMAs (1700 cycles) and 2 x 165 vector instructions, the block moves 290 KB through LDS (2300 cycles): 4100 cycles,
-// where the fp32 kernel takes 9580 for the same chunk.  64 images, C = K = 128 at 112 x 112: 568 us (417 TFLOP/s of a
-// direct convolution), C = K = 512 at 28 x 28: 521 us (454); 8 images 85 us.  VGG16's front stage 7.74 -> 6.07 ms a step,
+// where the fp32 kernel takes 9580 for the same chunk.  64 images, C = K = 128 at 112 x 112: 595 us (398 TFLOP/s of a
+// direct convolution; 564 with one scale for all channels and no tests), C = K = 512 at 28 x 28: 530 us (446); 8 images
+// 86 us.  VGG16's front stage 7.74 -> 6.07 ms a step,
 // all of VGG16 26.4 -> 20.0 ms, a validation pass over 2 x 8 images 3.70 -> 2.43 ms.  An item of 64 channels takes 27 500
 // cycles, 9000 of them behind its last product; before its divisions went to the ring of decoded items 35 000.
 // A block (512 threads, one per CU) owns 16 x 16 output pixels x 64 channels:
@@ -54,13 +66,20 @@ constexpr int H3_EXP_OFF = H3_ZERO_OFF + 512;          // [parity of the chunk][
 constexpr int H3_FLAG_OFF = H3_EXP_OFF + 2 * 64 * 4;
 constexpr int H3_ITEM_OFF = H3_FLAG_OFF + 16;          // the next work items, decoded
 constexpr int H3_ITEMS = 16;
-constexpr int H3_LDS = H3_ITEM_OFF + H3_ITEMS * 48;
+constexpr int H3_WIDE_OFF = H3_ITEM_OFF + H3_ITEMS * 48;   // a bit per block of 64 output channels: not for f16
+constexpr int H3_MAX_K_BLOCKS = 1024;
+constexpr int H3_LDS = H3_WIDE_OFF + H3_MAX_K_BLOCKS / 8;
 static_assert(H3_LDS <= 160 * 1024, "LDS budget of one CU");
 
-// Scales as biased exponents: a value field e (of the largest value) stands for the factor 2^(129 - e) on the input
-// and 2^(130 - e) on the filter.  Fields stop at 8 below (2^-119: the factor must stay finite) and reach 255 for
-// infinities.
-constexpr int H3_MIN_FIELD = 8;
+// Scales as biased exponents: a field e (of the largest value) stands for the factor 2^(H3_X_BASE - e) on the input and
+// 2^(H3_W_BASE - e) on the filter, so that the largest value becomes 2^11 to 2^12 and 2^13 to 2^14.
+constexpr int H3_X_BASE = 138, H3_W_BASE = 140;
+constexpr int H3_MIN_FIELD = 11;                       // (the factor must stay finite; denormals are still held exactly)
+constexpr int H3_MAX_FIELD = 190;                      // (below what an infinity has in any channel)
+constexpr int H3_SLACK = 1;                            // how far a tile's values may exceed its scale
+constexpr int H3_INNER = 8;                            // how far its inner pixels may stay below it
+constexpr int H3_MIN_SHIFT = -60;                      // range of s(c); a channel without weights has this too
+static_assert(255 + H3_MIN_SHIFT > H3_MAX_FIELD && H3_X_BASE - H3_MAX_FIELD + H3_MIN_SHIFT > -127, "fields");
 __device__ __forceinline__ float h3_scale(int field, int base) {
     return __builtin_bit_cast(float, (uint32_t)(base + 127 - field) << 23);
 }
@@ -82,71 +101,165 @@ __device__ __forceinline__ float h3_rest_hi(uint32_t p, float x) {
     return r;
 }
 
-// part[slice][k] = largest |w| (as bits) of output channel k over a slice of its filter.  Rows of the filter are
-// contiguous per k, or (rot180) k is the innermost index.
-__global__ __launch_bounds__(256) void winograd_amax_kernel(const float* __restrict__ w, uint32_t* __restrict__ part,
-                                                            int K, int C, int k_pad, int rot180, int slices) {
+// What the filter's buffer holds behind the fragments (byte offsets from its start).
+struct H3Layout {
+    size_t fields;      // [k_pad] int: R(k)
+    size_t shifts;      // [C] int: s(c)
+    size_t exps;        // [k_pad][C] bytes: e(k, c)
+    size_t part;        // [C / 16][k_pad] int: max of e over a slice of c (one slice where c is the innermost index of w)
+    size_t wide;        // [k_blocks][2 C / 16] int: not 0 where 32 output x 16 input channels lie as fp32, see below
+    size_t bytes;
+    __host__ __device__ H3Layout(int K, int C) {
+        const size_t k_blocks = (K + WG_BN - 1) / WG_BN, k_pad = k_blocks * WG_BN, chunks = C / H3_CC;
+        fields = k_blocks * chunks * H3_U_CHUNK;
+        shifts = fields + k_pad * 4;
+        exps = shifts + (size_t)C * 4;
+        part = exps + k_pad * C;
+        wide = part + chunks * k_pad * 4;
+        bytes = wide + k_blocks * chunks * 8;
+    }
+};
+
+// e(k, c) and its maxima over c.  0: all nine taps are zero (or NaN); denormals count as the smallest normal numbers.
+__global__ __launch_bounds__(256) void winograd_exps_kernel(const float* __restrict__ w, char* __restrict__ u, int K, int C,
+                                                            int k_pad, int rot180) {
+    const H3Layout at(K, C);
+    uint8_t* const exps = (uint8_t*)(u + at.exps);
+    int* const part = (int*)(u + at.part);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (!rot180) {                                     // a wave per output channel, one slice
+    auto exponent = [](float m) { return m > 0.f ? max((int)(__builtin_bit_cast(uint32_t, m) >> 23), 1) : 0; };
+    if (!rot180) {                                     // a wave per output channel, lanes along the input channels
         const int k = blockIdx.x * 4 + wave;
         if (k >= k_pad) return;
-        float m = 0.f;
+        int top = 0;
         if (k < K) {
             const float* row = w + (size_t)k * 9 * C;
-#pragma unroll 8
-            for (int i = lane; i < 9 * C; i += 64) m = fmaxf(m, fabsf(row[i]));
+            for (int c = lane; c < C; c += 64) {
+                float m = 0.f;
+#pragma unroll
+                for (int t = 0; t < 9; ++t) m = fmaxf(m, fabsf(row[(size_t)t * C + c]));
+                const int e = exponent(m);
+                exps[(size_t)k * C + c] = (uint8_t)e;
+                top = max(top, e);
+            }
         }
 #pragma unroll
-        for (int d = 32; d; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
-        if (lane == 0) part[k] = __builtin_bit_cast(uint32_t, m);
+        for (int d = 32; d; d >>= 1) top = max(top, __shfl_xor(top, d));
+        if (lane == 0) part[k] = top;
         return;
     }
-    __shared__ float red[256];
+    // lanes along the output channels, 16 input channels per block
+    __shared__ int red[256];
     const int k = blockIdx.x * 64 + lane, slice = blockIdx.y;
-    const int rows = 9 * C, per = (rows + slices - 1) / slices, r1 = min(rows, (slice + 1) * per);
-    float m = 0.f;
-    if (k < K)
-#pragma unroll 8
-        for (int r = slice * per + wave; r < r1; r += 4) m = fmaxf(m, fabsf(w[(size_t)r * K + k]));
-    red[threadIdx.x] = m;
+    int top = 0;
+    if (k < K) {
+        uint32_t packed = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float m = 0.f;
+#pragma unroll
+            for (int t = 0; t < 9; ++t) m = fmaxf(m, fabsf(w[((size_t)(slice * H3_CC + wave * 4 + i) * 9 + t) * K + k]));
+            const int e = exponent(m);
+            packed |= (uint32_t)e << (8 * i);
+            top = max(top, e);
+        }
+        *(uint32_t*)(exps + (size_t)k * C + slice * H3_CC + wave * 4) = packed;
+    }
+    red[threadIdx.x] = top;
     __syncthreads();
     if (wave == 0 && k < k_pad)
-        part[(size_t)slice * k_pad + k] =
-            __builtin_bit_cast(uint32_t, fmaxf(fmaxf(red[lane], red[64 + lane]), fmaxf(red[128 + lane], red[192 + lane])));
+        part[(size_t)slice * k_pad + k] = max(max(red[lane], red[64 + lane]), max(red[128 + lane], red[192 + lane]));
 }
 
 // U = G g G^T, scaled and split, in the order in which a wave consumes it:
-// [k / 64][c / 16][position][(k % 64) / 32][term][(c % 16) / 8][k % 32][c % 8].  Rows k >= K are zero.  Behind them
-// the fields of the channels' scales, [k_pad] ints.  A thread transforms one output channel and two consecutive input
-// channels; four neighbouring threads share a lane's 16 bytes.
+// [k / 64][c / 16][position][(k % 64) / 32][term][(c % 16) / 8][k % 32][c % 8].  Rows k >= K are zero.  A block makes
+// 32 output x 16 input channels; a thread transforms one output channel and two consecutive input channels, four
+// neighbouring threads share a lane's 16 bytes.  If the block holds a kernel that two terms do not hold (head of this
+// file; P is `range`), its U goes out in fp32, unscaled: the first four of a lane's eight channels in place of the first
+// terms, the others in place of the second ones.
 __global__ __launch_bounds__(256) void winograd_filter_f16x3_kernel(const float* __restrict__ w, char* __restrict__ u,
-                                                                    const uint32_t* __restrict__ part, int slices,
-                                                                    int* __restrict__ fields, int K, int C, int k_pad,
-                                                                    int rot180) {
+                                                                    int slices, int K, int C, int k_pad, int rot180,
+                                                                    int range) {
+    __shared__ int top_of[256];
+    __shared__ int s_part[4][H3_CC];
+    const H3Layout at(K, C);
+    const uint8_t* const exps = (const uint8_t*)(u + at.exps);
+    const int* const part = (const int*)(u + at.part);
     const int n_chunks = C / H3_CC;
     const int kb = blockIdx.y, chunk = blockIdx.x >> 1, kh = blockIdx.x & 1;
     const int tid = threadIdx.x;
     // the fast thread index runs along the contiguous index of w: input channels, or (rot180) output channels
     const int cp = rot180 ? tid >> 5 : tid & 7, k32 = rot180 ? tid & 31 : tid >> 3;
     const int k = kb * WG_BN + kh * 32 + k32, c0 = chunk * H3_CC + cp * 2;
-    uint32_t m = 0;
-    for (int s = 0; s < slices; ++s) m = max(m, part[(size_t)s * k_pad + k]);
-    const int field = max((int)(m >> 23), H3_MIN_FIELD);
-    if (chunk == 0 && cp == 0) fields[k] = field;
-    const float scale = h3_scale(field, 130);
+
+    // (the kernel's nine taps and R(k) are requested first: what follows waits for memory twice per 256 output channels)
     float g[3][3][2];
 #pragma unroll
     for (int r = 0; r < 3; ++r)
 #pragma unroll
         for (int s = 0; s < 3; ++s)
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                float v = 0.f;
-                if (k < K)
-                    v = rot180 ? w[((size_t)(c0 + e) * 9 + (2 - r) * 3 + (2 - s)) * K + k]
-                               : w[((size_t)k * 9 + r * 3 + s) * C + c0 + e];
-                g[r][s][e] = v * scale;
-            }
+            for (int e = 0; e < 2; ++e)
+                g[r][s][e] = k >= K ? 0.f : rot180 ? w[((size_t)(c0 + e) * 9 + (2 - r) * 3 + (2 - s)) * K + k]
+                                                   : w[((size_t)k * 9 + r * 3 + s) * C + c0 + e];
+    int top = 0;
+#pragma unroll 16
+    for (int sl = 0; sl < slices; ++sl) top = max(top, part[(size_t)sl * k_pad + k]);
+
+    // s(c) of the block's 16 channels, over all k in batches of 256: thread (k modulo 16, c)
+    constexpr int NONE = -1000;
+    int s_max = NONE;
+    for (int k0 = 0; k0 < K; k0 += 256) {
+        int e[16], row_top = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int kk = k0 + (tid >> 4) + 16 * i;
+            e[i] = kk < K ? exps[(size_t)kk * C + chunk * H3_CC + (tid & 15)] : 0;
+        }
+        if (k0 + tid < k_pad)
+#pragma unroll 16
+            for (int sl = 0; sl < slices; ++sl) row_top = max(row_top, part[(size_t)sl * k_pad + k0 + tid]);
+        __syncthreads();
+        top_of[tid] = row_top;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (e[i]) s_max = max(s_max, e[i] - top_of[(tid >> 4) + 16 * i]);
+    }
+    s_max = max(s_max, __shfl_xor(s_max, 16));
+    s_max = max(s_max, __shfl_xor(s_max, 32));
+    if ((tid & 63) < H3_CC) s_part[tid >> 6][tid & 15] = s_max;
+    __syncthreads();
+    int shift[2];
+    bool wide = top == 255;                                        // infinities
+    const int field = top ? top : 127;                             // (a row of zeros)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int c = cp * 2 + e;
+        const int s = max(max(s_part[0][c], s_part[1][c]), max(s_part[2][c], s_part[3][c]));
+        wide |= s != NONE && s < H3_MIN_SHIFT;
+        shift[e] = max(s, H3_MIN_SHIFT);
+        wide |= field + shift[e] < 13;                             // (the factor must stay finite)
+        if (top && s != NONE) {
+            const int own = exps[(size_t)k * C + c0 + e];
+            wide |= own == 0 || own - top - s < -range;
+        }
+    }
+    if (chunk == 0 && cp == 0) ((int*)(u + at.fields))[k] = field;
+    if (kb == 0 && kh == 0 && k32 == 0) {
+        ((int*)(u + at.shifts))[c0] = shift[0];
+        ((int*)(u + at.shifts))[c0 + 1] = shift[1];
+    }
+    wide = __syncthreads_or(wide);
+    if (tid == 0) ((int*)(u + at.wide))[(kb * n_chunks + chunk) * 2 + kh] = wide;
+    const float scale[2] = {wide ? 1.f : h3_scale(field + shift[0], H3_W_BASE),
+                            wide ? 1.f : h3_scale(field + shift[1], H3_W_BASE)};
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) g[r][s][e] *= scale[e];
     float t[4][3][2];
 #pragma unroll
     for (int s = 0; s < 3; ++s)
@@ -168,6 +281,12 @@ __global__ __launch_bounds__(256) void winograd_filter_f16x3_kernel(const float*
             for (int e = 0; e < 2; ++e)
                 o[e] = j == 0 ? t[i][0][e] : j == 3 ? t[i][2][e]
                               : 0.5f * (j == 1 ? t[i][0][e] + t[i][1][e] + t[i][2][e] : t[i][0][e] - t[i][1][e] + t[i][2][e]);
+            if (wide) {
+                char* to = u + (size_t)(kb * n_chunks + chunk) * H3_U_CHUNK + kh * (2 * H3_FRAG) + (cp >> 2) * 512 + k32 * 16 +
+                           (size_t)(i * 4 + j) * (4 * H3_FRAG) + ((cp >> 1) & 1) * H3_FRAG + (cp & 1) * 8;
+                *(float2_t*)to = float2_t{o[0], o[1]};
+                continue;
+            }
             const uint32_t p = h3_pack(o[0], o[1]);
             float r0 = h3_rest_lo(p, o[0]), r1 = h3_rest_hi(p, o[1]);
             if ((p & 0x7c00u) == 0x7c00u) r0 = 0.f;                // infinities and NaNs stand in the first term alone
@@ -203,6 +322,9 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
 
     int* const exps = (int*)(lds + H3_EXP_OFF);
     int* const flag = (int*)(lds + H3_FLAG_OFF);
+    uint32_t* const wide = (uint32_t*)(lds + H3_WIDE_OFF);
+    const H3Layout at(a.K, a.C);
+    const char* const u = (const char*)a.u;
 
     // ---- the block's items i .. i + H3_ITEMS - 1 lie decoded in a ring in LDS: the divisions are done by eight lanes for
     //      eight items at a time, instead of by everybody wherever an item begins.  Image, channel block, and first
@@ -292,6 +414,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
     const int tseg = SEG == 1 ? 0 : tx / (8 / SEG);
     const int src_tile = H3_RAW_OFF + ch8 * RAW_HALF + (2 * wave * 2 * P + tx + tseg) * 32 + (lane & 3) * 8;
     const int zeros = H3_ZERO_OFF + (lane & 3) * 8;
+    const int v_dst = (wave >> 2) * H3_FRAG + ch8 * 512 + ((wave & 3) * 8 + tx) * 16 + (lane & 3) * 4;
     const char* row0 = lds + src_tile;                             // patch rows 0 and 3: zeros at an image's edge
     const char* row3 = lds + src_tile + 3 * (2 * P * 32);
     auto set_patch_rows = [&](int i) {
@@ -302,38 +425,65 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
     };
     int p_i = 0, p_cc = 0;                                         // item and chunk of the next patch
     int field = H3_MIN_FIELD;                                      // scale of the tile
+    int inner = 0;                                                 // field of its inner pixels, all chunks of the item
+    int shift[2];                                                  // s(c) of the thread's two channels of the next patch
+    auto load_shift = [&]() {
+        typedef int int2_t __attribute__((ext_vector_type(2)));
+        const int2_t v = *(const int2_t*)(u + at.shifts + (size_t)(p_cc * H3_CC + ch8 * 8 + (lane & 3) * 2) * 4);
+        shift[0] = v[0];
+        shift[1] = v[1];
+    };
     float2_t d[4][4];                                              // patch, then B^T d
     auto read_patch_row = [&](int r) {
         const char* src = r == 0 ? row0 : r == 3 ? row3 : lds + src_tile + r * (2 * P * 32);
 #pragma unroll
         for (int s = 0; s < 4; ++s) d[r][s] = *(const float2_t*)(src + (s & 1) * (P * 32) + (s >> 1) * 32);
     };
-    float amax;
-    auto patch_max = [&](int r) {
-        float m = r == 0 ? 0.f : amax;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) m = fmaxf(fmaxf(m, fabsf(d[r][s][0])), fabsf(d[r][s][1]));
-        amax = m;
+    float pmax[2], imax[2];                                        // per channel: all of the patch, its inner pixels
+    auto patch_max = [&](int e) {
+        auto abs = [&](int r, int s) { return fabsf(d[r][s][e]); };
+        float m;                                                   // (fmaxf of two would first quiet both)
+        asm("v_max_f32 %0, |%1|, |%2|" : "=v"(m) : "v"(d[1][1][e]), "v"(d[1][2][e]));
+        imax[e] = m = fmaxf(fmaxf(m, abs(2, 1)), abs(2, 2));
+        m = fmaxf(fmaxf(m, abs(0, 0)), abs(0, 1));
+        m = fmaxf(fmaxf(m, abs(0, 2)), abs(0, 3));
+        m = fmaxf(fmaxf(m, abs(1, 0)), abs(1, 3));
+        m = fmaxf(fmaxf(m, abs(2, 0)), abs(2, 3));
+        m = fmaxf(fmaxf(m, abs(3, 0)), abs(3, 1));
+        pmax[e] = fmaxf(fmaxf(m, abs(3, 2)), abs(3, 3));
     };
-    auto set_scale = [&](int parity) {                             // over the tile's lanes
-        float m = amax;
-        m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0xB1, 0xf, 0xf, true)));
-        m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0x4E, 0xf, 0xf, true)));
+    auto tile_max = [&](int m) {                                   // over the tile's lanes
+        m = max(m, __builtin_amdgcn_mov_dpp(m, 0xB1, 0xf, 0xf, true));
+        m = max(m, __builtin_amdgcn_mov_dpp(m, 0x4E, 0xf, 0xf, true));
         // (the copy is made opaque: of a swap of one value with itself the compiler takes both results for the same)
-        uint32_t mb = __builtin_bit_cast(uint32_t, m), copy = mb;
+        int copy = m;
         asm("" : "+v"(copy));
-        const auto sw = __builtin_amdgcn_permlane32_swap(mb, copy, false, false);
-        mb = max(sw[0], sw[1]);                                    // (never negative: ordered like the floats)
-        const int f = (int)(mb >> 23);
-        if (p_cc == 0) field = H3_MIN_FIELD;                       // a new work item
-        field = f > field + 8 ? f : field;
-        if (f == 255) *flag = 1;
-        if ((lane & 35) == 0) exps[parity * 64 + tt] = field;
+        const auto sw = __builtin_amdgcn_permlane32_swap((uint32_t)m, (uint32_t)copy, false, false);
+        return max((int)sw[0], (int)sw[1]);
+    };
+    auto set_scale = [&](int parity) {
+        auto exponent = [](float m) { return (int)(__builtin_bit_cast(uint32_t, m) >> 23); };
+        const int f = tile_max(max(exponent(pmax[0]) + shift[0], exponent(pmax[1]) + shift[1]));
+        const int here = max(exponent(imax[0]) + shift[0], exponent(imax[1]) + shift[1]);
+        // (a new work item starts anew: p_cc is uniform, these are scalars)
+        const int forget = p_cc ? 0 : 1000, slack = p_cc ? H3_SLACK : 0;
+        inner = max(inner - forget, here);
+        const int before = max(field - forget, H3_MIN_FIELD);
+        field = f > before + slack ? f : before;
+        int to = v_dst;                                            // (tt formed anew: kept, it would be spilled)
+        asm volatile("" : "+v"(to));
+        if ((lane & 35) == 0) *(int*)(lds + H3_EXP_OFF + parity * 256 + (to >> 2) - (wave >> 2) * 128) = field;
+    };
+    auto look_inside = [&]() {                                     // the tile's inner pixels, all chunks of the item seen
+        if (tile_max(inner) + H3_INNER < field && field > H3_MIN_FIELD) {
+            const Item* it = items + (p_i - 1) % H3_ITEMS;         // (tiles beyond the image have none)
+            if (it->pos[tseg][0] + 2 * wave < a.H && it->pos[tseg][1] + 2 * (tx - tseg * (8 / SEG)) < a.W) *flag = 1;
+        }
     };
     auto transform_col = [&](int s) {                              // column s of the patch -> column s of B^T d, scaled
-        const float sc = h3_scale(field, 129);
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
+            const float sc = h3_scale(field - shift[e], H3_X_BASE);
             const float s1 = d[1][s][e] * sc, s2 = d[2][s][e] * sc;
             const float t0 = fmaf(d[0][s][e], sc, -s2), t3 = fmaf(d[3][s][e], -sc, s1);
             d[0][s][e] = t0;
@@ -342,7 +492,6 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
             d[3][s][e] = t3;
         }
     };
-    const int v_dst = (wave >> 2) * H3_FRAG + ch8 * 512 + ((wave & 3) * 8 + tx) * 16 + (lane & 3) * 4;
     auto write_v = [&](int row, int m) {                           // position (row, m), split, into the slot of its row
         float v[2];
 #pragma unroll
@@ -394,7 +543,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         uint32_t iw[UNPOOL ? 4 : 1];
     };
     typedef int int4_t __attribute__((ext_vector_type(4)));
-    const int* const k_fields = (const int*)((const char*)a.u + (size_t)a.k_blocks * a.n_chunks * H3_U_CHUNK);
+    const int* const k_fields = (const int*)(u + at.fields);
     const uint32_t out_elems = (uint32_t)a.H * a.W * a.K;
     float4_t b4;                               // of the channels: bias (past K, or without one, 0), scales
     int4_t kf;
@@ -516,41 +665,60 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         }
     };
 
-    // ---- prologue: chunk 0 transformed (rows 0, 1 in slot 0, rows 2, 3 in registers), chunk 1 in LDS, chunk 2 requested
+    // (marks of filters that are not for f16: requested here, looked at behind the first item's loads)
+    const int n_marks = a.k_blocks * a.n_chunks * 2;
+    const int* const marks = (const int*)(u + at.wide);
+    const int mark = tid < n_marks ? marks[tid] : 0;
     if (tid < H3_ITEMS && tid < n_my) decode_item(tid);
-    __syncthreads();
-    set_load_item(0);
-    load_raw(0);
-    advance_l();
-    load_u(0);
-    load_u(1);
+    if (tid < H3_MAX_K_BLOCKS / 32) wide[tid] = 0;
     if (tid < 128) ((float*)(lds + H3_ZERO_OFF))[tid] = 0.f;
-    if (tid == 0) *flag = 0;
-    store_raw();
-    load_raw(l_cc);
-    advance_l();
-    set_patch_rows(0);
     __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 4; ++r) { read_patch_row(r); patch_max(r); }
-    set_scale(0);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) transform_col(s);
-    __syncthreads();                                               // every patch is read
-    store_raw();
-    load_raw(l_cc);
-    advance_l();
-#pragma unroll
-    for (int m = 0; m < 8; ++m) write_v(m >> 2, m & 3);
     auto advance_p = [&]() {
         if (++p_cc == a.n_chunks) {
             p_cc = 0;
             set_patch_rows(++p_i);
         }
     };
-    advance_p();
-    __syncthreads();
-    read_v(0, 0);
+    int q = 0;                                                     // chunk of the whole sequence
+    // ---- start of the sequence, at item i: chunk 0 transformed (rows 0, 1 in slot 0, rows 2, 3 in registers), chunk 1 in
+    //      LDS, chunk 2 requested
+    auto prime = [&](int i) {
+        l_i = i;
+        l_cc = 0;
+        set_load_item(i);
+        load_raw(0);
+        advance_l();
+        u_i = i;
+        u_cc = 0;
+        u_kb = __builtin_amdgcn_readfirstlane(items[i % H3_ITEMS].kb);
+        load_u(0);
+        load_u(1);
+        p_i = i;
+        p_cc = 0;
+        load_shift();
+        if (tid == 0) *flag = 0;
+        store_raw();
+        load_raw(l_cc);
+        advance_l();
+        set_patch_rows(i);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) read_patch_row(r);
+        patch_max(0);
+        patch_max(1);
+        set_scale(q & 1);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) transform_col(s);
+        __syncthreads();                                           // every patch is read
+        store_raw();
+        load_raw(l_cc);
+        advance_l();
+#pragma unroll
+        for (int m = 0; m < 8; ++m) write_v(m >> 2, m & 3);
+        advance_p();
+        __syncthreads();
+        read_v(0, 0);
+    };
 
     auto clear = [&]() {                                           // (by MFMAs: eight instructions instead of 64)
         const half8_t none = {};
@@ -560,15 +728,32 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
 #pragma unroll
             for (int t = 0; t < 2; ++t) acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(none, none, zero, 0, 0, 0);
     };
-    int q = 0;                                                     // chunk of the whole sequence
-    bool plain = false;                                            // an infinity was met: fp32 MFMAs from here on
+    bool primed = false;
+    int penalty = 1, wait = 0;                                     // items that stay on the fp32 MFMAs after one that had to
+    auto note = [&](int i) {
+        const int kb = i / (a.n_chunks * 2);
+        atomicOr(&wide[kb >> 5], 1u << (kb & 31));
+    };
     for (int m_i = 0; m_i < n_my; ++m_i) {
         const int kb = __builtin_amdgcn_readfirstlane(items[m_i % H3_ITEMS].kb);
+        bool plain = wait > 0 || (m_i > 0 && __builtin_amdgcn_readfirstlane(wide[kb >> 5]) >> (kb & 31) & 1);
+        if (wait > 0) --wait;
+        if (!plain && !primed) {
+            prime(m_i);
+            primed = true;
+            if (m_i == 0) {
+                if (mark) note(tid);
+                for (int i = tid + WG_THREADS; i < n_marks; i += WG_THREADS)
+                    if (marks[i]) note(i);
+                __syncthreads();
+                plain = __builtin_amdgcn_readfirstlane(wide[kb >> 5]) >> (kb & 31) & 1;
+            }
+        }
         if (!plain) {
         clear();
-        if (wave == 0 && k_fields[kb * WG_BN + lane] == 255) *flag = 1;
 #pragma unroll
         for (int t = 0; t < 2; ++t) cur[t] = exps[(q & 1) * 64 + t * 32 + (lane & 31)];
+        plain = __any(max(cur[0], cur[1]) > H3_MAX_FIELD);         // (all 64 tiles: the same in every wave)
         for (int m_cc = 0; m_cc < a.n_chunks; ++m_cc, ++q) {
             // the tiles' scales of this chunk: sums held at another scale are brought to it
             {
@@ -576,6 +761,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
 #pragma unroll
                 for (int t = 0; t < 2; ++t) now[t] = exps[(q & 1) * 64 + t * 32 + (lane & 31)];
                 if (__any(now[0] != cur[0] || now[1] != cur[1])) {
+                    plain |= __any(max(now[0], now[1]) > H3_MAX_FIELD) != 0;
 #pragma unroll
                     for (int t = 0; t < 2; ++t) {
                         const float f = h3_scale(max(min(now[t] - cur[t] + 127, 254), 0) , 127);   // 2^(cur - now)
@@ -587,6 +773,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
                     }
                 }
             }
+            if (p_cc == 0) look_inside();
             // Two steps of four sections (position row, tile half) of three MFMAs.  Every MFMA is followed by a piece of
             // the other work, which the scheduler may not move across.  The barrier of a step sits before its last
             // section: by then what the next step reads is in LDS, and that section's operands are in registers.
@@ -603,6 +790,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
                     if (S == 0) {
                         if (k < 8) write_v(2 + (k >> 2), k & 3);
                         if (k < 2) read_patch_row(k);                   // (into rows of B^T d that are used up)
+                        if (k == 2) load_shift();
                         if (k == 4) read_patch_row(2);
                         if (k == 7) read_patch_row(3);
                     } else {
@@ -616,10 +804,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
                         __syncthreads();
                         read_v(S ^ 1, 0);
                     }
-                    if (S == 0 && k >= 9) {
-                        patch_max(k - 9);
-                        if (k == 11) patch_max(3);
-                    }
+                    if (S == 0 && k >= 10) patch_max(k - 10);
                     if (k == 5) {                                  // (the first row's filter fragments: their last use was here)
                         if (S == 0) load_u(2);
                         else { advance_u(); load_u(0); }
@@ -633,22 +818,34 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
             advance_l();
             advance_p();
         }
-        plain = __builtin_amdgcn_readfirstlane(*flag) != 0;        // (not written between the last two barriers of an item)
+        plain |= __builtin_amdgcn_readfirstlane(*flag) != 0;       // (written before the last two barriers of the item)
+        wait = plain ? penalty : 0;
+        penalty = plain ? min(2 * penalty, 1 << 20) : 1;
         }
         if (plain) {
-            // Infinities cannot be split: this item and the block's later ones on the fp32 MFMAs, one chunk after the
-            // other: halo tile -> LDS, all of V in fp32 -> LDS ([position][tile half][c half][tile][8]), products with
-            // the filter put together from its two terms.
+            // The item on the fp32 MFMAs, one chunk after the other: halo tile -> LDS, all of V in fp32 -> LDS
+            // ([position][tile half][c half][tile][8]), products with the filter put together from its two terms or, where
+            // these do not hold it, as it is.  128 -> 128 channels at 112 x 112, 64 images, every filter of that kind: 1.09 ms,
+            // the fp32 kernel 0.88, the f16 MFMAs 0.55
+            primed = false;
             clear();
             set_load_item(m_i);
             set_patch_rows(m_i);
-            const int kshift = k_fields[kb * WG_BN + kh * 32 + (lane & 31)] - 130;
+            const int kfield = k_fields[kb * WG_BN + kh * 32 + (lane & 31)];
             char* const v32 = lds + H3_SLOT1_OFF;
+            u_kb = kb;
+            u_cc = 0;
+            load_raw(0);
+            load_u(0);
+            load_u(1);
 #pragma unroll 1
             for (int cc = 0; cc < a.n_chunks; ++cc) {
-                load_raw(cc);
                 store_raw();
                 __syncthreads();
+                const bool as_is = marks[(kb * a.n_chunks + cc) * 2 + kh] != 0;
+                const int4_t* const s8 = (const int4_t*)(u + at.shifts) + cc * 4 + (lane >> 5) * 2;
+                const int4_t s_lo = s8[0], s_hi = s8[1];
+                if (cc + 1 < a.n_chunks) load_raw(cc + 1);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) read_patch_row(r);
 #pragma unroll
@@ -670,21 +867,27 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
                     *(float2_t*)(to + (4 * r + 3) * 4096) = d[r][1] - d[r][3];
                 }
                 __syncthreads();
-                u_kb = kb;
-                u_cc = cc;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    load_u(r);
-                    float u[8];
+                    float w[8];
+                    if (as_is) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) u[e] = __builtin_ldexpf((float)uf[r & 1][0][e] + (float)uf[r & 1][1][e], kshift);
+                        for (int e = 0; e < 8; ++e) w[e] = __builtin_bit_cast(float4_t, uf[r & 1][e >> 2])[e & 3];
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            w[e] = __builtin_ldexpf((float)uf[r & 1][0][e] + (float)uf[r & 1][1][e],
+                                                    kfield + (e < 4 ? s_lo[e & 3] : s_hi[e & 3]) - H3_W_BASE);
+                    }
+                    if (r >= 2 && cc + 1 < a.n_chunks) u_cc = cc + 1;
+                    load_u(r ^ 2);
 #pragma unroll
                     for (int t = 0; t < 2; ++t) {
                         const float* src = (const float*)(v32 + (r * 4 + j) * 4096 + t * 2048 + (lane >> 5) * 1024 + (lane & 31) * 32);
                         const float4_t v0 = *(const float4_t*)src, v1 = *(const float4_t*)(src + 4);
 #pragma unroll
                         for (int e = 0; e < 8; ++e)
-                            acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(u[e], e < 4 ? v0[e & 3] : v1[e & 3], acc[r][t], 0, 0, 0);
+                            acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[e], e < 4 ? v0[e & 3] : v1[e & 3], acc[r][t], 0, 0, 0);
                     }
                 }
                 // (the next chunk's halo tile is written behind this one's patch reads: the barrier above; its V behind
@@ -734,9 +937,9 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
             }
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                const int shift = plain ? 0 : tf + kf[c] - 259;
+                const int exponent = plain ? 0 : tf + kf[c] - (H3_X_BASE + H3_W_BASE);
 #pragma unroll
-                for (int px = 0; px < 4; ++px) y[px][c] = __builtin_ldexpf(y[px][c], shift);
+                for (int px = 0; px < 4; ++px) y[px][c] = __builtin_ldexpf(y[px][c], exponent);
             }
             finish(o, k4, y);
             __syncthreads();
@@ -752,13 +955,16 @@ namespace {
 int h3_shape(const char* who, int C, int K) {
     PD_REQUIRE(C > 0 && K > 0 && C % H3_CC == 0 && K % 4 == 0, PD_ESHAPE, "%s: needs C %% 16 == 0 and K %% 4 == 0 (C=%d K=%d)",
                who, C, K);
-    PD_REQUIRE((long)((K + WG_BN - 1) / WG_BN) * (C / H3_CC) * H3_U_CHUNK < (1L << 31), PD_ESHAPE,
-               "%s: too many channels (C=%d K=%d)", who, C, K);
+    PD_REQUIRE(pd_conv3x3_winograd_f16x3_supported(C, K), PD_ESHAPE, "%s: too many channels (C=%d K=%d)", who, C, K);
     return PD_OK;
 }
 
-// slices of the filter's rows per output channel when the channel is the innermost index
-int h3_slices(int C, int rot180) { return rot180 ? (C >= 256 ? 32 : 16) : 1; }
+// P of the head of this file
+int h3_range(int C) {
+    int bits = 0;
+    while (1 << bits < C) ++bits;
+    return 13 - (bits + 1) / 2;
+}
 
 template <bool STACKED, int SEG>
 void h3_launch(const WinoArgs& a, dim3 grid, hipStream_t s) {
@@ -771,16 +977,15 @@ void h3_launch(const WinoArgs& a, dim3 grid, hipStream_t s) {
 
 extern "C" int pd_conv3x3_winograd_f16x3_supported(int C, int K) {
     return C > 0 && K > 0 && C % H3_CC == 0 && K % 4 == 0 &&
-           (long)((K + WG_BN - 1) / WG_BN) * (C / H3_CC) * H3_U_CHUNK < (1L << 31);
+           (long)((K + WG_BN - 1) / WG_BN) * (C / H3_CC) * H3_U_CHUNK < (1L << 31) &&
+           (K + WG_BN - 1) / WG_BN <= H3_MAX_K_BLOCKS;
 }
 
 extern "C" int pd_conv3x3_winograd_f16x3_filter_bytes(int C, int K, uint64_t* bytes) {
     const char* who = "pd_conv3x3_winograd_f16x3_filter_bytes";
     PD_REQUIRE(bytes != nullptr, PD_EINVAL, "%s: NULL pointer", who);
     if (int rc = h3_shape(who, C, K)) return rc;
-    const uint64_t k_blocks = (K + WG_BN - 1) / WG_BN;
-    // the fragments, the fields of the channels' scales, the partial maxima they come from
-    *bytes = k_blocks * (C / H3_CC) * H3_U_CHUNK + k_blocks * WG_BN * 4 * (1 + 32);
+    *bytes = H3Layout(K, C).bytes;
     return PD_OK;
 }
 
@@ -790,15 +995,13 @@ extern "C" int pd_conv3x3_winograd_f16x3_filter_f32(const float* w, void* u, int
     if (int rc = h3_shape(who, C, K)) return rc;
     PD_REQUIRE(pd_aligned(u, 16), PD_EINVAL, "%s: u must be 16-byte aligned", who);
     const int k_blocks = (K + WG_BN - 1) / WG_BN, k_pad = k_blocks * WG_BN, n_chunks = C / H3_CC;
-    int* fields = (int*)((char*)u + (size_t)k_blocks * n_chunks * H3_U_CHUNK);
-    uint32_t* part = (uint32_t*)(fields + k_pad);
-    const int slices = h3_slices(C, rot180);
+    const int slices = rot180 ? n_chunks : 1;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid = rot180 ? dim3(k_blocks, slices) : dim3(k_pad / 4);
-    winograd_amax_kernel<<<grid, 256, 0, s>>>(w, part, K, C, k_pad, rot180, slices);
+    const dim3 grid = rot180 ? dim3(k_blocks, n_chunks) : dim3(k_pad / 4);
+    winograd_exps_kernel<<<grid, 256, 0, s>>>(w, (char*)u, K, C, k_pad, rot180);
     PD_CHECK_LAUNCH(who);
-    winograd_filter_f16x3_kernel<<<dim3(n_chunks * 2, k_blocks), 256, 0, s>>>(w, (char*)u, part, slices, fields, K, C, k_pad,
-                                                                              rot180);
+    winograd_filter_f16x3_kernel<<<dim3(n_chunks * 2, k_blocks), 256, 0, s>>>(w, (char*)u, slices, K, C, k_pad, rot180,
+                                                                              h3_range(C));
     PD_CHECK_LAUNCH(who);
     return PD_OK;
 }

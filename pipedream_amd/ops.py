@@ -681,16 +681,14 @@ def _winograd_conv(x, w, bias, in_mask, out_mask, n, h, wd, c, k, relu, rot180):
 
 def _winograd_run(x, w, bias, in_mask, out_mask, y, y_pool, pool_idx, unpool_idx, y_full, n, h, wd, c, k, relu, rot180):
     """Filter transform and convolution into the outputs given.  The products run on the f16 matrix pipes where the
-    kernel for that takes the channel counts (16 | c, every layer of VGG16 but the first), else on the fp32 ones.
+    kernel for that takes the channel counts (16 | c >= 32, every layer of VGG16 but the first), else on the fp32 ones.
     conv1_1 .. pool2 of VGG16 as one stage, 64 images: 7.74 ms a step with the fp32 kernel, 6.07 with this one."""
     lib = _cabi.lib()
     stream = _cabi.stream_ptr()
     nbytes = ctypes.c_uint64()
-    # one chunk of 16 channels saves less than the launch for the filter's scales costs (3 us) unless every block has two
-    # work items (16 x 16 pixels x 64 channels) or more: 16 -> 32 channels, 8 images of 64 x 64: 15.6 us fp32, 18.1 f16;
-    # 64 images of 112 x 112: 104 and 85; 32 -> 32 channels there 153 and 110
-    split = (lib.pd_conv3x3_winograd_f16x3_supported(c, k)
-             and (c >= 32 or n * h * wd * ((k + 63) // 64) > 512 * 256))
+    # (16 channels: the split's own error shows, 1.65e-7 of the result against 1.59e-7 of the fp32 kernel; with 32 it is
+    # 1.80e-7 against 2.00e-7, with 512 4.5e-7 against 6.9e-7)
+    split = lib.pd_conv3x3_winograd_f16x3_supported(c, k) and c >= 32
     if split:
         lib.pd_conv3x3_winograd_f16x3_filter_bytes(c, k, ctypes.byref(nbytes))
         u = torch.empty(nbytes.value // 4, dtype=torch.float32, device=x.device)
