@@ -249,14 +249,19 @@ def _resolve_tie(nf, trace, s, k, W, product_grad_in, product_grads, masks_entry
 
             candidates.sort(key=lambda t: (distance(t) > 0.15, t.margin))
     # greedy: keep a switched decision when it takes away part of the disagreement (decisions in different
-    # places contribute independently), stop when nothing is left
-    switch = ()
-    for t in candidates[:max_trials]:
-        trial, trial_grads, _ = disagreement(switch + (t,))
-        if trial < 0.8 * err:
-            switch, err, grads = switch + (t,), trial, trial_grads
-            if err <= tol:
-                return switch, grads
+    # places contribute independently), stop when nothing is left; a small part shows only once a larger one is
+    # gone, so the candidates are gone through again as long as one is kept
+    switch, kept = (), True
+    while kept:
+        kept = False
+        for t in candidates[:max_trials]:
+            if t in switch:
+                continue
+            trial, trial_grads, _ = disagreement(switch + (t,))
+            if trial < 0.8 * err:
+                switch, err, grads, kept = switch + (t,), trial, trial_grads, True
+                if err <= tol:
+                    return switch, grads
     return None
 
 
