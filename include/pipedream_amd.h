@@ -234,9 +234,11 @@ int pd_conv3x3_winograd_set_pieces(int mode);
 /* Tuning and test hook for pd_conv3x3_winograd_wgrad_nhwc_f32.  Its blocks sum over strips of eight 2 x 2 tiles:
  * 2 x 16 pixels of one image, or, upright, 16 rows x 2 columns of the batch taken as one image of N * H rows
  * (H, W even, H >= 14), which leaves no padding columns at widths that are no multiple of 16.  mode 0 (default):
- * upright strips exactly where the width is no multiple of 16, and long reductions on the f16 matrix pipes (operands
- * split as in pd_conv3x3_winograd_f16x3_fwd_nhwc_f32) without strips; 1: never; 2: wherever the shape allows.  Results
- * differ by the summation order only.  Process-wide.  No counterpart in the reference. */
+ * upright strips exactly where the width is no multiple of 16, and reductions of 32 tiles a block and more on the f16
+ * matrix pipes (operands split as in pd_conv3x3_winograd_f16x3_fwd_nhwc_f32, with a scale per channel that follows the
+ * values, and fp32 products for 16 tiles at a time where a channel's values there are too far apart) without strips;
+ * 1: never; 2: wherever the shape allows.  Modes 1 and 2 differ by the summation order, mode 0 also by the split: its
+ * error against 64 bits is 0.6 to 1.0 times theirs.  Process-wide.  No counterpart in the reference. */
 int pd_conv3x3_winograd_set_wgrad_strips(int mode);
 
 /* The same convolution (and, with rot180, its input gradient) by the Winograd algorithm

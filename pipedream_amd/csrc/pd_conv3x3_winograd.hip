@@ -984,8 +984,6 @@ __global__ __launch_bounds__(WW_THREADS, 1) void winograd_wgrad_kernel(const Win
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // behind the f16 kernel: all of it again if any of its blocks met an infinity
-    if (a.failed && !__syncthreads_or(threadIdx.x < WW_BLOCKS && a.failed[threadIdx.x])) return;
     int pair, rank;
     wino_wgrad_pair_rank(a, pair, rank);
     const int kb = pair / a.c_blocks, cb = pair % a.c_blocks;
@@ -1408,8 +1406,8 @@ extern "C" int pd_conv3x3_winograd_wgrad_workspace_bytes(int C, int K, uint64_t*
                "pd_conv3x3_winograd_wgrad_workspace_bytes: needs C and K multiples of 64 with C*K/4096 a power "
                "of two <= 256 (C=%d K=%d)", C, K);
     const uint64_t pairs = (uint64_t)(C / 64) * (K / 64);
-    // per block: partial dU, 2 x 64 partial dbias and the mark of the f16 kernel; per pair and rank group: summed dU and dbias
-    *bytes = ((uint64_t)WW_BLOCKS * (WW_PART_STRIDE + 128) + WW_SUM_GROUPS * pairs * (WW_PART_FLOATS + 64) + WW_BLOCKS) * sizeof(float);
+    // per block: partial dU and 2 x 64 partial dbias; per pair and rank group: summed dU and dbias
+    *bytes = ((uint64_t)WW_BLOCKS * (WW_PART_STRIDE + 128) + WW_SUM_GROUPS * pairs * (WW_PART_FLOATS + 64)) * sizeof(float);
     return PD_OK;
 }
 
@@ -1453,16 +1451,14 @@ extern "C" int pd_conv3x3_winograd_wgrad_nhwc_f32(const float* x, const float* d
     float* du = a.part_db + (size_t)WW_BLOCKS * 128;
     float* dbsum = du + (size_t)WW_SUM_GROUPS * a.n_pairs * WW_PART_FLOATS;
     hipStream_t s = (hipStream_t)stream;
-    // The f16 kernel, where its blocks have at least one full step of 16 tiles (below, its error against 64 bits is up to
-    // 6 % above the fp32 kernel's, which decides nothing about time), x and dY lie within its offsets, and no strips are
-    // asked for.  What it cannot split (infinities) the fp32 kernel does behind it, whose blocks otherwise leave at once.
-    // 64 images, C = K: 64 at 224 x 224 1147 -> 773 us, 128 at 112 975 -> 620, 256 at 56 1013 -> 603, 512 at 28 1021 -> 587,
-    // 512 at 14 292 -> 198.
+    // The f16 kernel, where its blocks have at least two steps of 16 tiles (its error against 64 bits is 4 to 7 % above the
+    // fp32 kernel's at 18 to 25 tiles a block, 8 % below it at 38, 40 % at 3000), x and dY lie within its offsets, and no
+    // strips are asked for.
+    // 64 images, C = K: 64 at 224 x 224 1005 -> 728 us, 128 at 112 968 -> 612, 512 at 28 1020 -> 601, 512 at 14 291 -> 199.
     const long tiles = (long)N * ((H + 1) / 2) * ((W + 1) / 2);
-    const bool split = g_wgrad_strips == 0 && tiles >= 16L * a.ranks && (long)N * H * W * (C > K ? C : K) * 4 < (1L << 30);
-    a.failed = split ? (int*)(dbsum + (size_t)WW_SUM_GROUPS * a.n_pairs * 64) : nullptr;
+    const bool split = g_wgrad_strips == 0 && tiles >= 32L * a.ranks && (long)N * H * W * (C > K ? C : K) * 4 < (1L << 30);
     if (split) pd_wino_wgrad_f16x3(a, s);
-    if (upright) winograd_wgrad_kernel<true><<<WW_BLOCKS, WW_THREADS, 0, s>>>(a);
+    else if (upright) winograd_wgrad_kernel<true><<<WW_BLOCKS, WW_THREADS, 0, s>>>(a);
     else winograd_wgrad_kernel<false><<<WW_BLOCKS, WW_THREADS, 0, s>>>(a);
     PD_CHECK_LAUNCH(who);
     const long sum_threads = (long)a.n_pairs * (WW_PART_FLOATS / 4);

@@ -94,7 +94,6 @@ struct WinoWgradArgs {
     int n_strips, strips_per_rank;
     int rows_all;        // upright strips: N * H, the rows of the batch taken as one tall image
     int c_blocks, n_pairs, ranks;
-    int* failed;         // [WW_BLOCKS], written by the f16 kernel: the block met an infinity; or null
 };
 // block -> (pair, rank): the 32 blocks of a die cover all pairs of a contiguous range of ranks, so that the pairs that
 // read the same x and dY run side by side on one L2
@@ -108,5 +107,5 @@ __device__ __forceinline__ void wino_wgrad_pair_rank(const WinoWgradArgs& a, int
         rank = blockIdx.x / a.n_pairs;
     }
 }
-// The f16 kernel: writes a.part, a.part_db and a.failed.
+// The f16 kernel: writes a.part and a.part_db.
 void pd_wino_wgrad_f16x3(const WinoWgradArgs& a, hipStream_t s);

@@ -818,3 +818,90 @@ def test_split_f16_weight_gradient_of_infinities(value, conv_algorithm):
     assert not torch.isfinite(dw[:, 5]).any()
     rest = [c for c in range(64) if c != 5]
     torch.testing.assert_close(dw[:, rest], clean[:, rest], rtol=1e-4, atol=1e-4)     # (sums of 3200 products: 57 typically)
+
+
+def _exact_weight_grad(x, dy):
+    N, C, H, W = x.shape
+    padded, rows = F.pad(x.double(), (1, 1, 1, 1)), dy.double().permute(1, 0, 2, 3).reshape(dy.size(1), -1)
+    return torch.stack([rows @ padded[:, :, r:r + H, s:s + W].permute(0, 2, 3, 1).reshape(-1, C)
+                        for r in range(3) for s in range(3)])      # [tap, K, C]
+
+
+def _fp32_weight_grad(x, dy):
+    ops.set_conv_wgrad_strips("flat")
+    try:
+        return ops.conv3x3_weight_grad(x, dy)
+    finally:
+        ops.set_conv_wgrad_strips("auto")
+
+
+# (all reach the f16 kernel, which needs 32 tiles per block: one pair of channel blocks, 256 blocks; 8 pairs, odd sizes,
+# units that end beyond the image; 64 pairs, blocks of three steps; blocks without a step)
+@pytest.mark.parametrize("N,C,K,H,W", [(11, 64, 64, 56, 56), (4, 128, 256, 33, 35), (3, 512, 512, 14, 14), (1, 256, 256, 66, 32)])
+@pytest.mark.parametrize("spread", ["plain", "x channels", "dy channels", "both", "outlier in x", "outlier in dy", "images",
+                                    "rows", "huge"])
+def test_split_f16_weight_gradient_keeps_small_values(N, C, K, H, W, spread, conv_algorithm):
+    """The gradient of a channel does not depend on how large its neighbours are, nor the contribution of a pixel on
+    pixels that contribute nothing: errors per input channel and per output channel are those of the fp32 kernel (1.1 on
+    average and 1.6 for a single channel: two samples of the same rounding)."""
+    if conv_algorithm != "winograd":
+        pytest.skip("the Winograd kernel's")
+    g = torch.Generator("cuda").manual_seed(N + C + H)
+    x = torch.randn(N, C, H, W, generator=g, device="cuda").relu_()
+    dy = torch.randn(N, K, H, W, generator=g, device="cuda") * 1e-3
+    dy = dy * (torch.rand(N, K, H, W, generator=g, device="cuda") < 0.5)
+    octaves = lambda n: torch.randint(-30, 31, (n, 1, 1), generator=g, device="cuda").float().exp2()
+    if spread in ("x channels", "both"):
+        x = x * octaves(C)
+    if spread in ("dy channels", "both"):
+        dy = dy * octaves(K)
+    if spread == "outlier in x":                           # seen by no output with a gradient
+        x[N // 2, :, 9, 7] = 2.0 ** 28
+        dy[N // 2, :, 8:11, 6:9] = 0
+    if spread == "outlier in dy":
+        dy[N // 2, :, 9, 7] = 2.0 ** 18
+        x[N // 2, :, 8:11, 6:9] = 0
+    if spread == "images":                                 # half of the rows far above the others, with no gradient in odd k
+        x[:, :, : H // 2] *= 2.0 ** 26
+        dy[:, 1::2, : H // 2 + 1] = 0
+    if spread == "rows":                                   # from one row of pixels to the next
+        x = x * (torch.arange(H, device="cuda") % 5 * 6.0).exp2()[:, None]
+        dy = dy * (-(torch.arange(H, device="cuda") % 5) * 6.0).exp2()[:, None]
+    if spread == "huge":
+        x = x * 2.0 ** 42
+    x, dy = (t.contiguous(memory_format=torch.channels_last) for t in (x, dy))
+    dw, db = ops.conv3x3_weight_grad(x, dy)
+    fp32, _ = _fp32_weight_grad(x, dy)
+    assert spread != "plain" or not torch.equal(dw, fp32)  # (it is the other kernel)
+    want = _exact_weight_grad(x, dy)
+    errors = [t.double().permute(2, 3, 0, 1).reshape(9, K, C) - want for t in (dw, fp32)]
+    parts = [slice(0, None, 2), slice(1, None, 2)]         # k
+    for part in parts:
+        for dims in ((0, 1), (0, 2)):                      # per input channel, per output channel
+            got, allowed = ((e[:, part] / want[:, part].pow(2).sum(0 if dims == (0, 2) else (0, 2), keepdim=True).sqrt().clamp_min(1e-300)
+                             ).pow(2).sum(dims).sqrt() for e in errors)
+            assert got.mean() <= 1.1 * allowed.mean(), (dims, got.mean(), allowed.mean())
+            assert (got <= 1.6 * allowed).all(), (dims, (got / allowed).max())
+    torch.testing.assert_close(db.double(), dy.double().sum((0, 2, 3)), rtol=1e-5, atol=float(dy.abs().max()) * 1e-5)
+    assert torch.equal(dw, ops.conv3x3_weight_grad(x, dy)[0])
+
+
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan")])
+@pytest.mark.parametrize("where", ["x", "dy"])
+@pytest.mark.parametrize("N,C,K,H,W", [(11, 64, 64, 56, 56), (4, 128, 256, 33, 35)])
+def test_split_f16_weight_gradient_of_infinities_and_nans(value, where, N, C, K, H, W, conv_algorithm):
+    """As the fp32 kernel: the channel of the infinity has no finite element, the others are as without it."""
+    if conv_algorithm != "winograd":
+        pytest.skip("the Winograd kernel's")
+    g = torch.Generator("cuda").manual_seed(5)
+    x = torch.randn(N, C, H, W, generator=g, device="cuda").contiguous(memory_format=torch.channels_last)
+    dy = torch.randn(N, K, H, W, generator=g, device="cuda").contiguous(memory_format=torch.channels_last)
+    clean = ops.conv3x3_weight_grad(x, dy)[0]
+    (x if where == "x" else dy)[1, 5, 7, 9] = value
+    dw, fp32 = ops.conv3x3_weight_grad(x, dy)[0], _fp32_weight_grad(x, dy)[0]
+    assert torch.equal(torch.isfinite(dw), torch.isfinite(fp32)) and not torch.equal(dw, fp32)
+    hit = dw[:, 5] if where == "x" else dw[5]
+    assert not torch.isfinite(hit).any()
+    rest = torch.isfinite(dw)
+    assert int(rest.sum()) == dw.numel() - hit.numel()
+    torch.testing.assert_close(dw[rest], clean[rest], rtol=1e-4, atol=1e-4 * (N * H * W / 3200) ** 0.5)
