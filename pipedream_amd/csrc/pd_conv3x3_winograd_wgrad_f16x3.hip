@@ -225,8 +225,11 @@ __global__ __launch_bounds__(WW_THREADS, 1) void winograd_wgrad_f16x3_kernel(con
 
     // Odd ranks sum up -dU.  The f16 MFMA rounds its sums towards minus infinity, and half an ulp of the same sign in each
     // of 600 additions and 256 blocks adds up where G^T . G only adds (tap 0, 0: an error of 6.9e-6 of the gradient over
-    // 64 images of 224 x 224, against 2.0e-6 of the fp32 kernel).
-    const float sign = rank & 1 ? -1.f : 1.f;
+    // 64 images of 224 x 224, against 2.0e-6 of the fp32 kernel).  A rank that is alone changes the sign every 32 steps
+    // (1024 -> 1024 channels, 64 images of 14 x 14: mean error of tap 0, 0 4.4e-7 of the gradient's size without it).
+    constexpr int TURN = 32;
+    float sign = rank & 1 ? -1.f : 1.f;
+    bool turned = false;                               // the step in the registers has the other sign than the sums
 
     // ---- transforms.  v: rows of B^T d of the two tiles (six columns); m: the columns of A dY (rows d0, d0 + d1,
     //      d0 - d1, d1; the signs of A's last row and column are left to the kernel behind this one)
@@ -343,6 +346,16 @@ __global__ __launch_bounds__(WW_THREADS, 1) void winograd_wgrad_f16x3_kernel(con
                 }
             moved = false;
         }
+        if (turned) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[s][i][j][e] = -acc[s][i][j][e];
+        }
         if (plain) {
             // fp32 MFMAs on the operands as they are, [position][V, dM][tile][channel] over both slots; the f16 MFMAs below
             // then have zeros to add (1.8 ms instead of 0.6 if every step is of this kind, the fp32
@@ -400,7 +413,12 @@ __global__ __launch_bounds__(WW_THREADS, 1) void winograd_wgrad_f16x3_kernel(con
                     if (k < 8) { write_v(2 + (k >> 2), k & 3); write_m(2 + (k >> 2), k & 3); }
                     if (k == 8) check();
                 } else {
-                    if (k == 0) { set_scales(); take(); }
+                    if (k == 0) {
+                        set_scales();
+                        turned = a.ranks == 1 && (q + 1) % TURN == 0 && q + 1 < n_steps;
+                        if (turned) sign = -sign;
+                        take();
+                    }
                     if (k == 1) load_rows();
                     if (k >= 1 && k < 9) load_part(k - 1);
                     if (k == 9) next_unit();

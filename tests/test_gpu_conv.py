@@ -905,3 +905,23 @@ def test_split_f16_weight_gradient_of_infinities_and_nans(value, where, N, C, K,
     rest = torch.isfinite(dw)
     assert int(rest.sum()) == dw.numel() - hit.numel()
     torch.testing.assert_close(dw[rest], clean[rest], rtol=1e-4, atol=1e-4 * (N * H * W / 3200) ** 0.5)
+
+
+@pytest.mark.parametrize("N,C,K,H,W", [(64, 1024, 1024, 14, 14), (32, 512, 2048, 14, 14)])
+def test_split_f16_weight_gradient_of_one_block_per_pair_has_no_bias(N, C, K, H, W, conv_algorithm):
+    """256 pairs of channel blocks: one block sums up all tiles of a pair, and there is no other whose sums are rounded
+    the other way.  The f16 MFMA rounds towards minus infinity: the mean error per tap must stay at what random rounding
+    leaves (the mean of C K / 9 errors; 2^-24 of a gradient's size is far above it and far below a bias of half an ulp in
+    each of 100 and more additions), and the error at that of the fp32 kernel."""
+    if conv_algorithm != "winograd":
+        pytest.skip("the Winograd kernel's")
+    g = torch.Generator("cuda").manual_seed(1)
+    x = torch.randn(N, C, H, W, generator=g, device="cuda").relu_().contiguous(memory_format=torch.channels_last)
+    dy = torch.randn(N, K, H, W, generator=g, device="cuda").contiguous(memory_format=torch.channels_last)
+    want = _exact_weight_grad(x, dy)
+    got, fp32 = (t[0].double().permute(2, 3, 0, 1).reshape(9, K, C) - want
+                 for t in (ops.conv3x3_weight_grad(x, dy), _fp32_weight_grad(x, dy)))
+    size = want.pow(2).mean((1, 2)).sqrt()
+    bias = (got.mean((1, 2)) / size).abs()
+    assert (bias <= 2.0 ** -24).all(), bias
+    assert (got.pow(2).mean((1, 2)) <= fp32.pow(2).mean((1, 2))).all(), got.pow(2).mean((1, 2)) / fp32.pow(2).mean((1, 2))
