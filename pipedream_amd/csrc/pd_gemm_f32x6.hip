@@ -302,13 +302,14 @@ __global__ __launch_bounds__(X_THREADS, 2) void pd_gemm_f32x6_kernel(const GemmX
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     acc[ti][tj][e] += low[ti][tj][e];
-                    bad |= acc[ti][tj][e] != acc[ti][tj][e];
+                    bad |= !(__builtin_fabsf(acc[ti][tj][e]) <= 3.4028235e38f);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
         if (__any(bad)) {
-            // Infinities and values that round to infinity in bf16 leave NaNs (inf - inf in the split): a wave that
-            // holds one computes its part again with fp32 MFMAs straight from memory, which gives what fp32 gives.
+            // Infinities and values that round to infinity in bf16 leave NaNs (inf - inf in the split), and the product of
+            // two leading terms, both rounded up, may overflow where the product itself does not: a wave that holds a NaN or
+            // an infinity computes its part again with fp32 MFMAs straight from memory, which gives what fp32 gives.
             const int k_end = min(a.K, it.k0 + a.k_per_split);
             clear();
             for (int k = it.k0; k < k_end; k += 2) {

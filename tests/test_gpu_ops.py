@@ -429,3 +429,23 @@ def test_gemm_f32x6_infinities_nans_and_values_that_round_to_infinity():
             ops.set_gemm_f32_algorithm("auto")
     assert bool(torch.isinf(outs["mfma_f32"]).any()) and bool(torch.isnan(outs["mfma_f32"]).any())
     torch.testing.assert_close(outs["split_bf16"], outs["mfma_f32"], rtol=1e-5, atol=1e-4, equal_nan=True)
+
+
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_gemm_f32x6_products_next_to_the_largest_float(trans_a, splits):
+    """a b = 3.3995e38 fits fp32; the product of the leading terms, both rounded up, does not.  The result is that of the
+    fp32 MFMA kernel, and so is a true overflow's."""
+    M, N, K = 256, 132, 128
+    a, b = torch.zeros(M, K), torch.zeros(K, N)
+    a[3, 5] = a[200, 70] = b[5, 7] = b[70, 100] = 1.99902 * 2.0 ** 63
+    a[40, 9], b[9, 9] = 2.0 ** 65, -2.0 ** 65
+    want = a.double() @ b.double()
+    a, b = (a.t() if trans_a else a).contiguous().cuda(), b.cuda()
+    out, part = torch.empty(M, N).cuda(), torch.empty(splits, M, N).cuda()
+    _cabi.lib().pd_gemm_f32x6(int(trans_a), 0, M, N, K, ops._ptr(a), a.stride(0), ops._ptr(b), b.stride(0), 0.0,
+                              ops._ptr(out), N, None, splits, ops._ptr(part), _cabi.stream_ptr())
+    assert int(torch.isinf(out).sum()) == 1 and float(out[40, 9]) == -float("inf")
+    want[40, 9], out[40, 9] = 0.0, 0.0
+    assert float(want.abs().max()) > 3.3e38
+    torch.testing.assert_close(out.cpu().double(), want, rtol=1e-6, atol=0.0)
