@@ -392,9 +392,9 @@ int pd_gemm_bf16_set_tile(int bm, int bn);
 
 /* The product of pd_gemm_f32 (same operands and layout flags, no ReLU) on the bf16 matrix pipes: the operands are
  * split into three bf16 terms each as they enter the kernel, six bf16 MFMAs stand for one fp32 MFMA, accumulation is
- * fp32.  At least as close to the exact product as the fp32 MFMA kernel, infinities and NaNs included.  
+ * fp32.  At least as close to the exact product as the fp32 MFMA kernel, infinities and NaNs included.
  * splits > 1: the reduction is cut into that many ranges, whose partial products go to partials[splits][M][N]
- * (16-byte aligned, N and ldc multiples of 4) and are added in index order.
+ * (partials, C and bias 16-byte aligned, N and ldc multiples of 4) and are added in index order.
  * An operand whose rows hold the reduction index (A not transposed, B transposed) must be 16-byte aligned with K and
  * its leading dimension multiples of 4. */
 int pd_gemm_f32x6(int trans_a, int trans_b, int M, int N, int K, const float* A, int lda, const float* B, int ldb,

@@ -385,8 +385,8 @@ extern "C" int pd_gemm_f32x6(int trans_a, int trans_b, int M, int N, int K, cons
     g.chunks = g.k_per_split / XK;
     splits = (K + g.k_per_split - 1) / g.k_per_split;       // (no empty range)
     if (splits > 1) {
-        PD_REQUIRE(N % 4 == 0 && ldc % 4 == 0 && pd_aligned(partials, 16) && pd_aligned(C, 16), PD_EINVAL,
-                   "pd_gemm_f32x6: a split reduction needs N and ldc multiples of 4 and aligned results");
+        PD_REQUIRE(N % 4 == 0 && ldc % 4 == 0 && pd_aligned(partials, 16) && pd_aligned(C, 16) && pd_aligned(bias, 16), PD_EINVAL,
+                   "pd_gemm_f32x6: a split reduction needs N and ldc multiples of 4, aligned results and an aligned bias");
         g.C = partials; g.ldc = N; g.bias = nullptr; g.beta = 0.f; g.c_split = (long long)M * N;
     } else {
         g.C = C; g.ldc = ldc; g.bias = bias; g.beta = beta; g.c_split = 0;

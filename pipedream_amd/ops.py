@@ -89,7 +89,9 @@ def gemm(a, b, trans_a=False, trans_b=False, bias=None, relu=False, out=None, be
     ldb = b.stride(0) if b.size(0) > 1 else b.size(1)
     ldc = out.stride(0) if out.size(0) > 1 else out.size(1)
     if _use_x6(M, N, K, trans_a, trans_b, relu, a, b, out, lda, ldb, ldc):
-        splits = _x6_splits(M, N, K, out.data_ptr() % 16 == 0 and ldc % 4 == 0)
+        # (the kernel that adds up the ranges reads out and bias 16 bytes at a time)
+        splits = _x6_splits(M, N, K, out.data_ptr() % 16 == 0 and ldc % 4 == 0 and
+                            (bias is None or bias.data_ptr() % 16 == 0))
         part = torch.empty((splits, M, N), dtype=torch.float32, device=a.device) if splits > 1 else None
         with _timed("gemm_f32_as_bf16x6", 2.0 * M * N * K):
             _cabi.lib().pd_gemm_f32x6(int(trans_a), int(trans_b), M, N, K, _ptr(a), lda, _ptr(b), ldb, float(beta),

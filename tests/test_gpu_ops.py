@@ -449,3 +449,24 @@ def test_gemm_f32x6_products_next_to_the_largest_float(trans_a, splits):
     want[40, 9], out[40, 9] = 0.0, 0.0
     assert float(want.abs().max()) > 3.3e38
     torch.testing.assert_close(out.cpu().double(), want, rtol=1e-6, atol=0.0)
+
+
+def test_gemm_with_a_bias_that_is_not_aligned():
+    """A contiguous view one element into a buffer, with a product whose reduction is split where the bias allows it: the
+    sum over the ranges reads the bias 16 bytes at a time, so this one runs unsplit.  The kernel's own entry refuses the
+    split before anything is launched."""
+    M, N, K = 6400, 1024, 4096
+    assert ops._x6_splits(M, N, K, True) > 1
+    g = torch.Generator("cuda").manual_seed(7)
+    a, b = torch.randn(M, K, generator=g, device="cuda"), torch.randn(K, N, generator=g, device="cuda")
+    bias = torch.randn(N + 1, generator=g, device="cuda")[1:]
+    assert bias.data_ptr() % 16 != 0
+    out = ops.gemm(a, b, bias=bias)
+    want = a.double() @ b.double() + bias.double()
+    assert float((out.double() - want).norm() / want.norm()) < 4e-7
+    part = torch.full((2, M, N), float("nan"), device="cuda")
+    with pytest.raises(RuntimeError):
+        _cabi.lib().pd_gemm_f32x6(0, 0, M, N, K, ops._ptr(a), K, ops._ptr(b), N, 0.0, ops._ptr(out), N, ops._ptr(bias), 2,
+                                  ops._ptr(part), _cabi.stream_ptr())
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(part).all())
