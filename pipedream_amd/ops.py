@@ -35,7 +35,8 @@ class _Timing(object):
     def __exit__(self, *exc):
         end = torch.cuda.Event(enable_timing=True)
         end.record()
-        kernel_timer.setdefault(self.name, []).append((self.start, end, self.work))
+        if kernel_timer is not None:               # (it may be reset inside the call)
+            kernel_timer.setdefault(self.name, []).append((self.start, end, self.work))
         return False
 
 

@@ -470,3 +470,15 @@ def test_gemm_with_a_bias_that_is_not_aligned():
                                   ops._ptr(part), _cabi.stream_ptr())
     torch.cuda.synchronize()
     assert bool(torch.isnan(part).all())
+
+
+def test_kernel_timer_may_be_reset_inside_a_timed_call():
+    timer = ops.kernel_timer = {}
+    try:
+        with ops._timed("kept", 1.0):
+            pass
+        with ops._timed("dropped", 1.0):
+            ops.kernel_timer = None
+    finally:
+        ops.kernel_timer = None
+    assert list(timer) == ["kept"] and len(timer["kept"]) == 1
