@@ -345,6 +345,35 @@ def test_gemm_as_six_bf16_products_is_closer_to_fp64_than_the_fp32_kernel(ta, tb
 
 
 @pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False)])
+@pytest.mark.parametrize("M,N,K,parts", [(256, 512, 128, 6), (4096, 3072, 64, 1)])
+def test_gemm_as_six_bf16_products_of_far_rows(M, N, K, parts, ta, tb, _gemm_algorithm_back_to_auto):
+    """An operand whose rows lie 2^20 elements and more apart is beyond the 32-bit offsets of pd_gemm_f32x6; its product
+    goes through memory, six bf16 slots of each operand and the bf16 kernel, unsplit and in ranges.  (The operand with
+    fewer rows is the far one: a row takes 4 MB.)"""
+    from pipedream_amd import ops
+    g = torch.Generator().manual_seed(23)
+    a = torch.randn((K, M) if ta else (M, K), generator=g).cuda()
+    b = torch.randn((N, K) if tb else (K, N), generator=g).cuda()
+    bias, prior = torch.randn(N, generator=g).cuda(), torch.randn(M, N, generator=g).cuda()
+    want = (a.double().t() if ta else a.double()) @ (b.double().t() if tb else b.double()) + bias.double() + 0.5 * prior.double()
+
+    def far(t):
+        view = torch.empty(t.size(0), 1 << 20, device="cuda")[:, :t.size(1)]
+        view.copy_(t)
+        return view
+
+    if a.size(0) < b.size(0):
+        a = far(a)
+    else:
+        b = far(b)
+    ops.set_gemm_f32_algorithm("split_bf16")
+    assert not ops._use_x6(M, N, K, ta, tb, False, a, b, prior, a.stride(0), b.stride(0), N)
+    assert ops._split_bf16_parts(M, N, K) == parts and ops._use_split_bf16(M, N, K, ta, tb, False, a, b, prior)
+    out = ops.gemm(a, b, trans_a=ta, trans_b=tb, bias=bias, out=prior.clone(), beta=0.5)
+    assert float((out.double() - want).norm() / want.norm()) < 4e-7
+
+
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False)])
 def test_gemm_as_six_bf16_products_with_few_output_tiles(ta, tb, _gemm_algorithm_back_to_auto):
     """A narrow output (1024 columns: 28 tiles of 256 x 256): the six-fold reduction is cut into ranges that run as
     batch entries, and their partial products are added in index order with bias and beta."""
