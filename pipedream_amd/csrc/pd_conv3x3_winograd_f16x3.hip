@@ -33,8 +33,8 @@
 // 48 MFMAs (1700 cycles) and 2 x 165 vector instructions, the block moves 290 KB through LDS (2300 cycles): 4100 cycles,
 // where the fp32 kernel takes 9580 for the same chunk.  64 images, C = K = 128 at 112 x 112: 595 us (398 TFLOP/s of a
 // direct convolution; 564 with one scale for all channels and no tests), C = K = 512 at 28 x 28: 530 us (446); 8 images
-// 86 us.  VGG16's front stage 7.74 -> 6.07 ms a step,
-// all of VGG16 26.4 -> 20.0 ms, a validation pass over 2 x 8 images 3.70 -> 2.43 ms.  An item of 64 channels takes 27 500
+// 86 us.  With the weight gradient's kernel VGG16's front stage 7.7 -> 5.1 ms a step, all of VGG16 26.3 -> 17.2 ms, a
+// validation pass over 2 x 8 images 3.68 -> 2.53 ms.  An item of 64 channels takes 28 000
 // cycles, 9000 of them behind its last product; before its divisions went to the ring of decoded items 35 000.
 // A block (512 threads, one per CU) owns 16 x 16 output pixels x 64 channels:
 // wave (j, kh) holds column j of the 4 x 4 transformed positions for 64 tiles x 32 channels (128 accumulators a lane);
@@ -82,23 +82,6 @@ constexpr int H3_MIN_SHIFT = -60;                      // range of s(c); a chann
 static_assert(255 + H3_MIN_SHIFT > H3_MAX_FIELD && H3_X_BASE - H3_MAX_FIELD + H3_MIN_SHIFT > -127, "fields");
 __device__ __forceinline__ float h3_scale(int field, int base) {
     return __builtin_bit_cast(float, (uint32_t)(base + 127 - field) << 23);
-}
-
-__device__ __forceinline__ uint32_t h3_pack(float lo, float hi) {
-    uint32_t p;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(p) : "v"(lo), "v"(hi));
-    return p;
-}
-// x - (the lower / upper half of p), exactly
-__device__ __forceinline__ float h3_rest_lo(uint32_t p, float x) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(p), "v"(x));
-    return r;
-}
-__device__ __forceinline__ float h3_rest_hi(uint32_t p, float x) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(p), "v"(x));
-    return r;
 }
 
 // What the filter's buffer holds behind the fragments (byte offsets from its start).
@@ -287,13 +270,13 @@ __global__ __launch_bounds__(256) void winograd_filter_f16x3_kernel(const float*
                 *(float2_t*)to = float2_t{o[0], o[1]};
                 continue;
             }
-            const uint32_t p = h3_pack(o[0], o[1]);
-            float r0 = h3_rest_lo(p, o[0]), r1 = h3_rest_hi(p, o[1]);
+            const uint32_t p = wino_f16_pack(o[0], o[1]);
+            float r0 = wino_f16_rest_lo(p, o[0]), r1 = wino_f16_rest_hi(p, o[1]);
             if ((p & 0x7c00u) == 0x7c00u) r0 = 0.f;                // infinities and NaNs stand in the first term alone
             if ((p & 0x7c000000u) == 0x7c000000u) r1 = 0.f;
             char* to = dst + (size_t)(i * 4 + j) * (4 * H3_FRAG);
             *(uint32_t*)to = p;
-            *(uint32_t*)(to + H3_FRAG) = h3_pack(r0, r1);
+            *(uint32_t*)(to + H3_FRAG) = wino_f16_pack(r0, r1);
         }
 }
 
@@ -498,8 +481,8 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         for (int e = 0; e < 2; ++e)
             v[e] = m == 0 ? d[row][0][e] - d[row][2][e] : m == 1 ? d[row][1][e] + d[row][2][e]
                  : m == 2 ? d[row][2][e] - d[row][1][e] : d[row][1][e] - d[row][3][e];
-        const uint32_t p = h3_pack(v[0], v[1]);
-        const uint32_t q = h3_pack(h3_rest_lo(p, v[0]), h3_rest_hi(p, v[1]));
+        const uint32_t p = wino_f16_pack(v[0], v[1]);
+        const uint32_t q = wino_f16_pack(wino_f16_rest_lo(p, v[0]), wino_f16_rest_hi(p, v[1]));
         char* to = lds + (row < 2 ? 0 : H3_SLOT1_OFF) + ((row & 1) * 4 + m) * (4 * H3_FRAG) + v_dst;
         *(uint32_t*)to = p;
         *(uint32_t*)(to + 2 * H3_FRAG) = q;

@@ -49,23 +49,6 @@ constexpr int W3_X_RANGE = 19, W3_Y_RANGE = 23;        // .. the values under on
 __device__ __forceinline__ float w3_scale(int field) {
     return __builtin_bit_cast(float, (uint32_t)(W3_BASE + 127 - field) << 23);
 }
-__device__ __forceinline__ uint32_t w3_pack(float lo, float hi) {
-    uint32_t p;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(p) : "v"(lo), "v"(hi));
-    return p;
-}
-// x - (the lower / upper half of p), exactly
-__device__ __forceinline__ float w3_rest_lo(uint32_t p, float x) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(p), "v"(x));
-    return r;
-}
-__device__ __forceinline__ float w3_rest_hi(uint32_t p, float x) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(p), "v"(x));
-    return r;
-}
-
 __global__ __launch_bounds__(WW_THREADS, 1) void winograd_wgrad_f16x3_kernel(const WinoWgradArgs a) {
     __shared__ __attribute__((aligned(1024))) char lds[W3_LDS];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -260,9 +243,9 @@ __global__ __launch_bounds__(WW_THREADS, 1) void winograd_wgrad_f16x3_kernel(con
     for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(dsts[i]), "+v"(srcs[i]));
     auto put = [&](int row, int pos, int op, float v0, float v1) {
         char* const to = lds + dsts[row >> 1] + ((row & 1) * 4 + pos) * W3_POS + op * 4096;
-        const uint32_t p = w3_pack(v0, v1);
+        const uint32_t p = wino_f16_pack(v0, v1);
         *(uint32_t*)to = p;
-        *(uint32_t*)(to + 2048) = w3_pack(w3_rest_lo(p, v0), w3_rest_hi(p, v1));
+        *(uint32_t*)(to + 2048) = wino_f16_pack(wino_f16_rest_lo(p, v0), wino_f16_rest_hi(p, v1));
     };
     auto v_of = [&](int row, int pos, int t) {         // position (row, pos) of tile t
         const float* w = &v[row][2 * t];

@@ -20,6 +20,23 @@ constexpr int WW_BLOCKS = 256;                       // persistent blocks: 8 die
 constexpr int WW_PART_FLOATS = 16 * 64 * 64;         // one block's partial dU
 constexpr int WW_PART_STRIDE = WW_PART_FLOATS;       // floats between two blocks' partials
 
+// Two fp32 values as two f16 terms each: the first terms, packed; what a first term leaves of its value, exactly.
+__device__ __forceinline__ uint32_t wino_f16_pack(float lo, float hi) {
+    uint32_t p;
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(p) : "v"(lo), "v"(hi));
+    return p;
+}
+__device__ __forceinline__ float wino_f16_rest_lo(uint32_t p, float x) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(p), "v"(x));
+    return r;
+}
+__device__ __forceinline__ float wino_f16_rest_hi(uint32_t p, float x) {
+    float r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(p), "v"(x));
+    return r;
+}
+
 }  // namespace
 
 struct WinoArgs {
