@@ -67,7 +67,8 @@ def _rowmajor2d(t, name):
 
 
 def gemm(a, b, trans_a=False, trans_b=False, bias=None, relu=False, out=None, beta=0.0):
-    """out[M,N] = op(a) @ op(b) (+ bias) (+ beta*out) (ReLU); fp32 MFMA kernel."""
+    """out[M,N] = op(a) @ op(b) (+ bias) (+ beta*out) (ReLU), in fp32 or on the bf16 matrix pipes with
+    fp32 accuracy (set_gemm_f32_algorithm)."""
     _rowmajor2d(a, "a")
     _rowmajor2d(b, "b")
     M, K = (a.size(1), a.size(0)) if trans_a else (a.size(0), a.size(1))
@@ -203,7 +204,7 @@ def _x6_splits(M, N, K, may_split):
 
 # The same arithmetic through memory: six bf16 slots of each operand written by pd_split3_bf16_f32 and multiplied by
 # the bf16 GEMM over a six-fold reduction.  Slower than pd_gemm_f32x6 everywhere; for operands whose leading dimension
-# is beyond that kernel's offsets.
+# is beyond that kernel's offsets (rows 2^20 elements and more apart).
 def _split_bf16_parts(M, N, K):
     """Number of ranges the six-fold reduction is cut into (partial products, one batch entry each, added by
     pd_splitk_reduce_f32) so that the bf16 kernel's 256 x 256 tiles fill the chip: 1 for at least 192 tiles, else
@@ -655,10 +656,10 @@ def set_conv_pieces(mode):
 
 
 def set_conv_wgrad_strips(mode):
-    """Strips of the fp32 Winograd weight-gradient kernel: "auto" (long reductions go to the f16 kernel, which has no
-    strips, the others take upright strips of 16 rows x 2 columns of the stacked batch where the width is no multiple
-    of 16 pixels), "flat" (2 x 16 pixels always), "upright" (wherever the shape allows).  The results differ by rounding
-    only."""
+    """Strips of the fp32 Winograd weight-gradient kernel: "auto" (reductions of 32 tiles a block and more go to the f16
+    kernel, which has no strips, the others take upright strips of 16 rows x 2 columns of the stacked batch where the
+    width is no multiple of 16 pixels), "flat" (2 x 16 pixels always), "upright" (wherever the shape allows), the last
+    two on the fp32 matrix pipes.  The results differ by rounding only."""
     _cabi.lib().pd_conv3x3_winograd_set_wgrad_strips({"auto": 0, "flat": 1, "upright": 2}[mode])
 
 

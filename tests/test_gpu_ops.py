@@ -319,7 +319,8 @@ def test_gemm_as_six_bf16_products_is_closer_to_fp64_than_the_fp32_kernel(ta, tb
     """Large fp32 products run on the bf16 matrix pipes: each operand as the exact sum of three bf16 terms, six
     products per term pair, fp32 accumulation.  Against torch's fp64 product the result must be at least as close
     as the fp32 MFMA kernel's (it is about three times closer: fewer roundings of the running sum), with bias and
-    beta applied; the default takes that path for this shape and not for a narrow or a small one."""
+    beta applied; the default takes that path for this shape.  (pd_gemm_f32x6 multiplies; the rule of the path through
+    memory, for wide outputs only, is looked at first.)"""
     from pipedream_amd import ops
     M, N, K = 4096, 3072, 1408
     assert ops._use_split_bf16(M, N, K, ta, tb, False, *(torch.empty(8, 8, device="cuda"),) * 3)
@@ -375,8 +376,8 @@ def test_gemm_as_six_bf16_products_of_far_rows(M, N, K, parts, ta, tb, _gemm_alg
 
 @pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False)])
 def test_gemm_as_six_bf16_products_with_few_output_tiles(ta, tb, _gemm_algorithm_back_to_auto):
-    """A narrow output (1024 columns: 28 tiles of 256 x 256): the six-fold reduction is cut into ranges that run as
-    batch entries, and their partial products are added in index order with bias and beta."""
+    """A narrow output (1024 columns): the reduction is cut into ranges, whose partial products are added in index order
+    with bias and beta (pd_gemm_f32x6; the path through memory would cut its six-fold one, too)."""
     from pipedream_amd import ops
     M, N, K = 1792, 1024, 1536
     assert ops._split_bf16_parts(M, N, K) == 6
