@@ -769,15 +769,15 @@ def test_split_f16_convolution_of_infinities(value, where, N, C, K, H, W, conv_a
     assert torch.isfinite(want).any() and not torch.isfinite(want).all()
 
 
-# (one unit of two tiles; ranks without a step; units that end beyond the image; more pairs of channel blocks than ranks;
-# reductions long enough for the rounding of the sums to show)
+# (the fifth and the last shape take the f16 kernel: few steps a block, and reductions long enough for the rounding of the
+# sums to show; the others have fewer than 32 tiles a block and take the fp32 kernel, which has to meet the same bound)
 @pytest.mark.parametrize("N,C,K,H,W", [(1, 64, 64, 1, 1), (1, 64, 64, 7, 5), (2, 128, 64, 33, 35), (3, 64, 128, 18, 20),
                                        (4, 512, 512, 14, 14), (1, 1024, 1024, 6, 6), (16, 64, 64, 112, 112)])
 @pytest.mark.parametrize("scales", ["plain", "channels", "growing"])
 def test_split_f16_weight_gradient(N, C, K, H, W, scales, conv_algorithm):
     """Against 64 bits.  Sums of P = N H W products of two terms each in fp32: 2^-23 for the terms and the transforms in
     front of them, times 4 for the cancellation in G^T dU G, and 2^-24 sqrt(P / 16) of the running sums; per tap, so
-    that a bias that adds up in one of them shows.  (The small ones take the fp32 kernel.)"""
+    that a bias that adds up in one of them shows."""
     if conv_algorithm != "winograd":
         pytest.skip("the Winograd kernel's")
     g = torch.Generator("cuda").manual_seed(N + C + H)
@@ -806,7 +806,8 @@ def test_split_f16_weight_gradient(N, C, K, H, W, scales, conv_algorithm):
 
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 def test_split_f16_weight_gradient_of_infinities(value, conv_algorithm):
-    """What the fp32 kernel gives: the channel of the infinity has no finite element, the others are as without it."""
+    """Too few tiles for the f16 kernel (see the test of infinities and NaNs below for that): the channel of the infinity
+    has no finite element, the others are as without it."""
     if conv_algorithm != "winograd":
         pytest.skip("the Winograd kernel's")
     g = torch.Generator("cuda").manual_seed(5)
