@@ -238,7 +238,8 @@ int pd_conv3x3_winograd_set_pieces(int mode);
  * matrix pipes (operands split as in pd_conv3x3_winograd_f16x3_fwd_nhwc_f32, with a scale per channel that follows the
  * values, and fp32 products for 16 tiles at a time where a channel's values there are too far apart) without strips;
  * 1: never; 2: wherever the shape allows.  Modes 1 and 2 differ by the summation order, mode 0 also by the split: its
- * error against 64 bits is 0.6 to 1.0 times theirs.  Process-wide.  No counterpart in the reference. */
+ * error against 64 bits is 0.6 to 1.0 times theirs (of single elements up to 8 times, where all their products lie beside
+ * gradients 2^20 times as large in the same tiles, with an input of zero).  Process-wide.  No counterpart in the reference. */
 int pd_conv3x3_winograd_set_wgrad_strips(int mode);
 
 /* The same convolution (and, with rot180, its input gradient) by the Winograd algorithm

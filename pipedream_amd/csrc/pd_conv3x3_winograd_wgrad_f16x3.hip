@@ -11,7 +11,10 @@
 // held to 2^-24.8 (rms) of the largest of its channel within a step.  What is far below that in the same step would lose
 // bits: where, in any channel, a dY value is below 2^-23 of the scale or all nine x values under an output pixel are below
 // 2^-19 of it, the step runs on fp32 MFMAs, and so does a step with infinities or with values 2^64 times those before.  A
-// sum then comes from values that are held to the rounding of fp32, whatever the other channels, images and pixels are like.
+// sum thus comes from values held to the rounding of fp32 against the largest of their channel in their own 16 tiles,
+// whatever the other channels, images and pixels are like.  (Over 500 random shapes, masks and ranges an element's error
+// stays below 1.9e-6 of the sum of its products' sizes, the fp32 kernel's below 0.5e-6: elements whose few products lie
+// beside dY values 2^20 times as large in the same tiles, where x is zero.)
 // (A step of VGG16: 12 to 28 % of the steps of a block look at their scales anew, 0.1 to 0.3 % run on fp32 MFMAs.)
 //
 // Bound: f16 MFMAs beside vector instructions and LDS traffic: a step takes 7500 cycles, of which 1700 are MFMAs and
