@@ -355,6 +355,30 @@ int pd_lstm_recurrence_fwd_f32(float* gates, const float* w_hh, const float* b_i
 int pd_lstm_recurrence_bwd_f32(const float* gates, const float* c, const float* dy, const float* w_hh,
                                float* dh_rec, int splits, float* dc, float* dgates, int T, int B, int H,
                                void* stream);
+/* The same time loops with the recurrent products on the bf16 matrix pipes at fp32 accuracy, for batches of at
+ * most 128 and H a multiple of 32 (pd_lstm_f32x6_supported).  Scratch (pd_lstm_f32x6_workspace_bytes, 16-byte
+ * aligned): w_split, which pd_lstm_split_weights_f32x6 fills from w_hh once per layer, direction and weight
+ * version (not needed for a single step), and tiles, which the time loop writes.
+ * Forward: steps t_begin .. t_end-1 of the tensors of pd_lstm_recurrence_fwd_f32, one launch each (step 0 starts
+ * from zero state; a later first step finds the tiles its predecessor left).
+ * Backward: the tensors of pd_lstm_recurrence_bwd_f32 with dh_rec[pd_lstm_dh_f32x6_splits(B, H)][B][H]; its two
+ * launches of a step by themselves: the cell (as pd_lstm_cell_bwd_f32, dgates also as tiles) and
+ * dh_rec = dgates w_hh as partial sums. */
+int pd_lstm_f32x6_supported(int B, int H);
+int pd_lstm_f32x6_workspace_bytes(int backward, int B, int H, uint64_t* weights, uint64_t* tiles);
+int pd_lstm_split_weights_f32x6(int backward, const float* w_hh, void* out, int H, void* stream);
+int pd_lstm_recurrence_fwd_f32x6(float* gates, const float* w_hh, const void* w_split, const float* b_ih,
+                                 const float* b_hh, float* h_tiles, float* c, float* y, int t_begin, int t_end, int B,
+                                 int H, void* stream);
+int pd_lstm_dh_f32x6_splits(int B, int H);
+int pd_lstm_cell_bwd_f32x6(const float* gates, const float* c_prev, const float* c, const float* dy, const float* dh_rec,
+                           int n_rec, float* dc_io, float* dgates, float* tiles, int B, int H, int first_step,
+                           void* stream);
+int pd_lstm_dh_f32x6(const float* tiles, const float* dgates, const float* w_hh, const void* w_split, float* dh_rec,
+                     int B, int H, void* stream);
+int pd_lstm_recurrence_bwd_f32x6(const float* gates, const float* c, const float* dy, const float* w_hh,
+                                 const void* w_split, float* tiles, float* dh_rec, float* dc, float* dgates, int T,
+                                 int B, int H, void* stream);
 /* y = a + b: the residual connections `out13 = out13 + out10` (stage0.py:32, 36). */
 int pd_add_f32(const float* a, const float* b, float* y, uint64_t n, void* stream);
 /* torch.nn.Embedding (stage0.py:10): out[p][:] = weight[ids[p]][:].  Backward writes the

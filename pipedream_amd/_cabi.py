@@ -105,6 +105,14 @@ SIGNATURES = {
     "pd_lstm_cell_bwd_f32": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _vp], True),
     "pd_lstm_recurrence_fwd_f32": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _vp], True),
     "pd_lstm_recurrence_bwd_f32": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _vp], True),
+    "pd_lstm_f32x6_supported": (_i, [_i, _i], False),
+    "pd_lstm_f32x6_workspace_bytes": (_i, [_i, _i, _i, ctypes.POINTER(_u64), ctypes.POINTER(_u64)], True),
+    "pd_lstm_split_weights_f32x6": (_i, [_i, _vp, _vp, _i, _vp], True),
+    "pd_lstm_recurrence_fwd_f32x6": (_i, [_vp] * 8 + [_i] * 4 + [_vp], True),
+    "pd_lstm_dh_f32x6_splits": (_i, [_i, _i], False),
+    "pd_lstm_cell_bwd_f32x6": (_i, [_vp] * 5 + [_i] + [_vp] * 3 + [_i] * 3 + [_vp], True),
+    "pd_lstm_dh_f32x6": (_i, [_vp] * 5 + [_i, _i, _vp], True),
+    "pd_lstm_recurrence_bwd_f32x6": (_i, [_vp] * 9 + [_i] * 3 + [_vp], True),
     "pd_add_f32": (_i, [_vp, _vp, _vp, _u64, _vp], True),
     "pd_embedding_fwd_f32": (_i, [_vp, _vp, _vp, _i, _i, _i64, _vp], True),
     "pd_embedding_bwd_f32": (_i, [_vp, _vp, _vp, _i, _i, _i64, _i64, _vp], True),

@@ -874,6 +874,23 @@ def add(a, b):
     return y
 
 
+def _lstm_x6(B, H, w_hh):
+    """Whether a layer's recurrence runs on the bf16 matrix pipes at fp32 accuracy (pd_lstm_f32x6.hip)."""
+    return (_GEMM_F32_ALGO != "never" and w_hh.is_contiguous() and w_hh.data_ptr() % 16 == 0 and
+            bool(_cabi.lib().pd_lstm_f32x6_supported(B, H)))
+
+
+def _lstm_x6_scratch(backward, T, B, H, w_hh):
+    """(split weights or None for a single step, tiles) for one pass over a layer."""
+    weights, tiles = ctypes.c_uint64(), ctypes.c_uint64()
+    _cabi.lib().pd_lstm_f32x6_workspace_bytes(backward, B, H, ctypes.byref(weights), ctypes.byref(tiles))
+    w_split = None
+    if T > 1:
+        w_split = torch.empty(weights.value, dtype=torch.uint8, device=w_hh.device)
+        _cabi.lib().pd_lstm_split_weights_f32x6(backward, _ptr(w_hh), _ptr(w_split), H, _cabi.stream_ptr())
+    return w_split, torch.empty(tiles.value, dtype=torch.uint8, device=w_hh.device)
+
+
 def lstm_forward(x, w_ih, w_hh, b_ih, b_hh):
     """Single-layer, uni-directional LSTM over x[T,B,I] from zero state.
     Returns (y[T,B,H], saved) where saved = (gates[T,B,4H] activated, c[T,B,H])."""
@@ -891,6 +908,20 @@ def lstm_forward(x, w_ih, w_hh, b_ih, b_hh):
     gates = gemm(x2, w_ih, trans_b=True).view(T, B, 4 * H)
     y = torch.empty((T, B, H), dtype=torch.float32, device=x.device)
     c = torch.empty((T, B, H), dtype=torch.float32, device=x.device)
+    if _lstm_x6(B, H, w_hh):
+        # product and cell of a step in one launch
+        w_split, tiles = _lstm_x6_scratch(0, T, B, H, w_hh)
+
+        def steps(t0, t1):
+            lib.pd_lstm_recurrence_fwd_f32x6(_ptr(gates), _ptr(w_hh), _ptr(w_split), _ptr(b_ih), _ptr(b_hh), _ptr(tiles),
+                                             _ptr(c), _ptr(y), t0, t1, B, H, s())
+        if kernel_timer is None:
+            steps(0, T)
+            return y, (gates, c)
+        for t in range(T):
+            with _timed("lstm_step_f32x6", 2.0 * B * 4 * H * H) if t > 0 else _UNTIMED:
+                steps(t, t + 1)
+        return y, (gates, c)
     # the recurrent product h_{t-1} W_hh^T has only B rows: split over k, summed inside the cell kernel
     rec = torch.empty((splitk_factor(B, 4 * H, H), B, 4 * H), dtype=torch.float32, device=x.device)
     if kernel_timer is None and w_hh.is_contiguous():
@@ -914,17 +945,22 @@ def lstm_backward(dy, x, y, gates, c, w_ih, w_hh, need_dx=True):
     lib, s = _cabi.lib(), _cabi.stream_ptr
     dgates = torch.empty((T, B, 4 * H), dtype=torch.float32, device=x.device)
     dc = torch.empty((B, H), dtype=torch.float32, device=x.device)
-    dh_rec = torch.empty((splitk_factor(B, H, 4 * H), B, H), dtype=torch.float32, device=x.device)
-    native = kernel_timer is None and w_hh.is_contiguous() and gates.is_contiguous() and c.is_contiguous()
-    if native:
-        lib.pd_lstm_recurrence_bwd_f32(_ptr(gates), _ptr(c), _ptr(dy), _ptr(w_hh), _ptr(dh_rec), dh_rec.size(0),
-                                       _ptr(dc), _ptr(dgates), T, B, H, s())
-    for t in (() if native else range(T - 1, -1, -1)):
-        lib.pd_lstm_cell_bwd_f32(_ptr(gates[t]), _ptr(c[t - 1]) if t > 0 else None, _ptr(c[t]), _ptr(dy[t]),
-                                 _ptr(dh_rec) if t < T - 1 else None, dh_rec.size(0), _ptr(dc), _ptr(dgates[t]), B, H,
-                                 int(t == T - 1), s())
-        if t > 0:
-            gemm_splitk(dgates[t], w_hh, False, False, dh_rec)      # [B,4H] @ [4H,H], split over 4H
+    if _lstm_x6(B, H, w_hh) and gates.is_contiguous() and c.is_contiguous():
+        splits = lib.pd_lstm_dh_f32x6_splits(B, H)
+        dh_rec = torch.empty((splits, B, H), dtype=torch.float32, device=x.device)
+        w_split, tiles = _lstm_x6_scratch(1, T, B, H, w_hh)
+        if kernel_timer is None:
+            lib.pd_lstm_recurrence_bwd_f32x6(_ptr(gates), _ptr(c), _ptr(dy), _ptr(w_hh), _ptr(w_split), _ptr(tiles),
+                                             _ptr(dh_rec), _ptr(dc), _ptr(dgates), T, B, H, s())
+        for t in (() if kernel_timer is None else range(T - 1, -1, -1)):
+            lib.pd_lstm_cell_bwd_f32x6(_ptr(gates[t]), _ptr(c[t - 1]) if t > 0 else None, _ptr(c[t]), _ptr(dy[t]),
+                                       _ptr(dh_rec), splits, _ptr(dc), _ptr(dgates[t]), _ptr(tiles), B, H,
+                                       int(t == T - 1), s())
+            if t > 0:
+                with _timed("gemm_f32_splitk", 2.0 * B * H * 4 * H):
+                    lib.pd_lstm_dh_f32x6(_ptr(tiles), _ptr(dgates[t]), _ptr(w_hh), _ptr(w_split), _ptr(dh_rec), B, H, s())
+    else:
+        _lstm_backward_loop(dy, gates, c, w_hh, dc, dgates)
     dg2 = dgates.view(T * B, 4 * H)
     x2 = x.contiguous().view(T * B, I)
     dw_ih = gemm(dg2, x2, trans_a=True)
@@ -936,6 +972,24 @@ def lstm_backward(dy, x, y, gates, c, w_ih, w_hh, need_dx=True):
     db = colsum(dg2)
     dx = gemm(dg2, w_ih).view(T, B, I) if need_dx else None
     return dx, dw_ih, dw_hh, db
+
+
+def _lstm_backward_loop(dy, gates, c, w_hh, dc, dgates):
+    """The backward time loop with fp32 MFMA products split over k."""
+    T, B = dy.shape[:2]
+    H = w_hh.shape[1]
+    lib, s = _cabi.lib(), _cabi.stream_ptr
+    dh_rec = torch.empty((splitk_factor(B, H, 4 * H), B, H), dtype=torch.float32, device=dy.device)
+    native = kernel_timer is None and w_hh.is_contiguous() and gates.is_contiguous() and c.is_contiguous()
+    if native:
+        lib.pd_lstm_recurrence_bwd_f32(_ptr(gates), _ptr(c), _ptr(dy), _ptr(w_hh), _ptr(dh_rec), dh_rec.size(0),
+                                       _ptr(dc), _ptr(dgates), T, B, H, s())
+    for t in (() if native else range(T - 1, -1, -1)):
+        lib.pd_lstm_cell_bwd_f32(_ptr(gates[t]), _ptr(c[t - 1]) if t > 0 else None, _ptr(c[t]), _ptr(dy[t]),
+                                 _ptr(dh_rec) if t < T - 1 else None, dh_rec.size(0), _ptr(dc), _ptr(dgates[t]), B, H,
+                                 int(t == T - 1), s())
+        if t > 0:
+            gemm_splitk(dgates[t], w_hh, False, False, dh_rec)      # [B,4H] @ [4H,H], split over 4H
 
 
 def embedding_forward(ids, weight):
