@@ -161,7 +161,6 @@ int pd_gemm_f32(int trans_a, int trans_b, int M, int N, int K,
 int pd_gemm_splitk_f32(int trans_a, int trans_b, int M, int N, int K,
                        const float* A, int lda, const float* B, int ldb,
                        float* partials, int splits, void* stream);
-/* C[M][ldc] = sum_s partials[s] (+ bias[N]) (+ beta*C) (ReLU); N and ldc multiples of 4. */
 int pd_splitk_reduce_f32(const float* partials, int splits, int M, int N, const float* bias, int relu,
                          float beta, float* C, int ldc, void* stream);
 

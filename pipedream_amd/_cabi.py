@@ -113,6 +113,8 @@ SIGNATURES = {
     "pd_lstm_cell_bwd_f32x6": (_i, [_vp] * 5 + [_i] + [_vp] * 3 + [_i] * 3 + [_vp], True),
     "pd_lstm_dh_f32x6": (_i, [_vp] * 5 + [_i, _i, _vp], True),
     "pd_lstm_recurrence_bwd_f32x6": (_i, [_vp] * 9 + [_i] * 3 + [_vp], True),
+    "pd_gemm_skinny_f32x6_splits": (_i, [_i, _i, _i], False),
+    "pd_gemm_skinny_f32x6": (_i, [_i, _i, _i, _i, _vp, _i, _vp, _i, _f, _vp, _i, _vp, _i, _i, _vp, _vp], True),
     "pd_add_f32": (_i, [_vp, _vp, _vp, _u64, _vp], True),
     "pd_embedding_fwd_f32": (_i, [_vp, _vp, _vp, _i, _i, _i64, _vp], True),
     "pd_embedding_bwd_f32": (_i, [_vp, _vp, _vp, _i, _i, _i64, _i64, _vp], True),
