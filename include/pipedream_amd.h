@@ -463,8 +463,8 @@ int pd_layernorm_bwd_bf16(const uint16_t* dy, const uint16_t* x, const float* ga
  * bf16 probabilities, and lse2 [batch][heads][seq] (fp32), log2 of the softmax denominator in the scaled
  * base-2 domain, from which the backward pass recomputes the probabilities:
  * P[q][k] = 2^(s_qk log2(e) / sqrt(head_dim) - lse2[q]).
- * Supported shapes: pd_attention_fwd_supported() != 0 (head_dim 64, seq 128 / 256 / 512); other shapes
- * use pd_gemm_bf16 + pd_softmax_fwd_bf16 / pd_softmax_bwd_bf16. */
+ * Supported shapes: pd_attention_fwd_supported() != 0 (head_dim 64, seq a multiple of 8; probs only with
+ * seq 128, 256 or 512); other shapes use pd_gemm_bf16 + pd_softmax_fwd_bf16 / pd_softmax_bwd_bf16. */
 int pd_attention_fwd_supported(int seq, int head_dim);
 int pd_attention_fwd_bf16(const uint16_t* qkv, uint16_t* ctx, uint16_t* probs, float* lse2, int batch, int seq,
                           int heads, int head_dim, void* stream);

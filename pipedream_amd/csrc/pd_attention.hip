@@ -11,7 +11,7 @@
 // Bound: MFMA bf16 / vector ALU (seq * seq exponentials per head); algorithmic HBM traffic = qkv
 // (and ctx, dctx in the backward) read once per kernel, ctx / dqkv written once.
 //
-// One block = one (batch, head) pair x 128 queries (or keys), 8 waves of 16.  The other side's two
+// seq 128, 256, 512 (others: "any sequence length" below).  One block = one (batch, head) pair x 128 queries (or keys), 8 waves of 16.  The other side's two
 // [seq][64] matrices are staged in LDS once per block with a row pitch of 72 bf16, which serves both
 // the 128-bit fragment reads (8 consecutive k per lane) and the transposing reads.  Everything is
 // computed in the orientation in which no accumulator ever has to change layout; shown for the
@@ -325,10 +325,293 @@ __global__ __launch_bounds__(AT_THREADS) void attention_bwd_kv_kernel(const uint
     }
 }
 
+// ---- any sequence length ---------------------------------------------------------------------------------
+// The other side's rows pass through LDS in chunks of AT_CH (the next chunk is on its way to the registers while one is
+// used), so seq is a run-time number: a multiple of 8, rows past it are zeros in LDS and masked.  A block has 64 queries
+// (keys), four waves of 16, 168 registers (three blocks a CU; with 212 and two, forward at 8 x 16 heads x 640 52 us instead
+// of 38).  The forward keeps a running maximum and sum per query and rescales what it has when the maximum rises.
+// us forward / backward, against the batched products and softmax kernels that took these shapes before: 3 x 12 heads x
+// 200 10 / 14 (23 / 31), 8 x 16 x 640 38 / 103 (115 / 192), 5 x 8 x 328 10 / 22 (32 / 53); error of the context (2-norm)
+// 2.2e-3 (4.2e-3: the scores went through bf16).  At 512 and 256 the kernels above are as fast forward and 4-17 % faster
+// backward, and stay.
+constexpr int AT_CH = 128;
+constexpr int AT_CT = 256;             // threads
+constexpr int AT_CQ = 64;              // queries (keys) per block
+
+// chunk of rows [r0, r0 + AT_CH) x 64 columns: global -> registers, registers -> LDS
+struct AtChunk {
+    static constexpr int ITERS = AT_CH * (AT_D / 8) / AT_CT;
+    u16x8 r[ITERS];
+    __device__ __forceinline__ void load(const uint16_t* __restrict__ g, int ld, int r0, int rows, int tid) {
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            const int id = tid + it * AT_CT;
+            r[it] = *(const u16x8*)(g + (size_t)min(r0 + id / (AT_D / 8), rows - 1) * ld + (id % (AT_D / 8)) * 8);
+        }
+    }
+    __device__ __forceinline__ void store(uint16_t* lds, int r0, int rows, int tid) const {
+        const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            const int id = tid + it * AT_CT;
+            *(u16x8*)(lds + (id / (AT_D / 8)) * AT_P + (id % (AT_D / 8)) * 8) = r0 + id / (AT_D / 8) < rows ? r[it] : zero;
+        }
+    }
+};
+
+__global__ __launch_bounds__(AT_CT, 3) void attention_any_fwd_kernel(const uint16_t* __restrict__ qkv,
+                                                                  uint16_t* __restrict__ ctx, float* __restrict__ lse2,
+                                                                  int S, int heads, float c) {
+    constexpr int NT = AT_CH / 16;
+    __shared__ __attribute__((aligned(16))) uint16_t k_lds[AT_CH * AT_P];
+    __shared__ __attribute__((aligned(16))) uint16_t v_lds[AT_CH * AT_P];
+
+    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+    const int li = lane % 16, g = lane / 16;
+    const int bh = blockIdx.y, b = bh / heads, h = bh % heads;
+    const int H = heads * AT_D, ld = 3 * H;
+    const uint16_t* base = qkv + (size_t)b * S * ld + h * AT_D;
+    AtChunk kc, vc;
+    kc.load(base + H, ld, 0, S, tid);
+    vc.load(base + 2 * H, ld, 0, S, tid);
+
+    const int q = blockIdx.x * AT_CQ + wave * 16 + li, qr = min(q, S - 1);
+    bf16x8 qf[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+        qf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)qr * ld + 32 * s + 8 * g));
+
+    float m = -INFINITY, sum = 0.f;
+    float4_t oacc[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) oacc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < S; k0 += AT_CH) {
+        if (k0) __syncthreads();                       // the last chunk's fragments are read
+        kc.store(k_lds, k0, S, tid);
+        vc.store(v_lds, k0, S, tid);
+        __syncthreads();
+        if (k0 + AT_CH < S) {
+            kc.load(base + H, ld, k0 + AT_CH, S, tid);
+            vc.load(base + 2 * H, ld, k0 + AT_CH, S, tid);
+        }
+        float4_t sc[NT];
+        float top = m;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            sc[t] = float4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+            if (k0 + 16 * t >= S) continue;
+            float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(k_lds, 16 * t + li, s, g), qf[s], acc, 0, 0, 0);
+            if (k0 + 16 * t + 4 * g < S) sc[t] = acc;  // (seq is a multiple of 4)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) top = fmaxf(top, sc[t][e]);
+        }
+        top = fmaxf(top, __shfl_xor(top, 16, 64));
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        const float fade = __builtin_amdgcn_exp2f((m - top) * c);
+        m = top;
+        sum *= fade;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) oacc[dt] *= fade;
+#pragma unroll
+        for (int u = 0; u < NT / 2; ++u) {
+            if (k0 + 32 * u >= S) continue;
+            u16x8 p;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float v = __builtin_amdgcn_exp2f((sc[2 * u + e / 4][e % 4] - m) * c);
+                sum += v;
+                p[e] = at_f2bf(v);
+            }
+            const bf16x8 pf = __builtin_bit_cast(bf16x8, p);
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+                oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(v_lds, u, dt, li, g), pf, oacc[dt], 0, 0, 0);
+        }
+    }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    if (q >= S) return;
+    const float inv = 1.0f / sum;
+    if (lse2 && g == 0) lse2[(size_t)bh * S + q] = m * c + __builtin_amdgcn_logf(sum);
+    uint16_t* crow = ctx + ((size_t)b * S + q) * H + h * AT_D + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) at_store4(crow + 16 * dt, oacc[dt] * inv);
+}
+
+__global__ __launch_bounds__(AT_CT, 3) void attention_any_bwd_q_kernel(const uint16_t* __restrict__ qkv,
+                                                                    const uint16_t* __restrict__ ctx,
+                                                                    const uint16_t* __restrict__ dctx,
+                                                                    const float* __restrict__ lse2,
+                                                                    float* __restrict__ delta_out,
+                                                                    uint16_t* __restrict__ dqkv, int S, int heads, float c,
+                                                                    float scale) {
+    constexpr int NT = AT_CH / 16;
+    __shared__ __attribute__((aligned(16))) uint16_t k_lds[AT_CH * AT_P];
+    __shared__ __attribute__((aligned(16))) uint16_t v_lds[AT_CH * AT_P];
+
+    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+    const int li = lane % 16, g = lane / 16;
+    const int bh = blockIdx.y, b = bh / heads, h = bh % heads;
+    const int H = heads * AT_D, ld = 3 * H;
+    const uint16_t* base = qkv + (size_t)b * S * ld + h * AT_D;
+    AtChunk kc, vc;
+    kc.load(base + H, ld, 0, S, tid);
+    vc.load(base + 2 * H, ld, 0, S, tid);
+
+    const int q = blockIdx.x * AT_CQ + wave * 16 + li, qr = min(q, S - 1);
+    const size_t orow = ((size_t)b * S + qr) * H + h * AT_D;
+    bf16x8 qf[2], dof[2];
+    float delta = 0.f;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        qf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)qr * ld + 32 * s + 8 * g));
+        const u16x8 d8 = *(const u16x8*)(dctx + orow + 32 * s + 8 * g);
+        const u16x8 o8 = *(const u16x8*)(ctx + orow + 32 * s + 8 * g);
+        dof[s] = __builtin_bit_cast(bf16x8, d8);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) delta += at_bf2f(d8[j]) * at_bf2f(o8[j]);
+    }
+    delta += __shfl_xor(delta, 16, 64);
+    delta += __shfl_xor(delta, 32, 64);
+    const float l2 = lse2[(size_t)bh * S + qr];
+    if (g == 0 && q < S) delta_out[(size_t)bh * S + q] = delta;
+
+    float4_t qacc[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) qacc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < S; k0 += AT_CH) {
+        if (k0) __syncthreads();
+        kc.store(k_lds, k0, S, tid);
+        vc.store(v_lds, k0, S, tid);
+        __syncthreads();
+        if (k0 + AT_CH < S) {
+            kc.load(base + H, ld, k0 + AT_CH, S, tid);
+            vc.load(base + 2 * H, ld, k0 + AT_CH, S, tid);
+        }
+#pragma unroll 2
+        for (int u = 0; u < NT / 2; ++u) {
+            if (k0 + 32 * u >= S) break;
+            u16x8 dsp;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const int t = 2 * u + half;
+                float4_t sa = {0.f, 0.f, 0.f, 0.f}, da = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(k_lds, 16 * t + li, s, g), qf[s], sa, 0, 0, 0);
+                    da = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(v_lds, 16 * t + li, s, g), dof[s], da, 0, 0, 0);
+                }
+                const float l = k0 + 16 * t + 4 * g < S ? l2 : INFINITY;      // (keys past the sequence: P = 0)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float p = at_bf2f(at_f2bf(__builtin_amdgcn_exp2f(sa[e] * c - l)));
+                    dsp[4 * half + e] = at_f2bf(scale * p * (da[e] - delta));
+                }
+            }
+            const bf16x8 dsf = __builtin_bit_cast(bf16x8, dsp);
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+                qacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(k_lds, u, dt, li, g), dsf, qacc[dt], 0, 0, 0);
+        }
+    }
+    if (q >= S) return;
+    uint16_t* qrow = dqkv + ((size_t)b * S + q) * ld + h * AT_D + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) at_store4(qrow + 16 * dt, qacc[dt]);
+}
+
+__global__ __launch_bounds__(AT_CT, 3) void attention_any_bwd_kv_kernel(const uint16_t* __restrict__ qkv,
+                                                                     const uint16_t* __restrict__ dctx,
+                                                                     const float* __restrict__ lse2,
+                                                                     const float* __restrict__ delta,
+                                                                     uint16_t* __restrict__ dqkv, int S, int heads, float c,
+                                                                     float scale) {
+    constexpr int NT = AT_CH / 16;
+    __shared__ __attribute__((aligned(16))) uint16_t q_lds[AT_CH * AT_P];
+    __shared__ __attribute__((aligned(16))) uint16_t do_lds[AT_CH * AT_P];
+    __shared__ __attribute__((aligned(16))) float row_lds[2 * AT_CH];       // lse2, delta of the chunk's queries
+
+    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+    const int li = lane % 16, g = lane / 16;
+    const int bh = blockIdx.y, b = bh / heads, h = bh % heads;
+    const int H = heads * AT_D, ld = 3 * H;
+    const uint16_t* base = qkv + (size_t)b * S * ld + h * AT_D;
+    const uint16_t* dbase = dctx + (size_t)b * S * H + h * AT_D;
+    const float* rows = (tid < AT_CH ? lse2 : delta) + (size_t)bh * S;
+    AtChunk qc, dc;
+    float row;
+    auto load = [&](int q0) {
+        qc.load(base, ld, q0, S, tid);
+        dc.load(dbase, H, q0, S, tid);
+        // (queries past the sequence: P = 0)
+        row = q0 + tid % AT_CH < S ? rows[q0 + tid % AT_CH] : tid < AT_CH ? INFINITY : 0.f;
+    };
+    load(0);
+
+    const int key = blockIdx.x * AT_CQ + wave * 16 + li, kr = min(key, S - 1);
+    bf16x8 kf[2], vf[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        kf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)kr * ld + H + 32 * s + 8 * g));
+        vf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)kr * ld + 2 * H + 32 * s + 8 * g));
+    }
+
+    float4_t kacc[4], vacc[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) kacc[dt] = vacc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int q0 = 0; q0 < S; q0 += AT_CH) {
+        if (q0) __syncthreads();
+        qc.store(q_lds, q0, S, tid);
+        dc.store(do_lds, q0, S, tid);
+        row_lds[tid] = row;
+        __syncthreads();
+        if (q0 + AT_CH < S) load(q0 + AT_CH);
+#pragma unroll 2
+        for (int u = 0; u < NT / 2; ++u) {
+            if (q0 + 32 * u >= S) break;
+            u16x8 pp, dsp;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const int t = 2 * u + half;
+                float4_t sa = {0.f, 0.f, 0.f, 0.f}, da = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(q_lds, 16 * t + li, s, g), kf[s], sa, 0, 0, 0);
+                    da = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(do_lds, 16 * t + li, s, g), vf[s], da, 0, 0, 0);
+                }
+                const float4_t l2 = *(const float4_t*)(row_lds + 16 * t + 4 * g);
+                const float4_t dl = *(const float4_t*)(row_lds + AT_CH + 16 * t + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint16_t pb = at_f2bf(__builtin_amdgcn_exp2f(sa[e] * c - l2[e]));
+                    pp[4 * half + e] = pb;
+                    dsp[4 * half + e] = at_f2bf(scale * at_bf2f(pb) * (da[e] - dl[e]));
+                }
+            }
+            const bf16x8 pf = __builtin_bit_cast(bf16x8, pp), dsf = __builtin_bit_cast(bf16x8, dsp);
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+                vacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(do_lds, u, dt, li, g), pf, vacc[dt], 0, 0, 0);
+                kacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(q_lds, u, dt, li, g), dsf, kacc[dt], 0, 0, 0);
+            }
+        }
+    }
+    if (key >= S) return;
+    uint16_t* krow = dqkv + ((size_t)b * S + key) * ld + H + h * AT_D + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+        at_store4(krow + 16 * dt, kacc[dt]);
+        at_store4(krow + H + 16 * dt, vacc[dt]);
+    }
+}
+
 int at_check(const char* who, int batch, int seq, int heads, int head_dim) {
     PD_REQUIRE(batch > 0 && heads > 0, PD_ESHAPE, "%s: batch and heads must be positive", who);
-    PD_REQUIRE(head_dim == AT_D && (seq == 512 || seq == 256 || seq == 128), PD_ESHAPE,
-               "%s: needs head_dim 64 and seq 128, 256 or 512 (got %d, %d)", who, head_dim, seq);
+    PD_REQUIRE(pd_attention_fwd_supported(seq, head_dim), PD_ESHAPE,
+               "%s: needs head_dim 64 and seq a multiple of 8 (got %d, %d)", who, head_dim, seq);
     PD_REQUIRE((long long)batch * heads <= 65535, PD_ESHAPE, "%s: too many (batch, head) pairs", who);
     return PD_OK;
 }
@@ -336,7 +619,7 @@ int at_check(const char* who, int batch, int seq, int heads, int head_dim) {
 }  // namespace
 
 extern "C" int pd_attention_fwd_supported(int seq, int head_dim) {
-    return head_dim == AT_D && (seq == 512 || seq == 256 || seq == 128);
+    return head_dim == AT_D && seq > 0 && seq % 8 == 0 && seq <= 65536;
 }
 
 extern "C" int pd_attention_fwd_bf16(const uint16_t* qkv, uint16_t* ctx, uint16_t* probs, float* lse2, int batch,
@@ -354,7 +637,11 @@ extern "C" int pd_attention_fwd_bf16(const uint16_t* qkv, uint16_t* ctx, uint16_
         if (probs) attention_fwd_kernel<S_, true><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c); \
         else attention_fwd_kernel<S_, false><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);      \
     } while (0)
-    if (seq == 512) PD_AT_FWD(512);
+    const bool whole = seq == 512 || seq == 256 || seq == 128;
+    PD_REQUIRE(whole || !probs, PD_ESHAPE, "pd_attention_fwd_bf16: probabilities only for seq 128, 256 and 512");
+    if (!whole)
+        attention_any_fwd_kernel<<<dim3((seq + AT_CQ - 1) / AT_CQ, batch * heads), AT_CT, 0, s>>>(qkv, ctx, lse2, seq, heads, c);
+    else if (seq == 512) PD_AT_FWD(512);
     else if (seq == 256) PD_AT_FWD(256);
     else PD_AT_FWD(128);
 #undef PD_AT_FWD
@@ -380,7 +667,13 @@ extern "C" int pd_attention_bwd_bf16(const uint16_t* qkv, const uint16_t* ctx, c
         PD_CHECK_LAUNCH("pd_attention_bwd_bf16(dQ)");                                                                  \
         attention_bwd_kv_kernel<S_><<<grid, AT_THREADS, 0, s>>>(qkv, dctx, lse2, delta, dqkv, heads, c, scale);         \
     } while (0)
-    if (seq == 512) PD_AT_BWD(512);
+    const bool whole = seq == 512 || seq == 256 || seq == 128;
+    if (!whole) {
+        const dim3 any((seq + AT_CQ - 1) / AT_CQ, batch * heads);
+        attention_any_bwd_q_kernel<<<any, AT_CT, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+        PD_CHECK_LAUNCH("pd_attention_bwd_bf16(dQ)");
+        attention_any_bwd_kv_kernel<<<any, AT_CT, 0, s>>>(qkv, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    } else if (seq == 512) PD_AT_BWD(512);
     else if (seq == 256) PD_AT_BWD(256);
     else PD_AT_BWD(128);
 #undef PD_AT_BWD

@@ -1178,8 +1178,8 @@ def _batched(ta, tb, M, N, K, A, a_off, lda, B, b_off, ldb, C, c_off, ldc, alpha
 
 def attention_forward(qkv, batch, seq, heads, need_probs=False):
     """qkv: [batch*seq, 3H] bf16 (Q | K | V, heads contiguous inside each).  Returns (ctx [batch*seq, H],
-    aux) where aux is what attention_backward needs: on the fused path (head dimension 64, seq 128 / 256 /
-    512) the fp32 vector lse2 [batch, heads, seq], otherwise -- or with need_probs -- the bf16
+    aux) where aux is what attention_backward needs: on the fused path (head dimension 64, seq a multiple of 8)
+    the fp32 vector lse2 [batch, heads, seq], otherwise -- or with need_probs -- the bf16
     probabilities [batch, heads, seq, seq]."""
     _mat_bf16(qkv, "qkv")
     H = qkv.size(1) // 3
@@ -1189,7 +1189,7 @@ def attention_forward(qkv, batch, seq, heads, need_probs=False):
                          % (tuple(qkv.shape), batch, seq, heads))
     dev = qkv.device
     ctx = torch.empty((batch * seq, H), dtype=BF16, device=dev)
-    if _cabi.lib().pd_attention_fwd_supported(seq, d):
+    if _cabi.lib().pd_attention_fwd_supported(seq, d) and (not need_probs or seq in (128, 256, 512)):
         probs = torch.empty((batch, heads, seq, seq), dtype=BF16, device=dev) if need_probs else None
         lse2 = None if need_probs else torch.empty((batch, heads, seq), dtype=torch.float32, device=dev)
         with _timed("attention_fwd", 4.0 * batch * heads * seq * seq * d):

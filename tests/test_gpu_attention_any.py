@@ -1,0 +1,65 @@
+"""Fused attention at any sequence length that is a multiple of 8 (chunks of 128 rows, blocks of 64 queries or keys, four
+waves of 16) against attention in fp32 from the same bf16 operands.
+
+Bound: P is rounded to bf16 once (2^-9 of it) and so is the result: 2-norm error below 2 x 2^-9 = 4e-3.  The backward
+rounds P, dS and its results, and reads a delta formed from the rounded context: 4 x 2^-9 = 8e-3."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+
+
+def _rel(a, b):
+    return float((a.double() - b.double()).norm() / b.double().norm())
+
+
+def _reference(qkv, dctx, B, S, h):
+    q, k, v = (t.reshape(B, S, h, 64).transpose(1, 2).float().contiguous().requires_grad_() for t in qkv.split(64 * h, 1))
+    o = torch.softmax(torch.matmul(q, k.transpose(2, 3).contiguous()) / 8, -1) @ v
+    o.backward(dctx.reshape(B, S, h, 64).transpose(1, 2).float().contiguous())
+    back = lambda t: t.transpose(1, 2).reshape(B * S, 64 * h)
+    return back(o.detach()), [back(t.grad) for t in (q, k, v)]
+
+
+@pytest.mark.parametrize("late", [False, True])
+@pytest.mark.parametrize("B,S,h", [(2, 8, 3), (1, 16, 2), (3, 24, 1), (2, 56, 2), (1, 64, 2), (2, 72, 3), (1, 120, 2), (2, 136, 2),
+                                   (3, 200, 12), (1, 248, 1), (2, 264, 2), (1, 384, 2), (1, 520, 2), (2, 640, 2)])
+def test_forward_and_backward(B, S, h, late):
+    """``late``: the largest scores of a query lie in its last keys, so that the running maximum rises with every chunk."""
+    from pipedream_amd import ops
+    g = torch.Generator().manual_seed(S)
+    qkv = torch.randn(B * S, 3 * 64 * h, generator=g)
+    if late:
+        ramp = torch.linspace(0.2, 4.0, S).repeat(B)[:, None]
+        qkv[:, 64 * h:128 * h] = qkv[:, 64 * h:128 * h].abs() * ramp * 0.5
+        qkv[:, :64 * h] = qkv[:, :64 * h].abs()
+    qkv, dctx = qkv.to(BF).cuda(), torch.randn(B * S, 64 * h, generator=g).to(BF).cuda()
+    ctx, lse2 = ops.attention_forward(qkv, B, S, h)
+    assert lse2.dtype == torch.float32 and lse2.shape == (B, h, S)
+    dqkv = ops.attention_backward(dctx, qkv, lse2, B, S, h, ctx=ctx)
+    ref, grads = _reference(qkv, dctx, B, S, h)
+    assert _rel(ctx, ref) < 4e-3
+    for name, got, want in zip("qkv", dqkv.split(64 * h, 1), grads):
+        # (late: nearly all weight on few keys, dS is a small difference of large numbers)
+        assert _rel(got, want) < (8e-3 if not late or name == "v" else 6e-2), name
+
+
+def test_rows_past_the_sequence_are_not_read_as_values():
+    """Each batch entry alone gives the same bits as inside the batch (its neighbour's rows lie behind its own), and a
+    NaN in one entry stays there."""
+    from pipedream_amd import ops
+    B, S, h = 3, 136, 2
+    g = torch.Generator().manual_seed(1)
+    qkv = torch.randn(B * S, 3 * 64 * h, generator=g).to(BF).cuda()
+    dctx = torch.randn(B * S, 64 * h, generator=g).to(BF).cuda()
+    qkv[2 * S:] = float("nan")
+    ctx, lse2 = ops.attention_forward(qkv, B, S, h)
+    dqkv = ops.attention_backward(dctx, qkv, lse2, B, S, h, ctx=ctx)
+    for b in range(2):
+        rows = slice(b * S, (b + 1) * S)
+        one, l1 = ops.attention_forward(qkv[rows].contiguous(), 1, S, h)
+        assert torch.equal(one, ctx[rows]) and torch.equal(l1[0], lse2[b])
+        assert torch.equal(ops.attention_backward(dctx[rows].contiguous(), qkv[rows].contiguous(), l1, 1, S, h, ctx=one), dqkv[rows])
+    assert torch.isnan(ctx[2 * S:].float()).all() and torch.isfinite(dqkv[:2 * S].float()).all()
