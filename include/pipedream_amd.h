@@ -496,6 +496,18 @@ int pd_colsum_batch(int n_jobs, const void* const* x, const int* is_bf16, float*
                     const int* N, const uint64_t* ld, const float* beta, float* workspace,
                     uint64_t workspace_floats, int splits, void* stream);
 
+/* A pre-LayerNorm transformer layer, x -> x2 = x + proj(attention(qkv(LN1(x)))) -> x2 + fc2(gelu(fc1(LN2(x2)))), on
+ * [batch*seq][hidden] activations: the launches of the entry points above as one call per pass.
+ * params / grads: weights and biases (fp32; the four matrices of params bf16) of ln1, qkv, proj, ln2, fc1, fc2 in this
+ * order, weight before bias, dense; bit i of `add`: grads[i] is added to, else written.  `saved` (written by the forward
+ * pass, read by the backward pass) and `work` (temporary) hold pd_transformer_layer_bytes() bytes, 256-byte aligned. */
+int pd_transformer_layer_bytes(int batch, int seq, int heads, int hidden, int ffn, uint64_t* saved, uint64_t* work);
+int pd_transformer_layer_fwd_bf16(const void* const* params, const uint16_t* x, void* saved, uint16_t* y, int batch,
+                                  int seq, int heads, int hidden, int ffn, float eps, void* stream);
+int pd_transformer_layer_bwd_bf16(const void* const* params, float* const* grads, uint32_t add, const uint16_t* x,
+                                  void* saved, const uint16_t* dy, void* work, uint16_t* dx, int batch, int seq,
+                                  int heads, int hidden, int ffn, void* stream);
+
 /* The label-smoothing criterion of the translation stages, LabelSmoothing.forward
  * (runtime/translation/seq2seq/train/smoothing.py:23-34): logits [R][V] (R = seq*batch rows of leading
  * dimension ld), fp32 log-softmax per row,

@@ -598,13 +598,22 @@ def _accumulate(p, fresh_fn, acc_fn):
 
 class _TransformerLayerFn(torch.autograd.Function):
     """x -> x + Attn(LN1(x)) -> . + FFN(LN2(.)), hand-written backward; every matrix product is
-    the bf16 MFMA GEMM, every reduction / pointwise op one of the bf16 HIP kernels."""
+    the bf16 MFMA GEMM, every reduction / pointwise op one of the bf16 HIP kernels.  Either pass is one native call
+    (pd_transformer_layer.hip); with the per-launch timer on, or operands that call does not take, its launches are
+    issued here, with the same results."""
 
     @staticmethod
     def forward(ctx, x, heads, eps, ln1_w, ln1_b, qkv_w, qkv_b, o_w, o_b, ln2_w, ln2_b, fc1_w, fc1_b, fc2_w, fc2_b):
         B, S, H = x.shape
         x2d = x.contiguous().view(B * S, H)
         bw = ops.bf16_weight
+        ctx.dims = (B, S, H, heads)
+        ctx.params = (ln1_w, ln1_b, qkv_w, qkv_b, o_w, o_b, ln2_w, ln2_b, fc1_w, fc1_b, fc2_w, fc2_b)
+        native = ops.transformer_layer_forward(x2d, ctx.params, B, S, heads, eps) if ops.kernel_timer is None else None
+        if native is not None:
+            y, saved = native
+            ctx.save_for_backward(x2d, saved)
+            return y.view(B, S, H)
         h1, mean1, rstd1 = ops.layernorm_forward(x2d, ln1_w, ln1_b, eps)
         qkv = ops.gemm_bf16(h1, bw(qkv_w), trans_b=True, bias=qkv_b)
         att, att_aux = ops.attention_forward(qkv, B, S, heads)
@@ -612,18 +621,23 @@ class _TransformerLayerFn(torch.autograd.Function):
         h2, mean2, rstd2 = ops.layernorm_forward(x2, ln2_w, ln2_b, eps)
         f, g = ops.gemm_bf16_gelu(h2, bw(fc1_w), trans_b=True, bias=fc1_b)      # g = gelu(f) in the epilogue
         y = ops.gemm_bf16(g, bw(fc2_w), trans_b=True, bias=fc2_b, residual=x2)
-        ctx.dims = (B, S, H, heads)
-        ctx.params = (ln1_w, ln1_b, qkv_w, qkv_b, o_w, o_b, ln2_w, ln2_b, fc1_w, fc1_b, fc2_w, fc2_b)
         ctx.save_for_backward(x2d, h1, mean1, rstd1, qkv, att_aux, att, x2, h2, mean2, rstd2, f, g)
         return y.view(B, S, H)
 
     @staticmethod
     def backward(ctx, dy):
         B, S, H, heads = ctx.dims
-        x2d, h1, mean1, rstd1, qkv, att_aux, att, x2, h2, mean2, rstd2, f, g = ctx.saved_tensors
+        x2d, *saved = ctx.saved_tensors
         ln1_w, ln1_b, qkv_w, qkv_b, o_w, o_b, ln2_w, ln2_b, fc1_w, fc1_b, fc2_w, fc2_b = ctx.params
         bw = ops.bf16_weight
         dy2 = dy.contiguous().view(B * S, H)
+        if len(saved) == 1:                       # of the native forward pass
+            if ops.kernel_timer is None:
+                dx = ops.transformer_layer_backward(dy2, x2d, saved[0], ctx.params, B, S, heads)
+                if dx is not None:
+                    return (dx.view(B, S, H), None, None) + (None,) * 12
+            saved = ops.transformer_layer_saved(saved[0], B, S, heads, H, fc1_w.size(0))
+        h1, mean1, rstd1, qkv, att_aux, att, x2, h2, mean2, rstd2, f, g = saved
         sums = ops.ColsumBatch()
 
         def linear_backward(d_out, inp, w, b, through_gelu_of=None):

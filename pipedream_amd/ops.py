@@ -1290,6 +1290,87 @@ def layernorm_backward(dy, x, gamma, mean, rstd, dgamma_acc=None, dbeta_acc=None
     return dx, outs[0], outs[1]
 
 
+_LAYER_MATRICES = frozenset((2, 4, 8, 10))      # qkv, proj, fc1, fc2 among a transformer layer's parameters
+
+
+@functools.lru_cache(maxsize=64)
+def _layer_bytes(batch, seq, heads, hidden, ffn):
+    saved, work = ctypes.c_uint64(), ctypes.c_uint64()
+    _cabi.lib().pd_transformer_layer_bytes(batch, seq, heads, hidden, ffn, ctypes.byref(saved), ctypes.byref(work))
+    return saved.value, work.value
+
+
+def _layer_params(params):
+    """A layer's parameters as the native calls take them (matrices as their bf16 images) and the tensors behind the
+    pointers, or None where one is not dense fp32 on the GPU."""
+    tensors = [bf16_weight(p) if i in _LAYER_MATRICES else p for i, p in enumerate(params)]
+    for i, t in enumerate(tensors):
+        if t.dtype != (BF16 if i in _LAYER_MATRICES else torch.float32) or not t.is_cuda or not t.is_contiguous():
+            return None
+    return (ctypes.c_void_p * 12)(*[t.data_ptr() for t in tensors]), tensors
+
+
+def transformer_layer_forward(x, params, batch, seq, heads, eps):
+    """(y, saved) of a pre-LayerNorm transformer layer on ``x`` [batch * seq, hidden], or None where the native call does not
+    take the operands.  ``params``: ln1, qkv, proj, ln2, fc1, fc2, each weight and bias."""
+    hidden, ffn = x.size(1), params[8].size(0)
+    if x.dtype != BF16 or not x.is_cuda or not x.is_contiguous() or x.numel() == 0 or hidden % heads:
+        return None
+    native = _layer_params(params)
+    if native is None:
+        return None
+    saved = torch.empty(_layer_bytes(batch, seq, heads, hidden, ffn)[0], dtype=torch.uint8, device=x.device)
+    y = torch.empty_like(x)
+    _cabi.lib().pd_transformer_layer_fwd_bf16(native[0], _ptr(x), _ptr(saved), _ptr(y), batch, seq, heads, hidden, ffn,
+                                              float(eps), _cabi.stream_ptr())
+    return y, saved
+
+
+def transformer_layer_saved(saved, batch, seq, heads, hidden, ffn):
+    """What the forward pass left in ``saved``, as tensors: h1, mean1, rstd1, qkv, attention's aux, attention, x2, h2, mean2,
+    rstd2, f, g (the order and 256-byte boundaries of pd_transformer_layer.hip)."""
+    rows = batch * seq
+    aux = (((batch, heads, seq), torch.float32) if _cabi.lib().pd_attention_fwd_supported(seq, hidden // heads)
+           else ((batch, heads, seq, seq), BF16))
+    wide, stat = ((rows, hidden), BF16), ((rows,), torch.float32)
+    out, at = [], 0
+    for shape, dtype in (wide, stat, stat, ((rows, 3 * hidden), BF16), aux, wide, wide, wide, stat, stat,
+                         ((rows, ffn), BF16), ((rows, ffn), BF16)):
+        n = dtype.itemsize
+        for d in shape:
+            n *= d
+        out.append(saved[at:at + n].view(dtype).view(shape))
+        at += -(-n // 256) * 256
+    return out
+
+
+def transformer_layer_backward(dy, x, saved, params, batch, seq, heads):
+    """dx of ``transformer_layer_forward``, or None where the native call does not take the operands; gradients are created
+    in, or added to, the parameters' ``grad``."""
+    hidden, ffn = x.size(1), params[8].size(0)
+    native = _layer_params(params)
+    if native is None or dy.dtype != BF16 or not dy.is_cuda or not dy.is_contiguous():
+        return None
+    grads = [p.grad for p in params]
+    if any(g is not None and (g.dtype != torch.float32 or not g.is_cuda or not g.is_contiguous()) for g in grads):
+        return None
+    add = 0
+    for i, p in enumerate(params):
+        if grads[i] is None:
+            grads[i] = torch.empty(p.shape, dtype=torch.float32, device=x.device)
+        else:
+            add |= 1 << i
+    work = torch.empty(_layer_bytes(batch, seq, heads, hidden, ffn)[1], dtype=torch.uint8, device=x.device)
+    dx = torch.empty_like(x)
+    _cabi.lib().pd_transformer_layer_bwd_bf16(native[0], (ctypes.c_void_p * 12)(*[g.data_ptr() for g in grads]), add, _ptr(x),
+                                              _ptr(saved), _ptr(dy), _ptr(work), _ptr(dx), batch, seq, heads, hidden, ffn,
+                                              _cabi.stream_ptr())
+    for i, p in enumerate(params):
+        if not add >> i & 1:
+            p.grad = grads[i]
+    return dx
+
+
 def gelu(x):
     y = torch.empty_like(x)
     _cabi.lib().pd_gelu_fwd_bf16(_ptr(x), _ptr(y), x.numel(), _cabi.stream_ptr())
