@@ -13,10 +13,12 @@
 // [K][lda] (trans_a = 1); op(B) is stored [K][ldb] (trans_b = 0) or [N][ldb]
 // (trans_b = 1, k-contiguous).
 //
-// A block of WM x WN waves owns a BM x BN tile; K runs in chunks of 64 through a
-// double-buffered LDS tile.  LDS bandwidth, not the matrix cores, limits small tiles: a
-// wave with a (32*TM) x (32*TN) tile reads (TM+TN) KB of fragments per TM*TN MFMAs, so the
-// large configuration gives every wave 128 x 64 and a block 256 x 256.
+// Three kernels: tiles of 64 x 64 to 256 x 256 fed by direct-to-LDS loads (nearly every product), k split over the waves of
+// a block (few tiles, deep reductions), and one that stages through registers, for operands whose rows lie 2^22 elements
+// and more apart.  LDS bandwidth, not the matrix cores, limits small tiles: a wave with a (32*TM) x (32*TN) tile reads
+// (TM+TN) KB of fragments per TM*TN MFMAs, so the largest gives every wave 128 x 128 and a block 256 x 256.
+// The staged kernel: a block of WM x WN waves owns a BM x BN tile; K runs in chunks of 64 through a double-buffered LDS
+// tile.
 //   * k-contiguous operand: LDS rows [row][64 k] with a pitch of 72 bf16; one
 //     conflict-free 128-bit read is one MFMA operand (8 k-values per lane).
 //   * row-contiguous operand (k is the slow index in memory): the tile is copied as it
@@ -104,11 +106,14 @@ __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint
 // element-wise path is used.
 // One staged 32-row block of a wave's tile -> C, for a block that lies inside the matrix: all LDS reads first,
 // then the operand loads, then the arithmetic and the 16-byte stores.  F32: fp32 output (BETA: accumulated into
-// C); RES: bf16 residual added; ACT: 1 = also store gelu(C) to aux_out, 2 = multiply by gelu'(aux_in).
-template <int TN, bool F32, bool BETA, bool RES, int ACT>
+// C); RES: bf16 residual added; ACT: 1 = also store gelu(C) to aux_out, 2 = multiply by gelu'(aux_in).  EDGE: rows past M
+// are left out (predicated, the batches stay).
+template <int TN, bool EDGE, bool F32, bool BETA, bool RES, int ACT>
 __device__ __forceinline__ void store_rows_full(const GemmBf16Args& a, const float* stage, int row0, int col0,
                                                 long long c_off, int lane) {
     constexpr int COLS = 32 * TN, P = COLS + 8;
+    const int rows = a.M - row0;
+    const auto inside = [&](int r) { return !EDGE || r < rows; };
     if constexpr (F32) {
         constexpr int LPR = COLS / 4, ITER = 32 * LPR / 64;
         const int c4 = (lane % LPR) * 4, r_in = lane / LPR;
@@ -118,10 +123,12 @@ __device__ __forceinline__ void store_rows_full(const GemmBf16Args& a, const flo
         float* const base = (float*)a.C + c_off + (long long)(row0 + r_in) * a.ldc + col0 + c4;
         if (BETA) {
 #pragma unroll
-            for (int it = 0; it < ITER; ++it) old[it] = *(const float4_t*)(base + (long long)it * (64 / LPR) * a.ldc);
+            for (int it = 0; it < ITER; ++it)
+                if (inside(it * (64 / LPR) + r_in)) old[it] = *(const float4_t*)(base + (long long)it * (64 / LPR) * a.ldc);
         }
 #pragma unroll
         for (int it = 0; it < ITER; ++it) {
+            if (!inside(it * (64 / LPR) + r_in)) continue;
             if (BETA) v[it] += a.beta * old[it];
             *(float4_t*)(base + (long long)it * (64 / LPR) * a.ldc) = v[it];
         }
@@ -139,16 +146,19 @@ __device__ __forceinline__ void store_rows_full(const GemmBf16Args& a, const flo
         if (RES) {
             const uint16_t* rb = a.residual + c_off + (long long)(row0 + r_in) * a.ldr + col0 + c8;
 #pragma unroll
-            for (int it = 0; it < ITER; ++it) extra[it] = *(const u16x8*)(rb + (long long)it * (64 / LPR) * a.ldr);
+            for (int it = 0; it < ITER; ++it)
+                if (inside(it * (64 / LPR) + r_in)) extra[it] = *(const u16x8*)(rb + (long long)it * (64 / LPR) * a.ldr);
         }
         if (ACT == 2) {
             const uint16_t* xb = a.aux_in + (long long)(row0 + r_in) * a.ld_aux + col0 + c8;
 #pragma unroll
-            for (int it = 0; it < ITER; ++it) extra[it] = *(const u16x8*)(xb + (long long)it * (64 / LPR) * a.ld_aux);
+            for (int it = 0; it < ITER; ++it)
+                if (inside(it * (64 / LPR) + r_in)) extra[it] = *(const u16x8*)(xb + (long long)it * (64 / LPR) * a.ld_aux);
         }
         uint16_t* const cb = (uint16_t*)a.C + c_off + (long long)(row0 + r_in) * a.ldc + col0 + c8;
 #pragma unroll
         for (int it = 0; it < ITER; ++it) {
+            if (!inside(it * (64 / LPR) + r_in)) continue;
             float v[8] = {v0[it][0], v0[it][1], v0[it][2], v0[it][3], v1[it][0], v1[it][1], v1[it][2], v1[it][3]};
             if (RES) {
 #pragma unroll
@@ -172,8 +182,8 @@ __device__ __forceinline__ void store_rows_full(const GemmBf16Args& a, const flo
     }
 }
 
-// A wave's whole tile, inside the matrix, in one output form: stage each 32-row block, then store it.
-template <int TM, int TN, bool F32, bool BETA, bool RES, int ACT>
+// A wave's whole tile, its columns inside the matrix, in one output form: stage each 32-row block, then store it.
+template <int TM, int TN, bool EDGE, bool F32, bool BETA, bool RES, int ACT>
 __device__ __forceinline__ void store_tile_full(const GemmBf16Args& a, float16_t (&acc)[TM][TN], const float (&bv)[TN],
                                                 int m0w, int n0w, long long c_off, float* stage, int lane) {
     constexpr int P = 32 * TN + 8;
@@ -185,8 +195,20 @@ __device__ __forceinline__ void store_tile_full(const GemmBf16Args& a, float16_t
 #pragma unroll
             for (int e = 0; e < 16; ++e)
                 stage[(8 * (e / 4) + 4 * h + (e % 4)) * P + j * 32 + idx] = a.alpha * acc[i][j][e] + bv[j];
-        store_rows_full<TN, F32, BETA, RES, ACT>(a, stage, m0w + i * 32, n0w, c_off, lane);
+        store_rows_full<TN, EDGE, F32, BETA, RES, ACT>(a, stage, m0w + i * 32, n0w, c_off, lane);
     }
+}
+
+template <int TM, int TN, bool EDGE>
+__device__ __forceinline__ void store_tile_form(const GemmBf16Args& a, float16_t (&acc)[TM][TN], const float (&bv)[TN],
+                                                int m0w, int n0w, long long c_off, float* stage, int lane) {
+    if (a.out_f32) {
+        if (a.beta != 0.f) store_tile_full<TM, TN, EDGE, true, true, false, 0>(a, acc, bv, m0w, n0w, c_off, stage, lane);
+        else store_tile_full<TM, TN, EDGE, true, false, false, 0>(a, acc, bv, m0w, n0w, c_off, stage, lane);
+    } else if (a.act == 1) store_tile_full<TM, TN, EDGE, false, false, false, 1>(a, acc, bv, m0w, n0w, c_off, stage, lane);
+    else if (a.act == 2) store_tile_full<TM, TN, EDGE, false, false, false, 2>(a, acc, bv, m0w, n0w, c_off, stage, lane);
+    else if (a.residual) store_tile_full<TM, TN, EDGE, false, false, true, 0>(a, acc, bv, m0w, n0w, c_off, stage, lane);
+    else store_tile_full<TM, TN, EDGE, false, false, false, 0>(a, acc, bv, m0w, n0w, c_off, stage, lane);
 }
 
 template <int TM, int TN>
@@ -229,18 +251,15 @@ __device__ __forceinline__ void store_tile(const GemmBf16Args& a, float16_t (&ac
         const int col = n0w + j * 32 + idx;
         bv[j] = (a.bias && col < a.N) ? a.bias[col] : 0.f;
     }
-    // The wave's tile lies inside the matrix (every transformer product): one loop per output form, without a
+    // The wave's columns lie inside the matrix (every transformer product): one loop per output form, without a
     // test inside, so that the LDS reads, the operand loads and the stores of a 32-row block are issued in
     // batches.  (With the form and the bounds tested per 16-byte vector every read waited for its own round
     // trip: 47 000 cycles for a 128 x 128 wave tile, more than the 256 x 256 kernel's whole k loop at K = 1024.)
-    if (m0w + 32 * TM <= a.M && n0w + 32 * TN <= a.N) {
-        if (a.out_f32) {
-            if (a.beta != 0.f) store_tile_full<TM, TN, true, true, false, 0>(a, acc, bv, m0w, n0w, c_off, stage, lane);
-            else store_tile_full<TM, TN, true, false, false, 0>(a, acc, bv, m0w, n0w, c_off, stage, lane);
-        } else if (a.act == 1) store_tile_full<TM, TN, false, false, false, 1>(a, acc, bv, m0w, n0w, c_off, stage, lane);
-        else if (a.act == 2) store_tile_full<TM, TN, false, false, false, 2>(a, acc, bv, m0w, n0w, c_off, stage, lane);
-        else if (a.residual) store_tile_full<TM, TN, false, false, true, 0>(a, acc, bv, m0w, n0w, c_off, stage, lane);
-        else store_tile_full<TM, TN, false, false, false, 0>(a, acc, bv, m0w, n0w, c_off, stage, lane);
+    // Tiles that stick out below the last row predicate the accesses instead.
+    if (n0w + 32 * TN <= a.N) {
+        if (m0w >= a.M) return;
+        if (m0w + 32 * TM <= a.M) store_tile_form<TM, TN, false>(a, acc, bv, m0w, n0w, c_off, stage, lane);
+        else store_tile_form<TM, TN, true>(a, acc, bv, m0w, n0w, c_off, stage, lane);
         return;
     }
 #pragma unroll
@@ -443,7 +462,7 @@ __global__ __launch_bounds__(64 * WM * WN) void pd_gemm_bf16_kernel(const GemmBf
 }
 
 // ---------------------------------------------------------------------------------------
-// Large-tile kernel: global -> LDS without passing through registers.
+// global -> LDS without passing through registers.
 //
 // With one 256 x 256 tile per CU, a chunk's loads must be issued several chunks ahead to
 // cover memory latency, and there are no registers to hold that much data in flight.
@@ -459,8 +478,8 @@ __global__ __launch_bounds__(64 * WM * WN) void pd_gemm_bf16_kernel(const GemmBf
 // The fragment reads are issued through inline assembly: the compiler cannot tell which
 // ring stage a direct-to-LDS load writes and would otherwise wait for *all* outstanding
 // loads before every LDS read; here the wait is an explicit vmcnt that leaves the younger
-// chunks in flight.  Requires K % 32 == 0 (no zero fill on this path); rows beyond M or N
-// are fetched from a clamped (valid) row and never stored.
+// chunks in flight.  Rows beyond M or N are fetched from a clamped (valid) row and never stored; for a K that the ring
+// does not divide a second instance of the kernel fetches zeros past its end.
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
 typedef __attribute__((address_space(1))) const void* global_void_ptr;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -471,6 +490,8 @@ constexpr int NS = 4;    // ring stages
 
 // One operand's part of the ring: where each lane fetches from and where the fragments are read.  NW waves fill it
 // together (4), or one fills and reads a ring of its own (1).
+__device__ __attribute__((aligned(16))) uint32_t g_zeros[4];      // what lies past the end of a reduction
+
 template <int ROWS, bool KC, int NW = 4>
 struct DmaTile {
     static constexpr int BYTES = ROWS * DK * 2;     // one stage
@@ -501,6 +522,11 @@ struct DmaTile {
     // different banks (256 bytes of them): a row of 128 or more elements always starts in the same bank, of 64 every
     // second row does, of 32 every fourth
     __device__ __forceinline__ static int granule_xor(int k) { return ROWS >= 128 ? k % 4 : ROWS == 64 ? (k >> 1) & 1 : 0; }
+    // k of this lane's 16 bytes of transfer t within its chunk
+    __device__ __forceinline__ static int k_of(int t, int wave, int lane) {
+        if (KC) return ((lane % 4) ^ ((lane / 16) & 3)) * 8;             // (row >> 2) & 3 = (lane / 16) & 3
+        return ((wave + NW * t) * 512 + lane * 8) / ROWS;
+    }
     // tile origin and per-chunk advance, in bytes (both wave-uniform)
     __device__ __forceinline__ static const char* origin(const uint16_t* g, int ld, int row0) {
         return (const char*)(KC ? g + (size_t)row0 * ld : g + row0);
@@ -578,7 +604,9 @@ __device__ __forceinline__ void wait_vmcnt() {
 //     every wave now holds all of chunk kt in registers, so stage kt is free
 //   step 1: MFMAs on the step-1 fragments; reads the step-0 fragments of stage kt+1 and
 //     issues the loads of chunk kt+NS into stage kt
-template <int BM, int BN, bool A_KC, bool B_KC>
+// TAIL: K is any multiple of 8.  The reduction is rounded up to whole ring rounds; a lane whose k lie past its end
+// fetches zeros instead (a compare and two selects per transfer), for both operands.
+template <int BM, int BN, bool A_KC, bool B_KC, bool TAIL>
 struct DmaGemm {
     static constexpr int TM = BM / 64, TN = BN / 64, NM = TM * TN;
     using TA = DmaTile<BM, A_KC>;
@@ -610,6 +638,7 @@ struct DmaGemm {
         size_t a_step, b_step;  // bytes per chunk
         char* ring;
         int wave;               // uniform
+        int K, lane;            // TAIL
         uint32_t fa_addr[TM][2], fb_addr[TN][2];   // LDS byte address of fragment (i, k-step s), stage 0
     };
 
@@ -631,15 +660,16 @@ struct DmaGemm {
     // direct-to-LDS load number d of chunk `chunk` into ring stage STG
     template <int STG>
     __device__ __forceinline__ static void dma_unit(const Ctx& c, int d, int chunk) {
+        const auto source = [&](const char* p, int k) { return !TAIL || chunk * DK + k < c.K ? p : (const char*)g_zeros; };
 #pragma unroll
         for (int t = 0; t < TA::PER_WAVE; ++t)
             if (d == t)
-                __builtin_amdgcn_global_load_lds((global_void_ptr)(c.a_org + chunk * c.a_step + c.ta.off[t]),
+                __builtin_amdgcn_global_load_lds((global_void_ptr)source(c.a_org + chunk * c.a_step + c.ta.off[t], TA::k_of(t, c.wave, c.lane)),
                                                  (lds_void_ptr)(c.ring + STG * TA::BYTES + (c.wave + 4 * t) * 1024), 16, 0, 0);
 #pragma unroll
         for (int t = 0; t < TB::PER_WAVE; ++t)
             if (d == TA::PER_WAVE + t)
-                __builtin_amdgcn_global_load_lds((global_void_ptr)(c.b_org + chunk * c.b_step + c.tb.off[t]),
+                __builtin_amdgcn_global_load_lds((global_void_ptr)source(c.b_org + chunk * c.b_step + c.tb.off[t], TB::k_of(t, c.wave, c.lane)),
                                                  (lds_void_ptr)(c.ring + RING_B + STG * TB::BYTES + (c.wave + 4 * t) * 1024), 16, 0, 0);
     }
 
@@ -679,9 +709,9 @@ struct DmaGemm {
     }
 };
 
-template <int BM, int BN, bool A_KC, bool B_KC>
+template <int BM, int BN, bool A_KC, bool B_KC, bool TAIL>
 __global__ __launch_bounds__(256, (BM * BN <= 128 * 128 ? 2 : 1)) void pd_gemm_bf16_dma_kernel(const GemmBf16Args a) {
-    using G = DmaGemm<BM, BN, A_KC, B_KC>;
+    using G = DmaGemm<BM, BN, A_KC, B_KC, TAIL>;
     using TA = typename G::TA;
     using TB = typename G::TB;
     constexpr int TM = G::TM, TN = G::TN, IPT = G::IPT;
@@ -714,7 +744,9 @@ __global__ __launch_bounds__(256, (BM * BN <= 128 * 128 ? 2 : 1)) void pd_gemm_b
     c.b_step = TB::chunk_bytes(a.ldb);
     c.ring = ring;
     c.wave = wave;
-    const int nk = a.K / DK;       // a multiple of NS
+    c.K = a.K;
+    c.lane = lane;
+    const int nk = TAIL ? (a.K + DK * NS - 1) / (DK * NS) * NS : a.K / DK;       // a multiple of NS
     // fill the ring: chunks 0 .. NS-1 into stages 0 .. NS-1
 #pragma unroll
     for (int d = 0; d < IPT; ++d) G::template dma_unit<0>(c, d, 0);
@@ -975,6 +1007,14 @@ int launch_gemm_bf16_ksplit(int tb, GemmBf16Args g, hipStream_t s) {
     return PD_OK;
 }
 
+template <int BM, int BN, bool TAIL>
+void launch_dma_layout(int ta, int tb, const GemmBf16Args& g, dim3 grid, hipStream_t s) {
+    if (!ta && tb) pd_gemm_bf16_dma_kernel<BM, BN, true, true, TAIL><<<grid, 256, 0, s>>>(g);
+    else if (!ta) pd_gemm_bf16_dma_kernel<BM, BN, true, false, TAIL><<<grid, 256, 0, s>>>(g);
+    else if (!tb) pd_gemm_bf16_dma_kernel<BM, BN, false, false, TAIL><<<grid, 256, 0, s>>>(g);
+    else if constexpr (BM == BN && BM <= 128) pd_gemm_bf16_dma_kernel<BM, BN, false, true, TAIL><<<grid, 256, 0, s>>>(g);
+}
+
 template <int BM, int BN>
 int launch_gemm_bf16_dma(int ta, int tb, GemmBf16Args g, int batch, hipStream_t s) {
     g.tiles_m = (g.M + BM - 1) / BM;
@@ -982,26 +1022,22 @@ int launch_gemm_bf16_dma(int ta, int tb, GemmBf16Args g, int batch, hipStream_t 
     g.total_tiles = g.tiles_m * g.tiles_n * batch;
     g.tiles_per_xcd = (g.total_tiles + N_XCD - 1) / N_XCD;
     const dim3 grid(g.tiles_per_xcd * N_XCD);
-    if (!ta && tb) pd_gemm_bf16_dma_kernel<BM, BN, true, true><<<grid, 256, 0, s>>>(g);
-    else if (!ta && !tb) pd_gemm_bf16_dma_kernel<BM, BN, true, false><<<grid, 256, 0, s>>>(g);
-    else if (ta && !tb) pd_gemm_bf16_dma_kernel<BM, BN, false, false><<<grid, 256, 0, s>>>(g);
-    else pd_gemm_bf16_dma_kernel<BM, BN, false, true><<<grid, 256, 0, s>>>(g);
+    if (g.K % (DK * NS) == 0) launch_dma_layout<BM, BN, false>(ta, tb, g, grid, s);
+    else if constexpr (BM < 256) launch_dma_layout<BM, BN, true>(ta, tb, g, grid, s);
     PD_CHECK_LAUNCH("pd_gemm_bf16");
     return PD_OK;
 }
 
-template <int BM, int BN, int WM, int WN>
-int launch_gemm_bf16(int ta, int tb, GemmBf16Args g, int batch, hipStream_t s) {
-    g.tiles_m = (g.M + BM - 1) / BM;
-    g.tiles_n = (g.N + BN - 1) / BN;
+int launch_gemm_bf16_staged(int ta, int tb, GemmBf16Args g, int batch, hipStream_t s) {
+    g.tiles_m = (g.M + 63) / 64;
+    g.tiles_n = (g.N + 63) / 64;
     g.total_tiles = g.tiles_m * g.tiles_n * batch;
     g.tiles_per_xcd = (g.total_tiles + N_XCD - 1) / N_XCD;
     const dim3 grid(g.tiles_per_xcd * N_XCD);
-    constexpr int NT = 64 * WM * WN;
-    if (!ta && tb) pd_gemm_bf16_kernel<BM, BN, WM, WN, true, true><<<grid, NT, 0, s>>>(g);
-    else if (!ta && !tb) pd_gemm_bf16_kernel<BM, BN, WM, WN, true, false><<<grid, NT, 0, s>>>(g);
-    else if (ta && !tb) pd_gemm_bf16_kernel<BM, BN, WM, WN, false, false><<<grid, NT, 0, s>>>(g);
-    else pd_gemm_bf16_kernel<BM, BN, WM, WN, false, true><<<grid, NT, 0, s>>>(g);
+    if (!ta && tb) pd_gemm_bf16_kernel<64, 64, 2, 2, true, true><<<grid, 256, 0, s>>>(g);
+    else if (!ta && !tb) pd_gemm_bf16_kernel<64, 64, 2, 2, true, false><<<grid, 256, 0, s>>>(g);
+    else if (ta && !tb) pd_gemm_bf16_kernel<64, 64, 2, 2, false, false><<<grid, 256, 0, s>>>(g);
+    else pd_gemm_bf16_kernel<64, 64, 2, 2, false, true><<<grid, 256, 0, s>>>(g);
     PD_CHECK_LAUNCH("pd_gemm_bf16");
     return PD_OK;
 }
@@ -1053,36 +1089,36 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     const int batch = batch_outer * batch_inner;
     hipStream_t s = (hipStream_t)stream;
     PD_REQUIRE((long long)((M + 63) / 64) * ((N + 63) / 64) * batch < (1ll << 28), PD_ESHAPE, "pd_gemm_bf16: too many tiles");
-    const long tiles256 = (long)((M + 255) / 256) * ((N + 255) / 256) * batch;
-    const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128) * batch;
-    // direct-to-LDS kernel: whole ring rounds of k, and per-lane byte offsets that fit 32 bits
-    const bool dma_ok = K % (DK * NS) == 0 && (long long)256 * (lda > ldb ? lda : ldb) * 2 < (1ll << 31);
-    const bool wide = M >= 256 && N >= 256;       // a 256 x 256 tile is mostly inside the matrix
-    if (g_force_bm && dma_ok) {
-        if (g_force_bm == 256 && g_force_bn == 256) return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
-        if (g_force_bm == 128 && g_force_bn == 128) return launch_gemm_bf16_dma<128, 128>(trans_a, trans_b, g, batch, s);
+    const auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
+    // direct-to-LDS kernels: per-lane byte offsets that fit 32 bits
+    const bool dma_ok = K > 0 && (long long)256 * (lda > ldb ? lda : ldb) * 2 < (1ll << 31);
+    if (!dma_ok) return launch_gemm_bf16_staged(trans_a, trans_b, g, batch, s);
+    const bool whole = K % (DK * NS) == 0, both_t = trans_a && trans_b;
+    if (g_force_bm && whole) {
+        if (g_force_bm == 256 && !both_t) return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
+        return launch_gemm_bf16_dma<128, 128>(trans_a, trans_b, g, batch, s);
     }
-    // Few output tiles: the reduction split over the waves of a block, with the smallest tile whose blocks still find a
-    // CU each (32 x 32, 32 x 64, 64 x 64).  us, weights from memory, against 128 x 128 tiles: 128 x 1024 x 4096 10.6 / 28,
-    // 128 x 1024 x 1024 5.0 / 8.8, 128 x 3072 x 1024 8.2 / 10.4, 600 x 768 x 3072 15.9 / 28.9, 600 x 768 x 768 8.1 / 8.8,
-    // 256 x 4096 x 1024 (256 blocks of 64 x 64) 10.4 / 10.4; with 360 blocks (600 x 2304 x 768) 15.2 / 9.4.
-    if (!g_force_bm && !trans_a && batch == 1 && g.vec_store && K % DK == 0 &&
-        (long long)64 * (lda > ldb ? lda : ldb) * 2 < (1ll << 31)) {
-        const auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    // Few output tiles and a deep reduction: k split over the waves of a block, with the smallest tile whose blocks still
+    // find a CU each (32 x 32, 32 x 64, 64 x 64).  What it saves grows with k, what it costs (more reads of the operands, a
+    // sum over eight waves) with the size of C: the line lies at k = 16 per tile of 64 x 64.  us, split / not, and k per
+    // tile: 128 x 1024 x 4096 8.7 / 14 (128), 88 x 768 x 768 4.6 / 5.4 (32), 600 x 768 x 3072 12.6 / 15.3 (26),
+    // 600 x 768 x 2304 9.5 / 11.3 (19), 640 x 1024 x 3072 15.2 / 15.5 (19), 200 x 768 x 768 5.2 / 5.4 (16), 1920 x 512 x 2048 15.3 / 11.4 (9), 600 x 768 x 768 7.9 / 4.9 (6),
+    // 200 x 3072 x 768 8.3 / 5.0 (4).
+    if (!trans_a && batch == 1 && g.vec_store && K % DK == 0 && K >= 16 * blocks(64, 64) && blocks(64, 64) <= 256) {
         if (blocks(32, 32) <= 256) return launch_gemm_bf16_ksplit<1, 1>(trans_b, g, s);
         if (blocks(32, 64) <= 256) return launch_gemm_bf16_ksplit<1, 2>(trans_b, g, s);
-        if (blocks(64, 64) <= 256) return launch_gemm_bf16_ksplit<2, 2>(trans_b, g, s);
+        return launch_gemm_bf16_ksplit<2, 2>(trans_b, g, s);
     }
     // 256 x 256 tiles (one block per CU, half the LDS reads per MFMA) from 192 tiles on, i.e. three quarters of
-    // the CUs busy: 4096 x 4096 x 1024 takes 41 us against 49 with 128 x 128 tiles, 4096 x 3072 x 1024 (192
-    // tiles) 34 against 39; products with fewer large tiles (4096 x 1024: 64) run two 128 x 128 blocks per CU.
-    if (dma_ok && wide && tiles256 >= 192) return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
-    if (dma_ok && M >= 128 && N >= 128) return launch_gemm_bf16_dma<128, 128>(trans_a, trans_b, g, batch, s);
-    if (wide && tiles256 >= 192) return launch_gemm_bf16<256, 256, 2, 4>(trans_a, trans_b, g, batch, s);
-    // narrow outputs (attention: N = head dimension): tall tiles, all waves stacked along M
-    if (N <= 64 && M >= 256) return launch_gemm_bf16<256, 64, 4, 1>(trans_a, trans_b, g, batch, s);
-    if (M >= 128 && N >= 128 && tiles128 >= 128) return launch_gemm_bf16<128, 128, 2, 2>(trans_a, trans_b, g, batch, s);
-    return launch_gemm_bf16<64, 64, 2, 2>(trans_a, trans_b, g, batch, s);
+    // the CUs busy: 4096 x 4096 x 1024 takes 39 us against 42 with 128 x 128 tiles.  Below, the largest tile that still
+    // gives every CU a block: us with 128 x 128, 64 x 128, 64 x 64: 2560 x 1024 x 1024 9.7 / 12.0 / 12.0 (160 blocks of
+    // 128 x 128), 600 x 2304 x 768 8.2 / 6.9 / 7.5 (180 of 64 x 128), 1240 x 1024 x 3072 25.8 / 18.6 / 23.3 (160),
+    // 1920 x 512 x 2048 17.7 / 13.1 / 11.4 (240 of 64 x 64), 768 x 768 x 600 9.9 / 8.2 / 6.5 (144).
+    if (whole && !both_t && M >= 256 && N >= 256 && blocks(256, 256) >= 192)
+        return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
+    if (blocks(64, 64) <= 256) return launch_gemm_bf16_dma<64, 64>(trans_a, trans_b, g, batch, s);
+    if (!both_t && blocks(64, 128) <= 256) return launch_gemm_bf16_dma<64, 128>(trans_a, trans_b, g, batch, s);
+    return launch_gemm_bf16_dma<128, 128>(trans_a, trans_b, g, batch, s);
 }
 
 extern "C" int pd_gemm_bf16_set_tile(int bm, int bn) {

@@ -1,0 +1,79 @@
+"""bf16 products at the edges of the kernels' tiles (32 to 256 rows and columns), of their rings (chunks of 32 k, rounds of
+128) and of the epilogue's row blocks, in all four layouts, against fp64 of the same bf16 operands.
+
+Bound: products of bf16 values are exact in fp32, a running sum is rounded once per 16 k and eight sums are added up at
+most: |error| <= (K / 16 + 16) 2^-24 sum |a| |b|, and for a bf16 result 2^-8 of its value."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+
+
+def _operand(rows, cols, g, pad=8):
+    """A matrix with NaNs behind every row and below the last one: nothing outside may be read as a value."""
+    big = torch.full((rows + 40, cols + pad), float("nan"), dtype=BF)
+    big[:rows, :cols] = torch.randn(rows, cols, generator=g).to(BF)
+    return big.cuda()[:rows, :cols]
+
+
+def _case(M, N, K, ta, tb, seed=0):
+    g = torch.Generator().manual_seed(seed + M + N + K)
+    a, b = _operand(*((K, M) if ta else (M, K)), g), _operand(*((N, K) if tb else (K, N)), g)
+    ad, bd = (a.t() if ta else a).double(), (b.t() if tb else b).double()
+    return a, b, ad @ bd, (K / 16 + 16) * 2.0 ** -24 * (ad.abs() @ bd.abs())
+
+
+SHAPES = [(8, 8, 8), (32, 64, 40), (64, 64, 128), (72, 56, 136), (64, 72, 3000), (88, 768, 768), (128, 128, 120), (136, 264, 600),
+          (200, 2304, 88), (600, 776, 200), (600, 3072, 256), (256, 1032, 1032), (1240, 1024, 72), (1920, 512, 512), (4096, 4104, 128),
+          (4040, 4096, 256), (64, 192, 4096), (640, 264, 2080), (200, 328, 7200)]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_product(M, N, K, ta, tb):
+    from pipedream_amd import ops
+    a, b, ref, bound = _case(M, N, K, ta, tb)
+    start = torch.randn(M, N).cuda()
+    out = start.clone()
+    ops.gemm_bf16(a, b, trans_a=bool(ta), trans_b=bool(tb), out=out, beta=1.0)
+    assert bool(((out.double() - ref - start.double()).abs() <= bound + 2.0 ** -22 * (ref.abs() + start.double().abs())).all())
+    y = ops.gemm_bf16(a, b, trans_a=bool(ta), trans_b=bool(tb))
+    assert bool(((y.double() - ref).abs() <= bound + 2.0 ** -8 * ref.abs()).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(72, 56, 136), (88, 768, 768), (600, 776, 200), (600, 3072, 256), (1240, 1024, 72), (640, 264, 2080),
+                                   (4040, 4096, 256)])
+def test_epilogues(M, N, K):
+    """Bias, residual, GELU and its derivative in tiles that stick out of the matrix; what lies behind the rows stays."""
+    from pipedream_amd import ops
+    a, b, ref, bound = _case(M, N, K, 0, 1)
+    bias, res = torch.randn(N).cuda(), torch.randn(M, N).to(BF).cuda()
+    wide = torch.zeros(M + 8, N + 8, dtype=BF).cuda()
+    ops.gemm_bf16(a, b, trans_b=True, bias=bias, residual=res, out=wide[:M, :N])
+    want = ref + bias.double() + res.double()
+    slack = bound + 2.0 ** -22 * (ref.abs() + bias.double().abs())
+    assert bool(((wide[:M, :N].double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all())
+    assert not wide[M:].any() and not wide[:, N:].any()
+    f, g = ops.gemm_bf16_gelu(a, b, trans_b=True, bias=bias)
+    assert bool(((f.double() - ref - bias.double()).abs() <= slack + 2.0 ** -8 * (ref + bias.double()).abs()).all())
+    torch.testing.assert_close(g.float(), torch.nn.functional.gelu(f.float()), rtol=2.0 ** -7, atol=2e-6)
+    w = b.t().contiguous()
+    df = ops.gemm_bf16_gelu_backward(a, w, f)
+    fr = f.double().requires_grad_()
+    torch.nn.functional.gelu(fr).sum().backward()
+    want = ref * fr.grad
+    assert bool(((df.double() - want).abs() <= (bound + 2.0 ** -8 * ref.abs()) * (fr.grad.abs() + 1e-6) + 2.0 ** -8 * want.abs() + 1e-6 * ref.abs()).all())
+
+
+def test_rows_far_apart():
+    """Leading dimensions of 2^22 elements: the kernel whose offsets are 64 bits wide."""
+    from pipedream_amd import ops
+    g = torch.Generator().manual_seed(3)
+    big = torch.zeros(20, 1 << 22, dtype=BF, device="cuda")
+    big[:, :200] = torch.randn(20, 200, generator=g).to(BF).cuda()
+    a, b = big[:, :200], torch.randn(72, 200, generator=g).to(BF).cuda()
+    y = ops.gemm_bf16(a, b, trans_b=True, out_f32=True)
+    ref = a.double() @ b.double().t()
+    assert bool(((y.double() - ref).abs() <= 32 * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t())).all())
