@@ -1295,90 +1295,106 @@ __global__ __launch_bounds__(WW_THREADS, 1) void winograd_wgrad_kernel(const Win
     if (gh == 0 && wn == 0) a.part_db[((size_t)(pair * a.ranks + rank) * 2 + h) * 64 + wm * 32 + cl] = db_acc;
 }
 
-constexpr int WW_SUM_GROUPS = 4;   // rank groups summed by different blocks (more loads in flight)
+// The ranks' partial dU of a pair lie as [element / 256][rank][element % 256]: a wave reads a rank's kilobyte.  All additions
+// are in a fixed order.
+// Few pairs have many ranks (256 / pairs) and few blocks in the final kernel: PER ranks at a time are first added up to one,
+// in the same layout.
+// us for the sums and the final kernel of 64 -> 64 / 64 -> 128 / 128 -> 128 / 512 -> 512 channels, 64 MB of partials each: 60 / 40 / 34 / 35 with
+// four groups of ranks whatever the pairs are, a test per load and a thread per filter element in the final kernel,
+// 18 / 17 / 18 / 13 now (64 MB at the rate of a large copy: 10).
+template <int PER>
+__global__ __launch_bounds__(256) void winograd_wgrad_sum_kernel(const float* __restrict__ part, float* __restrict__ out,
+                                                                 int ranks) {
+    const int groups = ranks / PER;
+    const long id = (long)blockIdx.x * 4 + (threadIdx.x >> 6);         // (pair and chunk of 256 elements, group)
+    const int lane = threadIdx.x & 63;
+    const float4_t* src = (const float4_t*)(part + (id / groups * ranks + id % groups * PER) * 256) + lane;
+    float4_t acc[8];
+#pragma unroll
+    for (int r = 0; r < PER; r += 8)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const float4_t v = src[(r + u) * 64];
+            acc[u] = r == 0 ? v : acc[u] + v;
+        }
+    const float4_t sum = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+    ((float4_t*)out)[id * 64 + lane] = sum;
+}
 
-// Sums of the ranks' partial dU (and partial dbias) of every pair: blockIdx.y picks a quarter of the
-// ranks, a thread owns four consecutive elements and keeps eight 16-byte loads in flight.  The order of
-// all additions is fixed.  du4 / db4: [group][pair][...].
-__global__ __launch_bounds__(256) void winograd_wgrad_sum_kernel(const float* __restrict__ part,
-                                                                 const float* __restrict__ part_db,
-                                                                 float* __restrict__ du4, float* __restrict__ db4,
-                                                                 int n_pairs, int ranks) {
-    const int per_pair = WW_PART_FLOATS / 4;
-    const int grp = blockIdx.y, r0 = grp * ranks / WW_SUM_GROUPS, r1 = (grp + 1) * ranks / WW_SUM_GROUPS;
-    const long id = (long)blockIdx.x * 256 + threadIdx.x;
-    if (id < (long)n_pairs * per_pair) {
-        const int pair = (int)(id / per_pair), i = (int)(id % per_pair);
-        // (layout [element / 256][rank][element % 256], see the kernel that writes it)
-        const float* src = part + (size_t)pair * ranks * WW_PART_STRIDE + (size_t)(i >> 6) * ranks * 256 + (i & 63) * 4;
-        float4_t acc[8];
+// dw[k][r][s][c] = (G^T dU[.][k][c] G)[r][s] with the signs of A's last row / column restored, and dbias.  A block has four
+// output channels and 64 input channels of a pair, wave i the transformed positions (i, 0..3): it adds up their ranks,
+// transforms along the columns, and the four waves meet in LDS for the other direction.
+template <int RANKS>
+__global__ __launch_bounds__(256) void winograd_wgrad_final_kernel(const float* __restrict__ part,
+                                                                   const float* __restrict__ part_db,
+                                                                   float* __restrict__ dw, float* __restrict__ db,
+                                                                   int C, int c_blocks, int db_ranks, int aligned) {
+    __shared__ __attribute__((aligned(16))) float4_t t_lds[4][3][64];
+    const int lane = threadIdx.x & 63, i = threadIdx.x >> 6;
+    const int pair = blockIdx.x / 16, kq = blockIdx.x % 16;
+    const float4_t* src = (const float4_t*)part + ((size_t)pair * (WW_PART_FLOATS / 256) + i * 64 + kq) * RANKS * 64 + lane;
+    float4_t u[4];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) acc[u] = float4_t{0.f, 0.f, 0.f, 0.f};
-        for (int r = r0; r < r1; r += 8) {
+    for (int m = 0; m < 4; ++m) {
+        float4_t v[RANKS];
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (r + u < r1) acc[u] += *(const float4_t*)(src + (size_t)(r + u) * 256);
-        }
-        ((float4_t*)du4)[(size_t)grp * n_pairs * per_pair + id] =
-            ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+        for (int r = 0; r < RANKS; ++r) v[r] = src[(m * 16 * RANKS + r) * 64];
+#pragma unroll
+        for (int w = 1; w < RANKS; w *= 2)             // neighbours first
+#pragma unroll
+            for (int r = 0; r < RANKS; r += 2 * w) v[r] += v[r + w];
+        u[m] = v[0];
     }
-    if (id < (long)n_pairs * 64) {
-        const int pair = (int)(id / 64), k = (int)(id % 64);
-        float sb[16];
+    if (i == 3) {
 #pragma unroll
-        for (int u = 0; u < 16; ++u) sb[u] = 0.f;
-        for (int r = 2 * r0; r < 2 * r1; r += 16) {
+        for (int m = 0; m < 3; ++m) u[m] = -u[m];
+    } else {
+        u[3] = -u[3];
+    }
+    t_lds[i][0][lane] = u[0] + 0.5f * (u[1] + u[2]);
+    t_lds[i][1][lane] = 0.5f * (u[1] - u[2]);
+    t_lds[i][2][lane] = u[3] + 0.5f * (u[1] + u[2]);
+    __syncthreads();
+    // (lane: four input channels of output channel lane / 16)
+    const int k = pair / c_blocks * 64 + kq * 4 + lane / 16, c = pair % c_blocks * 64 + lane % 16 * 4;
+    float* const out = dw + (size_t)k * 9 * C + c;
+    for (int p = i; p < 9; p += 4) {
+        const int row = p / 3, s = p % 3;
+        const float4_t t1 = t_lds[1][s][lane], t2 = t_lds[2][s][lane];
+        const float4_t o = row == 1 ? 0.5f * (t1 - t2) : t_lds[row == 0 ? 0 : 3][s][lane] + 0.5f * (t1 + t2);
+        if (aligned) *(float4_t*)(out + (size_t)p * C) = o;
+        else
 #pragma unroll
-            for (int u = 0; u < 16; ++u)
-                if (r + u < 2 * r1) sb[u] += part_db[((size_t)pair * ranks * 2 + r + u) * 64 + k];
+            for (int q = 0; q < 4; ++q) out[(size_t)p * C + q] = o[q];
+    }
+    if (db && pair % c_blocks == 0) {                  // wave i: output channel kq * 4 + i, a quarter of the ranks per 16 lanes
+        const float* e = part_db + (size_t)pair * db_ranks * 128 + kq * 4 + i;
+        const int end = 2 * ((lane / 16 + 1) * db_ranks / 4);
+        float v[8], sum = 0.f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {                  // (256 ranks at most)
+            const int at = 2 * (lane / 16 * db_ranks / 4) + lane % 16 + 16 * q;
+            v[q] = at < end ? e[(size_t)at * 64] : 0.f;
         }
 #pragma unroll
-        for (int w = 8; w >= 1; w >>= 1)
+        for (int q = 0; q < 8; ++q) sum += v[q];
 #pragma unroll
-            for (int u = 0; u < w; ++u) sb[u] += sb[u + w];
-        db4[(size_t)grp * n_pairs * 64 + id] = sb[0];
+        for (int d : {8, 4, 2, 1, 16, 32}) sum += __shfl_xor(sum, d);
+        if (lane == 0) db[pair / c_blocks * 64 + kq * 4 + i] = sum;
     }
 }
 
-// dw[k][r][s][c] = (G^T dU[.][k][c] G)[r][s] with the signs of A's last row / column restored, and dbias.
-__global__ __launch_bounds__(256) void winograd_wgrad_final_kernel(const float* __restrict__ du4,
-                                                                   const float* __restrict__ db4,
-                                                                   float* __restrict__ dw, float* __restrict__ db,
-                                                                   int K, int C, int c_blocks, int n_pairs) {
-    const long id = (long)blockIdx.x * 256 + threadIdx.x;
-    if (id >= (long)K * C) return;
-    const int c = (int)(id % C), k = (int)(id / C);
-    const int pair = (k / 64) * c_blocks + c / 64;
-    const float* src = du4 + (size_t)pair * WW_PART_FLOATS + (k % 64) * 64 + (c % 64);
-    const size_t gstride = (size_t)n_pairs * WW_PART_FLOATS;
-    float u[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const float* e = src + (i * 4 + m) * 64 * 64;
-            const float v = (e[0] + e[gstride]) + (e[2 * gstride] + e[3 * gstride]);
-            u[i][m] = ((i == 3) != (m == 3)) ? -v : v;
-        }
-    float t[4][3];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        t[i][0] = u[i][0] + 0.5f * (u[i][1] + u[i][2]);
-        t[i][1] = 0.5f * (u[i][1] - u[i][2]);
-        t[i][2] = u[i][3] + 0.5f * (u[i][1] + u[i][2]);
-    }
-    float* out = dw + (size_t)k * 9 * C + c;
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-        out[(0 * 3 + s) * C] = t[0][s] + 0.5f * (t[1][s] + t[2][s]);
-        out[(1 * 3 + s) * C] = 0.5f * (t[1][s] - t[2][s]);
-        out[(2 * 3 + s) * C] = t[3][s] + 0.5f * (t[1][s] + t[2][s]);
-    }
-    if (db && c == 0) {
-        const float* e = db4 + (size_t)((k / 64) * c_blocks) * 64 + (k % 64);
-        const size_t bs = (size_t)n_pairs * 64;
-        db[k] = (e[0] + e[bs]) + (e[2 * bs] + e[3 * bs]);
-    }
+// How many ranks the sum kernel adds up to one before the final kernel (to four in all; with eight and sixteen left the
+// final kernel takes 3 and 8 us longer); 1: the final kernel adds up all of them.
+int wino_wgrad_per(int pairs) {
+    const int ranks = WW_BLOCKS / pairs;
+    return ranks >= 32 ? ranks / 4 : 1;
+}
+
+template <int PER>
+void launch_wgrad_sum(const WinoWgradArgs& a, float* out, hipStream_t s) {
+    winograd_wgrad_sum_kernel<PER><<<dim3((unsigned)(a.n_pairs * (WW_PART_FLOATS / 256) * (a.ranks / PER) / 4)), 256, 0, s>>>(
+        a.part, out, a.ranks);
 }
 
 bool wino_wgrad_shape_ok(int C, int K) {
@@ -1406,8 +1422,9 @@ extern "C" int pd_conv3x3_winograd_wgrad_workspace_bytes(int C, int K, uint64_t*
                "pd_conv3x3_winograd_wgrad_workspace_bytes: needs C and K multiples of 64 with C*K/4096 a power "
                "of two <= 256 (C=%d K=%d)", C, K);
     const uint64_t pairs = (uint64_t)(C / 64) * (K / 64);
-    // per block: partial dU and 2 x 64 partial dbias; per pair and rank group: summed dU and dbias
-    *bytes = ((uint64_t)WW_BLOCKS * (WW_PART_STRIDE + 128) + WW_SUM_GROUPS * pairs * (WW_PART_FLOATS + 64)) * sizeof(float);
+    // per block: partial dU and 2 x 64 partial dbias; per pair and group of ranks: summed dU
+    const uint64_t per = wino_wgrad_per((int)pairs);
+    *bytes = ((uint64_t)WW_BLOCKS * (WW_PART_STRIDE + 128) + (per > 1 ? WW_BLOCKS / per * WW_PART_FLOATS : 0)) * sizeof(float);
     return PD_OK;
 }
 
@@ -1448,8 +1465,6 @@ extern "C" int pd_conv3x3_winograd_wgrad_nhwc_f32(const float* x, const float* d
     float* ws = (float*)workspace;
     a.part = ws;
     a.part_db = ws + (size_t)WW_BLOCKS * WW_PART_STRIDE;
-    float* du = a.part_db + (size_t)WW_BLOCKS * 128;
-    float* dbsum = du + (size_t)WW_SUM_GROUPS * a.n_pairs * WW_PART_FLOATS;
     hipStream_t s = (hipStream_t)stream;
     // The f16 kernel, where its blocks have at least two steps of 16 tiles (its error against 64 bits is 4 to 7 % above the
     // fp32 kernel's at 18 to 25 tiles a block, 8 % below it at 38, 40 % at 3000), x and dY lie within its offsets, and no
@@ -1461,12 +1476,22 @@ extern "C" int pd_conv3x3_winograd_wgrad_nhwc_f32(const float* x, const float* d
     else if (upright) winograd_wgrad_kernel<true><<<WW_BLOCKS, WW_THREADS, 0, s>>>(a);
     else winograd_wgrad_kernel<false><<<WW_BLOCKS, WW_THREADS, 0, s>>>(a);
     PD_CHECK_LAUNCH(who);
-    const long sum_threads = (long)a.n_pairs * (WW_PART_FLOATS / 4);
-    winograd_wgrad_sum_kernel<<<dim3((unsigned)((sum_threads + 255) / 256), WW_SUM_GROUPS), 256, 0, s>>>(
-        a.part, a.part_db, du, dbsum, a.n_pairs, a.ranks);
-    PD_CHECK_LAUNCH(who);
-    winograd_wgrad_final_kernel<<<(unsigned)(((long)K * C + 255) / 256), 256, 0, s>>>(du, dbsum, dw, dbias, K, C,
-                                                                                     a.c_blocks, a.n_pairs);
+    const int per = wino_wgrad_per(a.n_pairs);
+    const float* sums = a.part;
+    if (per > 1) {
+        float* const du = a.part_db + (size_t)WW_BLOCKS * 128;
+        if (per == 64) launch_wgrad_sum<64>(a, du, s);
+        else if (per == 32) launch_wgrad_sum<32>(a, du, s);
+        else if (per == 16) launch_wgrad_sum<16>(a, du, s);
+        else launch_wgrad_sum<8>(a, du, s);
+        PD_CHECK_LAUNCH(who);
+        sums = du;
+    }
+    const int left = a.ranks / per;
+    const auto final_kernel = left == 16 ? winograd_wgrad_final_kernel<16> : left == 8 ? winograd_wgrad_final_kernel<8>
+                              : left == 4 ? winograd_wgrad_final_kernel<4> : left == 2 ? winograd_wgrad_final_kernel<2>
+                                                                                       : winograd_wgrad_final_kernel<1>;
+    final_kernel<<<dim3(a.n_pairs * 16), 256, 0, s>>>(sums, a.part_db, dw, dbias, C, a.c_blocks, a.ranks, pd_aligned(dw, 16));
     PD_CHECK_LAUNCH(who);
     return PD_OK;
 }
