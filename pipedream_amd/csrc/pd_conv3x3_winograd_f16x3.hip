@@ -104,20 +104,23 @@ struct H3Layout {
 };
 
 // e(k, c) and its maxima over c.  0: all nine taps are zero (or NaN); denormals count as the smallest normal numbers.
+// (lanes: threads per output channel where the input channels are the innermost index of w, 64, 128 or 256: as many as
+// there are input channels to read, so that a thread waits for memory once.  A wave for all 512 took 7 us, 256 threads 4)
 __global__ __launch_bounds__(256) void winograd_exps_kernel(const float* __restrict__ w, char* __restrict__ u, int K, int C,
-                                                            int k_pad, int rot180) {
+                                                            int k_pad, int rot180, int lanes) {
+    __shared__ int red[256];
     const H3Layout at(K, C);
     uint8_t* const exps = (uint8_t*)(u + at.exps);
     int* const part = (int*)(u + at.part);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     auto exponent = [](float m) { return m > 0.f ? max((int)(__builtin_bit_cast(uint32_t, m) >> 23), 1) : 0; };
-    if (!rot180) {                                     // a wave per output channel, lanes along the input channels
-        const int k = blockIdx.x * 4 + wave;
-        if (k >= k_pad) return;
+    if (!rot180) {
+        const int k = blockIdx.x * (256 / lanes) + threadIdx.x / lanes;
         int top = 0;
         if (k < K) {
             const float* row = w + (size_t)k * 9 * C;
-            for (int c = lane; c < C; c += 64) {
+#pragma unroll 2
+            for (int c = threadIdx.x % lanes; c < C; c += lanes) {
                 float m = 0.f;
 #pragma unroll
                 for (int t = 0; t < 9; ++t) m = fmaxf(m, fabsf(row[(size_t)t * C + c]));
@@ -128,11 +131,15 @@ __global__ __launch_bounds__(256) void winograd_exps_kernel(const float* __restr
         }
 #pragma unroll
         for (int d = 32; d; d >>= 1) top = max(top, __shfl_xor(top, d));
-        if (lane == 0) part[k] = top;
+        if (lane == 0) red[wave] = top;
+        __syncthreads();
+        if (threadIdx.x % lanes == 0 && k < k_pad) {
+            for (int i = 1; i < lanes / 64; ++i) top = max(top, red[wave + i]);
+            part[k] = top;
+        }
         return;
     }
     // lanes along the output channels, 16 input channels per block
-    __shared__ int red[256];
     const int k = blockIdx.x * 64 + lane, slice = blockIdx.y;
     int top = 0;
     if (k < K) {
@@ -163,8 +170,7 @@ __global__ __launch_bounds__(256) void winograd_exps_kernel(const float* __restr
 __global__ __launch_bounds__(256) void winograd_filter_f16x3_kernel(const float* __restrict__ w, char* __restrict__ u,
                                                                     int slices, int K, int C, int k_pad, int rot180,
                                                                     int range) {
-    __shared__ int top_of[256];
-    __shared__ int s_part[4][H3_CC];
+    __shared__ uint32_t s_part[4][H3_CC / 2];
     const H3Layout at(K, C);
     const uint8_t* const exps = (const uint8_t*)(u + at.exps);
     const int* const part = (const int*)(u + at.part);
@@ -175,7 +181,7 @@ __global__ __launch_bounds__(256) void winograd_filter_f16x3_kernel(const float*
     const int cp = rot180 ? tid >> 5 : tid & 7, k32 = rot180 ? tid & 31 : tid >> 3;
     const int k = kb * WG_BN + kh * 32 + k32, c0 = chunk * H3_CC + cp * 2;
 
-    // (the kernel's nine taps and R(k) are requested first: what follows waits for memory twice per 256 output channels)
+    // (everything is requested before anything is waited for: taps, exponents and maxima of up to 512 output channels)
     float g[3][3][2];
 #pragma unroll
     for (int r = 0; r < 3; ++r)
@@ -185,46 +191,78 @@ __global__ __launch_bounds__(256) void winograd_filter_f16x3_kernel(const float*
             for (int e = 0; e < 2; ++e)
                 g[r][s][e] = k >= K ? 0.f : rot180 ? w[((size_t)(c0 + e) * 9 + (2 - r) * 3 + (2 - s)) * K + k]
                                                    : w[((size_t)k * 9 + r * 3 + s) * C + c0 + e];
+    const uint32_t own2 = k < K ? *(const uint16_t*)(exps + (size_t)k * C + c0) : 0;
+    // s(c) of the block's 16 channels over all k: a thread takes whole rows of them, 255 + e - R as 16 bits, 0 for no weights
+    typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+    u16x2_t best[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) best[i] = u16x2_t{0, 0};
     int top = 0;
-#pragma unroll 16
-    for (int sl = 0; sl < slices; ++sl) top = max(top, part[(size_t)sl * k_pad + k]);
-
-    // s(c) of the block's 16 channels, over all k in batches of 256: thread (k modulo 16, c)
-    constexpr int NONE = -1000;
-    int s_max = NONE;
-    for (int k0 = 0; k0 < K; k0 += 256) {
-        int e[16], row_top = 0;
+    for (int sl = 0; sl < slices; sl += 8) {
+        int v[8];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int kk = k0 + (tid >> 4) + 16 * i;
-            e[i] = kk < K ? exps[(size_t)kk * C + chunk * H3_CC + (tid & 15)] : 0;
-        }
-        if (k0 + tid < k_pad)
-#pragma unroll 16
-            for (int sl = 0; sl < slices; ++sl) row_top = max(row_top, part[(size_t)sl * k_pad + k0 + tid]);
-        __syncthreads();
-        top_of[tid] = row_top;
-        __syncthreads();
+        for (int q = 0; q < 8; ++q) v[q] = part[(size_t)min(sl + q, slices - 1) * k_pad + k];
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (e[i]) s_max = max(s_max, e[i] - top_of[(tid >> 4) + 16 * i]);
+        for (int q = 0; q < 8; ++q) top = max(top, v[q]);
     }
-    s_max = max(s_max, __shfl_xor(s_max, 16));
-    s_max = max(s_max, __shfl_xor(s_max, 32));
-    if ((tid & 63) < H3_CC) s_part[tid >> 6][tid & 15] = s_max;
+    for (int k0 = 0; k0 < K; k0 += 512) {
+        u32x4_t e[2];
+        int row_top[2] = {0, 0};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int kk = k0 + 256 * h + tid;
+            e[h] = kk < K ? *(const u32x4_t*)(exps + (size_t)kk * C + chunk * H3_CC) : u32x4_t{0, 0, 0, 0};
+        }
+        // (rows past the filter read the last one's maximum beside exponents of zero)
+        const int* const p0 = part + min(k0 + tid, k_pad - 1);
+        const int* const p1 = part + min(k0 + 256 + tid, k_pad - 1);
+        for (int sl = 0; sl < slices; sl += 8) {
+            int v[8][2];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const size_t at_slice = (size_t)min(sl + q, slices - 1) * k_pad;
+                v[q][0] = p0[at_slice];
+                v[q][1] = p1[at_slice];
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                row_top[0] = max(row_top[0], v[q][0]);
+                row_top[1] = max(row_top[1], v[q][1]);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t pair = e[h][i / 2] >> (16 * (i % 2));
+                const int lo = pair & 255, hi = pair >> 8 & 255;
+                const u16x2_t v = {(uint16_t)(lo ? 255 + lo - row_top[h] : 0), (uint16_t)(hi ? 255 + hi - row_top[h] : 0)};
+                best[i] = __builtin_elementwise_max(best[i], v);
+            }
+    }
+#pragma unroll
+    for (int d = 32; d; d >>= 1)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            best[i] = __builtin_elementwise_max(
+                best[i], __builtin_bit_cast(u16x2_t, __shfl_xor(__builtin_bit_cast(int, best[i]), d)));
+    if ((tid & 63) == 0)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s_part[tid >> 6][i] = __builtin_bit_cast(uint32_t, best[i]);
     __syncthreads();
+    constexpr int NONE = -1000;
     int shift[2];
     bool wide = top == 255;                                        // infinities
     const int field = top ? top : 127;                             // (a row of zeros)
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-        const int c = cp * 2 + e;
-        const int s = max(max(s_part[0][c], s_part[1][c]), max(s_part[2][c], s_part[3][c]));
+        const auto of = [&](int i) { return (int)(s_part[i][cp] >> (16 * e) & 0xffffu); };
+        const int v = max(max(of(0), of(1)), max(of(2), of(3))), s = v ? v - 255 : NONE;
         wide |= s != NONE && s < H3_MIN_SHIFT;
         shift[e] = max(s, H3_MIN_SHIFT);
         wide |= field + shift[e] < 13;                             // (the factor must stay finite)
         if (top && s != NONE) {
-            const int own = exps[(size_t)k * C + c0 + e];
+            const int own = own2 >> (8 * e) & 255;
             wide |= own == 0 || own - top - s < -range;
         }
     }
@@ -980,8 +1018,9 @@ extern "C" int pd_conv3x3_winograd_f16x3_filter_f32(const float* w, void* u, int
     const int k_blocks = (K + WG_BN - 1) / WG_BN, k_pad = k_blocks * WG_BN, n_chunks = C / H3_CC;
     const int slices = rot180 ? n_chunks : 1;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid = rot180 ? dim3(k_blocks, n_chunks) : dim3(k_pad / 4);
-    winograd_exps_kernel<<<grid, 256, 0, s>>>(w, (char*)u, K, C, k_pad, rot180);
+    const int lanes = C >= 256 ? 256 : C >= 128 ? 128 : 64;
+    const dim3 grid = rot180 ? dim3(k_blocks, n_chunks) : dim3(k_pad / (256 / lanes));
+    winograd_exps_kernel<<<grid, 256, 0, s>>>(w, (char*)u, K, C, k_pad, rot180, lanes);
     PD_CHECK_LAUNCH(who);
     winograd_filter_f16x3_kernel<<<dim3(n_chunks * 2, k_blocks), 256, 0, s>>>(w, (char*)u, slices, K, C, k_pad, rot180,
                                                                               h3_range(C));
