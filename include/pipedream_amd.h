@@ -161,6 +161,15 @@ int pd_gemm_f32(int trans_a, int trans_b, int M, int N, int K,
 int pd_gemm_splitk_f32(int trans_a, int trans_b, int M, int N, int K,
                        const float* A, int lda, const float* B, int ldb,
                        float* partials, int splits, void* stream);
+/* pd_gemm_f32 for at most 128 rows of an untransposed A, on the bf16 matrix pipes at fp32 accuracy (K a multiple
+ * of 8, lda and ldb of 4, for a plain B also N; A and B 16-byte aligned).  `splits` ranges of k
+ * (pd_gemm_skinny_f32x6_splits: about one block per CU) through partials[splits][M][N]; a split needs N and ldc
+ * multiples of 4 and 16-byte aligned C, bias and partials. */
+int pd_gemm_skinny_f32x6_splits(int M, int N, int K);
+int pd_gemm_skinny_f32x6(int trans_b, int M, int N, int K, const float* A, int lda, const float* B, int ldb,
+                         float beta, float* C, int ldc, const float* bias, int relu, int splits, float* partials,
+                         void* stream);
+/* C[M][ldc] = sum_s partials[s] (+ bias[N]) (+ beta*C) (ReLU); N and ldc multiples of 4. */
 int pd_splitk_reduce_f32(const float* partials, int splits, int M, int N, const float* bias, int relu,
                          float beta, float* C, int ldc, void* stream);
 
