@@ -302,6 +302,14 @@ int pd_conv3x3_winograd_f16x3_fwd_nhwc_f32(const float* x, const void* u, const 
                                            const float* out_mask, float* y, float* y_pool, uint8_t* pool_idx, const uint8_t* unpool_idx,
                                            float* y_full, int N, int H, int W, int C, int K, int relu,
                                            void* stream);
+/* The same convolution where a launch has few work items and many input channels: ranges of these by different blocks,
+ * into `partials` (pd_conv3x3_winograd_f16x3_split_bytes; 0 bytes: the shape is not split and this call refuses it),
+ * then their sum with bias, ReLU and output mask, or with ReLU and pooling. */
+int pd_conv3x3_winograd_f16x3_split_bytes(int N, int H, int W, int C, int K, uint64_t* bytes);
+int pd_conv3x3_winograd_f16x3_fwd_split_nhwc_f32(const float* x, const void* u, const float* bias, const float* out_mask,
+                                                 float* y, float* y_pool, uint8_t* pool_idx, void* partials,
+                                                 uint64_t partials_bytes, int N, int H, int W, int C, int K, int relu,
+                                                 void* stream);
 /* Weight (and optional bias) gradient of the same convolution in the Winograd domain: sums
  * dU = sum over 2x2 output tiles of (A dY A^T) (B^T d B) in persistent blocks, adds the blocks' partial
  * sums in fixed order and applies G^T . G.  Deterministic; agrees with pd_conv3x3_wgrad_nhwc_f32 to

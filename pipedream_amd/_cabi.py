@@ -96,6 +96,8 @@ SIGNATURES = {
     "pd_conv3x3_winograd_f16x3_filter_bytes": (_i, [_i, _i, ctypes.POINTER(_u64)], True),
     "pd_conv3x3_winograd_f16x3_filter_f32": (_i, [_vp, _vp, _i, _i, _i, _vp], True),
     "pd_conv3x3_winograd_f16x3_fwd_nhwc_f32": (_i, [_vp] * 10 + [_i] * 6 + [_vp], True),
+    "pd_conv3x3_winograd_f16x3_split_bytes": (_i, [_i] * 5 + [ctypes.POINTER(_u64)], True),
+    "pd_conv3x3_winograd_f16x3_fwd_split_nhwc_f32": (_i, [_vp] * 8 + [_u64] + [_i] * 6 + [_vp], True),
     "pd_conv3x3_winograd_wgrad_supported": (_i, [_i, _i], False),
     "pd_conv3x3_winograd_wgrad_workspace_bytes": (_i, [_i, _i, ctypes.POINTER(_u64)], True),
     "pd_conv3x3_winograd_wgrad_nhwc_f32": (_i, [_vp, _vp, _vp, _vp, _vp, _u64, _i, _i, _i, _i, _i, _vp], True),

@@ -319,10 +319,14 @@ __global__ __launch_bounds__(256) void winograd_filter_f16x3_kernel(const float*
 }
 
 // POOL, UNPOOL, STACKED, SEG: as in the fp32 kernel (a.u is the split filter, a.n_chunks counts chunks of 16).
-// MASK: the input is taken as 0 where a.mask <= 0.
-template <bool POOL, bool UNPOOL, bool STACKED, int SEG, bool MASK = false>
+// MASK: the input is taken as 0 where a.mask <= 0.  SPLIT: an item reduces over one of 2^split_log2 ranges of the input
+// channels and stores its sums alone (no bias, ReLU, mask); winograd_split_sum_kernel does the rest.
+template <bool POOL, bool UNPOOL, bool STACKED, int SEG, bool MASK = false, bool SPLIT = false>
 __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const WinoArgs a) {
-    static_assert((SEG == 1 || STACKED) && !(MASK && (STACKED || POOL || UNPOOL)), "variants that exist");
+    static_assert((SEG == 1 || STACKED) && !(MASK && (STACKED || POOL || UNPOOL)) && !(SPLIT && (MASK || POOL || UNPOOL)),
+                  "variants that exist");
+    const auto block_of = [&](int kb) { return SPLIT ? kb >> a.split_log2 : kb; };            // of output channels
+    const auto range_of = [&](int kb) { return SPLIT ? kb & ((1 << a.split_log2) - 1) : 0; };  // of input channels
     constexpr int SEGW = WG_PIX / SEG;
     constexpr int HALO_W = WG_PIX + 2 * SEG;
     constexpr int P = HALO_W / 2;                                  // columns of one parity
@@ -385,6 +389,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
             ximg = a.x + img;
             if (MASK) mimg = a.mask + img;
         }
+        const uint32_t range = SPLIT && i < n_my ? (uint32_t)(range_of(it->kb) * a.n_chunks) * (H3_CC * 4) : 0u;
         int t = tid;
         asm volatile("" : "+v"(t));            // (rows and columns are formed anew: kept, they would be spilled)
 #pragma unroll
@@ -395,7 +400,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
             const int gy = it->pos[sg][0] - 1 + row, gx = it->pos[sg][1] - 1 + col - sg * (SEGW + 2);
             // out of the buffer: reads 0
             const bool in = i < n_my && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W && p < PIECES;
-            loff[j] = in ? (uint32_t)((gy * a.W + gx) * a.C) * 4 + quarter * 16 : 0x80000000u;
+            loff[j] = in ? (uint32_t)((gy * a.W + gx) * a.C) * 4 + quarter * 16 + range : 0x80000000u;
         }
     };
     float4_t rawr[NP], rawm[MASK ? NP : 1];
@@ -445,12 +450,16 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         row3 = lds + ((r0 + 2) % a.img_h == 0 ? zeros : src_tile + 3 * (2 * P * 32));
     };
     int p_i = 0, p_cc = 0;                                         // item and chunk of the next patch
+    int p_range = 0;                                               // SPLIT: first chunk of its range
+    auto set_patch_range = [&](int i) {
+        if (SPLIT && i < n_my) p_range = __builtin_amdgcn_readfirstlane(range_of(items[i % H3_ITEMS].kb)) * a.n_chunks;
+    };
     int field = H3_MIN_FIELD;                                      // scale of the tile
     int inner = 0;                                                 // field of its inner pixels, all chunks of the item
     int shift[2];                                                  // s(c) of the thread's two channels of the next patch
     auto load_shift = [&]() {
         typedef int int2_t __attribute__((ext_vector_type(2)));
-        const int2_t v = *(const int2_t*)(u + at.shifts + (size_t)(p_cc * H3_CC + ch8 * 8 + (lane & 3) * 2) * 4);
+        const int2_t v = *(const int2_t*)(u + at.shifts + (size_t)((p_range + p_cc) * H3_CC + ch8 * 8 + (lane & 3) * 2) * 4);
         shift[0] = v[0];
         shift[1] = v[1];
     };
@@ -583,6 +592,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         o.ok = o.y < a.H && o.x < a.W && k < a.K;
         o.n = SEG == 1 ? __builtin_amdgcn_readfirstlane(it->n) : 0;
         o.img = (size_t)o.n * a.H * a.W * a.K;
+        if (SPLIT) o.img += __builtin_amdgcn_readfirstlane(range_of(it->kb)) * a.part_elems;
         o.off = (uint32_t)((o.y * a.W + o.x) * a.K + k);
         if (UNPOOL) {
             const __amdgpu_buffer_rsrc_t ir =
@@ -698,6 +708,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         if (++p_cc == a.n_chunks) {
             p_cc = 0;
             set_patch_rows(++p_i);
+            set_patch_range(p_i);
         }
     };
     int q = 0;                                                     // chunk of the whole sequence
@@ -716,6 +727,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         load_u(1);
         p_i = i;
         p_cc = 0;
+        set_patch_range(i);
         load_shift();
         if (tid == 0) *flag = 0;
         store_raw();
@@ -852,7 +864,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
             clear();
             set_load_item(m_i);
             set_patch_rows(m_i);
-            const int kfield = k_fields[kb * WG_BN + kh * 32 + (lane & 31)];
+            const int kfield = k_fields[block_of(kb) * WG_BN + kh * 32 + (lane & 31)];
             char* const v32 = lds + H3_SLOT1_OFF;
             u_kb = kb;
             u_cc = 0;
@@ -864,7 +876,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
                 store_raw();
                 __syncthreads();
                 const bool as_is = marks[(kb * a.n_chunks + cc) * 2 + kh] != 0;
-                const int4_t* const s8 = (const int4_t*)(u + at.shifts) + cc * 4 + (lane >> 5) * 2;
+                const int4_t* const s8 = (const int4_t*)(u + at.shifts) + (range_of(kb) * a.n_chunks + cc) * 4 + (lane >> 5) * 2;
                 const int4_t s_lo = s8[0], s_hi = s8[1];
                 if (cc + 1 < a.n_chunks) load_raw(cc + 1);
 #pragma unroll
@@ -920,7 +932,7 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
         // ---- epilogue of item m_i, 32 tiles at a time: a lane folds its four rows of M to two (A^T M), the staged
         //      sums are [column of positions][row][tile][channel]; then a thread has a tile and four channels, adds up the
         //      columns and stores the tile's 2 x 2 pixels.
-        const int k4 = kb * WG_BN + (tid & 15) * 4;
+        const int k4 = block_of(kb) * WG_BN + (tid & 15) * 4;
         load_channels(k4);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -969,6 +981,87 @@ __global__ __launch_bounds__(WG_THREADS, 1) void winograd_fwd_f16x3_kernel(const
     }
 }
 
+// y = the sum of the ranges' results + bias, ReLU, output mask; or its 2 x 2 maxima and index bytes (as the epilogue above
+// forms them).  A thread has four channels of a pixel or of a window.
+struct SplitSumArgs {
+    const float* part;
+    const float* bias;
+    const float* out_mask;
+    float* y;
+    float* pool_y;
+    uint8_t* pool_idx;
+    size_t part_elems;
+    int N, H, W, K, splits, relu;
+};
+template <bool POOL>
+__global__ __launch_bounds__(256) void winograd_split_sum_kernel(const SplitSumArgs a) {
+    const int K4 = a.K / 4, Ho = POOL ? a.H / 2 : a.H, Wo = POOL ? a.W / 2 : a.W;
+    const long id = (long)blockIdx.x * 256 + threadIdx.x;
+    if (id >= (long)a.N * Ho * Wo * K4) return;
+    const int k = (int)(id % K4) * 4;
+    const long pix = id / K4;
+    const int x = (int)(pix % Wo), y = (int)(pix / Wo % Ho);
+    const long n = pix / ((long)Wo * Ho);
+    constexpr int PX = POOL ? 4 : 1;
+    size_t at[PX];
+    float4_t v[PX];
+#pragma unroll
+    for (int p = 0; p < PX; ++p) {
+        at[p] = POOL ? ((size_t)(n * a.H + 2 * y + (p >> 1)) * a.W + 2 * x + (p & 1)) * a.K + k : (size_t)pix * a.K + k;
+        v[p] = *(const float4_t*)(a.part + at[p]);
+    }
+    for (int s = 1; s < a.splits; s += 3) {            // (2^n - 1 more of them, three in flight)
+        float4_t q[3][PX];
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+#pragma unroll
+            for (int p = 0; p < PX; ++p) q[u][p] = *(const float4_t*)(a.part + min(s + u, a.splits - 1) * a.part_elems + at[p]);
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+            if (s + u < a.splits)
+#pragma unroll
+                for (int p = 0; p < PX; ++p) v[p] += q[u][p];
+    }
+    if (a.bias) {
+#pragma unroll
+        for (int p = 0; p < PX; ++p)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[p][c] += a.bias[k + c];
+    }
+    if (a.relu) {
+#pragma unroll
+        for (int p = 0; p < PX; ++p)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[p][c] = v[p][c] > 0.f ? v[p][c] : 0.f;
+    }
+    if constexpr (POOL) {
+        float4_t best;
+        uint32_t packed = 0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            float b = v[0][c];
+            uint32_t arg = 0;
+#pragma unroll
+            for (int p = 1; p < 4; ++p) {
+                const bool take = v[p][c] > b || v[p][c] != v[p][c];
+                b = take ? v[p][c] : b;
+                arg = take ? (uint32_t)p : arg;
+            }
+            best[c] = b;
+            packed |= (arg | (b > 0.f ? 4u : 0u)) << (8 * c);
+        }
+        *(float4_t*)(a.pool_y + (size_t)pix * a.K + k) = best;
+        *(uint32_t*)(a.pool_idx + (size_t)pix * a.K + k) = packed;
+    } else {
+        if (a.out_mask) {
+            const float4_t m = *(const float4_t*)(a.out_mask + at[0]);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[0][c] = m[c] > 0.f ? v[0][c] : 0.f;
+        }
+        *(float4_t*)(a.y + at[0]) = v[0];
+    }
+}
+
 }  // namespace
 
 namespace {
@@ -985,6 +1078,21 @@ int h3_range(int C) {
     int bits = 0;
     while (1 << bits < C) ++bits;
     return 13 - (bits + 1) / 2;
+}
+
+// Into how many ranges of the input channels a launch's reduction is cut (1: it is not).  An item of 64 channels is
+// 28 000 cycles and every 16 more 4100, so a launch of few items with many channels leaves most CUs idle for long.  A cut
+// writes and reads the result once per range and costs a launch: from four chunks a range on, and while every item still
+// finds a CU.  us for 512 -> 512 channels with the filter's launches, uncut / cut: 8 images of 14 x 14 78 / 49 (4 ranges),
+// 1 image 77 / 35 (8), 4 images of 28 x 28 78 / 62 (2); 256 -> 256, 1 image of 56 x 56 50 / 35 (4).  With 128 input
+// channels there is nothing left to gain (1 image of 112 x 112 33 / 34).
+int h3_splits(const WinoArgs& a) {
+    int splits = 1;
+    if (a.n_chunks < 16) return 1;
+    while (2 * splits * (long)a.n_items <= 256 && a.n_chunks % (2 * splits) == 0 && a.n_chunks / (2 * splits) >= 4 &&
+           2 * splits * a.k_blocks <= H3_MAX_K_BLOCKS)
+        splits *= 2;
+    return splits;
 }
 
 template <bool STACKED, int SEG>
@@ -1063,6 +1171,67 @@ extern "C" int pd_conv3x3_winograd_f16x3_fwd_nhwc_f32(const float* x, const void
     else if (plan.seg == 4) h3_launch<true, 4>(a, grid, s);
     else if (plan.stacked) h3_launch<true, 1>(a, grid, s);
     else h3_launch<false, 1>(a, grid, s);
+    PD_CHECK_LAUNCH(who);
+    return PD_OK;
+}
+
+extern "C" int pd_conv3x3_winograd_f16x3_split_bytes(int N, int H, int W, int C, int K, uint64_t* bytes) {
+    const char* who = "pd_conv3x3_winograd_f16x3_split_bytes";
+    PD_REQUIRE(bytes && N > 0 && H > 0 && W > 0, PD_EINVAL, "%s: NULL pointer or empty tensor", who);
+    if (int rc = h3_shape(who, C, K)) return rc;
+    PD_REQUIRE((long)H * W * (C > K ? C : K) < (1L << 29), PD_ESHAPE, "%s: image too large", who);
+    WinoArgs a;
+    a.unpool_y = nullptr;
+    WinoPlan plan;
+    if (int rc = pd_wino_plan(who, a, N, H, W, C, K, H3_CC, true, &plan)) return rc;
+    const int splits = h3_splits(a);
+    *bytes = splits > 1 ? (uint64_t)splits * N * H * W * K * sizeof(float) : 0;
+    return PD_OK;
+}
+
+extern "C" int pd_conv3x3_winograd_f16x3_fwd_split_nhwc_f32(const float* x, const void* u, const float* bias,
+                                                            const float* out_mask, float* y, float* y_pool, uint8_t* pool_idx,
+                                                            void* partials, uint64_t partials_bytes, int N, int H, int W,
+                                                            int C, int K, int relu, void* stream) {
+    const char* who = "pd_conv3x3_winograd_f16x3_fwd_split_nhwc_f32";
+    uint64_t need = 0;
+    if (int rc = pd_conv3x3_winograd_f16x3_split_bytes(N, H, W, C, K, &need)) return rc;
+    PD_REQUIRE(need > 0, PD_ESHAPE, "%s: the reduction of this shape is not split", who);
+    PD_REQUIRE(x && u && partials && partials_bytes >= need, PD_EINVAL, "%s: NULL pointer or too few bytes", who);
+    PD_REQUIRE(y_pool ? pool_idx && !y && !out_mask && H >= 2 && W >= 2 : y && !pool_idx, PD_EINVAL,
+               "%s: y, or a pooled output with its index bytes", who);
+    PD_REQUIRE(pd_aligned(x, 16) && pd_aligned(u, 16) && pd_aligned(y, 16) && pd_aligned(out_mask, 16) && pd_aligned(y_pool, 16) &&
+                   pd_aligned(partials, 16) && pd_aligned(pool_idx, 4), PD_EINVAL,
+               "%s: tensors must be 16-byte aligned, index bytes 4-byte aligned", who);
+    WinoArgs a;
+    a.x = x; a.u = (const float*)u; a.bias = nullptr; a.mask = nullptr; a.out_mask = nullptr; a.y = (float*)partials;
+    a.pool_y = nullptr; a.pool_idx = nullptr; a.unpool_idx = nullptr; a.unpool_y = nullptr;
+    a.relu = 0;
+    WinoPlan plan;
+    if (int rc = pd_wino_plan(who, a, N, H, W, C, K, H3_CC, true, &plan)) return rc;
+    SplitSumArgs f;
+    f.splits = h3_splits(a);
+    a.split_log2 = __builtin_ctz((unsigned)f.splits);
+    a.part_elems = (size_t)N * H * W * K;
+    a.k_blocks *= f.splits;
+    a.n_chunks /= f.splits;
+    a.n_items *= f.splits;                             // (at most 256: a block each)
+    a.items_per_xcd = (a.n_items + WG_XCD - 1) / WG_XCD;
+    const dim3 grid((unsigned)a.items_per_xcd * WG_XCD);
+    hipStream_t s = (hipStream_t)stream;
+    if (plan.seg == 2) winograd_fwd_f16x3_kernel<false, false, true, 2, false, true><<<grid, WG_THREADS, 0, s>>>(a);
+    else if (plan.seg == 4) winograd_fwd_f16x3_kernel<false, false, true, 4, false, true><<<grid, WG_THREADS, 0, s>>>(a);
+    else if (plan.stacked) winograd_fwd_f16x3_kernel<false, false, true, 1, false, true><<<grid, WG_THREADS, 0, s>>>(a);
+    else winograd_fwd_f16x3_kernel<false, false, false, 1, false, true><<<grid, WG_THREADS, 0, s>>>(a);
+    PD_CHECK_LAUNCH(who);
+    f.part = (const float*)partials;
+    f.bias = bias; f.out_mask = out_mask; f.y = y; f.pool_y = y_pool; f.pool_idx = pool_idx;
+    f.part_elems = a.part_elems;
+    f.N = N; f.H = H; f.W = W; f.K = K; f.relu = relu != 0;
+    const long threads = y_pool ? (long)N * (H / 2) * (W / 2) * (K / 4) : (long)N * H * W * (K / 4);
+    const dim3 sum_grid((unsigned)((threads + 255) / 256));
+    if (y_pool) winograd_split_sum_kernel<true><<<sum_grid, 256, 0, s>>>(f);
+    else winograd_split_sum_kernel<false><<<sum_grid, 256, 0, s>>>(f);
     PD_CHECK_LAUNCH(who);
     return PD_OK;
 }

@@ -57,6 +57,8 @@ struct WinoArgs {
     int tiles_x, tiles_y, k_blocks, n_chunks;
     int segs_per_row, n_segs;     // segmented variant: pieces per 16 rows of the stacked batch, pieces in all
     int n_items, items_per_xcd;   // work items (pixel tile x channel block) in all / per die
+    int split_log2;         // f16 kernel, split reduction: k_blocks counts (channel block, range of input channels) pairs,
+    size_t part_elems;      // n_chunks the chunks of a range, y holds a result per range, part_elems apart
 };
 
 // How a launch divides its work (a's sizes, tiles, segments and items are filled in): persistent blocks, segments

@@ -702,6 +702,12 @@ def _winograd_conv(x, w, bias, in_mask, out_mask, n, h, wd, c, k, relu, rot180):
     return y
 
 
+def _conv_split_bytes(n, h, wd, c, k):
+    nbytes = ctypes.c_uint64()
+    _cabi.lib().pd_conv3x3_winograd_f16x3_split_bytes(n, h, wd, c, k, ctypes.byref(nbytes))
+    return nbytes.value
+
+
 def _winograd_run(x, w, bias, in_mask, out_mask, y, y_pool, pool_idx, unpool_idx, y_full, n, h, wd, c, k, relu, rot180):
     """Filter transform and convolution into the outputs given.  The products run on the f16 matrix pipes where the
     kernel for that takes the channel counts (16 | c >= 32, every layer of VGG16 but the first), else on the fp32 ones.
@@ -721,7 +727,16 @@ def _winograd_run(x, w, bias, in_mask, out_mask, y, y_pool, pool_idx, unpool_idx
         u = torch.empty(nbytes.value // 4, dtype=torch.float32, device=x.device)
         lib.pd_conv3x3_winograd_filter_f32(_ptr(w), _ptr(u), c, k, int(rot180), stream)
     with _timed("conv3x3_winograd_kernel", 18.0 * c * k * n * h * wd):
-        if split:
+        part_bytes = 0
+        if split and in_mask is None and y_full is None:
+            # (few work items with many input channels: ranges of these, added up by a second launch)
+            part_bytes = _conv_split_bytes(n, h, wd, c, k)
+        if part_bytes:
+            part = torch.empty(part_bytes, dtype=torch.uint8, device=x.device)
+            lib.pd_conv3x3_winograd_f16x3_fwd_split_nhwc_f32(_ptr(x), _ptr(u), _ptr(bias), _ptr(out_mask), _ptr(y),
+                                                             _ptr(y_pool), _ptr(pool_idx), _ptr(part), part_bytes, n, h,
+                                                             wd, c, k, int(relu), stream)
+        elif split:
             lib.pd_conv3x3_winograd_f16x3_fwd_nhwc_f32(_ptr(x), _ptr(u), _ptr(bias), _ptr(in_mask), _ptr(out_mask),
                                                        _ptr(y), _ptr(y_pool), _ptr(pool_idx), _ptr(unpool_idx),
                                                        _ptr(y_full), n, h, wd, c, k, int(relu), stream)
