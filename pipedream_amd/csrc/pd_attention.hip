@@ -11,10 +11,10 @@
 // Bound: MFMA bf16 / vector ALU (seq * seq exponentials per head); algorithmic HBM traffic = qkv
 // (and ctx, dctx in the backward) read once per kernel, ctx / dqkv written once.
 //
-// seq 128, 256, 512 (others: "any sequence length" below).  One block = one (batch, head) pair x 128 queries (or keys), 8 waves of 16.  The other side's two
-// [seq][64] matrices are staged in LDS once per block with a row pitch of 72 bf16, which serves both
-// the 128-bit fragment reads (8 consecutive k per lane) and the transposing reads.  Everything is
-// computed in the orientation in which no accumulator ever has to change layout; shown for the
+// Forward at seq 128 and 256 (all else: "any sequence length" below): one block = one (batch, head)
+// pair x 128 queries, 8 waves of 16, K and V of the head staged in LDS once
+// per block with a row pitch of 72 bf16, which serves both the 128-bit fragment reads (8 consecutive
+// k per lane) and the transposing reads.  Everything is computed in the orientation in which no accumulator ever has to change layout; shown for the
 // forward (v_mfma_f32_16x16x32_bf16: lane l holds A row / B column l % 16, k-slots 8 (l / 16) + 0..7,
 // and accumulator column l % 16, rows 4 (l / 16) + 0..3):
 //   S^T = K Q^T   A = K rows from LDS (k = head dimension), B = this wave's Q rows straight from
@@ -173,170 +173,26 @@ __global__ __launch_bounds__(AT_THREADS) void attention_fwd_kernel(const uint16_
     for (int dt = 0; dt < 4; ++dt) at_store4(crow + 16 * dt, oacc[dt]);
 }
 
-// ---- backward, query side -----------------------------------------------------------------------------
-// Per query block: P^T = 2^(K Q^T c - lse2), dP^T = V dO^T, dS^T = P^T o (dP^T - delta) / sqrt(d) with
-// delta_q = sum_d dO[q][d] O[q][d] (= sum_k dP[q][k] P[q][k]), dQ^T = K^T dS^T.  The key tiles are
-// processed two at a time, so nothing of size seq lives in registers.  delta is also written out
-// for the key-side kernel.
-template <int S>
-__global__ __launch_bounds__(AT_THREADS) void attention_bwd_q_kernel(const uint16_t* __restrict__ qkv,
-                                                                    const uint16_t* __restrict__ ctx,
-                                                                    const uint16_t* __restrict__ dctx,
-                                                                    const float* __restrict__ lse2,
-                                                                    float* __restrict__ delta_out,
-                                                                    uint16_t* __restrict__ dqkv, int heads, float c,
-                                                                    float scale) {
-    constexpr int NT = S / 16;
-    __shared__ __attribute__((aligned(16))) uint16_t k_lds[S * AT_P];
-    __shared__ __attribute__((aligned(16))) uint16_t v_lds[S * AT_P];
-
-    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-    const int li = lane % 16, g = lane / 16;
-    const int bh = blockIdx.y, b = bh / heads, h = bh % heads;
-    const int H = heads * AT_D, ld = 3 * H;
-    const uint16_t* base = qkv + (size_t)b * S * ld + h * AT_D;
-    at_stage<S>(k_lds, base + H, ld, tid);
-    at_stage<S>(v_lds, base + 2 * H, ld, tid);
-
-    const int q = blockIdx.x * AT_QB + wave * 16 + li;
-    const size_t orow = ((size_t)b * S + q) * H + h * AT_D;
-    bf16x8 qf[2], dof[2];
-    float delta = 0.f;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        qf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)q * ld + 32 * s + 8 * g));
-        const u16x8 d8 = *(const u16x8*)(dctx + orow + 32 * s + 8 * g);
-        const u16x8 o8 = *(const u16x8*)(ctx + orow + 32 * s + 8 * g);
-        dof[s] = __builtin_bit_cast(bf16x8, d8);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) delta += at_bf2f(d8[j]) * at_bf2f(o8[j]);
-    }
-    delta += __shfl_xor(delta, 16, 64);
-    delta += __shfl_xor(delta, 32, 64);
-    const float l2 = lse2[(size_t)bh * S + q];
-    if (g == 0) delta_out[(size_t)bh * S + q] = delta;
-    __syncthreads();
-
-    float4_t qacc[4];
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) qacc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int u = 0; u < NT / 2; ++u) {
-        u16x8 dsp;
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int t = 2 * u + half;
-            float4_t sa = {0.f, 0.f, 0.f, 0.f}, da = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(k_lds, 16 * t + li, s, g), qf[s], sa, 0, 0, 0);
-                da = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(v_lds, 16 * t + li, s, g), dof[s], da, 0, 0, 0);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                // P is rounded to bf16 as the forward pass did before using it
-                const float p = at_bf2f(at_f2bf(__builtin_amdgcn_exp2f(sa[e] * c - l2)));
-                dsp[4 * half + e] = at_f2bf(scale * p * (da[e] - delta));
-            }
-        }
-        const bf16x8 dsf = __builtin_bit_cast(bf16x8, dsp);
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-            qacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(k_lds, u, dt, li, g), dsf, qacc[dt], 0, 0, 0);
-    }
-
-    uint16_t* qrow = dqkv + ((size_t)b * S + q) * ld + h * AT_D + 4 * g;     // the Q third of dqkv
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) at_store4(qrow + 16 * dt, qacc[dt]);
-}
-
-// ---- backward, key side --------------------------------------------------------------------------------
-// Per key block, looping over all queries: S = Q K^T and dP = dO V^T now have the queries on the MFMA
-// rows (A operands = Q and dO rows from LDS, B = this wave's K and V rows from global memory), so lane
-// l holds key l % 16 and queries 16 t + 4 (l / 16) + e: P and dS land packed as B operands of the sums
-// over queries dV^T = dO^T P and dK^T = Q^T dS, whose A operands are transposing reads of dO and Q.
-template <int S>
-__global__ __launch_bounds__(AT_THREADS) void attention_bwd_kv_kernel(const uint16_t* __restrict__ qkv,
-                                                                     const uint16_t* __restrict__ dctx,
-                                                                     const float* __restrict__ lse2,
-                                                                     const float* __restrict__ delta,
-                                                                     uint16_t* __restrict__ dqkv, int heads, float c,
-                                                                     float scale) {
-    constexpr int NT = S / 16;
-    __shared__ __attribute__((aligned(16))) uint16_t q_lds[S * AT_P];
-    __shared__ __attribute__((aligned(16))) uint16_t do_lds[S * AT_P];
-
-    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-    const int li = lane % 16, g = lane / 16;
-    const int bh = blockIdx.y, b = bh / heads, h = bh % heads;
-    const int H = heads * AT_D, ld = 3 * H;
-    const uint16_t* base = qkv + (size_t)b * S * ld + h * AT_D;
-    at_stage<S>(q_lds, base, ld, tid);
-    at_stage<S>(do_lds, dctx + (size_t)b * S * H + h * AT_D, H, tid);
-
-    const int key = blockIdx.x * AT_QB + wave * 16 + li;
-    bf16x8 kf[2], vf[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        kf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)key * ld + H + 32 * s + 8 * g));
-        vf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)key * ld + 2 * H + 32 * s + 8 * g));
-    }
-    const float* l2p = lse2 + (size_t)bh * S + 4 * g;
-    const float* dlp = delta + (size_t)bh * S + 4 * g;
-    __syncthreads();
-
-    float4_t kacc[4], vacc[4];
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) kacc[dt] = vacc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int u = 0; u < NT / 2; ++u) {
-        u16x8 pp, dsp;
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int t = 2 * u + half;
-            float4_t sa = {0.f, 0.f, 0.f, 0.f}, da = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(q_lds, 16 * t + li, s, g), kf[s], sa, 0, 0, 0);
-                da = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(do_lds, 16 * t + li, s, g), vf[s], da, 0, 0, 0);
-            }
-            const float4_t l2 = *(const float4_t*)(l2p + 16 * t);       // queries 16 t + 4 g + (0..3)
-            const float4_t dl = *(const float4_t*)(dlp + 16 * t);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint16_t pb = at_f2bf(__builtin_amdgcn_exp2f(sa[e] * c - l2[e]));
-                pp[4 * half + e] = pb;
-                dsp[4 * half + e] = at_f2bf(scale * at_bf2f(pb) * (da[e] - dl[e]));
-            }
-        }
-        const bf16x8 pf = __builtin_bit_cast(bf16x8, pp), dsf = __builtin_bit_cast(bf16x8, dsp);
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-            vacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(do_lds, u, dt, li, g), pf, vacc[dt], 0, 0, 0);
-            kacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(q_lds, u, dt, li, g), dsf, kacc[dt], 0, 0, 0);
-        }
-    }
-
-    uint16_t* krow = dqkv + ((size_t)b * S + key) * ld + H + h * AT_D + 4 * g;    // the K third; V third at +H
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-        at_store4(krow + 16 * dt, kacc[dt]);
-        at_store4(krow + H + 16 * dt, vacc[dt]);
-    }
-}
-
-// ---- any sequence length ---------------------------------------------------------------------------------
+// ---- any sequence length: forward, backward -----------------------------------------------------------------
 // The other side's rows pass through LDS in chunks of AT_CH (the next chunk is on its way to the registers while one is
-// used), so seq is a run-time number: a multiple of 8, rows past it are zeros in LDS and masked.  A block has 64 queries
-// (keys), four waves of 16, 168 registers (three blocks a CU; with 212 and two, forward at 8 x 16 heads x 640 52 us instead
-// of 38).  The forward keeps a running maximum and sum per query and rescales what it has when the maximum rises.
-// us forward / backward, against the batched products and softmax kernels that took these shapes before: 3 x 12 heads x
-// 200 10 / 14 (23 / 31), 8 x 16 x 640 38 / 103 (115 / 192), 5 x 8 x 328 10 / 22 (32 / 53); error of the context (2-norm)
-// 2.2e-3 (4.2e-3: the scores went through bf16).  At 512 and 256 the kernels above are as fast forward and 4-17 % faster
-// backward, and stay.
+// used), so seq is a run-time number: a multiple of 8, rows past it are zeros in LDS and masked.  A wave has QT times 16
+// queries (keys), a block four waves.
+// Forward: a running maximum and sum per query; what is there is rescaled when the maximum rises.
+// Backward, query side: P^T = 2^(K Q^T c - lse2), dP^T = V dO^T, dS^T = P^T o (dP^T - delta) / sqrt(d) with
+// delta_q = sum_d dO[q][d] O[q][d] (= sum_k dP[q][k] P[q][k]), dQ^T = K^T dS^T; delta is also written out for the key side.
+// Backward, key side: S = Q K^T and dP = dO V^T have the queries on the MFMA rows (A operands = Q and dO rows from LDS, B =
+// this wave's K and V rows from global memory), so lane l holds key l % 16 and queries 16 t + 4 (l / 16) + e: P and dS land
+// packed as B operands of the sums over queries dV^T = dO^T P and dK^T = Q^T dS, whose A operands are transposing reads.
+//
+// Bound: fragment reads from LDS, a kilobyte per MFMA of 16 cycles with QT = 1 (256 bytes a cycle for four SIMDs), half of
+// that with QT = 2; registers (116-160 and 163-213) leave three and two blocks a CU.
+// us forward / backward: 8 x 16 heads x 512 24 / 62 (30 / 74 with QT = 1 or a head's K and V whole in LDS, 105 / 183 as
+// batched products with softmax kernels), 8 x 16 x 640 37 / 90 (115 / 192 as batched products), 3 x 12 x 200 6 / 14 (QT = 2:
+// 7 / 18; 23 / 31 with launches as batched products).  QT = 2 from 256 of its blocks on, one per CU: 8 x 16 x 256 (256
+// blocks) 9 / 23 against 11 / 28, 5 x 8 x 328 (120) 10 / 24 against 8 / 22.  Error of the context (2-norm) 2.2e-3, as batched
+// products, whose scores go through bf16, 4.2e-3.
 constexpr int AT_CH = 128;
 constexpr int AT_CT = 256;             // threads
-constexpr int AT_CQ = 64;              // queries (keys) per block
 
 // chunk of rows [r0, r0 + AT_CH) x 64 columns: global -> registers, registers -> LDS
 struct AtChunk {
@@ -359,9 +215,13 @@ struct AtChunk {
     }
 };
 
-__global__ __launch_bounds__(AT_CT, 3) void attention_any_fwd_kernel(const uint16_t* __restrict__ qkv,
-                                                                  uint16_t* __restrict__ ctx, float* __restrict__ lse2,
-                                                                  int S, int heads, float c) {
+// WRITE_P: the probabilities, which need the sums, by a second pass over the keys (the first pass' bits stay the same).
+template <int QT, bool WRITE_P>
+__global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_fwd_kernel(const uint16_t* __restrict__ qkv,
+                                                                                   uint16_t* __restrict__ ctx,
+                                                                                   uint16_t* __restrict__ probs,
+                                                                                   float* __restrict__ lse2, int S, int heads,
+                                                                                   float c) {
     constexpr int NT = AT_CH / 16;
     __shared__ __attribute__((aligned(16))) uint16_t k_lds[AT_CH * AT_P];
     __shared__ __attribute__((aligned(16))) uint16_t v_lds[AT_CH * AT_P];
@@ -375,16 +235,23 @@ __global__ __launch_bounds__(AT_CT, 3) void attention_any_fwd_kernel(const uint1
     kc.load(base + H, ld, 0, S, tid);
     vc.load(base + 2 * H, ld, 0, S, tid);
 
-    const int q = blockIdx.x * AT_CQ + wave * 16 + li, qr = min(q, S - 1);
-    bf16x8 qf[2];
+    const int q0 = (blockIdx.x * 4 + wave) * 16 * QT + li;            // tile j of the wave: query q0 + 16 j
+    bf16x8 qf[QT][2];
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
-        qf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)qr * ld + 32 * s + 8 * g));
+    for (int j = 0; j < QT; ++j)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            qf[j][s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)min(q0 + 16 * j, S - 1) * ld + 32 * s + 8 * g));
 
-    float m = -INFINITY, sum = 0.f;
-    float4_t oacc[4];
+    float m[QT], sum[QT];
+    float4_t oacc[QT][4];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) oacc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < QT; ++j) {
+        m[j] = -INFINITY;
+        sum[j] = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) oacc[j][dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    }
     for (int k0 = 0; k0 < S; k0 += AT_CH) {
         if (k0) __syncthreads();                       // the last chunk's fragments are read
         kc.store(k_lds, k0, S, tid);
@@ -394,60 +261,108 @@ __global__ __launch_bounds__(AT_CT, 3) void attention_any_fwd_kernel(const uint1
             kc.load(base + H, ld, k0 + AT_CH, S, tid);
             vc.load(base + 2 * H, ld, k0 + AT_CH, S, tid);
         }
-        float4_t sc[NT];
-        float top = m;
+        float4_t sc[QT][NT];
+        float top[QT];
+#pragma unroll
+        for (int j = 0; j < QT; ++j) top[j] = m[j];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            sc[t] = float4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+            for (int j = 0; j < QT; ++j) sc[j][t] = float4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
             if (k0 + 16 * t >= S) continue;
-            float4_t acc = {0.f, 0.f, 0.f, 0.f};
+            float4_t acc[QT];
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(k_lds, 16 * t + li, s, g), qf[s], acc, 0, 0, 0);
-            if (k0 + 16 * t + 4 * g < S) sc[t] = acc;  // (seq is a multiple of 4)
+            for (int j = 0; j < QT; ++j) acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) top = fmaxf(top, sc[t][e]);
+            for (int s = 0; s < 2; ++s) {
+                const bf16x8 kf = at_frag(k_lds, 16 * t + li, s, g);
+#pragma unroll
+                for (int j = 0; j < QT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[j][s], acc[j], 0, 0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < QT; ++j) {
+                if (k0 + 16 * t + 4 * g < S) sc[j][t] = acc[j];       // (seq is a multiple of 4)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) top[j] = fmaxf(top[j], sc[j][t][e]);
+            }
         }
-        top = fmaxf(top, __shfl_xor(top, 16, 64));
-        top = fmaxf(top, __shfl_xor(top, 32, 64));
-        const float fade = __builtin_amdgcn_exp2f((m - top) * c);
-        m = top;
-        sum *= fade;
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) oacc[dt] *= fade;
+        for (int j = 0; j < QT; ++j) {
+            top[j] = fmaxf(top[j], __shfl_xor(top[j], 16, 64));
+            top[j] = fmaxf(top[j], __shfl_xor(top[j], 32, 64));
+            const float fade = __builtin_amdgcn_exp2f((m[j] - top[j]) * c);
+            m[j] = top[j];
+            sum[j] *= fade;
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) oacc[j][dt] *= fade;
+        }
 #pragma unroll
         for (int u = 0; u < NT / 2; ++u) {
             if (k0 + 32 * u >= S) continue;
-            u16x8 p;
+            bf16x8 pf[QT];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float v = __builtin_amdgcn_exp2f((sc[2 * u + e / 4][e % 4] - m) * c);
-                sum += v;
-                p[e] = at_f2bf(v);
+            for (int j = 0; j < QT; ++j) {
+                u16x8 p;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float v = __builtin_amdgcn_exp2f((sc[j][2 * u + e / 4][e % 4] - m[j]) * c);
+                    sum[j] += v;
+                    p[e] = at_f2bf(v);
+                }
+                pf[j] = __builtin_bit_cast(bf16x8, p);
             }
-            const bf16x8 pf = __builtin_bit_cast(bf16x8, p);
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
-                oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(v_lds, u, dt, li, g), pf, oacc[dt], 0, 0, 0);
+            for (int dt = 0; dt < 4; ++dt) {
+                const bf16x8 vt = at_frag_t(v_lds, u, dt, li, g);
+#pragma unroll
+                for (int j = 0; j < QT; ++j)
+                    oacc[j][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, pf[j], oacc[j][dt], 0, 0, 0);
+            }
         }
     }
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
-    if (q >= S) return;
-    const float inv = 1.0f / sum;
-    if (lse2 && g == 0) lse2[(size_t)bh * S + q] = m * c + __builtin_amdgcn_logf(sum);
-    uint16_t* crow = ctx + ((size_t)b * S + q) * H + h * AT_D + 4 * g;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) at_store4(crow + 16 * dt, oacc[dt] * inv);
+    for (int j = 0; j < QT; ++j) {
+        const int q = q0 + 16 * j;
+        sum[j] += __shfl_xor(sum[j], 16, 64);
+        sum[j] += __shfl_xor(sum[j], 32, 64);
+        if (q >= S) continue;
+        const float inv = 1.0f / sum[j];
+        if (lse2 && g == 0) lse2[(size_t)bh * S + q] = m[j] * c + __builtin_amdgcn_logf(sum[j]);
+        uint16_t* crow = ctx + ((size_t)b * S + q) * H + h * AT_D + 4 * g;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) at_store4(crow + 16 * dt, oacc[j][dt] * inv);
+    }
+    if (!WRITE_P) return;
+    for (int k0 = 0; k0 < S; k0 += AT_CH) {
+        __syncthreads();
+        kc.load(base + H, ld, k0, S, tid);
+        kc.store(k_lds, k0, S, tid);
+        __syncthreads();
+        for (int t = 0; t < NT; ++t) {
+            const int key = k0 + 16 * t + 4 * g;
+#pragma unroll
+            for (int j = 0; j < QT; ++j) {
+                float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(k_lds, 16 * t + li, s, g), qf[j][s], acc, 0, 0, 0);
+                const float inv = 1.0f / sum[j];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = __builtin_amdgcn_exp2f((acc[e] - m[j]) * c) * inv;
+                if (key < S && q0 + 16 * j < S) at_store4(probs + ((size_t)bh * S + q0 + 16 * j) * S + key, acc);
+            }
+        }
+    }
 }
 
-__global__ __launch_bounds__(AT_CT, 3) void attention_any_bwd_q_kernel(const uint16_t* __restrict__ qkv,
-                                                                    const uint16_t* __restrict__ ctx,
-                                                                    const uint16_t* __restrict__ dctx,
-                                                                    const float* __restrict__ lse2,
-                                                                    float* __restrict__ delta_out,
-                                                                    uint16_t* __restrict__ dqkv, int S, int heads, float c,
-                                                                    float scale) {
+template <int QT>
+__global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_bwd_q_kernel(const uint16_t* __restrict__ qkv,
+                                                                                     const uint16_t* __restrict__ ctx,
+                                                                                     const uint16_t* __restrict__ dctx,
+                                                                                     const float* __restrict__ lse2,
+                                                                                     float* __restrict__ delta_out,
+                                                                                     uint16_t* __restrict__ dqkv, int S,
+                                                                                     int heads, float c, float scale) {
     constexpr int NT = AT_CH / 16;
     __shared__ __attribute__((aligned(16))) uint16_t k_lds[AT_CH * AT_P];
     __shared__ __attribute__((aligned(16))) uint16_t v_lds[AT_CH * AT_P];
@@ -461,27 +376,34 @@ __global__ __launch_bounds__(AT_CT, 3) void attention_any_bwd_q_kernel(const uin
     kc.load(base + H, ld, 0, S, tid);
     vc.load(base + 2 * H, ld, 0, S, tid);
 
-    const int q = blockIdx.x * AT_CQ + wave * 16 + li, qr = min(q, S - 1);
-    const size_t orow = ((size_t)b * S + qr) * H + h * AT_D;
-    bf16x8 qf[2], dof[2];
-    float delta = 0.f;
+    const int q0 = (blockIdx.x * 4 + wave) * 16 * QT + li;
+    bf16x8 qf[QT][2], dof[QT][2];
+    float delta[QT], l2[QT];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        qf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)qr * ld + 32 * s + 8 * g));
-        const u16x8 d8 = *(const u16x8*)(dctx + orow + 32 * s + 8 * g);
-        const u16x8 o8 = *(const u16x8*)(ctx + orow + 32 * s + 8 * g);
-        dof[s] = __builtin_bit_cast(bf16x8, d8);
+    for (int j = 0; j < QT; ++j) {
+        const int q = q0 + 16 * j, qr = min(q, S - 1);
+        const size_t orow = ((size_t)b * S + qr) * H + h * AT_D;
+        delta[j] = 0.f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) delta += at_bf2f(d8[j]) * at_bf2f(o8[j]);
+        for (int s = 0; s < 2; ++s) {
+            qf[j][s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)qr * ld + 32 * s + 8 * g));
+            const u16x8 d8 = *(const u16x8*)(dctx + orow + 32 * s + 8 * g);
+            const u16x8 o8 = *(const u16x8*)(ctx + orow + 32 * s + 8 * g);
+            dof[j][s] = __builtin_bit_cast(bf16x8, d8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) delta[j] += at_bf2f(d8[e]) * at_bf2f(o8[e]);
+        }
+        delta[j] += __shfl_xor(delta[j], 16, 64);
+        delta[j] += __shfl_xor(delta[j], 32, 64);
+        l2[j] = lse2[(size_t)bh * S + qr];
+        if (g == 0 && q < S) delta_out[(size_t)bh * S + q] = delta[j];
     }
-    delta += __shfl_xor(delta, 16, 64);
-    delta += __shfl_xor(delta, 32, 64);
-    const float l2 = lse2[(size_t)bh * S + qr];
-    if (g == 0 && q < S) delta_out[(size_t)bh * S + q] = delta;
 
-    float4_t qacc[4];
+    float4_t qacc[QT][4];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) qacc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < QT; ++j)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) qacc[j][dt] = float4_t{0.f, 0.f, 0.f, 0.f};
     for (int k0 = 0; k0 < S; k0 += AT_CH) {
         if (k0) __syncthreads();
         kc.store(k_lds, k0, S, tid);
@@ -494,41 +416,60 @@ __global__ __launch_bounds__(AT_CT, 3) void attention_any_bwd_q_kernel(const uin
 #pragma unroll 2
         for (int u = 0; u < NT / 2; ++u) {
             if (k0 + 32 * u >= S) break;
-            u16x8 dsp;
+            u16x8 dsp[QT];
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
                 const int t = 2 * u + half;
-                float4_t sa = {0.f, 0.f, 0.f, 0.f}, da = {0.f, 0.f, 0.f, 0.f};
+                float4_t sa[QT], da[QT];
+#pragma unroll
+                for (int j = 0; j < QT; ++j) sa[j] = da[j] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(k_lds, 16 * t + li, s, g), qf[s], sa, 0, 0, 0);
-                    da = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(v_lds, 16 * t + li, s, g), dof[s], da, 0, 0, 0);
-                }
-                const float l = k0 + 16 * t + 4 * g < S ? l2 : INFINITY;      // (keys past the sequence: P = 0)
+                    const bf16x8 kf = at_frag(k_lds, 16 * t + li, s, g), vf = at_frag(v_lds, 16 * t + li, s, g);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float p = at_bf2f(at_f2bf(__builtin_amdgcn_exp2f(sa[e] * c - l)));
-                    dsp[4 * half + e] = at_f2bf(scale * p * (da[e] - delta));
+                    for (int j = 0; j < QT; ++j) {
+                        sa[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[j][s], sa[j], 0, 0, 0);
+                        da[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, dof[j][s], da[j], 0, 0, 0);
+                    }
+                }
+                const bool live = k0 + 16 * t + 4 * g < S;            // (keys past the sequence: P = 0)
+#pragma unroll
+                for (int j = 0; j < QT; ++j) {
+                    const float l = live ? l2[j] : INFINITY;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        // P is rounded to bf16 as the forward pass did before using it
+                        const float p = at_bf2f(at_f2bf(__builtin_amdgcn_exp2f(sa[j][e] * c - l)));
+                        dsp[j][4 * half + e] = at_f2bf(scale * p * (da[j][e] - delta[j]));
+                    }
                 }
             }
-            const bf16x8 dsf = __builtin_bit_cast(bf16x8, dsp);
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
-                qacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(k_lds, u, dt, li, g), dsf, qacc[dt], 0, 0, 0);
+            for (int dt = 0; dt < 4; ++dt) {
+                const bf16x8 kt = at_frag_t(k_lds, u, dt, li, g);
+#pragma unroll
+                for (int j = 0; j < QT; ++j)
+                    qacc[j][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt, __builtin_bit_cast(bf16x8, dsp[j]), qacc[j][dt], 0, 0, 0);
+            }
         }
     }
-    if (q >= S) return;
-    uint16_t* qrow = dqkv + ((size_t)b * S + q) * ld + h * AT_D + 4 * g;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) at_store4(qrow + 16 * dt, qacc[dt]);
+    for (int j = 0; j < QT; ++j) {
+        const int q = q0 + 16 * j;
+        if (q >= S) continue;
+        uint16_t* qrow = dqkv + ((size_t)b * S + q) * ld + h * AT_D + 4 * g;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) at_store4(qrow + 16 * dt, qacc[j][dt]);
+    }
 }
 
-__global__ __launch_bounds__(AT_CT, 3) void attention_any_bwd_kv_kernel(const uint16_t* __restrict__ qkv,
-                                                                     const uint16_t* __restrict__ dctx,
-                                                                     const float* __restrict__ lse2,
-                                                                     const float* __restrict__ delta,
-                                                                     uint16_t* __restrict__ dqkv, int S, int heads, float c,
-                                                                     float scale) {
+template <int QT>
+__global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_bwd_kv_kernel(const uint16_t* __restrict__ qkv,
+                                                                                      const uint16_t* __restrict__ dctx,
+                                                                                      const float* __restrict__ lse2,
+                                                                                      const float* __restrict__ delta,
+                                                                                      uint16_t* __restrict__ dqkv, int S,
+                                                                                      int heads, float c, float scale) {
     constexpr int NT = AT_CH / 16;
     __shared__ __attribute__((aligned(16))) uint16_t q_lds[AT_CH * AT_P];
     __shared__ __attribute__((aligned(16))) uint16_t do_lds[AT_CH * AT_P];
@@ -543,25 +484,31 @@ __global__ __launch_bounds__(AT_CT, 3) void attention_any_bwd_kv_kernel(const ui
     const float* rows = (tid < AT_CH ? lse2 : delta) + (size_t)bh * S;
     AtChunk qc, dc;
     float row;
-    auto load = [&](int q0) {
-        qc.load(base, ld, q0, S, tid);
-        dc.load(dbase, H, q0, S, tid);
+    auto load = [&](int r0) {
+        qc.load(base, ld, r0, S, tid);
+        dc.load(dbase, H, r0, S, tid);
         // (queries past the sequence: P = 0)
-        row = q0 + tid % AT_CH < S ? rows[q0 + tid % AT_CH] : tid < AT_CH ? INFINITY : 0.f;
+        row = r0 + tid % AT_CH < S ? rows[r0 + tid % AT_CH] : tid < AT_CH ? INFINITY : 0.f;
     };
     load(0);
 
-    const int key = blockIdx.x * AT_CQ + wave * 16 + li, kr = min(key, S - 1);
-    bf16x8 kf[2], vf[2];
+    const int key0 = (blockIdx.x * 4 + wave) * 16 * QT + li;
+    bf16x8 kf[QT][2], vf[QT][2];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        kf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)kr * ld + H + 32 * s + 8 * g));
-        vf[s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(base + (size_t)kr * ld + 2 * H + 32 * s + 8 * g));
+    for (int j = 0; j < QT; ++j) {
+        const uint16_t* krow = base + (size_t)min(key0 + 16 * j, S - 1) * ld + H;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            kf[j][s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(krow + 32 * s + 8 * g));
+            vf[j][s] = __builtin_bit_cast(bf16x8, *(const u16x8*)(krow + H + 32 * s + 8 * g));
+        }
     }
 
-    float4_t kacc[4], vacc[4];
+    float4_t kacc[QT][4], vacc[QT][4];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) kacc[dt] = vacc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < QT; ++j)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) kacc[j][dt] = vacc[j][dt] = float4_t{0.f, 0.f, 0.f, 0.f};
     for (int q0 = 0; q0 < S; q0 += AT_CH) {
         if (q0) __syncthreads();
         qc.store(q_lds, q0, S, tid);
@@ -572,39 +519,54 @@ __global__ __launch_bounds__(AT_CT, 3) void attention_any_bwd_kv_kernel(const ui
 #pragma unroll 2
         for (int u = 0; u < NT / 2; ++u) {
             if (q0 + 32 * u >= S) break;
-            u16x8 pp, dsp;
+            u16x8 pp[QT], dsp[QT];
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
                 const int t = 2 * u + half;
-                float4_t sa = {0.f, 0.f, 0.f, 0.f}, da = {0.f, 0.f, 0.f, 0.f};
+                float4_t sa[QT], da[QT];
+#pragma unroll
+                for (int j = 0; j < QT; ++j) sa[j] = da[j] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(q_lds, 16 * t + li, s, g), kf[s], sa, 0, 0, 0);
-                    da = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag(do_lds, 16 * t + li, s, g), vf[s], da, 0, 0, 0);
+                    const bf16x8 qf = at_frag(q_lds, 16 * t + li, s, g), df = at_frag(do_lds, 16 * t + li, s, g);
+#pragma unroll
+                    for (int j = 0; j < QT; ++j) {
+                        sa[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf, kf[j][s], sa[j], 0, 0, 0);
+                        da[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(df, vf[j][s], da[j], 0, 0, 0);
+                    }
                 }
                 const float4_t l2 = *(const float4_t*)(row_lds + 16 * t + 4 * g);
                 const float4_t dl = *(const float4_t*)(row_lds + AT_CH + 16 * t + 4 * g);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint16_t pb = at_f2bf(__builtin_amdgcn_exp2f(sa[e] * c - l2[e]));
-                    pp[4 * half + e] = pb;
-                    dsp[4 * half + e] = at_f2bf(scale * at_bf2f(pb) * (da[e] - dl[e]));
-                }
+                for (int j = 0; j < QT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint16_t pb = at_f2bf(__builtin_amdgcn_exp2f(sa[j][e] * c - l2[e]));
+                        pp[j][4 * half + e] = pb;
+                        dsp[j][4 * half + e] = at_f2bf(scale * at_bf2f(pb) * (da[j][e] - dl[e]));
+                    }
             }
-            const bf16x8 pf = __builtin_bit_cast(bf16x8, pp), dsf = __builtin_bit_cast(bf16x8, dsp);
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) {
-                vacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(do_lds, u, dt, li, g), pf, vacc[dt], 0, 0, 0);
-                kacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at_frag_t(q_lds, u, dt, li, g), dsf, kacc[dt], 0, 0, 0);
+                const bf16x8 dot = at_frag_t(do_lds, u, dt, li, g), qt = at_frag_t(q_lds, u, dt, li, g);
+#pragma unroll
+                for (int j = 0; j < QT; ++j) {
+                    vacc[j][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dot, __builtin_bit_cast(bf16x8, pp[j]), vacc[j][dt], 0, 0, 0);
+                    kacc[j][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qt, __builtin_bit_cast(bf16x8, dsp[j]), kacc[j][dt], 0, 0, 0);
+                }
             }
         }
     }
-    if (key >= S) return;
-    uint16_t* krow = dqkv + ((size_t)b * S + key) * ld + H + h * AT_D + 4 * g;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-        at_store4(krow + 16 * dt, kacc[dt]);
-        at_store4(krow + H + 16 * dt, vacc[dt]);
+    for (int j = 0; j < QT; ++j) {
+        const int key = key0 + 16 * j;
+        if (key >= S) continue;
+        uint16_t* krow = dqkv + ((size_t)b * S + key) * ld + H + h * AT_D + 4 * g;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+            at_store4(krow + 16 * dt, kacc[j][dt]);
+            at_store4(krow + H + 16 * dt, vacc[j][dt]);
+        }
     }
 }
 
@@ -615,6 +577,9 @@ int at_check(const char* who, int batch, int seq, int heads, int head_dim) {
     PD_REQUIRE((long long)batch * heads <= 65535, PD_ESHAPE, "%s: too many (batch, head) pairs", who);
     return PD_OK;
 }
+
+// Whether a wave takes 32 queries (keys).
+bool at_wide(int batch, int seq, int heads) { return (long)((seq + 127) / 128) * batch * heads >= 256; }
 
 }  // namespace
 
@@ -632,19 +597,21 @@ extern "C" int pd_attention_fwd_bf16(const uint16_t* qkv, uint16_t* ctx, uint16_
     const float c = AT_LOG2E / sqrtf((float)head_dim);
     const dim3 grid(seq / AT_QB, batch * heads);
     hipStream_t s = (hipStream_t)stream;
-#define PD_AT_FWD(S_)                                                                                        \
-    do {                                                                                                     \
-        if (probs) attention_fwd_kernel<S_, true><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c); \
-        else attention_fwd_kernel<S_, false><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);      \
-    } while (0)
-    const bool whole = seq == 512 || seq == 256 || seq == 128;
-    PD_REQUIRE(whole || !probs, PD_ESHAPE, "pd_attention_fwd_bf16: probabilities only for seq 128, 256 and 512");
-    if (!whole)
-        attention_any_fwd_kernel<<<dim3((seq + AT_CQ - 1) / AT_CQ, batch * heads), AT_CT, 0, s>>>(qkv, ctx, lse2, seq, heads, c);
-    else if (seq == 512) PD_AT_FWD(512);
-    else if (seq == 256) PD_AT_FWD(256);
-    else PD_AT_FWD(128);
-#undef PD_AT_FWD
+    PD_REQUIRE(!probs || seq == 512 || seq == 256 || seq == 128, PD_ESHAPE,
+               "pd_attention_fwd_bf16: probabilities only for seq 128, 256 and 512");
+    // (8 x 16 heads of 256: 7.0 us with a head's K and V whole in LDS, 8.6 in chunks; of 128 4.5 / 4.2)
+    if (seq == 128 && probs) attention_fwd_kernel<128, true><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);
+    else if (seq == 128) attention_fwd_kernel<128, false><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);
+    else if (seq == 256 && probs) attention_fwd_kernel<256, true><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);
+    else if (seq == 256) attention_fwd_kernel<256, false><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);
+    else {
+        const bool wide = at_wide(batch, seq, heads);
+        const dim3 blocks((seq + (wide ? 127 : 63)) / (wide ? 128 : 64), batch * heads);
+        if (wide && probs) attention_any_fwd_kernel<2, true><<<blocks, AT_CT, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+        else if (wide) attention_any_fwd_kernel<2, false><<<blocks, AT_CT, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+        else if (probs) attention_any_fwd_kernel<1, true><<<blocks, AT_CT, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+        else attention_any_fwd_kernel<1, false><<<blocks, AT_CT, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+    }
     PD_CHECK_LAUNCH("pd_attention_fwd_bf16");
     return PD_OK;
 }
@@ -659,24 +626,14 @@ extern "C" int pd_attention_bwd_bf16(const uint16_t* qkv, const uint16_t* ctx, c
                    pd_aligned(delta, 16) && pd_aligned(dqkv, 8),
                PD_EINVAL, "pd_attention_bwd_bf16: qkv, ctx, dctx, lse2, delta must be 16-byte, dqkv 8-byte aligned");
     const float scale = 1.0f / sqrtf((float)head_dim), c = AT_LOG2E * scale;
-    const dim3 grid(seq / AT_QB, batch * heads);
     hipStream_t s = (hipStream_t)stream;
-#define PD_AT_BWD(S_)                                                                                                  \
-    do {                                                                                                               \
-        attention_bwd_q_kernel<S_><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, heads, c, scale);     \
-        PD_CHECK_LAUNCH("pd_attention_bwd_bf16(dQ)");                                                                  \
-        attention_bwd_kv_kernel<S_><<<grid, AT_THREADS, 0, s>>>(qkv, dctx, lse2, delta, dqkv, heads, c, scale);         \
-    } while (0)
-    const bool whole = seq == 512 || seq == 256 || seq == 128;
-    if (!whole) {
-        const dim3 any((seq + AT_CQ - 1) / AT_CQ, batch * heads);
-        attention_any_bwd_q_kernel<<<any, AT_CT, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, seq, heads, c, scale);
-        PD_CHECK_LAUNCH("pd_attention_bwd_bf16(dQ)");
-        attention_any_bwd_kv_kernel<<<any, AT_CT, 0, s>>>(qkv, dctx, lse2, delta, dqkv, seq, heads, c, scale);
-    } else if (seq == 512) PD_AT_BWD(512);
-    else if (seq == 256) PD_AT_BWD(256);
-    else PD_AT_BWD(128);
-#undef PD_AT_BWD
+    const bool wide = at_wide(batch, seq, heads);
+    const dim3 blocks((seq + (wide ? 127 : 63)) / (wide ? 128 : 64), batch * heads);
+    if (wide) attention_any_bwd_q_kernel<2><<<blocks, AT_CT, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    else attention_any_bwd_q_kernel<1><<<blocks, AT_CT, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    PD_CHECK_LAUNCH("pd_attention_bwd_bf16(dQ)");
+    if (wide) attention_any_bwd_kv_kernel<2><<<blocks, AT_CT, 0, s>>>(qkv, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    else attention_any_bwd_kv_kernel<1><<<blocks, AT_CT, 0, s>>>(qkv, dctx, lse2, delta, dqkv, seq, heads, c, scale);
     PD_CHECK_LAUNCH("pd_attention_bwd_bf16(dK, dV)");
     return PD_OK;
 }

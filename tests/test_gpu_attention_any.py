@@ -1,5 +1,5 @@
 """Fused attention at any sequence length that is a multiple of 8 (chunks of 128 rows, blocks of 64 queries or keys, four
-waves of 16) against attention in fp32 from the same bf16 operands.
+waves of 16; from 256 blocks of 128 on, waves of 32) against attention in fp32 from the same bf16 operands.
 
 Bound: P is rounded to bf16 once (2^-9 of it) and so is the result: 2-norm error below 2 x 2^-9 = 4e-3.  The backward
 rounds P, dS and its results, and reads a delta formed from the rounded context: 4 x 2^-9 = 8e-3."""
@@ -25,7 +25,8 @@ def _reference(qkv, dctx, B, S, h):
 
 @pytest.mark.parametrize("late", [False, True])
 @pytest.mark.parametrize("B,S,h", [(2, 8, 3), (1, 16, 2), (3, 24, 1), (2, 56, 2), (1, 64, 2), (2, 72, 3), (1, 120, 2), (2, 136, 2),
-                                   (3, 200, 12), (1, 248, 1), (2, 264, 2), (1, 384, 2), (1, 520, 2), (2, 640, 2)])
+                                   (3, 200, 12), (1, 248, 1), (2, 264, 2), (1, 384, 2), (1, 520, 2), (2, 640, 2),
+                                   (128, 8, 2), (64, 72, 4), (128, 120, 2), (64, 128, 4), (65, 136, 2), (43, 264, 2), (26, 520, 2)])
 def test_forward_and_backward(B, S, h, late):
     """``late``: the largest scores of a query lie in its last keys, so that the running maximum rises with every chunk."""
     from pipedream_amd import ops
@@ -63,3 +64,17 @@ def test_rows_past_the_sequence_are_not_read_as_values():
         assert torch.equal(one, ctx[rows]) and torch.equal(l1[0], lse2[b])
         assert torch.equal(ops.attention_backward(dctx[rows].contiguous(), qkv[rows].contiguous(), l1, 1, S, h, ctx=one), dqkv[rows])
     assert torch.isnan(ctx[2 * S:].float()).all() and torch.isfinite(dqkv[:2 * S].float()).all()
+
+
+@pytest.mark.parametrize("batch,heads", [(1, 2), (4, 16)])
+def test_probabilities_at_512(batch, heads):
+    """Written by a second pass, with blocks of 64 and of 128 queries: the context keeps its bits, a probability is one
+    rounding to bf16 (half a unit in the last of 8 bits: 2^-8 at most) off, and a little for the exponential of the hardware."""
+    from pipedream_amd import ops
+    S, g = 512, torch.Generator().manual_seed(5)
+    qkv = torch.randn(batch * S, 3 * 64 * heads, generator=g).to(BF).cuda()
+    ctx, probs = ops.attention_forward(qkv, batch, S, heads, need_probs=True)
+    assert torch.equal(ctx, ops.attention_forward(qkv, batch, S, heads)[0])
+    q, k = (t.reshape(batch, S, heads, 64).transpose(1, 2).float().contiguous() for t in qkv.split(64 * heads, 1)[:2])
+    want = torch.softmax(torch.matmul(q, k.transpose(2, 3).contiguous()) / 8, -1)
+    assert float(((probs.float() - want).abs() / want).max()) < 2.0 ** -8 + 1e-4
