@@ -74,21 +74,23 @@ struct GemmBf16Args {
     int ld_aux;
 };
 
-// erf by Abramowitz & Stegun 7.1.26 (absolute error below 1.5e-7, far inside a bf16 result's rounding): a
-// few multiply-adds, one reciprocal and one exponential, instead of the library erff, whose register demand
-// inside the 256 x 256 kernels' epilogue (all 256 registers hold accumulators there) spilled a kilobyte per lane.
-__device__ __forceinline__ float erf_as(float x) {
-    const float ax = fabsf(x);
-    const float t = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * ax);
-    const float poly = t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
-    const float r = 1.0f - poly * __expf(-ax * ax);
-    return x < 0.f ? -r : r;
+// Normal distribution by Abramowitz & Stegun 7.1.26 for erf (absolute error of the cdf below 1e-7, far inside a bf16
+// result's rounding): a few multiply-adds, one reciprocal and one exponential, instead of the library erff, whose register
+// demand inside the 256 x 256 kernels' epilogue (all 256 registers hold accumulators there) spilled a kilobyte per lane.
+// bell = exp(-x^2 / 2) is the factor of the polynomial and, for the derivative, of the density: the epilogues are bound by
+// the vector ALU (with two exponentials and erf's own sign and halves 4096 x 4096 x 1024 with 256 x 256 tiles 50 and 55 us
+// forward and backward, now 47 and 50).
+__device__ __forceinline__ float normal_cdf(float x, float bell) {
+    const float t = __builtin_amdgcn_rcpf(1.0f + 0.2316418882f * fabsf(x));
+    const float poly = t * (0.127414796f + t * (-0.142248368f + t * (0.7107068705f + t * (-0.7265760135f + t * 0.5307027145f))));
+    const float tail = poly * bell;
+    return x < 0.f ? tail : 1.0f - tail;
 }
-__device__ __forceinline__ float gelu_f(float x) { return 0.5f * x * (1.0f + erf_as(x * 0.70710678118654752f)); }
+__device__ __forceinline__ float bell_f(float x) { return __builtin_amdgcn_exp2f(x * x * -0.72134752044448170f); }
+__device__ __forceinline__ float gelu_f(float x) { return x * normal_cdf(x, bell_f(x)); }
 __device__ __forceinline__ float gelu_grad_f(float x) {
-    const float cdf = 0.5f * (1.0f + erf_as(x * 0.70710678118654752f));
-    const float pdf = 0.39894228040143268f * __expf(-0.5f * x * x);
-    return cdf + x * pdf;
+    const float bell = bell_f(x);
+    return normal_cdf(x, bell) + x * 0.39894228040143268f * bell;
 }
 
 __device__ __forceinline__ uint16_t f2bf(float f) { return pd_f2bf(f); }
@@ -1044,6 +1046,22 @@ int launch_gemm_bf16_staged(int ta, int tb, GemmBf16Args g, int batch, hipStream
 
 }  // namespace
 
+// Whether, from three quarters of the CUs busy on, tiles of 256 x 256 (one block per CU, half the LDS reads per MFMA;
+// nothing hides the epilogue) take less time than tiles of 128 x 128 (three blocks per CU, whose epilogues run under the
+// others' products).  Both as a time in us, fitted to 60 shapes of 2560 to 16384 rows, 768 to 4096 columns, k = 512 to 4096
+// (the tile taken is at most 10 % slower than the other one there):
+// 256 x 256: per turn of the CUs an epilogue (plain 7.5, with GELU 17.5, with its derivative 20) and 28.5 per 1024 k; a
+// turn that leaves CUs idle clocks higher.  128 x 128: per block on a CU 1.1 (2.5) and 9 (B as [N][K]: 10) per 1024 k.
+// us, 256 / 128: 4096 x 4096 x 1024 36.6 / 42.5, 4608 rows 57.5 / 49.5; with GELU 45.4 / 48.6 and 78.4 / 56.8, 3000 rows
+// 41.8 / 38.8; derivative, 4096 rows 49.4 / 45.2, k = 4096 127 / 158.
+static bool wide_tiles(long b256, long b128, int K, int trans_b, int act) {
+    if (b256 < 192) return false;
+    const float k = K / 1024.f, turns = (float)((b256 + 255) / 256), fill = b256 / (256.f * turns);
+    const float t256 = ((act == 0 ? 7.5f : act == 1 ? 17.5f : 20.f) + 28.5f * k) * turns * (0.48f + 0.52f * fill);
+    const float t128 = ((act ? 2.5f : 1.1f) + (trans_b ? 10.f : 9.f) * k) * (float)((b128 + 255) / 256);
+    return t256 <= t128;
+}
+
 // tile choice forced by pd_gemm_bf16_set_tile (0 = the built-in choice)
 static int g_force_bm = 0, g_force_bn = 0;
 
@@ -1102,20 +1120,18 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     // find a CU each (32 x 32, 32 x 64, 64 x 64).  What it saves grows with k, what it costs (more reads of the operands, a
     // sum over eight waves) with the size of C: the line lies at k = 16 per tile of 64 x 64.  us, split / not, and k per
     // tile: 128 x 1024 x 4096 8.7 / 14 (128), 88 x 768 x 768 4.6 / 5.4 (32), 600 x 768 x 3072 12.6 / 15.3 (26),
-    // 600 x 768 x 2304 9.5 / 11.3 (19), 640 x 1024 x 3072 15.2 / 15.5 (19), 200 x 768 x 768 5.2 / 5.4 (16), 1920 x 512 x 2048 15.3 / 11.4 (9), 600 x 768 x 768 7.9 / 4.9 (6),
-    // 200 x 3072 x 768 8.3 / 5.0 (4).
+    // 600 x 768 x 2304 9.5 / 11.3 (19), 640 x 1024 x 3072 15.2 / 15.5 (19), 200 x 768 x 768 5.2 / 5.4 (16),
+    // 1920 x 512 x 2048 15.3 / 11.4 (9), 600 x 768 x 768 7.9 / 4.9 (6), 200 x 3072 x 768 8.3 / 5.0 (4).
     if (!trans_a && batch == 1 && g.vec_store && K % DK == 0 && K >= 16 * blocks(64, 64) && blocks(64, 64) <= 256) {
         if (blocks(32, 32) <= 256) return launch_gemm_bf16_ksplit<1, 1>(trans_b, g, s);
         if (blocks(32, 64) <= 256) return launch_gemm_bf16_ksplit<1, 2>(trans_b, g, s);
         return launch_gemm_bf16_ksplit<2, 2>(trans_b, g, s);
     }
-    // 256 x 256 tiles (one block per CU, half the LDS reads per MFMA) from 192 tiles on, i.e. three quarters of
-    // the CUs busy: 4096 x 4096 x 1024 takes 39 us against 42 with 128 x 128 tiles.  Below, the largest tile that still
-    // gives every CU a block: us with 128 x 128, 64 x 128, 64 x 64: 2560 x 1024 x 1024 9.7 / 12.0 / 12.0 (160 blocks of
-    // 128 x 128), 600 x 2304 x 768 8.2 / 6.9 / 7.5 (180 of 64 x 128), 1240 x 1024 x 3072 25.8 / 18.6 / 23.3 (160),
-    // 1920 x 512 x 2048 17.7 / 13.1 / 11.4 (240 of 64 x 64), 768 x 768 x 600 9.9 / 8.2 / 6.5 (144).
-    if (whole && !both_t && M >= 256 && N >= 256 && blocks(256, 256) >= 192)
+    if (whole && !both_t && M >= 256 && N >= 256 && wide_tiles(blocks(256, 256), blocks(128, 128), K, trans_b, act))
         return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
+    // Below, the largest tile that still gives every CU a block: us with 128 x 128, 64 x 128, 64 x 64: 2560 x 1024 x 1024
+    // 9.7 / 12.0 / 12.0 (160 blocks of 128 x 128), 600 x 2304 x 768 8.2 / 6.9 / 7.5 (180 of 64 x 128), 1240 x 1024 x 3072
+    // 25.8 / 18.6 / 23.3 (160), 1920 x 512 x 2048 17.7 / 13.1 / 11.4 (240 of 64 x 64), 768 x 768 x 600 9.9 / 8.2 / 6.5 (144).
     if (blocks(64, 64) <= 256) return launch_gemm_bf16_dma<64, 64>(trans_a, trans_b, g, batch, s);
     if (!both_t && blocks(64, 128) <= 256) return launch_gemm_bf16_dma<64, 128>(trans_a, trans_b, g, batch, s);
     return launch_gemm_bf16_dma<128, 128>(trans_a, trans_b, g, batch, s);
