@@ -235,8 +235,10 @@ __global__ __launch_bounds__(LX_THREADS, 2) void lstm_step_f32x6_kernel(const Ls
         float s = 0.f;
 #pragma unroll
         for (int w = 0; w < LX_WAVES; ++w) s += part[w][(col + 4 * q) * P + row];
-        pre[q] += s;
-        if (a.b_ih) pre[q] += a.b_ih[(size_t)q * H + unit] + a.b_hh[(size_t)q * H + unit];
+        // (four terms, rounded once)
+        double z = (double)pre[q] + (double)s;
+        if (a.b_ih) z += (double)a.b_ih[(size_t)q * H + unit] + (double)a.b_hh[(size_t)q * H + unit];
+        pre[q] = (float)z;
     }
     const float gi = lx_sigmoid(pre[0]), gf = lx_sigmoid(pre[1]), gg = tanhf(pre[2]), go = lx_sigmoid(pre[3]);
     const float c = gf * cp + gi * gg;
