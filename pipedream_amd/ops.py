@@ -186,10 +186,17 @@ def _use_x6(M, N, K, trans_a, trans_b, relu, a, b, out, lda, ldb, ldc):
     return not trans_b or (K % 4 == 0 and ldb % 4 == 0 and b.data_ptr() % 16 == 0)
 
 
+SKINNY_X6_MIN_WEIGHTS = 1 << 22
+
+
 def _use_skinny_x6(M, N, K, trans_a, trans_b, a, b, lda, ldb):
     """Whether ``gemm`` takes pd_gemm_skinny_f32x6: at most 128 rows of an untransposed A, operands it can fetch 16 bytes at
-    a time.  Faster than the fp32 kernels on all of 25 shapes from 1 x 8 x 8 to 100 x 32320 x 1024 (1.1 to 3.8 times)."""
-    return (_GEMM_F32_ALGO != "never" and not trans_a and 0 < M <= 128 and N > 0 and K > 0 and K % 8 == 0 and
+    a time, and more than 2^22 weights (16 MB).  Those are read at 5.4 instead of 2.7 TB/s: 8 x 4096 x 25088 76 us against
+    154.  With fewer a product takes 4-10 us either way (30 x 32 x 128 4.2 / 7.3, 100 x 512 x 512 10.5 / 10.0), in passes
+    that the host's launches bound (32 rows through 784-1024-1024-10: 617-675 us either way), and the fp32 kernels keep
+    their bits, so that no pre-activation next to zero falls on the other side of a ReLU (1 of 100 runs of four such
+    passes)."""
+    return (_GEMM_F32_ALGO != "never" and not trans_a and 0 < M <= 128 and N * K > SKINNY_X6_MIN_WEIGHTS and K % 8 == 0 and
             (trans_b or N % 4 == 0) and lda % 4 == 0 and ldb % 4 == 0 and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0)
 
 
