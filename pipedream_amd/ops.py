@@ -735,8 +735,8 @@ def _winograd_run(x, w, bias, in_mask, out_mask, y, y_pool, pool_idx, unpool_idx
         lib.pd_conv3x3_winograd_filter_f32(_ptr(w), _ptr(u), c, k, int(rot180), stream)
     with _timed("conv3x3_winograd_kernel", 18.0 * c * k * n * h * wd):
         part_bytes = 0
-        if split and in_mask is None and y_full is None:
-            # (few work items with many input channels: ranges of these, added up by a second launch)
+        if split and c >= 256 and in_mask is None and y_full is None:
+            # (few work items with at least 256 input channels: ranges of these, added up by a second launch)
             part_bytes = _conv_split_bytes(n, h, wd, c, k)
         if part_bytes:
             part = torch.empty(part_bytes, dtype=torch.uint8, device=x.device)
