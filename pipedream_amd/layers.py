@@ -612,8 +612,10 @@ class _TransformerLayerFn(torch.autograd.Function):
         native = ops.transformer_layer_forward(x2d, ctx.params, B, S, heads, eps) if ops.kernel_timer is None else None
         if native is not None:
             y, saved = native
+            ctx.ffn = fc1_w.size(0)
             ctx.save_for_backward(x2d, saved)
             return y.view(B, S, H)
+        ops.check_layer_vectors(ctx.params, H)
         h1, mean1, rstd1 = ops.layernorm_forward(x2d, ln1_w, ln1_b, eps)
         qkv = ops.gemm_bf16(h1, bw(qkv_w), trans_b=True, bias=qkv_b)
         att, att_aux = ops.attention_forward(qkv, B, S, heads)
@@ -632,11 +634,12 @@ class _TransformerLayerFn(torch.autograd.Function):
         bw = ops.bf16_weight
         dy2 = dy.contiguous().view(B * S, H)
         if len(saved) == 1:                       # of the native forward pass
-            if ops.kernel_timer is None:
+            if ops.kernel_timer is None and fc1_w.size(0) == ctx.ffn:
                 dx = ops.transformer_layer_backward(dy2, x2d, saved[0], ctx.params, B, S, heads)
                 if dx is not None:
                     return (dx.view(B, S, H), None, None) + (None,) * 12
-            saved = ops.transformer_layer_saved(saved[0], B, S, heads, H, fc1_w.size(0))
+            saved = ops.transformer_layer_saved(saved[0], B, S, heads, H, ctx.ffn)
+        ops.check_layer_vectors(ctx.params, H)
         h1, mean1, rstd1, qkv, att_aux, att, x2, h2, mean2, rstd2, f, g = saved
         sums = ops.ColsumBatch()
 

@@ -1322,9 +1322,37 @@ def _layer_bytes(batch, seq, heads, hidden, ffn):
     return saved.value, work.value
 
 
-def _layer_params(params):
+@functools.lru_cache(maxsize=64)
+def _layer_shapes(hidden, ffn):
+    vec, wide = (hidden,), (3 * hidden, hidden)
+    return (vec, vec, wide, wide[:1], (hidden, hidden), vec, vec, vec, (ffn, hidden), (ffn,), (hidden, ffn), vec)
+
+
+def _layer_fits(params, hidden):
+    """Whether a transformer layer's parameters are the twelve tensors of the shapes that the native calls, which see
+    pointers alone, take for granted on ``hidden`` features.  (Others, an attention of another width for instance or no
+    bias, are left to the single launches and their checks.)"""
+    if any(p is None for p in params):
+        return False
+    return tuple([p.shape for p in params]) == _layer_shapes(hidden, params[8].shape[0] if params[8].dim() else 0)
+
+
+def check_layer_vectors(params, hidden):
+    """The single launches check the matrices against each other; a normalisation's parameters and the biases have to
+    reach as far as the kernels read, and as their gradients are written."""
+    for i in (0, 1, 6, 7):
+        if params[i] is not None and params[i].numel() < hidden:
+            raise ValueError("transformer layer: a normalisation over %d features got %d" % (params[i].numel(), hidden))
+    for i in (3, 5, 9, 11):
+        if params[i] is not None and params[i].numel() < params[i - 1].size(0):
+            raise ValueError("transformer layer: %d biases for %d rows of a weight" % (params[i].numel(), params[i - 1].size(0)))
+
+
+def _layer_params(params, hidden):
     """A layer's parameters as the native calls take them (matrices as their bf16 images) and the tensors behind the
-    pointers, or None where one is not dense fp32 on the GPU."""
+    pointers, or None where they do not fit or one is not dense fp32 on the GPU."""
+    if not _layer_fits(params, hidden):
+        return None
     tensors = [bf16_weight(p) if i in _LAYER_MATRICES else p for i, p in enumerate(params)]
     for i, t in enumerate(tensors):
         if t.dtype != (BF16 if i in _LAYER_MATRICES else torch.float32) or not t.is_cuda or not t.is_contiguous():
@@ -1335,12 +1363,13 @@ def _layer_params(params):
 def transformer_layer_forward(x, params, batch, seq, heads, eps):
     """(y, saved) of a pre-LayerNorm transformer layer on ``x`` [batch * seq, hidden], or None where the native call does not
     take the operands.  ``params``: ln1, qkv, proj, ln2, fc1, fc2, each weight and bias."""
-    hidden, ffn = x.size(1), params[8].size(0)
+    hidden = x.size(1)
     if x.dtype != BF16 or not x.is_cuda or not x.is_contiguous() or x.numel() == 0 or hidden % heads:
         return None
-    native = _layer_params(params)
+    native = _layer_params(params, hidden)
     if native is None:
         return None
+    ffn = params[8].size(0)
     saved = torch.empty(_layer_bytes(batch, seq, heads, hidden, ffn)[0], dtype=torch.uint8, device=x.device)
     y = torch.empty_like(x)
     _cabi.lib().pd_transformer_layer_fwd_bf16(native[0], _ptr(x), _ptr(saved), _ptr(y), batch, seq, heads, hidden, ffn,
@@ -1369,10 +1398,11 @@ def transformer_layer_saved(saved, batch, seq, heads, hidden, ffn):
 def transformer_layer_backward(dy, x, saved, params, batch, seq, heads):
     """dx of ``transformer_layer_forward``, or None where the native call does not take the operands; gradients are created
     in, or added to, the parameters' ``grad``."""
-    hidden, ffn = x.size(1), params[8].size(0)
-    native = _layer_params(params)
+    hidden = x.size(1)
+    native = _layer_params(params, hidden)
     if native is None or dy.dtype != BF16 or not dy.is_cuda or not dy.is_contiguous():
         return None
+    ffn = params[8].size(0)
     grads = [p.grad for p in params]
     if any(g is not None and (g.dtype != torch.float32 or not g.is_cuda or not g.is_contiguous()) for g in grads):
         return None
