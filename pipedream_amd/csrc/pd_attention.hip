@@ -29,6 +29,8 @@
 //                 matching keys.
 // The backward kernels use the same two moves: "first product lands in the layout of the second
 // product's B operand" and "transposed A operand through ds_read_b64_tr_b16".
+#include <cfloat>
+
 #include "pd_internal.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -177,7 +179,9 @@ __global__ __launch_bounds__(AT_THREADS) void attention_fwd_kernel(const uint16_
 // The other side's rows pass through LDS in chunks of AT_CH (the next chunk is on its way to the registers while one is
 // used), so seq is a run-time number: a multiple of 8, rows past it are zeros in LDS and masked.  A wave has QT times 16
 // queries (keys), a block four waves.
-// Forward: a running maximum and sum per query; what is there is rescaled when the maximum rises.
+// Forward: a running maximum and sum per query; what is there is rescaled when the maximum rises.  It starts at the lowest
+// finite number, so that keys whose scores are all -inf count as zeros until another one comes (and a query that has no
+// other keys ends as 0 / 0, as in a softmax).
 // Backward, query side: P^T = 2^(K Q^T c - lse2), dP^T = V dO^T, dS^T = P^T o (dP^T - delta) / sqrt(d) with
 // delta_q = sum_d dO[q][d] O[q][d] (= sum_k dP[q][k] P[q][k]), dQ^T = K^T dS^T; delta is also written out for the key side.
 // Backward, key side: S = Q K^T and dP = dO V^T have the queries on the MFMA rows (A operands = Q and dO rows from LDS, B =
@@ -247,7 +251,7 @@ __global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_fwd_kern
     float4_t oacc[QT][4];
 #pragma unroll
     for (int j = 0; j < QT; ++j) {
-        m[j] = -INFINITY;
+        m[j] = -FLT_MAX;
         sum[j] = 0.f;
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) oacc[j][dt] = float4_t{0.f, 0.f, 0.f, 0.f};

@@ -78,3 +78,35 @@ def test_probabilities_at_512(batch, heads):
     q, k = (t.reshape(batch, S, heads, 64).transpose(1, 2).float().contiguous() for t in qkv.split(64 * heads, 1)[:2])
     want = torch.softmax(torch.matmul(q, k.transpose(2, 3).contiguous()) / 8, -1)
     assert float(((probs.float() - want).abs() / want).max()) < 2.0 ** -8 + 1e-4
+
+
+@pytest.mark.parametrize("B,S,h", [(1, 200, 2), (2, 512, 2), (1, 264, 1), (8, 512, 8), (43, 264, 2)])
+def test_scores_that_are_infinite(B, S, h):
+    """Query 0: the first 128 keys at -inf (finite operands whose products overflow), finite ones after them.  Query 1: all
+    but the last key.  Query 2: every key at -inf, query 3: one at +inf, both NaN as in fp32.  The others are ordinary."""
+    from pipedream_amd import ops
+    g = torch.Generator().manual_seed(S + 1)
+    qkv, dctx = torch.randn(B * S, 3 * 64 * h, generator=g), torch.randn(B * S, 64 * h, generator=g)
+    q, k, _ = (t.view(B, S, h, 64) for t in qkv.split(64 * h, 1))
+    q[..., :4], k[..., :4] = 0.0, 0.0
+    for i in range(4):
+        q[:, i, :, i] = 1e30
+    k[:, :128, :, 0] = -1e30
+    k[:, :S - 1, :, 1] = -1e30
+    k[:, :, :, 2] = -1e30
+    k[:, 150, :, 3] = 1e30
+    qkv, dctx = qkv.to(BF).cuda(), dctx.to(BF).cuda()
+    ctx, lse2 = ops.attention_forward(qkv, B, S, h)
+    ref, grads = _reference(qkv.cpu(), dctx.cpu(), B, S, h)
+    got, want = ctx.cpu().view(B, S, -1), ref.view(B, S, -1)
+    ordinary = [0, 1] + list(range(4, S))
+    assert torch.isnan(want[:, 2:4]).all() and torch.isnan(got[:, 2:4].float()).all()
+    assert torch.isfinite(want[:, ordinary]).all() and _rel(got[:, ordinary], want[:, ordinary]) < 4e-3
+    for i in (0, 1):
+        assert _rel(got[:, i], want[:, i]) < 8e-3          # (one row: a rounding of P and one of the result each)
+    # the gradients of the queries, without the NaNs that reach every key from queries 2 and 3
+    dq = ops.attention_backward(dctx, qkv, lse2, B, S, h, ctx=ctx)[:, :64 * h].cpu().view(B, S, -1)
+    want = grads[0].view(B, S, -1)
+    rows = list(range(4, S))
+    cols = [64 * i + j for i in range(h) for j in range(4, 64)]        # (the first four columns of K hold the 1e30)
+    assert _rel(dq[:, rows][..., cols], want[:, rows][..., cols]) < 8e-3
