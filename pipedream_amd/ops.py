@@ -1404,6 +1404,8 @@ def transformer_layer_backward(dy, x, saved, params, batch, seq, heads):
         return None
     ffn = params[8].size(0)
     grads = [p.grad for p in params]
+    if len(set(map(id, params))) < len(params):      # one parameter in two places: its gradients are added one by one
+        return None
     if any(g is not None and (g.dtype != torch.float32 or not g.is_cuda or not g.is_contiguous()) for g in grads):
         return None
     add = 0

@@ -74,3 +74,19 @@ def test_weights_read_by_the_backward_pass_are_the_current_ones():
         y.backward(dy)
         xs.append(xi.grad)
     assert not torch.equal(xs[0], xs[1])
+
+
+def test_one_matrix_in_two_places_gets_both_gradients():
+    """fc1 and fc2 as one parameter: what separate copies get, added up, in a first pass and in an accumulated one."""
+    layer = _layer(64, 1, 64)
+    g = torch.Generator().manual_seed(3)
+    x, dy = (torch.randn(2, 16, 64, generator=g).bfloat16().cuda() for _ in range(2))
+    layer.fc2.weight.data = layer.fc1.weight.data.clone()
+    _passes(layer, [x, x], [dy, dy], True, True)
+    want = layer.fc1.weight.grad.double() + layer.fc2.weight.grad.double()
+    others = [p.grad.clone() for p in layer.parameters() if p is not layer.fc1.weight and p is not layer.fc2.weight]
+    layer.fc2.weight = layer.fc1.weight
+    _passes(layer, [x, x], [dy, dy], True, True)
+    assert float((layer.fc1.weight.grad.double() - want).norm() / want.norm()) < 1e-6
+    for a, b in zip([p.grad for p in layer.parameters() if p is not layer.fc1.weight], others):
+        assert torch.equal(a, b)
