@@ -1232,8 +1232,8 @@ def attention_forward(qkv, batch, seq, heads, need_probs=False):
 
 
 def attention_backward(dctx, qkv, aux, batch, seq, heads, ctx=None):
-    """Gradient with respect to qkv; `aux` is the second result of attention_forward (lse2 needs `ctx`,
-    the forward output, as well)."""
+    """Gradient with respect to qkv; `aux` is the second result of attention_forward.  lse2 needs `ctx`, the forward
+    output, as well; at lengths other than 128, 256 and 512 it is computed once more where it is not given."""
     _mat_bf16(dctx, "dctx")
     H = qkv.size(1) // 3
     d = H // heads
@@ -1244,7 +1244,9 @@ def attention_backward(dctx, qkv, aux, batch, seq, heads, ctx=None):
     dqkv = torch.empty_like(qkv)
     if aux.dtype == torch.float32:
         if ctx is None:
-            raise ValueError("attention_backward: the fused path needs ctx")
+            if seq in (128, 256, 512):
+                raise ValueError("attention_backward: the fused path needs ctx")
+            ctx = attention_forward(qkv, batch, seq, heads)[0]
         _mat_bf16(ctx, "ctx")
         if tuple(ctx.shape) != (batch * seq, H) or not ctx.is_contiguous() or tuple(aux.shape) != (batch, heads, seq):
             raise ValueError("attention_backward: ctx must be a contiguous [batch*seq, H] matrix, lse2 [batch, heads, seq]")

@@ -110,3 +110,22 @@ def test_scores_that_are_infinite(B, S, h):
     rows = list(range(4, S))
     cols = [64 * i + j for i in range(h) for j in range(4, 64)]        # (the first four columns of K hold the 1e30)
     assert _rel(dq[:, rows][..., cols], want[:, rows][..., cols]) < 8e-3
+
+
+@pytest.mark.parametrize("S", [8, 200, 264])
+def test_backward_without_the_context(S):
+    from pipedream_amd import ops
+    g = torch.Generator().manual_seed(S)
+    qkv, dctx = torch.randn(2 * S, 3 * 128, generator=g).to(BF).cuda(), torch.randn(2 * S, 128, generator=g).to(BF).cuda()
+    ctx, aux = ops.attention_forward(qkv, 2, S, 2)
+    assert torch.equal(ops.attention_backward(dctx, qkv, aux, 2, S, 2), ops.attention_backward(dctx, qkv, aux, 2, S, 2, ctx=ctx))
+    with pytest.raises(ValueError):
+        ops.attention_backward(dctx, qkv, aux, 2, S, 2, ctx=ctx[:S])
+
+
+def test_lengths_that_always_needed_the_context_still_do():
+    from pipedream_amd import ops
+    qkv = torch.randn(128, 3 * 64).to(BF).cuda()
+    ctx, aux = ops.attention_forward(qkv, 1, 128, 1)
+    with pytest.raises(ValueError):
+        ops.attention_backward(torch.ones_like(ctx), qkv, aux, 1, 128, 1)
