@@ -14,8 +14,8 @@
 // (trans_b = 1, k-contiguous).
 //
 // Three kernels: tiles of 64 x 64 to 256 x 256 fed by direct-to-LDS loads (nearly every product), k split over the waves of
-// a block (few tiles, deep reductions), and one that stages through registers, for operands whose rows lie 2^22 elements
-// and more apart.  LDS bandwidth, not the matrix cores, limits small tiles: a wave with a (32*TM) x (32*TN) tile reads
+// a block (few tiles, deep reductions), and one that stages through registers, for reductions of at most 192 and operands
+// whose rows lie 2^22 elements and more apart.  LDS bandwidth, not the matrix cores, limits small tiles: a wave with a (32*TM) x (32*TN) tile reads
 // (TM+TN) KB of fragments per TM*TN MFMAs, so the largest gives every wave 128 x 128 and a block 256 x 256.
 // The staged kernel: a block of WM x WN waves owns a BM x BN tile; K runs in chunks of 64 through a double-buffered LDS
 // tile.
@@ -1030,16 +1030,17 @@ int launch_gemm_bf16_dma(int ta, int tb, GemmBf16Args g, int batch, hipStream_t 
     return PD_OK;
 }
 
+template <int B>
 int launch_gemm_bf16_staged(int ta, int tb, GemmBf16Args g, int batch, hipStream_t s) {
-    g.tiles_m = (g.M + 63) / 64;
-    g.tiles_n = (g.N + 63) / 64;
+    g.tiles_m = (g.M + B - 1) / B;
+    g.tiles_n = (g.N + B - 1) / B;
     g.total_tiles = g.tiles_m * g.tiles_n * batch;
     g.tiles_per_xcd = (g.total_tiles + N_XCD - 1) / N_XCD;
     const dim3 grid(g.tiles_per_xcd * N_XCD);
-    if (!ta && tb) pd_gemm_bf16_kernel<64, 64, 2, 2, true, true><<<grid, 256, 0, s>>>(g);
-    else if (!ta && !tb) pd_gemm_bf16_kernel<64, 64, 2, 2, true, false><<<grid, 256, 0, s>>>(g);
-    else if (ta && !tb) pd_gemm_bf16_kernel<64, 64, 2, 2, false, false><<<grid, 256, 0, s>>>(g);
-    else pd_gemm_bf16_kernel<64, 64, 2, 2, false, true><<<grid, 256, 0, s>>>(g);
+    if (!ta && tb) pd_gemm_bf16_kernel<B, B, 2, 2, true, true><<<grid, 256, 0, s>>>(g);
+    else if (!ta && !tb) pd_gemm_bf16_kernel<B, B, 2, 2, true, false><<<grid, 256, 0, s>>>(g);
+    else if (ta && !tb) pd_gemm_bf16_kernel<B, B, 2, 2, false, false><<<grid, 256, 0, s>>>(g);
+    else pd_gemm_bf16_kernel<B, B, 2, 2, false, true><<<grid, 256, 0, s>>>(g);
     PD_CHECK_LAUNCH("pd_gemm_bf16");
     return PD_OK;
 }
@@ -1110,7 +1111,7 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     const auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
     // direct-to-LDS kernels: per-lane byte offsets that fit 32 bits
     const bool dma_ok = K > 0 && (long long)256 * (lda > ldb ? lda : ldb) * 2 < (1ll << 31);
-    if (!dma_ok) return launch_gemm_bf16_staged(trans_a, trans_b, g, batch, s);
+    if (!dma_ok) return launch_gemm_bf16_staged<64>(trans_a, trans_b, g, batch, s);
     const bool whole = K % (DK * NS) == 0, both_t = trans_a && trans_b;
     if (g_force_bm && whole) {
         if (g_force_bm == 256 && !both_t) return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
@@ -1127,12 +1128,26 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
         if (blocks(32, 64) <= 256) return launch_gemm_bf16_ksplit<1, 2>(trans_b, g, s);
         return launch_gemm_bf16_ksplit<2, 2>(trans_b, g, s);
     }
+    // Short reductions: the staged kernel, whose chunks of 64 k need no ring (a round of the ring is 128 k; what K leaves of
+    // it are zeros).  us, staged / direct: k = 64 4096 x 4096 12.2 / 14.6, 600 x 3072 4.0 / 4.7, 512 times 512 x 512 93 / 115, 2048
+    // times 64 x 64 10 / 13; k = 136 4096 x 4096 17.5 / 19.0, 2400 x 768 5.3 / 5.4; beyond 192 the ring: k = 200 2400 x 768
+    // 5.9 / 5.4, 4096 x 4096 19.8 / 19.6, 2400 x 512 x 328 6.8 / 5.7.  Tiles of 128 x 128 once there is one per CU:
+    // 4096 x 768 x 64 (192 of them) 5.4, with 64 x 64 4.8; 128 times 200 x 200 x 64 (512) 7.1, with 64 x 64 8.5.
+    // A whole round (k = 128) only where most of a wider tile would lie outside: 2048 times 64 x 64 15.2 / 17.8.
+    const bool narrow = M <= 64 || N <= 64;
+    if (K <= 192 && (!whole || (narrow && blocks(64, 64) > 256))) {
+        if (!narrow && blocks(128, 128) >= 256) return launch_gemm_bf16_staged<128>(trans_a, trans_b, g, batch, s);
+        return launch_gemm_bf16_staged<64>(trans_a, trans_b, g, batch, s);
+    }
     if (whole && !both_t && M >= 256 && N >= 256 && wide_tiles(blocks(256, 256), blocks(128, 128), K, trans_b, act))
         return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
     // Below, the largest tile that still gives every CU a block: us with 128 x 128, 64 x 128, 64 x 64: 2560 x 1024 x 1024
     // 9.7 / 12.0 / 12.0 (160 blocks of 128 x 128), 600 x 2304 x 768 8.2 / 6.9 / 7.5 (180 of 64 x 128), 1240 x 1024 x 3072
     // 25.8 / 18.6 / 23.3 (160), 1920 x 512 x 2048 17.7 / 13.1 / 11.4 (240 of 64 x 64), 768 x 768 x 600 9.9 / 8.2 / 6.5 (144).
-    if (blocks(64, 64) <= 256) return launch_gemm_bf16_dma<64, 64>(trans_a, trans_b, g, batch, s);
+    // Narrow results (one side at most 64: attention's products with few features per head) leave half of a wider tile empty:
+    // 264 x 64 x 264 512 times 22 with 64 x 64, 29 with 128 x 128, 200 x 32 x 200 512 times 15 / 20.  From 1024 rows on
+    // the larger tile's fewer reads make up for it: 1024 x 48 x 1024 128 times 64 / 55.
+    if (blocks(64, 64) <= 256 || (narrow && M < 1024 && N < 1024)) return launch_gemm_bf16_dma<64, 64>(trans_a, trans_b, g, batch, s);
     if (!both_t && blocks(64, 128) <= 256) return launch_gemm_bf16_dma<64, 128>(trans_a, trans_b, g, batch, s);
     return launch_gemm_bf16_dma<128, 128>(trans_a, trans_b, g, batch, s);
 }

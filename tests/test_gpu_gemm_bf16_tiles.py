@@ -27,7 +27,9 @@ def _case(M, N, K, ta, tb, seed=0):
 
 SHAPES = [(8, 8, 8), (32, 64, 40), (64, 64, 128), (72, 56, 136), (64, 72, 3000), (88, 768, 768), (128, 128, 120), (136, 264, 600),
           (200, 2304, 88), (600, 776, 200), (600, 3072, 256), (256, 1032, 1032), (1240, 1024, 72), (1920, 512, 512), (4096, 4104, 128),
-          (4040, 4096, 256), (64, 192, 4096), (640, 264, 2080), (200, 328, 7200)]
+          (4040, 4096, 256), (64, 192, 4096), (640, 264, 2080), (200, 328, 7200),
+          # reductions of at most 192: staged, in tiles of 128 x 128 from 256 of them on
+          (72, 56, 8), (136, 2056, 64), (2056, 2056, 40), (2040, 2056, 192), (4104, 1032, 136), (2056, 2056, 200)]
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
@@ -65,6 +67,24 @@ def test_epilogues(M, N, K):
     torch.nn.functional.gelu(fr).sum().backward()
     want = ref * fr.grad
     assert bool(((df.double() - want).abs() <= (bound + 2.0 ** -8 * ref.abs()) * (fr.grad.abs() + 1e-6) + 2.0 ** -8 * want.abs() + 1e-6 * ref.abs()).all())
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("batch,M,N,K", [(300, 64, 64, 128), (520, 40, 32, 40), (130, 136, 64, 264), (80, 200, 24, 200),
+                                         (260, 72, 128, 64), (130, 136, 136, 192), (257, 64, 72, 128), (80, 1032, 48, 256)])
+def test_batches_of_small_products(batch, M, N, K, ta, tb):
+    """Attention's products at head dimensions without a fused kernel: many entries, narrow sides, short reductions."""
+    from pipedream_amd import ops
+    g = torch.Generator().manual_seed(batch + M)
+    a = torch.randn(*((batch, K, M) if ta else (batch, M, K)), generator=g).to(BF).cuda()
+    b = torch.randn(*((batch, N, K) if tb else (batch, K, N)), generator=g).to(BF).cuda()
+    out = torch.full((batch * M + 8, N), float("nan"), dtype=BF, device="cuda")
+    ops._batched(ta, tb, M, N, K, a, 0, a.size(2), b, 0, b.size(2), out, 0, N, 1.0, batch, 1, (M * K, 0, N * K, 0, M * N, 0))
+    ad, bd = (a.transpose(1, 2) if ta else a).double().contiguous(), (b.transpose(1, 2) if tb else b).double().contiguous()
+    ref = torch.bmm(ad, bd)
+    bound = (K / 16 + 16) * 2.0 ** -24 * torch.bmm(ad.abs(), bd.abs()) + 2.0 ** -8 * ref.abs()
+    assert bool(((out[:batch * M].view(batch, M, N).double() - ref).abs() <= bound).all())
+    assert torch.isnan(out[batch * M:].float()).all()
 
 
 def test_rows_far_apart():
