@@ -12,8 +12,8 @@
 // Bound: reading B from memory, 5.4 TB/s at 8 rows; from 64 rows on also the conversions (both operands, once per block)
 // beside the MFMAs.  us, launches and sums included, before (fp32 MFMA kernel with 64 rows a block whatever M is,
 // operands through an LDS ring with a barrier per 16 k) / now: 8 x 4096 x 25088 154 / 76, 64 x 4096 x 25088 176 / 123,
-// its input gradient 202 / 126, 64 x 4096 x 4096 32 / 27 and 32 / 24, 32 x 10 x 1024 34 / 9.  Error against 64 bits
-// (2-norm) 2.9e-7 / 1.6e-7 at K = 1024, 1.0e-6 / 4.8e-7 at 25088.
+// its input gradient 202 / 126, 64 x 4096 x 4096 30 / 27 and 30 / 24.  Error against 64 bits (2-norm) 2.9e-7 / 1.6e-7 at
+// K = 1024, 1.0e-6 / 4.8e-7 at 25088.
 #include "pd_f32x6.hpp"
 
 namespace {
@@ -204,10 +204,12 @@ void launch_skinny(const SkinnyX6Args& g, int trans_b, hipStream_t s) {
 // Columns of C per block, 64 or 32.
 static int skinny_cols(int M, int N) { return (N + 63) / 64 * ((M + 63) / 64) <= 16 ? 32 : 64; }
 
-// Ranges of k: one block per CU and a chunk of k per wave.  Up to 32 chunks stay in one piece: 32 x 1024 x 1024 takes
-// 6.3 us in one launch and 4.4 in four ranges, whose sums cost a launch of 3 us more.
+// Ranges of k: one block per CU and a chunk of k per wave.  Up to 32 chunks (24 from 33 rows on, whose conversions spread
+// over the CUs as well) stay in one piece, since the launch that adds up the ranges costs what they save: us, one piece /
+// two ranges, 8 x 8192 x 768 11.3 / 11.4 and, B as [K][N], 8.1 / 10.1, x 1024 13.4 / 12.6 and 9.8 / 11.3,
+// 64 x 8192 x 768 18.4 / 19.2 and 15.3 / 18.3, x 1024 22.4 / 19.6 and 18.2 / 18.4.
 extern "C" int pd_gemm_skinny_f32x6_splits(int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K <= 1024) return 1;
+    if (M <= 0 || N <= 0 || K <= (M > 32 ? 768 : 1024)) return 1;
     const int cols = skinny_cols(M, N);
     const long blocks = (long)((N + cols - 1) / cols) * ((M + 63) / 64);
     const long most = (K + 31) / 32 / KX_WAVES, want = 256 / blocks;

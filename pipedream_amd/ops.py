@@ -191,12 +191,20 @@ SKINNY_X6_MIN_WEIGHTS = 1 << 22
 
 def _use_skinny_x6(M, N, K, trans_a, trans_b, a, b, lda, ldb):
     """Whether ``gemm`` takes pd_gemm_skinny_f32x6: at most 128 rows of an untransposed A, operands it can fetch 16 bytes at
-    a time, and more than 2^22 weights (16 MB).  Those are read at 5.4 instead of 2.7 TB/s: 8 x 4096 x 25088 76 us against
-    154.  With fewer a product takes 4-10 us either way (30 x 32 x 128 4.2 / 7.3, 100 x 512 x 512 10.5 / 10.0), in passes
-    that the host's launches bound (32 rows through 784-1024-1024-10: 617-675 us either way), and the fp32 kernels keep
-    their bits, so that no pre-activation next to zero falls on the other side of a ReLU (1 of 100 runs of four such
-    passes)."""
-    return (_GEMM_F32_ALGO != "never" and not trans_a and 0 < M <= 128 and N * K > SKINNY_X6_MIN_WEIGHTS and K % 8 == 0 and
+    a time, and more than 2^22 weights (16 MB), for [N][K] weights and more than 96 rows 2^23 at least.  us, fp32
+    kernels / this one, weights from memory, at 8, 32, 64, 96 and 128 rows:
+      [N][K]  2048 x 2304  14.5 / 10.9  16.0 / 12.9  18.0 / 17.1  19.4 / 18.6  19.5 / 20.6
+              3072 x 2048  16.4 / 11.4  18.1 / 14.0  18.5 / 18.3  23.2 / 23.0  23.3 / 26.0
+              4096 x 2048  17.5 / 12.5  19.1 / 14.6  19.9 / 19.4  26.4 / 23.3  26.8 / 26.6
+              4096 x 4096  28.3 / 20.5  30.2 / 23.4  30.5 / 29.0  45.3 / 36.7  45.6 / 41.4
+      [K][N]  2048 x 2304  14.1 / 9.7   15.8 / 11.8  17.8 / 16.0  19.7 / 16.3  19.7 / 19.1
+    Below 2^22 it loses from 64 rows on (64 x 2048 x 1024 13.1 / 21.7) and wins or loses with few by the shape (8 rows:
+    1024 x 1024 11.1 / 8.6, 2048 x 1024 11.5 / 13.0, 10 x 1024 33 / 6).  The fp32 kernels keep their bits there: products
+    of few weights are found in front of a ReLU in passes that the host's launches bound, which gain nothing, while a
+    pre-activation next to zero that falls on the other side moves a result (1 of 100 runs of four passes at 32 rows)."""
+    if N * K <= SKINNY_X6_MIN_WEIGHTS or (trans_b and M > 96 and N * K < 2 * SKINNY_X6_MIN_WEIGHTS):
+        return False
+    return (_GEMM_F32_ALGO != "never" and not trans_a and 0 < M <= 128 and K % 8 == 0 and
             (trans_b or N % 4 == 0) and lda % 4 == 0 and ldb % 4 == 0 and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0)
 
 
