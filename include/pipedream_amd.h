@@ -425,11 +425,13 @@ int pd_gemm_bf16(int trans_a, int trans_b, int M, int N, int K,
                  void* C, int ldc, int out_f32, float alpha, float beta,
                  const float* bias, const uint16_t* residual, int ldr,
                  int batch_outer, int batch_inner, const int64_t* strides, void* stream);
+/* Ranges of tokens into which the weight gradient dy[T][n]^T x[T][k] of a bf16 Linear layer is cut (partial products as
+ * batch entries of pd_gemm_bf16, added up by pd_splitk_reduce_f32) so that few output tiles keep the chip busy; 1: not cut. */
+int pd_gemm_bf16_wgrad_splits(uint64_t T, int n, int k);
 /* Tuning and test hook: force the tile of the direct-to-LDS kernel behind pd_gemm_bf16 / pd_gemm_bf16_gelu
- * for products it can take (K a multiple of 128): (128, 128) or (256, 256); (0, 0) restores the built-in
- * choice (256 x 256 when there are at least 192 such tiles, 32 x 32 to 64 x 64 with the reduction split over the waves of
- * a block when these are at most 256, else 128 x 128).  Process-wide,
- * not thread-safe against concurrent GEMM calls.  No counterpart in the reference (its GEMMs are library calls). */
+ * for products whose K is a multiple of 128: (128, 128) or (256, 256); (0, 0) restores the built-in choice (by the time
+ * each tile takes).  Process-wide, not thread-safe against concurrent GEMM calls.  No counterpart in the reference
+ * (its GEMMs are library calls). */
 int pd_gemm_bf16_set_tile(int bm, int bn);
 
 /* The product of pd_gemm_f32 (same operands and layout flags, no ReLU) on the bf16 matrix pipes: the operands are
@@ -519,6 +521,10 @@ int pd_colsum_batch(int n_jobs, const void* const* x, const int* is_bf16, float*
  * order, weight before bias, dense; bit i of `add`: grads[i] is added to, else written.  `saved` (written by the forward
  * pass, read by the backward pass) and `work` (temporary) hold pd_transformer_layer_bytes() bytes, 256-byte aligned. */
 int pd_transformer_layer_bytes(int batch, int seq, int heads, int hidden, int ffn, uint64_t* saved, uint64_t* work);
+/* Where the twelve tensors of `saved` begin, in bytes: h1 = LN1(x), its mean and rstd (fp32), qkv, lse2 (fp32) or, where
+ * pd_attention_fwd_supported() is 0, the probabilities, the attention's result, x2, h2 = LN2(x2), its mean and rstd, fc1's
+ * result, its GELU. */
+int pd_transformer_layer_saved_offsets(int batch, int seq, int heads, int hidden, int ffn, uint64_t* offsets);
 int pd_transformer_layer_fwd_bf16(const void* const* params, const uint16_t* x, void* saved, uint16_t* y, int batch,
                                   int seq, int heads, int hidden, int ffn, float eps, void* stream);
 int pd_transformer_layer_bwd_bf16(const void* const* params, float* const* grads, uint32_t add, const uint16_t* x,

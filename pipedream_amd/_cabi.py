@@ -141,6 +141,8 @@ SIGNATURES = {
     "pd_colsum_bf16": (_i, [_vp, _vp, _u64, _i, _u64, _i, _vp], True),
     "pd_colsum_batch_workspace_floats": (_i, [_i, _vp, _vp, _i, ctypes.POINTER(_u64)], True),
     "pd_colsum_batch": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _u64, _i, _vp], True),
+    "pd_gemm_bf16_wgrad_splits": (_i, [_u64, _i, _i], False),
+    "pd_transformer_layer_saved_offsets": (_i, [_i] * 5 + [ctypes.POINTER(_u64)], True),
     "pd_transformer_layer_bytes": (_i, [_i] * 5 + [ctypes.POINTER(_u64)] * 2, True),
     "pd_transformer_layer_fwd_bf16": (_i, [_vp] * 4 + [_i] * 5 + [_f, _vp], True),
     "pd_transformer_layer_bwd_bf16": (_i, [_vp, _vp, ctypes.c_uint32] + [_vp] * 5 + [_i] * 5 + [_vp], True),

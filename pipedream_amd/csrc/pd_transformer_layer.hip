@@ -16,10 +16,12 @@ constexpr int COLSUM_SPLITS = 64;              // row ranges of the batched colu
 struct Regions {
     char* base;
     uint64_t at = 0;
-    explicit Regions(void* p) : base((char*)p) {}
+    uint64_t* starts;                          // of the regions so far, where somebody asks for them
+    explicit Regions(void* p, uint64_t* starts = nullptr) : base((char*)p), starts(starts) {}
     template <typename T>
     T* take(uint64_t count) {
         T* p = base ? (T*)(base + at) : nullptr;
+        if (starts) *starts++ = at;
         at += (count * sizeof(T) + 255) / 256 * 256;
         return p;
     }
@@ -49,13 +51,13 @@ struct Saved {
     float* lse2;
     uint16_t* probs;
     uint64_t bytes;
-    Saved(const Dims& d, void* p) {
-        Regions r(p);
+    Saved(const Dims& d, void* p, uint64_t* starts = nullptr) {
+        Regions r(p, starts);
         h1 = r.take<uint16_t>(d.T * d.H);
         mean1 = r.take<float>(d.T);
         rstd1 = r.take<float>(d.T);
         qkv = r.take<uint16_t>(d.T * 3 * d.H);
-        lse2 = d.fused ? r.take<float>(d.scores) : nullptr;
+        lse2 = d.fused ? r.take<float>(d.scores) : nullptr;      // (either of the two)
         probs = d.fused ? nullptr : r.take<uint16_t>(d.scores);
         att = r.take<uint16_t>(d.T * d.H);
         x2 = r.take<uint16_t>(d.T * d.H);
@@ -67,16 +69,6 @@ struct Saved {
         bytes = r.at;
     }
 };
-
-// A weight gradient dy^T x [n][k] with few output tiles is cut over the tokens into partial products (1: it is not).
-int wgrad_splits(uint64_t T, int n, int k) {
-    const long tiles = (long)((n + 127) / 128) * ((k + 127) / 128);
-    if (tiles > 64) return 1;
-    long s = 256 / tiles;
-    if ((long)(T / 1024) < s) s = (long)(T / 1024);
-    if (s > 8) s = 8;
-    return s < 2 || T % (s * 128) != 0 || n % 4 != 0 || k % 4 != 0 ? 1 : (int)s;
-}
 
 // Temporaries of the backward pass.
 struct Work {
@@ -99,7 +91,7 @@ struct Work {
         const int shapes[4][2] = {{d.H, d.F}, {d.F, d.H}, {d.H, d.H}, {3 * d.H, d.H}};
         uint64_t most = 0;
         for (const auto& s : shapes) {
-            const int splits = wgrad_splits(d.T, s[0], s[1]);
+            const int splits = pd_gemm_bf16_wgrad_splits(d.T, s[0], s[1]);
             const uint64_t n = splits > 1 ? (uint64_t)splits * s[0] * s[1] : 0;
             if (n > most) most = n;
         }
@@ -152,7 +144,7 @@ int attention_backward(const Dims& d, const Saved& s, const Work& w, void* strea
 // dw [n][k] (+)= dy^T x
 int weight_gradient(const uint16_t* dy, const uint16_t* x, float* dw, bool add, uint64_t T, int n, int k, float* partials,
                     void* stream) {
-    const int splits = wgrad_splits(T, n, k);
+    const int splits = pd_gemm_bf16_wgrad_splits(T, n, k);
     if (splits == 1)
         return pd_gemm_bf16(1, 0, n, k, (int)T, dy, n, x, k, dw, k, 1, 1.f, add ? 1.f : 0.f, nullptr, nullptr, 0, 1, 1, nullptr, stream);
     const int rows = (int)(T / splits);
@@ -170,6 +162,24 @@ int check_params(const char* who, const void* const* params) {
 }
 
 }  // namespace
+
+extern "C" int pd_gemm_bf16_wgrad_splits(uint64_t T, int n, int k) {
+    if (n <= 0 || k <= 0) return 1;
+    const long tiles = (long)((n + 127) / 128) * ((k + 127) / 128);
+    if (tiles > 64) return 1;
+    long s = 256 / tiles;
+    if ((long)(T / 1024) < s) s = (long)(T / 1024);
+    if (s > 8) s = 8;
+    return s < 2 || T % (s * 128) != 0 || n % 4 != 0 || k % 4 != 0 ? 1 : (int)s;
+}
+
+extern "C" int pd_transformer_layer_saved_offsets(int batch, int seq, int heads, int hidden, int ffn, uint64_t* offsets) {
+    Dims d;
+    PD_STEP(make_dims("pd_transformer_layer_saved_offsets", batch, seq, heads, hidden, ffn, &d));
+    PD_REQUIRE(offsets, PD_EINVAL, "pd_transformer_layer_saved_offsets: NULL pointer");
+    Saved(d, nullptr, offsets);
+    return PD_OK;
+}
 
 extern "C" int pd_transformer_layer_bytes(int batch, int seq, int heads, int hidden, int ffn, uint64_t* saved, uint64_t* work) {
     Dims d;

@@ -8,6 +8,7 @@ torch's current stream.
 import contextlib
 import ctypes
 import functools
+import math
 
 import torch
 
@@ -1178,9 +1179,8 @@ def gemm_bf16_wgrad(dy, x, acc=None):
     _mat_bf16(x, "x")
     T, N = dy.shape
     K = x.shape[1]
-    tiles = -(-N // 128) * -(-K // 128)
-    splits = min(256 // tiles, T // 1024, 8) if tiles <= 64 else 1
-    if splits < 2 or T % (splits * 128) != 0 or N % 4 != 0 or K % 4 != 0:
+    splits = _cabi.lib().pd_gemm_bf16_wgrad_splits(T, N, K)
+    if splits < 2:
         if acc is None:
             return gemm_bf16(dy, x, trans_a=True, out_f32=True)
         return gemm_bf16(dy, x, trans_a=True, out=acc, beta=1.0)
@@ -1389,20 +1389,17 @@ def transformer_layer_forward(x, params, batch, seq, heads, eps):
 
 def transformer_layer_saved(saved, batch, seq, heads, hidden, ffn):
     """What the forward pass left in ``saved``, as tensors: h1, mean1, rstd1, qkv, attention's aux, attention, x2, h2, mean2,
-    rstd2, f, g (the order and 256-byte boundaries of pd_transformer_layer.hip)."""
+    rstd2, f, g."""
     rows = batch * seq
+    starts = (ctypes.c_uint64 * 12)()
+    _cabi.lib().pd_transformer_layer_saved_offsets(batch, seq, heads, hidden, ffn, starts)
     aux = (((batch, heads, seq), torch.float32) if _cabi.lib().pd_attention_fwd_supported(seq, hidden // heads)
            else ((batch, heads, seq, seq), BF16))
     wide, stat = ((rows, hidden), BF16), ((rows,), torch.float32)
-    out, at = [], 0
-    for shape, dtype in (wide, stat, stat, ((rows, 3 * hidden), BF16), aux, wide, wide, wide, stat, stat,
-                         ((rows, ffn), BF16), ((rows, ffn), BF16)):
-        n = dtype.itemsize
-        for d in shape:
-            n *= d
-        out.append(saved[at:at + n].view(dtype).view(shape))
-        at += -(-n // 256) * 256
-    return out
+    tensors = (wide, stat, stat, ((rows, 3 * hidden), BF16), aux, wide, wide, wide, stat, stat, ((rows, ffn), BF16),
+               ((rows, ffn), BF16))
+    return [saved[at:at + math.prod(shape) * dtype.itemsize].view(dtype).view(shape)
+            for at, (shape, dtype) in zip(starts, tensors)]
 
 
 def transformer_layer_backward(dy, x, saved, params, batch, seq, heads):

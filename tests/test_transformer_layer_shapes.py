@@ -44,6 +44,18 @@ def test_a_parameter_that_is_too_short_is_refused(place):
             ops.check_layer_vectors(params, 64)
 
 
+@pytest.mark.parametrize("B,S,hidden,heads,ffn", [(2, 16, 64, 1, 96), (3, 200, 768, 12, 3072), (1, 8, 64, 2, 8), (2, 24, 96, 3, 104)])
+def test_the_tensors_a_forward_pass_leaves_lie_side_by_side(B, S, hidden, heads, ffn):
+    """Every tensor on a 256-byte boundary, in order, none over another, the last one inside the buffer."""
+    saved = torch.zeros(ops._layer_bytes(B, S, heads, hidden, ffn)[0], dtype=torch.uint8)
+    at = 0
+    for t in ops.transformer_layer_saved(saved, B, S, heads, hidden, ffn):
+        start = t.data_ptr() - saved.data_ptr()
+        assert start % 256 == 0 and at <= start < at + 256
+        at = start + t.numel() * t.element_size()
+    assert at <= saved.numel() < at + 256
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("timer", [None, {}])
 @pytest.mark.parametrize("built,given", [(128, 256), (256, 128)])
