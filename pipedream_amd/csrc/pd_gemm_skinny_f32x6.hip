@@ -111,6 +111,7 @@ __global__ __launch_bounds__(KX_THREADS, 2) void pd_gemm_skinny_f32x6_kernel(con
         load_b(0);
 #pragma unroll
         for (int i = 0; i < RT; ++i) load_a(i, 0);
+        const float sign = pd_x6_sign(chunks, ways, way);
         for (int c = 0; c < n; ++c) {
             const int next = min(c + 1, n - 1);    // (past the end the last chunk is fetched again)
             u32x4_t bt[CT][3];
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(KX_THREADS, 2) void pd_gemm_skinny_f32x6_kernel(con
 #pragma unroll
             for (int i = 0; i < RT; ++i) {
                 u32x4_t at[3];
-                pd_x6_split8(ar[i], at);
+                pd_x6_split8<true>(ar[i], at, sign);
                 load_a(i, next);
 #pragma unroll
                 for (int s = 0; s < 6; ++s)
@@ -129,6 +130,10 @@ __global__ __launch_bounds__(KX_THREADS, 2) void pd_gemm_skinny_f32x6_kernel(con
                     for (int j = 0; j < CT; ++j) acc[i][j] = pd_x6_mfma(at[PD_X6_A[s]], bt[j][PD_X6_B[s]], acc[i][j]);
             }
         }
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) acc[i][j] *= sign;
 
         bool bad = false;
 #pragma unroll

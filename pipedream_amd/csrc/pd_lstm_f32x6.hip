@@ -40,10 +40,10 @@ __device__ __forceinline__ size_t tile_offset(int row, int k, int chunks) {
 }
 
 // One wave's product: rows of `x` (tiles; 16 RT of them, from its first chunk on) with the split weights `w` (16 CT
-// columns), n chunks of 32 k.
+// columns), n chunks of 32 k, summed up with `sign`.
 template <int RT, int CT>
 __device__ __forceinline__ void wave_product(f32x4_t (&acc)[RT][CT], const float* x, const u32x4_t* w, int chunks, int n,
-                                             int lane) {
+                                             int lane, float sign) {
     f32x4_t raw[RT][2];
     u32x4_t wt[2][CT][3];
     auto load_x = [&](int i, int c) {
@@ -65,7 +65,7 @@ __device__ __forceinline__ void wave_product(f32x4_t (&acc)[RT][CT], const float
             const float v[8] = {raw[i][0][0], raw[i][0][1], raw[i][0][2], raw[i][0][3],
                                 raw[i][1][0], raw[i][1][1], raw[i][1][2], raw[i][1][3]};
             u32x4_t xt[3];
-            pd_x6_split8(v, xt);
+            pd_x6_split8<true>(v, xt, sign);
             load_x(i, next);
 #pragma unroll
             for (int s = 0; s < 6; ++s)
@@ -80,6 +80,10 @@ __device__ __forceinline__ void wave_product(f32x4_t (&acc)[RT][CT], const float
         step(integral_constant<int, 0>{}, c);
         if (c + 1 < n) step(integral_constant<int, 1>{}, c + 1);
     }
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) acc[i][j] *= sign;
 }
 
 // Whether a sum is NaN or infinite.  Infinities and values that round to infinity in bf16 leave NaNs: the wave then
@@ -198,7 +202,7 @@ __global__ __launch_bounds__(LX_THREADS, 2) void lstm_step_f32x6_kernel(const Ls
     const int c0 = chunks * wave / LX_WAVES, n = a.h_prev ? chunks * (wave + 1) / LX_WAVES - c0 : 0;
     if (n > 0) {
         wave_product(acc, a.h_in + ((size_t)row0 / 16 * chunks + c0) * 512, a.w_split + ((size_t)group0 * chunks + c0) * 192,
-                     chunks, n, lane);
+                     chunks, n, lane, pd_x6_sign(chunks, LX_WAVES, wave));
         if (not_finite(acc)) {
             clear(acc);
             const int idx = lane & 15;
@@ -330,7 +334,7 @@ __global__ __launch_bounds__(LX_THREADS, 2) void lstm_dh_f32x6_kernel(const Lstm
     const int c0 = chunks * way / ways, n = chunks * (way + 1) / ways - c0;
     if (n > 0) {
         wave_product(acc, a.tiles + ((size_t)row0 / 16 * chunks + c0) * 512, a.w_split + ((size_t)j0 / 16 * chunks + c0) * 192,
-                     chunks, n, lane);
+                     chunks, n, lane, pd_x6_sign(chunks, ways, way));
         if (not_finite(acc)) {
             clear(acc);
             const int idx = lane & 15;

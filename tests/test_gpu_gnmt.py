@@ -40,11 +40,13 @@ def test_lstm_layer_matches_torch():
         torch.testing.assert_close(p.grad.cpu(), q.grad, rtol=1e-5, atol=2e-6, msg=k)
 
 
-@pytest.mark.parametrize("T,B,I,H", [(7, 5, 24, 32), (1, 3, 16, 16), (12, 128, 256, 256), (6, 100, 128, 1024)])
+@pytest.mark.parametrize("T,B,I,H", [(7, 5, 24, 32), (1, 3, 16, 16), (12, 128, 256, 256), (6, 100, 128, 1024),
+                                     (6, 129, 24, 64), (5, 7, 24, 48), (4, 200, 16, 96)])
 def test_lstm_time_loop_in_native_code_equals_the_step_by_step_calls(T, B, I, H):
-    """ops.lstm_forward / lstm_backward issue a layer's time loop through pd_lstm_recurrence_fwd/bwd_f32; with the
-    per-launch timer on they call the product and the cell once per step instead.  Same kernels on the same
-    operands: every result bit for bit.  (100 and 128 rows: the recurrence product's two block rows of 64.)"""
+    """ops.lstm_forward / lstm_backward issue a layer's time loop through pd_lstm_recurrence_fwd/bwd_f32x6, and for more than
+    128 rows or an H that 32 does not divide (the last three, and the single step) through pd_lstm_recurrence_fwd/bwd_f32;
+    with the per-launch timer on they launch one step at a time instead.  Same kernels on the same operands: every result
+    bit for bit.  (100 and 128 rows: the recurrence product's two block rows of 64.)"""
     from pipedream_amd import ops
     g = torch.Generator().manual_seed(5)
     x = torch.randn(T, B, I, generator=g).cuda()
