@@ -442,7 +442,7 @@ __global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_bwd_q_ke
                     const float l = live ? l2[j] : INFINITY;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        // P is rounded to bf16 as the forward pass did before using it
+                        // (P in bf16, as the forward pass uses it at 128 and 256; in chunks that rounds P times the sum)
                         const float p = at_bf2f(at_f2bf(__builtin_amdgcn_exp2f(sa[j][e] * c - l)));
                         dsp[j][4 * half + e] = at_f2bf(scale * p * (da[j][e] - delta[j]));
                     }
@@ -603,7 +603,8 @@ extern "C" int pd_attention_fwd_bf16(const uint16_t* qkv, uint16_t* ctx, uint16_
     hipStream_t s = (hipStream_t)stream;
     PD_REQUIRE(!probs || seq == 512 || seq == 256 || seq == 128, PD_ESHAPE,
                "pd_attention_fwd_bf16: probabilities only for seq 128, 256 and 512");
-    // (8 x 16 heads of 256: 7.0 us with a head's K and V whole in LDS, 8.6 in chunks; of 128 4.5 / 4.2)
+    // A head's K and V whole in LDS where they fit: us, whole / in chunks, 1 x 16 heads of 128 4.1 / 3.9, 8 x 16 4.4 / 4.2,
+    // 16 x 16 4.7 / 5.7, 32 x 16 7.0 / 7.7, 64 x 16 15.4 / 16.1; of 256 1 x 16 5.9 / 5.8, 8 x 16 6.8 / 8.3, 32 x 16 23 / 26.
     if (seq == 128 && probs) attention_fwd_kernel<128, true><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);
     else if (seq == 128) attention_fwd_kernel<128, false><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);
     else if (seq == 256 && probs) attention_fwd_kernel<256, true><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);

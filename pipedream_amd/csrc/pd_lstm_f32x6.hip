@@ -15,14 +15,15 @@
 // Everything the products read lies in memory in the order in which lanes read it.  W_hh is laid out, and split into its
 // terms, once per layer and direction (24 H^2 bytes; 7 us at H = 1024); a cell writes h (dgates) a second time in
 // "tiles": 16 rows x 32 k, as two halves of four k per lane.  Rows of 4H floats fetched 16 at a time start in the same
-// L2 channel: with h read row by row a forward step took 15.6 us where tiles give 12.4.  A row tile is split just before
-// its MFMAs (all of a chunk at once: 12.4, so 11.2: the two waves of a SIMD then overlap one's conversions with the
-// other's MFMAs).  fp32 weights split in the loop instead of the three terms: 11.5 us; sixteen waves a block: 11.6-12.8.
+// L2 channel: with h read row by row a forward step took 15.6 us where tiles gave 12.4.  A row tile is split just before
+// its MFMAs (all of a chunk at once: 12.4, so 11.2 before the sums took turns in sign: the two waves of a SIMD then overlap
+// one's conversions with the other's MFMAs).  fp32 weights split in the loop instead of the three terms: 11.5 us; sixteen
+// waves a block: 11.6-12.8.
 //
 // Bound: reads from L2, 448 KB per CU and forward step at 128 x 1024, 26 bytes a cycle; MFMAs 2.6 us of it.
-// us per time step with its launches, before (fp32 MFMA product and cell) / now: forward at H = 1024 19.2 / 11.2 (batch
-// 128), 14.4 / 7.6 (40), 12.9 / 5.5 (16), at H = 512 and batch 128 12.0 / 6.9; kernels of a backward step 19.0 / 15.4 (128),
-// 15.9 / 10.5 (40).  Error of h against 64 bits after 50 steps 9.5e-8 / 8.9e-8 (2-norm).
+// us per time step in a chain of 20, before (fp32 MFMA product and cell) / now: forward at H = 1024 18.5 / 12.0 (batch 128),
+// 14.3 / 8.1 (40), 12.8 / 5.8 (16), at H = 512 and batch 128 12.1 / 7.2; backward 18.9 / 15.0, 14.8 / 10.0, 12.8 / 7.5 and
+// 12.1 / 8.6.  2-norm errors against 64 bits after 50 steps of 128 x 1024: h 1.1e-7 / 9.9e-8, bias gradient 1.6e-7 / 1.5e-7.
 #include <type_traits>
 
 #include "pd_f32x6.hpp"

@@ -87,13 +87,25 @@ def test_batches_of_small_products(batch, M, N, K, ta, tb):
     assert torch.isnan(out[batch * M:].float()).all()
 
 
-def test_rows_far_apart():
-    """Leading dimensions of 2^22 elements: the kernel whose offsets are 64 bits wide."""
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("far", ["a", "b"])
+def test_rows_far_apart(far, ta, tb):
+    """Leading dimensions of 2^22 elements: the kernel that stages through registers, whose offsets are 64 bits wide, for a
+    reduction that the direct-to-LDS kernels would otherwise have taken."""
     from pipedream_amd import ops
     g = torch.Generator().manual_seed(3)
-    big = torch.zeros(20, 1 << 22, dtype=BF, device="cuda")
-    big[:, :200] = torch.randn(20, 200, generator=g).to(BF).cuda()
-    a, b = big[:, :200], torch.randn(72, 200, generator=g).to(BF).cuda()
-    y = ops.gemm_bf16(a, b, trans_b=True, out_f32=True)
-    ref = a.double() @ b.double().t()
-    assert bool(((y.double() - ref).abs() <= 32 * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t())).all())
+    M, N, K = 24, 72, 328
+
+    def operand(rows, cols, wide):
+        t = torch.randn(rows, cols, generator=g).to(BF).cuda()
+        if not wide:
+            return t
+        big = torch.full((rows, 1 << 22), float("nan"), dtype=BF, device="cuda")
+        big[:, :cols] = t
+        return big[:, :cols]
+    a = operand(*((K, M) if ta else (M, K)), far == "a")
+    b = operand(*((N, K) if tb else (K, N)), far == "b")
+    y = ops.gemm_bf16(a, b, trans_a=bool(ta), trans_b=bool(tb), out_f32=True)
+    ad, bd = (a.t() if ta else a).double(), (b.t() if tb else b).double()
+    bound = (K / 16 + 16) * 2.0 ** -24 * (ad.abs() @ bd.abs())
+    assert bool(((y.double() - ad @ bd).abs() <= bound).all())

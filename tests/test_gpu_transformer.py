@@ -61,9 +61,10 @@ def test_gemm_bf16_epilogues():
 @pytest.mark.parametrize("tile", [128, 256])
 def test_gemm_bf16_large_tiles(M, N, K, ta, tb, tile):
     """K a multiple of 128 runs the direct-to-LDS ring kernel (one to three ring rounds), here with each of
-    its two tile sizes forced in turn (the built-in choice takes 256 x 256 tiles from 192 of them on); other K
-    the register-staged kernels; M and N that are not tile multiples exercise the clamped loads and the masked
-    vector stores.  The fp32 reference product is computed on the device by torch from the same bf16 inputs."""
+    its two tile sizes forced in turn (the built-in choice is by the time each takes); other K cannot be forced and run
+    the built-in choice both times, the ring with a masked last round (224) or the register-staged kernel (96); M and N
+    that are not tile multiples exercise the clamped loads and the masked vector stores.  The fp32 reference product
+    is computed on the device by torch from the same bf16 inputs."""
     from pipedream_amd import _cabi, ops
     g = torch.Generator().manual_seed(M + N + K)
     a = torch.randn((K, M) if ta else (M, K), generator=g).to(BF).cuda()
@@ -81,7 +82,7 @@ def test_gemm_bf16_large_tiles(M, N, K, ta, tb, tile):
 
 
 def test_gemm_bf16_built_in_tile_choice_and_hook_errors():
-    """Whatever tile the built-in choice takes (256 x 256 from 192 such tiles on, else 128 x 128), it agrees with
+    """Whatever tile the built-in choice takes (the faster of 256 x 256 and 128 x 128, or a smaller one), it agrees with
     both forced runs bit for bit (the tile size does not change the order of a dot product's additions)."""
     from pipedream_amd import _cabi, ops
     lib = _cabi.lib()
