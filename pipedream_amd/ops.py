@@ -924,9 +924,14 @@ def add(a, b):
     return y
 
 
-def _lstm_x6(B, H, w_hh):
-    """Whether a layer's recurrence runs on the bf16 matrix pipes at fp32 accuracy (pd_lstm_f32x6.hip)."""
-    return (_GEMM_F32_ALGO != "never" and w_hh.is_contiguous() and w_hh.data_ptr() % 16 == 0 and
+def _lstm_x6(T, B, H, w_hh):
+    """Whether a layer's recurrence of T steps runs on the bf16 matrix pipes at fp32 accuracy (pd_lstm_f32x6.hip).  Splitting
+    W_hh takes as long as one to three steps, which a short sequence does not earn back.  us for forward + backward, fp32
+    loop / this one, at 40 rows: H = 256, 2 steps 28 / 23; H = 512, 2 steps 28 / 28, 3 53 / 41; H = 1024, 3 65 / 72,
+    4 95 / 90, 6 153 / 127; H = 2560, 4 275 / 297, 5 363 / 353; H = 3072, 4 394 / 413, 5 524 / 494; H = 4096 (whose split
+    weights do not stay in the cache), 6 939 / 1149, 12 2054 / 2168, each further one 186 / 178."""
+    enough = 2 if H <= 256 else 3 if H <= 512 else 5 if H <= 3072 else 16
+    return (T >= enough and _GEMM_F32_ALGO != "never" and w_hh.is_contiguous() and w_hh.data_ptr() % 16 == 0 and
             bool(_cabi.lib().pd_lstm_f32x6_supported(B, H)))
 
 
@@ -958,7 +963,7 @@ def lstm_forward(x, w_ih, w_hh, b_ih, b_hh):
     gates = gemm(x2, w_ih, trans_b=True).view(T, B, 4 * H)
     y = torch.empty((T, B, H), dtype=torch.float32, device=x.device)
     c = torch.empty((T, B, H), dtype=torch.float32, device=x.device)
-    if _lstm_x6(B, H, w_hh):
+    if _lstm_x6(T, B, H, w_hh):
         # product and cell of a step in one launch
         w_split, tiles = _lstm_x6_scratch(0, T, B, H, w_hh)
 
@@ -995,7 +1000,7 @@ def lstm_backward(dy, x, y, gates, c, w_ih, w_hh, need_dx=True):
     lib, s = _cabi.lib(), _cabi.stream_ptr
     dgates = torch.empty((T, B, 4 * H), dtype=torch.float32, device=x.device)
     dc = torch.empty((B, H), dtype=torch.float32, device=x.device)
-    if _lstm_x6(B, H, w_hh) and gates.is_contiguous() and c.is_contiguous():
+    if _lstm_x6(T, B, H, w_hh) and gates.is_contiguous() and c.is_contiguous():
         splits = lib.pd_lstm_dh_f32x6_splits(B, H)
         dh_rec = torch.empty((splits, B, H), dtype=torch.float32, device=x.device)
         w_split, tiles = _lstm_x6_scratch(1, T, B, H, w_hh)

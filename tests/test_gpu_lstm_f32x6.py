@@ -60,7 +60,7 @@ def _no_worse_than_fp32(params, dy):
 def test_layer_matches_64_bits(B, H, scale):
     from pipedream_amd import _cabi
     assert _cabi.lib().pd_lstm_f32x6_supported(B, H)
-    params, dy = _layer(4, B, H)
+    params, dy = _layer(5, B, H)
     params[2] *= scale
     _no_worse_than_fp32(params, dy)
 
