@@ -178,7 +178,7 @@ __global__ __launch_bounds__(AT_THREADS) void attention_fwd_kernel(const uint16_
 // ---- any sequence length: forward, backward -----------------------------------------------------------------
 // The other side's rows pass through LDS in chunks of AT_CH (the next chunk is on its way to the registers while one is
 // used), so seq is a run-time number: a multiple of 8, rows past it are zeros in LDS and masked.  A wave has QT times 16
-// queries (keys), a block four waves.
+// queries (keys).
 // Forward: a running maximum and sum per query; what is there is rescaled when the maximum rises.  It starts at the lowest
 // finite number, so that keys whose scores are all -inf count as zeros until another one comes (and a query that has no
 // other keys ends as 0 / 0, as in a softmax).
@@ -189,23 +189,25 @@ __global__ __launch_bounds__(AT_THREADS) void attention_fwd_kernel(const uint16_
 // packed as B operands of the sums over queries dV^T = dO^T P and dK^T = Q^T dS, whose A operands are transposing reads.
 //
 // Bound: fragment reads from LDS, a kilobyte per MFMA of 16 cycles with QT = 1 (256 bytes a cycle for four SIMDs), half of
-// that with QT = 2; registers (116-160 and 163-213) leave three and two blocks a CU.
-// us forward / backward: 8 x 16 heads x 512 24 / 62 (30 / 74 with QT = 1 or a head's K and V whole in LDS, 105 / 183 as
-// batched products with softmax kernels), 8 x 16 x 640 37 / 90 (115 / 192 as batched products), 3 x 12 x 200 6 / 14 (QT = 2:
-// 7 / 18; 23 / 31 with launches as batched products).  QT = 2 from 256 of its blocks on, one per CU: 8 x 16 x 256 (256
-// blocks) 9 / 23 against 11 / 28, 5 x 8 x 328 (120) 10 / 24 against 8 / 22.  Error of the context (2-norm) 2.2e-3, as batched
-// products, whose scores go through bf16, 4.2e-3.
-constexpr int AT_CH = 128;
-constexpr int AT_CT = 256;             // threads
+// that with QT = 2; registers (116-161 and 163-213) leave three and two blocks of four waves a CU.
+// Three blocks, by what keeps one on every CU (at_block): four waves of 16 rows; eight of 16 and chunks of 256 rows, which
+// need half the barriers; four of 32.  us forward / backward: 512 keys for 32 heads 10.5 / 30, 10.0 / 28, 12 / 31; for 48
+// (384 blocks of 64 or 192 of 128) 14.5 / 36, 11.1 / 31, 13 / 34; for 96 22 / 53, 24 / 56, 20 / 52; 328 keys for 56 9.9 / 28,
+// 9.2 / 24, 9.9 / 25; 200 keys for 64 (256 blocks of 64) 5.9 / 15, 6.2 / 16, 7.5 / 18; for 96 7.4 / 20, 6.3 / 17, 7.7 / 19;
+// 1024 keys for 24 22 / 57, 21 / 55, 23 / 58.
+// 8 x 16 heads x 512 24 / 62 (105 / 183 as batched products with softmax kernels), 8 x 16 x 640 37 / 90 (115 / 192),
+// 3 x 12 x 200 6 / 14 (23 / 31 with launches).  Error of the context (2-norm) 2.2e-3, as batched products, whose scores go
+// through bf16, 4.2e-3.
 
-// chunk of rows [r0, r0 + AT_CH) x 64 columns: global -> registers, registers -> LDS
+// chunk of rows [r0, r0 + THREADS / 2) x 64 columns: global -> registers, registers -> LDS
+template <int THREADS>
 struct AtChunk {
-    static constexpr int ITERS = AT_CH * (AT_D / 8) / AT_CT;
+    static constexpr int ITERS = THREADS / 2 * (AT_D / 8) / THREADS;
     u16x8 r[ITERS];
     __device__ __forceinline__ void load(const uint16_t* __restrict__ g, int ld, int r0, int rows, int tid) {
 #pragma unroll
         for (int it = 0; it < ITERS; ++it) {
-            const int id = tid + it * AT_CT;
+            const int id = tid + it * THREADS;
             r[it] = *(const u16x8*)(g + (size_t)min(r0 + id / (AT_D / 8), rows - 1) * ld + (id % (AT_D / 8)) * 8);
         }
     }
@@ -213,20 +215,20 @@ struct AtChunk {
         const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int it = 0; it < ITERS; ++it) {
-            const int id = tid + it * AT_CT;
+            const int id = tid + it * THREADS;
             *(u16x8*)(lds + (id / (AT_D / 8)) * AT_P + (id % (AT_D / 8)) * 8) = r0 + id / (AT_D / 8) < rows ? r[it] : zero;
         }
     }
 };
 
 // WRITE_P: the probabilities, which need the sums, by a second pass over the keys (the first pass' bits stay the same).
-template <int QT, bool WRITE_P>
-__global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_fwd_kernel(const uint16_t* __restrict__ qkv,
+template <int QT, int WAVES, bool WRITE_P>
+__global__ __launch_bounds__(64 * WAVES, QT == 1 && WAVES == 4 ? 3 : 2) void attention_any_fwd_kernel(const uint16_t* __restrict__ qkv,
                                                                                    uint16_t* __restrict__ ctx,
                                                                                    uint16_t* __restrict__ probs,
                                                                                    float* __restrict__ lse2, int S, int heads,
                                                                                    float c) {
-    constexpr int NT = AT_CH / 16;
+    constexpr int AT_CH = 32 * WAVES, NT = AT_CH / 16;
     __shared__ __attribute__((aligned(16))) uint16_t k_lds[AT_CH * AT_P];
     __shared__ __attribute__((aligned(16))) uint16_t v_lds[AT_CH * AT_P];
 
@@ -235,11 +237,11 @@ __global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_fwd_kern
     const int bh = blockIdx.y, b = bh / heads, h = bh % heads;
     const int H = heads * AT_D, ld = 3 * H;
     const uint16_t* base = qkv + (size_t)b * S * ld + h * AT_D;
-    AtChunk kc, vc;
+    AtChunk<64 * WAVES> kc, vc;
     kc.load(base + H, ld, 0, S, tid);
     vc.load(base + 2 * H, ld, 0, S, tid);
 
-    const int q0 = (blockIdx.x * 4 + wave) * 16 * QT + li;            // tile j of the wave: query q0 + 16 j
+    const int q0 = (blockIdx.x * WAVES + wave) * 16 * QT + li;            // tile j of the wave: query q0 + 16 j
     bf16x8 qf[QT][2];
 #pragma unroll
     for (int j = 0; j < QT; ++j)
@@ -359,15 +361,15 @@ __global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_fwd_kern
     }
 }
 
-template <int QT>
-__global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_bwd_q_kernel(const uint16_t* __restrict__ qkv,
+template <int QT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, QT == 1 && WAVES == 4 ? 3 : 2) void attention_any_bwd_q_kernel(const uint16_t* __restrict__ qkv,
                                                                                      const uint16_t* __restrict__ ctx,
                                                                                      const uint16_t* __restrict__ dctx,
                                                                                      const float* __restrict__ lse2,
                                                                                      float* __restrict__ delta_out,
                                                                                      uint16_t* __restrict__ dqkv, int S,
                                                                                      int heads, float c, float scale) {
-    constexpr int NT = AT_CH / 16;
+    constexpr int AT_CH = 32 * WAVES, NT = AT_CH / 16;
     __shared__ __attribute__((aligned(16))) uint16_t k_lds[AT_CH * AT_P];
     __shared__ __attribute__((aligned(16))) uint16_t v_lds[AT_CH * AT_P];
 
@@ -376,11 +378,11 @@ __global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_bwd_q_ke
     const int bh = blockIdx.y, b = bh / heads, h = bh % heads;
     const int H = heads * AT_D, ld = 3 * H;
     const uint16_t* base = qkv + (size_t)b * S * ld + h * AT_D;
-    AtChunk kc, vc;
+    AtChunk<64 * WAVES> kc, vc;
     kc.load(base + H, ld, 0, S, tid);
     vc.load(base + 2 * H, ld, 0, S, tid);
 
-    const int q0 = (blockIdx.x * 4 + wave) * 16 * QT + li;
+    const int q0 = (blockIdx.x * WAVES + wave) * 16 * QT + li;
     bf16x8 qf[QT][2], dof[QT][2];
     float delta[QT], l2[QT];
 #pragma unroll
@@ -467,14 +469,14 @@ __global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_bwd_q_ke
     }
 }
 
-template <int QT>
-__global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_bwd_kv_kernel(const uint16_t* __restrict__ qkv,
+template <int QT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, QT == 1 && WAVES == 4 ? 3 : 2) void attention_any_bwd_kv_kernel(const uint16_t* __restrict__ qkv,
                                                                                       const uint16_t* __restrict__ dctx,
                                                                                       const float* __restrict__ lse2,
                                                                                       const float* __restrict__ delta,
                                                                                       uint16_t* __restrict__ dqkv, int S,
                                                                                       int heads, float c, float scale) {
-    constexpr int NT = AT_CH / 16;
+    constexpr int AT_CH = 32 * WAVES, NT = AT_CH / 16;
     __shared__ __attribute__((aligned(16))) uint16_t q_lds[AT_CH * AT_P];
     __shared__ __attribute__((aligned(16))) uint16_t do_lds[AT_CH * AT_P];
     __shared__ __attribute__((aligned(16))) float row_lds[2 * AT_CH];       // lse2, delta of the chunk's queries
@@ -486,7 +488,7 @@ __global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_bwd_kv_k
     const uint16_t* base = qkv + (size_t)b * S * ld + h * AT_D;
     const uint16_t* dbase = dctx + (size_t)b * S * H + h * AT_D;
     const float* rows = (tid < AT_CH ? lse2 : delta) + (size_t)bh * S;
-    AtChunk qc, dc;
+    AtChunk<64 * WAVES> qc, dc;
     float row;
     auto load = [&](int r0) {
         qc.load(base, ld, r0, S, tid);
@@ -496,7 +498,7 @@ __global__ __launch_bounds__(AT_CT, QT == 1 ? 3 : 2) void attention_any_bwd_kv_k
     };
     load(0);
 
-    const int key0 = (blockIdx.x * 4 + wave) * 16 * QT + li;
+    const int key0 = (blockIdx.x * WAVES + wave) * 16 * QT + li;
     bf16x8 kf[QT][2], vf[QT][2];
 #pragma unroll
     for (int j = 0; j < QT; ++j) {
@@ -582,8 +584,13 @@ int at_check(const char* who, int batch, int seq, int heads, int head_dim) {
     return PD_OK;
 }
 
-// Whether a wave takes 32 queries (keys).
-bool at_wide(int batch, int seq, int heads) { return (long)((seq + 127) / 128) * batch * heads >= 256; }
+// What a block takes: 64 queries (keys) by four waves of 16, 128 by eight waves of 16, or 128 by four waves of 32.
+enum AtBlock { AT_64, AT_128, AT_128_WIDE };
+AtBlock at_block(int batch, int seq, int heads) {
+    const long pairs = (long)batch * heads;
+    if ((seq + 63) / 64 * pairs <= 256) return AT_64;
+    return (seq + 127) / 128 * pairs <= 256 ? AT_128 : AT_128_WIDE;
+}
 
 }  // namespace
 
@@ -610,12 +617,14 @@ extern "C" int pd_attention_fwd_bf16(const uint16_t* qkv, uint16_t* ctx, uint16_
     else if (seq == 256 && probs) attention_fwd_kernel<256, true><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);
     else if (seq == 256) attention_fwd_kernel<256, false><<<grid, AT_THREADS, 0, s>>>(qkv, ctx, probs, lse2, heads, c);
     else {
-        const bool wide = at_wide(batch, seq, heads);
-        const dim3 blocks((seq + (wide ? 127 : 63)) / (wide ? 128 : 64), batch * heads);
-        if (wide && probs) attention_any_fwd_kernel<2, true><<<blocks, AT_CT, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
-        else if (wide) attention_any_fwd_kernel<2, false><<<blocks, AT_CT, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
-        else if (probs) attention_any_fwd_kernel<1, true><<<blocks, AT_CT, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
-        else attention_any_fwd_kernel<1, false><<<blocks, AT_CT, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+        const AtBlock block = at_block(batch, seq, heads);
+        const dim3 blocks(block == AT_64 ? (seq + 63) / 64 : (seq + 127) / 128, batch * heads);
+        if (block == AT_64 && probs) attention_any_fwd_kernel<1, 4, true><<<blocks, 256, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+        else if (block == AT_64) attention_any_fwd_kernel<1, 4, false><<<blocks, 256, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+        else if (block == AT_128 && probs) attention_any_fwd_kernel<1, 8, true><<<blocks, 512, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+        else if (block == AT_128) attention_any_fwd_kernel<1, 8, false><<<blocks, 512, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+        else if (probs) attention_any_fwd_kernel<2, 4, true><<<blocks, 256, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
+        else attention_any_fwd_kernel<2, 4, false><<<blocks, 256, 0, s>>>(qkv, ctx, probs, lse2, seq, heads, c);
     }
     PD_CHECK_LAUNCH("pd_attention_fwd_bf16");
     return PD_OK;
@@ -632,13 +641,15 @@ extern "C" int pd_attention_bwd_bf16(const uint16_t* qkv, const uint16_t* ctx, c
                PD_EINVAL, "pd_attention_bwd_bf16: qkv, ctx, dctx, lse2, delta must be 16-byte, dqkv 8-byte aligned");
     const float scale = 1.0f / sqrtf((float)head_dim), c = AT_LOG2E * scale;
     hipStream_t s = (hipStream_t)stream;
-    const bool wide = at_wide(batch, seq, heads);
-    const dim3 blocks((seq + (wide ? 127 : 63)) / (wide ? 128 : 64), batch * heads);
-    if (wide) attention_any_bwd_q_kernel<2><<<blocks, AT_CT, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, seq, heads, c, scale);
-    else attention_any_bwd_q_kernel<1><<<blocks, AT_CT, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    const AtBlock block = at_block(batch, seq, heads);
+    const dim3 blocks(block == AT_64 ? (seq + 63) / 64 : (seq + 127) / 128, batch * heads);
+    if (block == AT_64) attention_any_bwd_q_kernel<1, 4><<<blocks, 256, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    else if (block == AT_128) attention_any_bwd_q_kernel<1, 8><<<blocks, 512, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    else attention_any_bwd_q_kernel<2, 4><<<blocks, 256, 0, s>>>(qkv, ctx, dctx, lse2, delta, dqkv, seq, heads, c, scale);
     PD_CHECK_LAUNCH("pd_attention_bwd_bf16(dQ)");
-    if (wide) attention_any_bwd_kv_kernel<2><<<blocks, AT_CT, 0, s>>>(qkv, dctx, lse2, delta, dqkv, seq, heads, c, scale);
-    else attention_any_bwd_kv_kernel<1><<<blocks, AT_CT, 0, s>>>(qkv, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    if (block == AT_64) attention_any_bwd_kv_kernel<1, 4><<<blocks, 256, 0, s>>>(qkv, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    else if (block == AT_128) attention_any_bwd_kv_kernel<1, 8><<<blocks, 512, 0, s>>>(qkv, dctx, lse2, delta, dqkv, seq, heads, c, scale);
+    else attention_any_bwd_kv_kernel<2, 4><<<blocks, 256, 0, s>>>(qkv, dctx, lse2, delta, dqkv, seq, heads, c, scale);
     PD_CHECK_LAUNCH("pd_attention_bwd_bf16(dK, dV)");
     return PD_OK;
 }
