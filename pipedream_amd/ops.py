@@ -1327,7 +1327,8 @@ def layernorm_backward(dy, x, gamma, mean, rstd, dgamma_acc=None, dbeta_acc=None
     return dx, outs[0], outs[1]
 
 
-_LAYER_MATRICES = frozenset((2, 4, 8, 10))      # qkv, proj, fc1, fc2 among a transformer layer's parameters
+_LAYER_MATRICES = (2, 4, 8, 10)                 # qkv, proj, fc1, fc2 among a transformer layer's parameters
+_LAYER_DTYPES = [BF16 if i in _LAYER_MATRICES else torch.float32 for i in range(12)]
 
 
 @functools.lru_cache(maxsize=64)
@@ -1340,16 +1341,18 @@ def _layer_bytes(batch, seq, heads, hidden, ffn):
 @functools.lru_cache(maxsize=64)
 def _layer_shapes(hidden, ffn):
     vec, wide = (hidden,), (3 * hidden, hidden)
-    return (vec, vec, wide, wide[:1], (hidden, hidden), vec, vec, vec, (ffn, hidden), (ffn,), (hidden, ffn), vec)
+    return [vec, vec, wide, wide[:1], (hidden, hidden), vec, vec, vec, (ffn, hidden), (ffn,), (hidden, ffn), vec]
 
 
 def _layer_fits(params, hidden):
     """Whether a transformer layer's parameters are the twelve tensors of the shapes that the native calls, which see
     pointers alone, take for granted on ``hidden`` features.  (Others, an attention of another width for instance or no
     bias, are left to the single launches and their checks.)"""
-    if any(p is None for p in params):
+    try:
+        shapes = [p.shape for p in params]
+    except AttributeError:                           # no bias
         return False
-    return tuple([p.shape for p in params]) == _layer_shapes(hidden, params[8].shape[0] if params[8].dim() else 0)
+    return len(shapes[8]) == 2 and shapes == _layer_shapes(hidden, shapes[8][0])
 
 
 def check_layer_vectors(params, hidden):
@@ -1368,10 +1371,12 @@ def _layer_params(params, hidden):
     pointers, or None where they do not fit or one is not dense fp32 on the GPU."""
     if not _layer_fits(params, hidden):
         return None
-    tensors = [bf16_weight(p) if i in _LAYER_MATRICES else p for i, p in enumerate(params)]
-    for i, t in enumerate(tensors):
-        if t.dtype != (BF16 if i in _LAYER_MATRICES else torch.float32) or not t.is_cuda or not t.is_contiguous():
-            return None
+    tensors = list(params)
+    for i in _LAYER_MATRICES:
+        tensors[i] = bf16_weight(params[i])
+    if ([t.dtype for t in tensors] != _LAYER_DTYPES or
+            not all([t.is_cuda for t in tensors]) or not all([t.is_contiguous() for t in tensors])):
+        return None
     return (ctypes.c_void_p * 12)(*[t.data_ptr() for t in tensors]), tensors
 
 
