@@ -1184,6 +1184,8 @@ def gemm_bf16_wgrad(dy, x, acc=None):
     _mat_bf16(x, "x")
     T, N = dy.shape
     K = x.shape[1]
+    if acc is not None and tuple(acc.shape) != (N, K):
+        raise ValueError("gemm_bf16_wgrad: a gradient of %s for a weight of %s" % (tuple(acc.shape), (N, K)))
     splits = _cabi.lib().pd_gemm_bf16_wgrad_splits(T, N, K)
     if splits < 2:
         if acc is None:
@@ -1423,7 +1425,8 @@ def transformer_layer_backward(dy, x, saved, params, batch, seq, heads):
     grads = [p.grad for p in params]
     if len(set(map(id, params))) < len(params):      # one parameter in two places: its gradients are added one by one
         return None
-    if any(g is not None and (g.dtype != torch.float32 or not g.is_cuda or not g.is_contiguous()) for g in grads):
+    if any(g is not None and (g.dtype != torch.float32 or not g.is_cuda or not g.is_contiguous() or g.shape != p.shape)
+           for g, p in zip(grads, params)):          # (a parameter's data may have changed its shape under a gradient)
         return None
     add = 0
     for i, p in enumerate(params):

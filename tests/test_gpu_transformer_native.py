@@ -90,3 +90,19 @@ def test_one_matrix_in_two_places_gets_both_gradients():
     assert float((layer.fc1.weight.grad.double() - want).norm() / want.norm()) < 1e-6
     for a, b in zip([p.grad for p in layer.parameters() if p is not layer.fc1.weight], others):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,S", [(2, 16), (4, 512)])
+@pytest.mark.parametrize("name,shape", [("fc2.weight", (64, 32)), ("fc1.weight", (128, 64)), ("qkv.bias", (64,)),
+                                        ("ln1.weight", (72,))])
+def test_a_gradient_of_another_shape_raises(B, S, name, shape):
+    """A parameter whose data had another shape when its gradient was made: the kernels would write past the gradient's end."""
+    layer = _layer(64, 1, 64)
+    p = layer.get_parameter(name)
+    kept = p.data
+    p.data = torch.zeros(shape, device="cuda")
+    p.grad = torch.zeros(shape, device="cuda")
+    p.data = kept
+    y = layer(torch.randn(B, S, 64).bfloat16().cuda().requires_grad_())
+    with pytest.raises((ValueError, RuntimeError)):
+        y.backward(torch.ones_like(y))
