@@ -1419,9 +1419,15 @@ def transformer_layer_backward(dy, x, saved, params, batch, seq, heads):
     in, or added to, the parameters' ``grad``."""
     hidden = x.size(1)
     native = _layer_params(params, hidden)
-    if native is None or dy.dtype != BF16 or not dy.is_cuda or not dy.is_contiguous():
+    if native is None or x.shape != dy.shape:
+        return None
+    if any(t.dtype != BF16 or not t.is_cuda or not t.is_contiguous() for t in (x, dy)):
         return None
     ffn = params[8].size(0)
+    saved_bytes, work_bytes = _layer_bytes(batch, seq, heads, hidden, ffn)
+    # (saved-tensor hooks may have put it somewhere else)
+    if not saved.is_cuda or not saved.is_contiguous() or saved.nbytes < saved_bytes or saved.data_ptr() % 256:
+        return None
     grads = [p.grad for p in params]
     if len(set(map(id, params))) < len(params):      # one parameter in two places: its gradients are added one by one
         return None
@@ -1434,7 +1440,7 @@ def transformer_layer_backward(dy, x, saved, params, batch, seq, heads):
             grads[i] = torch.empty(p.shape, dtype=torch.float32, device=x.device)
         else:
             add |= 1 << i
-    work = torch.empty(_layer_bytes(batch, seq, heads, hidden, ffn)[1], dtype=torch.uint8, device=x.device)
+    work = torch.empty(work_bytes, dtype=torch.uint8, device=x.device)
     dx = torch.empty_like(x)
     _cabi.lib().pd_transformer_layer_bwd_bf16(native[0], (ctypes.c_void_p * 12)(*[g.data_ptr() for g in grads]), add, _ptr(x),
                                               _ptr(saved), _ptr(dy), _ptr(work), _ptr(dx), batch, seq, heads, hidden, ffn,

@@ -92,6 +92,24 @@ def test_one_matrix_in_two_places_gets_both_gradients():
         assert torch.equal(a, b)
 
 
+def test_saved_tensors_may_come_back_at_another_address():
+    """Hooks that keep what the forward pass saved in a buffer of their own, on boundaries of 16 bytes only."""
+    layer = _layer(64, 1, 64)
+    x, dy = torch.randn(2, 16, 64).bfloat16().cuda(), torch.randn(2, 16, 64).bfloat16().cuda()
+    want = _passes(layer, [x], [dy], True, True)
+
+    def elsewhere(t):
+        n = t.numel() * t.element_size()
+        buf = torch.empty(n + 16, dtype=torch.uint8, device=t.device)[16:]
+        buf.copy_(t.reshape(-1).view(torch.uint8))
+        return buf.view(t.dtype).view(t.shape)
+
+    with torch.autograd.graph.saved_tensors_hooks(elsewhere, lambda t: t):
+        got = _passes(layer, [x], [dy], True, True)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("B,S", [(2, 16), (4, 512)])
 @pytest.mark.parametrize("name,shape", [("fc2.weight", (64, 32)), ("fc1.weight", (128, 64)), ("qkv.bias", (64,)),
                                         ("ln1.weight", (72,))])
