@@ -190,10 +190,26 @@ def _use_x6(M, N, K, trans_a, trans_b, relu, a, b, out, lda, ldb, ldc):
 SKINNY_X6_MIN_WEIGHTS = 1 << 22
 
 
+def _skinny_x6_min_k(M, trans_b):
+    """The shortest reduction for which pd_gemm_skinny_f32x6 reads more than 2^22 weights faster than the fp32 kernels.  Its
+    waves share k in chunks of 32 and split A's rows again for every 64 columns, so a short reduction leaves waves without
+    a chunk and many rows cost more than the weights.  us, fp32 kernels / this one, at 2^24 weights:
+      [N][K]  16 rows k = 64 55 / 43; 32 rows 64 63 / 65, 128 53 / 42; 48 rows 64 69 / 87, 128 54 / 52; 64 rows 256 40 / 45,
+              384 46 / 40 (2^25: 69 / 77), 512 32 / 32; 96 rows 256 64 / 75, 384 59 / 66, 512 53 / 51; 128 rows 256 66 / 85,
+              512 54 / 58, 768 69 / 56
+      [K][N]  16 rows 64 53 / 43; 32 rows 64 62 / 65, 128 50 / 38; 64 rows 64 67 / 101, 128 55 / 57, 192 56 / 51; 96 rows 128
+              59 / 90, 256 65 / 57; 128 rows 128 54 / 106, 256 68 / 69, 384 64 / 67, 512 54 / 47"""
+    if M <= 16:
+        return 64
+    if M <= (48 if trans_b else 64):
+        return 128
+    return (512 if M <= 96 else 768) if trans_b else (256 if M <= 96 else 512)
+
+
 def _use_skinny_x6(M, N, K, trans_a, trans_b, a, b, lda, ldb):
     """Whether ``gemm`` takes pd_gemm_skinny_f32x6: at most 128 rows of an untransposed A, operands it can fetch 16 bytes at
-    a time, and more than 2^22 weights (16 MB), for [N][K] weights and more than 96 rows 2^23 at least.  us, fp32
-    kernels / this one, weights from memory, at 8, 32, 64, 96 and 128 rows:
+    a time, a reduction that is not short (_skinny_x6_min_k), and more than 2^22 weights (16 MB), for [N][K] weights and more
+    than 96 rows 2^23 at least.  us, fp32 kernels / this one, weights from memory, at 8, 32, 64, 96 and 128 rows:
       [N][K]  2048 x 2304  14.5 / 10.9  16.0 / 12.9  18.0 / 17.1  19.4 / 18.6  19.5 / 20.6
               3072 x 2048  16.4 / 11.4  18.1 / 14.0  18.5 / 18.3  23.2 / 23.0  23.3 / 26.0
               4096 x 2048  17.5 / 12.5  19.1 / 14.6  19.9 / 19.4  26.4 / 23.3  26.8 / 26.6
@@ -204,6 +220,8 @@ def _use_skinny_x6(M, N, K, trans_a, trans_b, a, b, lda, ldb):
     of few weights are found in front of a ReLU in passes that the host's launches bound, which gain nothing, while a
     pre-activation next to zero that falls on the other side moves a result (1 of 100 runs of four passes at 32 rows)."""
     if N * K <= SKINNY_X6_MIN_WEIGHTS or (trans_b and M > 96 and N * K < 2 * SKINNY_X6_MIN_WEIGHTS):
+        return False
+    if K < _skinny_x6_min_k(M, trans_b):
         return False
     return (_GEMM_F32_ALGO != "never" and not trans_a and 0 < M <= 128 and K % 8 == 0 and
             (trans_b or N % 4 == 0) and lda % 4 == 0 and ldb % 4 == 0 and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0)

@@ -16,6 +16,17 @@ def test_rows_and_weights(M, N, K, rows_of_k, columns_of_k):
     assert not ops._use_skinny_x6(M, N, K, True, True, a, b, K, K)
 
 
+@pytest.mark.parametrize("M,k_of_rows,k_of_columns", [(1, 64, 64), (16, 64, 64), (17, 128, 128), (48, 128, 128), (49, 512, 128),
+                                                      (64, 512, 128), (65, 512, 256), (96, 512, 256), (97, 768, 512), (128, 768, 512)])
+def test_short_reductions(M, k_of_rows, k_of_columns):
+    """The shortest reduction, whatever the number of weights."""
+    for trans_b, least in ((True, k_of_rows), (False, k_of_columns)):
+        for K in (least - 8, least):
+            N = (1 << 24) // K // 8 * 8
+            a, b = torch.empty(M, K, device="meta"), torch.empty(*((N, K) if trans_b else (K, N)), device="meta")
+            assert ops._use_skinny_x6(M, N, K, False, trans_b, a, b, K, b.stride(0)) == (K == least)
+
+
 @pytest.mark.parametrize("T,B,H,takes", [(1, 8, 64, False), (2, 8, 64, True), (2, 128, 256, True), (2, 8, 512, False), (3, 8, 512, True),
                                          (4, 40, 1024, False), (5, 40, 1024, True), (5, 129, 1024, False), (5, 40, 1000, False)])
 def test_lstm_steps(T, B, H, takes):

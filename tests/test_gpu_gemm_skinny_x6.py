@@ -17,9 +17,10 @@ SHAPES = [(1, 8, 8), (16, 4, 32), (17, 36, 40), (31, 100, 256), (32, 64, 264), (
 
 
 @pytest.fixture(autouse=True)
-def _any_number_of_weights(monkeypatch):
+def _any_weights(monkeypatch):
     from pipedream_amd import ops
     monkeypatch.setattr(ops, "SKINNY_X6_MIN_WEIGHTS", 0)
+    monkeypatch.setattr(ops, "_skinny_x6_min_k", lambda M, trans_b: 0)
 
 
 def _operands(M, N, K, trans_b, seed=1):
