@@ -209,12 +209,13 @@ void launch_skinny(const SkinnyX6Args& g, int trans_b, hipStream_t s) {
 // Columns of C per block, 64 or 32.
 static int skinny_cols(int M, int N) { return (N + 63) / 64 * ((M + 63) / 64) <= 16 ? 32 : 64; }
 
-// Ranges of k: one block per CU and a chunk of k per wave.  Up to 32 chunks (24 from 33 rows on, whose conversions spread
+// Ranges of k: one block per CU and a chunk of k per wave.  Up to 32 chunks (24 from 17 rows on, whose conversions spread
 // over the CUs as well) stay in one piece, since the launch that adds up the ranges costs what they save: us, one piece /
 // two ranges, 8 x 8192 x 768 11.3 / 11.4 and, B as [K][N], 8.1 / 10.1, x 1024 13.4 / 12.6 and 9.8 / 11.3,
+// 32 x 5120 x 1024 16.5 / 14.0 and 11.2 / 10.9, x 8192 x 1024 17.0 / 14.7 and 11.6 / 12.1, x 768 13.7 / 13.5 and 9.3 / 11.5,
 // 64 x 8192 x 768 18.4 / 19.2 and 15.3 / 18.3, x 1024 22.4 / 19.6 and 18.2 / 18.4.
 extern "C" int pd_gemm_skinny_f32x6_splits(int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K <= (M > 32 ? 768 : 1024)) return 1;
+    if (M <= 0 || N <= 0 || K <= (M > 16 ? 768 : 1024)) return 1;
     const int cols = skinny_cols(M, N);
     const long blocks = (long)((N + cols - 1) / cols) * ((M + 63) / 64);
     const long most = (K + 31) / 32 / KX_WAVES, want = 256 / blocks;
