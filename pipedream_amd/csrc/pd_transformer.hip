@@ -557,12 +557,16 @@ __global__ __launch_bounds__(TR_THREADS) void colsum_batch_partial_kernel(const 
     }
 }
 
-// Bound: the chain of loads over up to 512 rows of partial results.  16 waves a block, thread (w, h, column) adds the rows
-// 4 (2 h) + w and 4 (2 h + 1) + w of every 32, in order: 13312 columns with 64 rows and, of the normalisations', 512:
-// 5.2 us (four waves a block with 8 loads in flight 8.6; the same order of additions).
-constexpr int CB_FINAL_THREADS = 1024;
-__global__ __launch_bounds__(CB_FINAL_THREADS) void colsum_batch_final_kernel(const ColsumBatch b, int splits) {
-    __shared__ float part[4][4][64];
+// Bound: the chain of loads over up to 512 rows of partial results.  4 WAYS waves a block; eight sums per wave of four and
+// column, each over every eighth of its rows, are spread over WAYS threads: thread (w, h, column) adds the rows 4 u + w of
+// every 32 for its 8 / WAYS values of u, in order, and the order in which the sums are added up is the same for any WAYS.
+// 13312 columns with 64 rows and, of the normalisations', 512: 5.2 us with WAYS = 4, 8.6 with 1.  With at most 128 rows the
+// larger blocks cost 0.3-0.6 us more than they save (both launches for 600 tokens of 768 features 7.5 / 7.1, for 128 of 2048
+// 9.8 / 9.2; 1240 tokens, 155 rows, 9.2 / 9.3).
+template <int WAYS>
+__global__ __launch_bounds__(256 * WAYS) void colsum_batch_final_kernel(const ColsumBatch b, int splits) {
+    constexpr int U = 8 / WAYS;
+    __shared__ float part[4][WAYS][64];
     int j = 0;
 #pragma unroll
     for (int q = 1; q < CB_MAX_JOBS; ++q) j += (q < b.n && (int)blockIdx.x >= b.job[q].tile2) ? 1 : 0;
@@ -571,25 +575,39 @@ __global__ __launch_bounds__(CB_FINAL_THREADS) void colsum_batch_final_kernel(co
     const uint64_t M = job.is_bf16 ? (uint64_t)splits : job.M, ld = job.is_bf16 ? (uint64_t)job.N : job.ld;
     const int N = job.N, c = threadIdx.x % 64, w = threadIdx.x / 64 % 4, h = threadIdx.x / 256;
     const int col = ((int)blockIdx.x - job.tile2) * 64 + c;
+    // (a tree over a power of two of neighbours)
+    const auto add_up = [](auto& v, int n) {
+#pragma unroll
+        for (int step = 1; step < n; step *= 2)
+#pragma unroll
+            for (int q = 0; q + step < n; q += 2 * step) v[q] += v[q + step];
+        return v[0];
+    };
     float s = 0.f;
     if (col < N) {
-        float t0 = 0.f, t1 = 0.f;
+        float t[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) t[u] = 0.f;
         uint64_t r = w;
-#pragma unroll 4
-        for (; r + 28 < M; r += 32) {
-            t0 += x[(r + 8 * h) * ld + col];
-            t1 += x[(r + 8 * h + 4) * ld + col];
-        }
+#pragma unroll WAYS
+        for (; r + 28 < M; r += 32)
+#pragma unroll
+            for (int u = 0; u < U; ++u) t[u] += x[(r + 4 * (U * h + u)) * ld + col];
         if (h == 0)
-            for (; r < M; r += 4) t0 += x[r * ld + col];
-        s = t0 + t1;
+            for (; r < M; r += 4) t[0] += x[r * ld + col];
+        s = add_up(t, U);
     }
     part[w][h][c] = s;
     __syncthreads();
     if (threadIdx.x < 64 && col < N) {
         float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = (part[q][0][c] + part[q][1][c]) + (part[q][2][c] + part[q][3][c]);
+        for (int q = 0; q < 4; ++q) {
+            float p[WAYS];
+#pragma unroll
+            for (int k = 0; k < WAYS; ++k) p[k] = part[q][k][c];
+            v[q] = add_up(p, WAYS);
+        }
         const float t = (v[0] + v[1]) + (v[2] + v[3]);
         float* o = job.out + col;
         *o = job.beta != 0.f ? t + job.beta * *o : t;
@@ -620,7 +638,7 @@ extern "C" int pd_colsum_batch(int n_jobs, const void* const* x, const int* is_b
     PD_REQUIRE(x && is_bf16 && out && M && N && ld && beta, PD_EINVAL, "%s: NULL argument array", who);
     ColsumBatch b;
     b.n = n_jobs;
-    uint64_t used = 0;
+    uint64_t used = 0, rows = 0;
     int tiles1 = 0, tiles2 = 0;
     for (int j = 0; j < n_jobs; ++j) {
         PD_REQUIRE(x[j] && out[j], PD_EINVAL, "%s: NULL operand in job %d", who, j);
@@ -636,6 +654,8 @@ extern "C" int pd_colsum_batch(int n_jobs, const void* const* x, const int* is_b
             tiles1 += (N[j] + 511) / 512;
         }
         tiles2 += (N[j] + 63) / 64;
+        const uint64_t job_rows = job.is_bf16 ? (uint64_t)splits : job.M;
+        if (job_rows > rows) rows = job_rows;
     }
     PD_REQUIRE(used == 0 || (workspace && workspace_floats >= used), PD_EINVAL,
                "%s: workspace too small (%llu < %llu floats)", who, (unsigned long long)workspace_floats,
@@ -644,7 +664,8 @@ extern "C" int pd_colsum_batch(int n_jobs, const void* const* x, const int* is_b
         colsum_batch_partial_kernel<<<dim3(tiles1, splits), dim3(TR_THREADS), 0, (hipStream_t)stream>>>(b);
         PD_CHECK_LAUNCH(who);
     }
-    colsum_batch_final_kernel<<<dim3(tiles2), dim3(CB_FINAL_THREADS), 0, (hipStream_t)stream>>>(b, splits);
+    if (rows <= 128) colsum_batch_final_kernel<1><<<dim3(tiles2), dim3(256), 0, (hipStream_t)stream>>>(b, splits);
+    else colsum_batch_final_kernel<4><<<dim3(tiles2), dim3(1024), 0, (hipStream_t)stream>>>(b, splits);
     PD_CHECK_LAUNCH(who);
     return PD_OK;
 }
