@@ -14,8 +14,8 @@
 // (trans_b = 1, k-contiguous).
 //
 // Three kernels: tiles of 64 x 64 to 256 x 256 fed by direct-to-LDS loads (nearly every product), k split over the waves of
-// a block (few tiles, deep reductions), and one that stages through registers, for reductions of at most 192 and operands
-// whose rows lie 2^22 elements and more apart.  LDS bandwidth, not the matrix cores, limits small tiles: a wave with a (32*TM) x (32*TN) tile reads
+// a block (few tiles, deep reductions), and one that stages through registers, for reductions of at most 192, longer ones of
+// large products that 128 does not divide, and operands whose rows lie 2^22 elements and more apart.  LDS bandwidth, not the matrix cores, limits small tiles: a wave with a (32*TM) x (32*TN) tile reads
 // (TM+TN) KB of fragments per TM*TN MFMAs, so the largest gives every wave 128 x 128 and a block 256 x 256.
 // The staged kernel: a block of WM x WN waves owns a BM x BN tile; K runs in chunks of 64 through a double-buffered LDS
 // tile.
@@ -1037,10 +1037,11 @@ int launch_gemm_bf16_staged(int ta, int tb, GemmBf16Args g, int batch, hipStream
     g.total_tiles = g.tiles_m * g.tiles_n * batch;
     g.tiles_per_xcd = (g.total_tiles + N_XCD - 1) / N_XCD;
     const dim3 grid(g.tiles_per_xcd * N_XCD);
-    if (!ta && tb) pd_gemm_bf16_kernel<B, B, 2, 2, true, true><<<grid, 256, 0, s>>>(g);
-    else if (!ta && !tb) pd_gemm_bf16_kernel<B, B, 2, 2, true, false><<<grid, 256, 0, s>>>(g);
-    else if (ta && !tb) pd_gemm_bf16_kernel<B, B, 2, 2, false, false><<<grid, 256, 0, s>>>(g);
-    else pd_gemm_bf16_kernel<B, B, 2, 2, false, true><<<grid, 256, 0, s>>>(g);
+    constexpr int WN = B == 256 ? 4 : 2, NT = 128 * WN;
+    if (!ta && tb) pd_gemm_bf16_kernel<B, B, 2, WN, true, true><<<grid, NT, 0, s>>>(g);
+    else if (!ta && !tb) pd_gemm_bf16_kernel<B, B, 2, WN, true, false><<<grid, NT, 0, s>>>(g);
+    else if (ta && !tb) pd_gemm_bf16_kernel<B, B, 2, WN, false, false><<<grid, NT, 0, s>>>(g);
+    else pd_gemm_bf16_kernel<B, B, 2, WN, false, true><<<grid, NT, 0, s>>>(g);
     PD_CHECK_LAUNCH("pd_gemm_bf16");
     return PD_OK;
 }
@@ -1131,14 +1132,27 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     // Short reductions: the staged kernel, whose chunks of 64 k need no ring (a round of the ring is 128 k; what K leaves of
     // it are zeros).  us, staged / direct: k = 64 4096 x 4096 12.2 / 14.6, 600 x 3072 4.0 / 4.7, 512 times 512 x 512 93 / 115, 2048
     // times 64 x 64 10 / 13; k = 136 4096 x 4096 17.5 / 19.0, 2400 x 768 5.3 / 5.4; beyond 192 the ring: k = 200 2400 x 768
-    // 5.9 / 5.4, 4096 x 4096 19.8 / 19.6, 2400 x 512 x 328 6.8 / 5.7.  Tiles of 128 x 128 once there is one per CU:
-    // 4096 x 768 x 64 (192 of them) 5.4, with 64 x 64 4.8; 128 times 200 x 200 x 64 (512) 7.1, with 64 x 64 8.5.
-    // A whole round (k = 128) only where most of a wider tile would lie outside: 2048 times 64 x 64 15.2 / 17.8.
+    // 5.9 / 5.4, 2400 x 512 x 328 6.8 / 5.7.  A whole round (k = 128) only where most of a wider tile would lie outside: 2048
+    // times 64 x 64 15.2 / 17.8.  Its tile is the one whose blocks, that each keep a CU busy, take the least time for the area
+    // they cover, 1, 0.87 and 0.82 for the same area in tiles of 64, 128 and 256: us with the three, k = 96: 4096 x 4096 - /
+    // 16.7 / 15.3, 128 times 512 x 512 30.5 / 27.8 / 25.7, 93 times 600 x 600 37.4 / 31.8 / 39.2, 218 times 392 x 392 38.3 / 40.6 /
+    // 42.8, 256 times 264 x 264 24.6 / 28.5 / 39.7, 200 x 200 17.0 / 15.4 / 14.1, 136 x 136 11.0 / 13.9 / 11.9, 104 x 104 6.6 / 7.3 /
+    // 10.9; 4096 x 768 x 64 (192 of 128 x 128) 4.8 / 5.4 / -.
     const bool narrow = M <= 64 || N <= 64;
+    const long area64 = blocks(64, 64) * 100, area128 = blocks(128, 128) * 4 * 87, area256 = blocks(256, 256) * 16 * 82;
     if (K <= 192 && (!whole || (narrow && blocks(64, 64) > 256))) {
-        if (!narrow && blocks(128, 128) >= 256) return launch_gemm_bf16_staged<128>(trans_a, trans_b, g, batch, s);
+        const bool can128 = M >= 128 && N >= 128 && blocks(128, 128) >= 256 && area128 < area64;
+        if (blocks(256, 256) >= 192 && area256 < (can128 ? area128 : area64))
+            return launch_gemm_bf16_staged<256>(trans_a, trans_b, g, batch, s);
+        if (can128) return launch_gemm_bf16_staged<128>(trans_a, trans_b, g, batch, s);
         return launch_gemm_bf16_staged<64>(trans_a, trans_b, g, batch, s);
     }
+    // Large products of longer reductions that 128 does not divide, for which there are no direct-to-LDS tiles of 256 x 256:
+    // staged 256 x 256 / direct 128 x 128, B as [N][K] and [K][N]: 4096 x 4096 x 200 20.3 / 21.8 and 19.6 / 20.5, x 1000 49 / 61 and
+    // 45 / 47, x 4104 157 / 214 and 149 / 172; both operands with their rows along k 16384 x 1024 x 328 26.1 / 28.7, x 1000 47.7 / 46.4,
+    // x 3000 114 / 114.
+    if (!whole && (!trans_a || K <= 600) && blocks(256, 256) >= 192 && area256 <= area128)
+        return launch_gemm_bf16_staged<256>(trans_a, trans_b, g, batch, s);
     if (whole && !both_t && M >= 256 && N >= 256 && wide_tiles(blocks(256, 256), blocks(128, 128), K, trans_b, act))
         return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
     // Below, the largest tile that still gives every CU a block: us with 128 x 128, 64 x 128, 64 x 64: 2560 x 1024 x 1024

@@ -29,7 +29,9 @@ SHAPES = [(8, 8, 8), (32, 64, 40), (64, 64, 128), (72, 56, 136), (64, 72, 3000),
           (200, 2304, 88), (600, 776, 200), (600, 3072, 256), (256, 1032, 1032), (1240, 1024, 72), (1920, 512, 512), (4096, 4104, 128),
           (4040, 4096, 256), (64, 192, 4096), (640, 264, 2080), (200, 328, 7200),
           # reductions of at most 192: staged, in tiles of 128 x 128 from 256 of them on
-          (72, 56, 8), (136, 2056, 64), (2056, 2056, 40), (2040, 2056, 192), (4104, 1032, 136), (2056, 2056, 200)]
+          (72, 56, 8), (136, 2056, 64), (2056, 2056, 40), (2040, 2056, 192), (4104, 1032, 136), (2056, 2056, 200),
+          # staged 256 x 256 from 192 tiles on, whatever 128 leaves of k
+          (4104, 3080, 40), (4104, 3080, 136), (4096, 3072, 328)]
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
@@ -71,7 +73,8 @@ def test_epilogues(M, N, K):
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("batch,M,N,K", [(300, 64, 64, 128), (520, 40, 32, 40), (130, 136, 64, 264), (80, 200, 24, 200),
-                                         (260, 72, 128, 64), (130, 136, 136, 192), (257, 64, 72, 128), (80, 1032, 48, 256)])
+                                         (260, 72, 128, 64), (130, 136, 136, 192), (257, 64, 72, 128), (80, 1032, 48, 256),
+                                         (200, 200, 200, 96)])
 def test_batches_of_small_products(batch, M, N, K, ta, tb):
     """Attention's products at head dimensions without a fused kernel: many entries, narrow sides, short reductions."""
     from pipedream_amd import ops
