@@ -1123,8 +1123,17 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     // sum over eight waves) with the size of C: the line lies at k = 16 per tile of 64 x 64.  us, split / not, and k per
     // tile: 128 x 1024 x 4096 8.7 / 14 (128), 88 x 768 x 768 4.6 / 5.4 (32), 600 x 768 x 3072 12.6 / 15.3 (26),
     // 600 x 768 x 2304 9.5 / 11.3 (19), 640 x 1024 x 3072 15.2 / 15.5 (19), 200 x 768 x 768 5.2 / 5.4 (16),
-    // 1920 x 512 x 2048 15.3 / 11.4 (9), 600 x 768 x 768 7.9 / 4.9 (6), 200 x 3072 x 768 8.3 / 5.0 (4).
-    if (!trans_a && batch == 1 && g.vec_store && K % DK == 0 && K >= 16 * blocks(64, 64) && blocks(64, 64) <= 256) {
+    // 1920 x 512 x 2048 15.3 / 11.4 (9), 600 x 768 x 768 7.9 / 4.9 (6), 200 x 3072 x 768 8.3 / 5.0 (4).  For B as [K][N], whose
+    // long reductions the direct-to-LDS kernel reads more slowly, at 10 from k = 1000 on: 300 x 1024 x 1024 6.2 / 7.1 (13), 900 x
+    // 512 x 1536 7.6 / 8.3 (13), 100 x 3072 x 1024 6.4 / 6.9 (11), 360 x 1280 x 1280 7.6 / 7.6 (11), 500 x 1024 x 1024 6.9 / 6.9
+    // (8), 300 x 768 x 768 6.6 / 5.9 (13).
+    const long tiles = blocks(64, 64);
+    const bool deep = K >= (trans_b || K < 800 ? 16 : 10) * tiles;
+    // And reductions that would leave a part of the direct-to-LDS ring's last round empty, in launches that fill a quarter of
+    // the CUs: 304 x 512 x 160 4.1 / 4.6, x 96 3.9 / 4.2, x 64 3.8 / 3.9, x 416 4.7 / 5.4 (B as [K][N] 4.9 / 6.0), 256 x 1000 x 800
+    // 6.2 / 6.8 (7.7 / 7.8); 80 tiles of 300 x 1000 x 800 7.3 / 6.7, of 2400 x 104 x 160 with GELU's derivative 5.1 / 5.6.
+    const bool ragged = !whole && K >= 96 && tiles <= (K <= 192 ? 80 : 64);
+    if (!trans_a && batch == 1 && g.vec_store && K % DK == 0 && (deep || ragged) && tiles <= 256) {
         if (blocks(32, 32) <= 256) return launch_gemm_bf16_ksplit<1, 1>(trans_b, g, s);
         if (blocks(32, 64) <= 256) return launch_gemm_bf16_ksplit<1, 2>(trans_b, g, s);
         return launch_gemm_bf16_ksplit<2, 2>(trans_b, g, s);
