@@ -1162,6 +1162,12 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     // x 3000 114 / 114.
     if (!whole && (!trans_a || K <= 600) && blocks(256, 256) >= 192 && area256 <= area128)
         return launch_gemm_bf16_staged<256>(trans_a, trans_b, g, batch, s);
+    // With both operands' rows along k the ring's chunks of 32 k of a row lie in two cache lines each, and from one to two blocks
+    // of 128 x 128 per CU on nothing hides that: staged / direct 2400 x 2304 x 600 19.8 / 19.3, x 1000 26.9 / 29.4, x 3000 64 / 74,
+    // 5120 x 1024 x 1000 (320 blocks) 25.3 / 28.8, 8000 x 1000 x 1000 (504) 28 / 32; 2048 x 2048 x 1000 (256) 20.7 / 18.2,
+    // 3000 x 3000 x 1000 (576) 43 / 42; B as [K][N] 2400 x 2304 x 1000 26.5 / 24.2.
+    if (!whole && !trans_a && trans_b && K >= 700 && blocks(128, 128) > 256 && blocks(128, 128) <= 512 && area128 < area64)
+        return launch_gemm_bf16_staged<128>(trans_a, trans_b, g, batch, s);
     if (whole && !both_t && M >= 256 && N >= 256 && wide_tiles(blocks(256, 256), blocks(128, 128), K, trans_b, act))
         return launch_gemm_bf16_dma<256, 256>(trans_a, trans_b, g, batch, s);
     // Below, the largest tile that still gives every CU a block: us with 128 x 128, 64 x 128, 64 x 64: 2560 x 1024 x 1024

@@ -30,8 +30,8 @@ SHAPES = [(8, 8, 8), (32, 64, 40), (64, 64, 128), (72, 56, 136), (64, 72, 3000),
           (4040, 4096, 256), (64, 192, 4096), (640, 264, 2080), (200, 328, 7200),
           # reductions of at most 192: staged, in tiles of 128 x 128 from 256 of them on
           (72, 56, 8), (136, 2056, 64), (2056, 2056, 40), (2040, 2056, 192), (4104, 1032, 136), (2056, 2056, 200),
-          # staged 256 x 256 from 192 tiles on, whatever 128 leaves of k
-          (4104, 3080, 40), (4104, 3080, 136), (4096, 3072, 328),
+          # staged 256 x 256 from 192 tiles on, whatever 128 leaves of k; staged 128 x 128 of longer reductions
+          (4104, 3080, 40), (4104, 3080, 136), (4096, 3072, 328), (2312, 2056, 712),
           # ragged reductions of few tiles and, for B as [K][N], long ones of more, over the waves of a block
           (304, 520, 160), (104, 1000, 800), (304, 1024, 1056)]
 
