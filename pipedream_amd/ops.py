@@ -1439,8 +1439,9 @@ def transformer_layer_backward(dy, x, saved, params, batch, seq, heads):
     native = _layer_params(params, hidden)
     if native is None or x.shape != dy.shape:
         return None
-    if any(t.dtype != BF16 or not t.is_cuda or not t.is_contiguous() for t in (x, dy)):
-        return None
+    for t in (x, dy):
+        if t.dtype != BF16 or not t.is_cuda or not t.is_contiguous():
+            return None
     ffn = params[8].size(0)
     saved_bytes, work_bytes = _layer_bytes(batch, seq, heads, hidden, ffn)
     # (saved-tensor hooks may have put it somewhere else)
@@ -1449,9 +1450,9 @@ def transformer_layer_backward(dy, x, saved, params, batch, seq, heads):
     grads = [p.grad for p in params]
     if len(set(map(id, params))) < len(params):      # one parameter in two places: its gradients are added one by one
         return None
-    if any(g is not None and (g.dtype != torch.float32 or not g.is_cuda or not g.is_contiguous() or g.shape != p.shape)
-           for g, p in zip(grads, params)):          # (a parameter's data may have changed its shape under a gradient)
-        return None
+    for g, shape in zip(grads, _layer_shapes(hidden, ffn)):      # (a parameter's data may have changed its shape under a gradient)
+        if g is not None and (g.shape != shape or g.dtype != torch.float32 or not g.is_cuda or not g.is_contiguous()):
+            return None
     add = 0
     for i, p in enumerate(params):
         if grads[i] is None:
