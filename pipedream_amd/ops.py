@@ -1394,6 +1394,8 @@ def _layer_params(params, hidden):
     tensors = list(params)
     for i in _LAYER_MATRICES:
         tensors[i] = bf16_weight(params[i])
+        if tensors[i].shape != params[i].shape:      # an optimizer's image of the data before a replacement
+            return None
     if ([t.dtype for t in tensors] != _LAYER_DTYPES or
             not all([t.is_cuda for t in tensors]) or not all([t.is_contiguous() for t in tensors])):
         return None

@@ -1,5 +1,7 @@
 """Which parameters the native calls of a transformer layer take: they see pointers alone, so every shape is compared before
 one is handed over, and what the single launches do not compare themselves is refused."""
+import types
+
 import pytest
 import torch
 
@@ -85,6 +87,17 @@ def test_a_replaced_linear_raises_in_either_pass(name, rows, cols):
     kept.weight.data, kept.bias.data = other.weight.data, other.bias.data       # between the passes
     with pytest.raises((ValueError, RuntimeError)):
         y.backward(torch.ones_like(y))
+
+
+@pytest.mark.gpu
+def test_a_bf16_image_of_another_shape_raises():
+    """The image that an optimizer keeps of a weight is what the kernels read: one of fewer rows than the weight, from before its
+    data was replaced."""
+    layer = layers.TransformerLayer(128, 2, 256).cuda()
+    layer.fc2.weight._pd_arena = types.SimpleNamespace(live_slot=0)
+    layer.fc2.weight._pd_bf16_views = [torch.zeros(64, 256, dtype=torch.bfloat16, device="cuda")]
+    with pytest.raises(ValueError):
+        layer(torch.zeros(2, 16, 128, dtype=torch.bfloat16, device="cuda"))
 
 
 @pytest.mark.gpu
