@@ -1126,9 +1126,10 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     // 1920 x 512 x 2048 15.3 / 11.4 (9), 600 x 768 x 768 7.9 / 4.9 (6), 200 x 3072 x 768 8.3 / 5.0 (4).  For B as [K][N], whose
     // long reductions the direct-to-LDS kernel reads more slowly, at 10 from k = 1000 on: 300 x 1024 x 1024 6.2 / 7.1 (13), 900 x
     // 512 x 1536 7.6 / 8.3 (13), 100 x 3072 x 1024 6.4 / 6.9 (11), 360 x 1280 x 1280 7.6 / 7.6 (11), 500 x 1024 x 1024 6.9 / 6.9
-    // (8), 300 x 768 x 768 6.6 / 5.9 (13).
+    // (8), 300 x 768 x 768 6.6 / 5.9 (13); but not with more than 128 tiles: 1240 x 512 x 2048 (160, 13 k a tile) 13.7 / 10.8,
+    // 1240 x 768 x 3072 (240, 13) 19.1 / 16.8, 600 x 1024 x 2048 (160, 13) 10.3 / 10.9.
     const long tiles = blocks(64, 64);
-    const bool deep = K >= (trans_b || K < 800 ? 16 : 10) * tiles;
+    const bool deep = K >= (trans_b || K < 800 || tiles > 128 ? 16 : 10) * tiles;
     // And reductions that would leave a part of the direct-to-LDS ring's last round empty, in launches that fill a quarter of
     // the CUs: 304 x 512 x 160 4.1 / 4.6, x 96 3.9 / 4.2, x 64 3.8 / 3.9, x 416 4.7 / 5.4 (B as [K][N] 4.9 / 6.0), 256 x 1000 x 800
     // 6.2 / 6.8 (7.7 / 7.8); 80 tiles of 300 x 1000 x 800 7.3 / 6.7, of 2400 x 104 x 160 with GELU's derivative 5.1 / 5.6.
@@ -1143,14 +1144,15 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     // times 64 x 64 10 / 13; k = 136 4096 x 4096 17.5 / 19.0, 2400 x 768 5.3 / 5.4; beyond 192 the ring: k = 200 2400 x 768
     // 5.9 / 5.4, 2400 x 512 x 328 6.8 / 5.7.  A whole round (k = 128) only where most of a wider tile would lie outside: 2048
     // times 64 x 64 15.2 / 17.8.  Its tile is the one whose blocks, that each keep a CU busy, take the least time for the area
-    // they cover, 1, 0.87 and 0.82 for the same area in tiles of 64, 128 and 256: us with the three, k = 96: 4096 x 4096 - /
+    // they cover, 1, 0.87 and 0.82 for the same area in tiles of 64, 128 and 256 (and 64 for entries within 128 x 128, whose
+    // blocks of 128 are too few to overlap): us with the three, k = 96: 4096 x 4096 - /
     // 16.7 / 15.3, 128 times 512 x 512 30.5 / 27.8 / 25.7, 93 times 600 x 600 37.4 / 31.8 / 39.2, 218 times 392 x 392 38.3 / 40.6 /
     // 42.8, 256 times 264 x 264 24.6 / 28.5 / 39.7, 200 x 200 17.0 / 15.4 / 14.1, 136 x 136 11.0 / 13.9 / 11.9, 104 x 104 6.6 / 7.3 /
     // 10.9; 4096 x 768 x 64 (192 of 128 x 128) 4.8 / 5.4 / -.
     const bool narrow = M <= 64 || N <= 64;
     const long area64 = blocks(64, 64) * 100, area128 = blocks(128, 128) * 4 * 87, area256 = blocks(256, 256) * 16 * 82;
     if (K <= 192 && (!whole || (narrow && blocks(64, 64) > 256))) {
-        const bool can128 = M >= 128 && N >= 128 && blocks(128, 128) >= 256 && area128 < area64;
+        const bool can128 = (M >= 128 || N >= 128) && !narrow && blocks(128, 128) >= 256 && area128 < area64;
         if (blocks(256, 256) >= 192 && area256 < (can128 ? area128 : area64))
             return launch_gemm_bf16_staged<256>(trans_a, trans_b, g, batch, s);
         if (can128) return launch_gemm_bf16_staged<128>(trans_a, trans_b, g, batch, s);
@@ -1158,9 +1160,10 @@ static int gemm_bf16_run(int trans_a, int trans_b, int M, int N, int K, const ui
     }
     // Large products of longer reductions that 128 does not divide, for which there are no direct-to-LDS tiles of 256 x 256:
     // staged 256 x 256 / direct 128 x 128, B as [N][K] and [K][N]: 4096 x 4096 x 200 20.3 / 21.8 and 19.6 / 20.5, x 1000 49 / 61 and
-    // 45 / 47, x 4104 157 / 214 and 149 / 172; both operands with their rows along k 16384 x 1024 x 328 26.1 / 28.7, x 1000 47.7 / 46.4,
-    // x 3000 114 / 114.
-    if (!whole && (!trans_a || K <= 600) && blocks(256, 256) >= 192 && area256 <= area128)
+    // 45 / 47, x 4104 157 / 214 and 149 / 172; A as [K][M] 16384 x 1024 x 328 26.1 / 28.7, x 1000 47.7 / 46.4, x 3000 114 / 114.
+    // Tiles that lie in the result but for a seventh: 218 times 392 x 256 x 392 (three quarters) 47.6 / 45.
+    const bool full256 = (long long)M * N * batch * 100 >= blocks(256, 256) * 65536ll * 85;
+    if (!whole && (!trans_a || K <= 600) && blocks(256, 256) >= 192 && full256)
         return launch_gemm_bf16_staged<256>(trans_a, trans_b, g, batch, s);
     // With both operands' rows along k the ring's chunks of 32 k of a row lie in two cache lines each, and from one to two blocks
     // of 128 x 128 per CU on nothing hides that: staged / direct 2400 x 2304 x 600 19.8 / 19.3, x 1000 26.9 / 29.4, x 3000 64 / 74,
