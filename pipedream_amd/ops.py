@@ -193,23 +193,24 @@ SKINNY_X6_MIN_WEIGHTS = 1 << 22
 def _skinny_x6_min_k(M, trans_b):
     """The shortest reduction for which pd_gemm_skinny_f32x6 reads more than 2^22 weights faster than the fp32 kernels.  Its
     waves share k in chunks of 32 and split A's rows again for every 64 columns, so a short reduction leaves waves without
-    a chunk and many rows cost more than the weights.  us, fp32 kernels / this one, at 2^24 weights:
-      [N][K]  16 rows k = 64 55 / 43; 32 rows 64 63 / 65, 128 53 / 42; 48 rows 64 69 / 87, 128 54 / 52; 64 rows 256 40 / 45,
-              384 46 / 40 (2^25: 69 / 77), 512 32 / 32; 96 rows 256 64 / 75, 384 59 / 66, 512 53 / 51; 128 rows 256 66 / 85,
-              512 54 / 58, 768 69 / 56
-      [K][N]  16 rows 64 53 / 43; 32 rows 64 62 / 65, 128 50 / 38; 64 rows 64 67 / 101, 128 55 / 57, 192 56 / 51; 96 rows 128
-              59 / 90, 256 65 / 57; 128 rows 128 54 / 106, 256 68 / 69, 384 64 / 67, 512 54 / 47"""
-    if M <= 16:
-        return 64
-    if M <= (48 if trans_b else 64):
-        return 128
-    return (512 if M <= 96 else 768) if trans_b else (256 if M <= 96 else 512)
+    a chunk and many rows cost more than the weights.  us, fp32 kernels (which vary by a third with how N falls on their
+    blocks) / this one, at 2^23 and 2^24 weights:
+      [N][K]  16 rows k = 64 33 / 23, 55 / 43; 32 rows 64 34 / 34, 63 / 65, 128 28 / 23, 53 / 42; 64 rows 64 38 / 51, 70 / 99, 128
+              34 / 33, 57 / 59, 192 41 / 29, 56 / 55, 256 22 / 24, 40 / 45, 384 25 / 27, 46 / 40; 96 rows 256 34 / 39, 64 / 75, 384
+              41 / 35, 59 / 66, 512 29 / 27, 53 / 51; 128 rows 384 42 / 42, 63 / 76, 512 30 / 31, 54 / 58, 768 37 / 36, 69 / 56
+      [K][N]  16 rows 64 30 / 24, 53 / 43; 32 rows 64 33 / 34, 62 / 65, 128 28 / 20, 50 / 38; 64 rows 64 38 / 53, 67 / 101, 128 33 / 31,
+              55 / 57, 192 42 / 26, 56 / 51; 96 rows 128 33 / 48, 59 / 90, 192 42 / 41, 54 / 71, 256 33 / 31, 65 / 57; 128 rows 192
+              43 / 47, 55 / 83, 256 34 / 37, 68 / 69, 384 41 / 35, 64 / 67, 512 30 / 25, 54 / 47"""
+    if M <= 64:
+        return 64 if M <= 16 else 128
+    return (384 if M <= 96 else 768) if trans_b else 256
 
 
 def _use_skinny_x6(M, N, K, trans_a, trans_b, a, b, lda, ldb):
     """Whether ``gemm`` takes pd_gemm_skinny_f32x6: at most 128 rows of an untransposed A, operands it can fetch 16 bytes at
-    a time, a reduction that is not short (_skinny_x6_min_k), and more than 2^22 weights (16 MB), for [N][K] weights and more
-    than 96 rows 2^23 at least.  us, fp32 kernels / this one, weights from memory, at 8, 32, 64, 96 and 128 rows:
+    a time, a reduction that is not short (_skinny_x6_min_k), and more than 2^22 weights (16 MB); for [N][K] weights of at most
+    4096 rows, which take several ranges of k, and more than 96 rows of A 2^23 at least (128 x 6000 x 1000 37 / 20, x 8192 x 768
+    24 / 20 in one range).  us, fp32 kernels / this one, weights from memory, at 8, 32, 64, 96 and 128 rows:
       [N][K]  2048 x 2304  14.5 / 10.9  16.0 / 12.9  18.0 / 17.1  19.4 / 18.6  19.5 / 20.6
               3072 x 2048  16.4 / 11.4  18.1 / 14.0  18.5 / 18.3  23.2 / 23.0  23.3 / 26.0
               4096 x 2048  17.5 / 12.5  19.1 / 14.6  19.9 / 19.4  26.4 / 23.3  26.8 / 26.6
@@ -219,9 +220,9 @@ def _use_skinny_x6(M, N, K, trans_a, trans_b, a, b, lda, ldb):
     1024 x 1024 11.1 / 8.6, 2048 x 1024 11.5 / 13.0, 10 x 1024 33 / 6).  The fp32 kernels keep their bits there: products
     of few weights are found in front of a ReLU in passes that the host's launches bound, which gain nothing, while a
     pre-activation next to zero that falls on the other side moves a result (1 of 100 runs of four passes at 32 rows)."""
-    if N * K <= SKINNY_X6_MIN_WEIGHTS or (trans_b and M > 96 and N * K < 2 * SKINNY_X6_MIN_WEIGHTS):
+    if N * K <= SKINNY_X6_MIN_WEIGHTS or K < _skinny_x6_min_k(M, trans_b):
         return False
-    if K < _skinny_x6_min_k(M, trans_b):
+    if trans_b and M > 96 and N <= 4096 and N * K < 2 * SKINNY_X6_MIN_WEIGHTS:
         return False
     return (_GEMM_F32_ALGO != "never" and not trans_a and 0 < M <= 128 and K % 8 == 0 and
             (trans_b or N % 4 == 0) and lda % 4 == 0 and ldb % 4 == 0 and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0)
@@ -945,10 +946,11 @@ def add(a, b):
 def _lstm_x6(T, B, H, w_hh):
     """Whether a layer's recurrence of T steps runs on the bf16 matrix pipes at fp32 accuracy (pd_lstm_f32x6.hip).  Splitting
     W_hh takes as long as one to three steps, which a short sequence does not earn back.  us for forward + backward, fp32
-    loop / this one, at 40 rows: H = 256, 2 steps 28 / 23; H = 512, 2 steps 28 / 28, 3 53 / 41; H = 1024, 3 65 / 72,
+    loop / this one, at 40 rows: H = 256, 2 steps 28 / 23; H = 512, 2 steps 28 / 28, 3 53 / 41; H = 768, 3 (with
+    the layer's other products) 119 / 115; H = 1024, 3 65 / 72,
     4 95 / 90, 6 153 / 127; H = 2560, 4 275 / 297, 5 363 / 353; H = 3072, 4 394 / 413, 5 524 / 494; H = 4096 (whose split
     weights do not stay in the cache), 6 939 / 1149, 12 2054 / 2168, each further one 186 / 178."""
-    enough = 2 if H <= 256 else 3 if H <= 512 else 5 if H <= 3072 else 16
+    enough = 2 if H <= 256 else 3 if H <= 768 else 4 if H <= 1024 else 5 if H <= 3072 else 16
     return (T >= enough and _GEMM_F32_ALGO != "never" and w_hh.is_contiguous() and w_hh.data_ptr() % 16 == 0 and
             bool(_cabi.lib().pd_lstm_f32x6_supported(B, H)))
 
