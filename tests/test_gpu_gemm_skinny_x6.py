@@ -13,7 +13,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 8, 8), (16, 4, 32), (17, 36, 40), (31, 100, 256), (32, 64, 264), (48, 1028, 72), (49, 32, 2048), (64, 516, 1096),
-          (65, 1000, 128), (128, 132, 3080), (100, 2052, 520), (8, 4096, 4104), (40, 260, 1000)]
+          (65, 1000, 128), (128, 132, 3080), (100, 2052, 520), (8, 4096, 4104), (40, 260, 1000), (24, 516, 904)]
 
 
 @pytest.fixture(autouse=True)
