@@ -946,10 +946,9 @@ def add(a, b):
 def _lstm_x6(T, B, H, w_hh):
     """Whether a layer's recurrence of T steps runs on the bf16 matrix pipes at fp32 accuracy (pd_lstm_f32x6.hip).  Splitting
     W_hh takes as long as one to three steps, which a short sequence does not earn back.  us for forward + backward, fp32
-    loop / this one, at 40 rows: H = 256, 2 steps 28 / 23; H = 512, 2 steps 28 / 28, 3 53 / 41; H = 768, 3 (with
-    the layer's other products) 119 / 115; H = 1024, 3 65 / 72,
-    4 95 / 90, 6 153 / 127; H = 2560, 4 275 / 297, 5 363 / 353; H = 3072, 4 394 / 413, 5 524 / 494; H = 4096 (whose split
-    weights do not stay in the cache), 6 939 / 1149, 12 2054 / 2168, each further one 186 / 178."""
+    loop / this one, at 40 rows: H = 256, 2 steps 28 / 23; H = 512, 2 steps 28 / 28, 3 53 / 41; H = 768, 3 (with the
+    layer's other products) 119 / 115; H = 1024, 3 65 / 72, 4 95 / 90, 6 153 / 127; H = 2560, 4 275 / 297, 5 363 / 353; H = 3072, 4
+    394 / 413, 5 524 / 494; H = 4096 (whose split weights do not stay in the cache), 6 939 / 1149, 12 2054 / 2168, each further one 186 / 178."""
     enough = 2 if H <= 256 else 3 if H <= 768 else 4 if H <= 1024 else 5 if H <= 3072 else 16
     return (T >= enough and _GEMM_F32_ALGO != "never" and w_hh.is_contiguous() and w_hh.data_ptr() % 16 == 0 and
             bool(_cabi.lib().pd_lstm_f32x6_supported(B, H)))
